@@ -118,11 +118,12 @@ int taco_profile_enable(taco_ctx* ctx, int on);
 int taco_profile_reset(taco_ctx* ctx);
 int taco_profile_get(taco_ctx* ctx, int kernel, double* total_ms, long* launches, double* algo_bytes);
 
-/* Tile configuration the autotuner chose for FFT length 2^log2_nfft in this
- * context, per phase A, B, C (0: 8192 values/512 threads, 1: 4096/256,
- * 2: 4096/512, 3: 2048/256, 4: 4096/1024, 5: 2048/512; -1 if not tuned
- * yet).  TACO_FFT_TILE=<0..5> forces one.  No reference counterpart (the reference's cuFFT plans are
- * internal, tcl4_fcr_kernels.cu:602-622). */
+/* Shape of the FFT passes of length 2^log2_nfft last run in this context, per
+ * phase A, B, C (3: tiles of 2048 values; 10, 11: groups of 2^10, 2^11 values,
+ * one workgroup each; -1 if none ran yet).  Every shape performs the same
+ * butterflies.  TACO_FFT_TILE forces one: 0, 1 the tiles on 256 / 512 threads,
+ * 2, 3 groups of 2^10, 2^11.  No reference counterpart (the
+ * reference's cuFFT plans are internal, tcl4_fcr_kernels.cu:602-622). */
 int taco_fft_tile_choice(taco_ctx* ctx, int log2_nfft, int* cfg3);
 
 /* Correctly rounded sin/cos of each x[i] (|x| < 2^30): the phase routine of

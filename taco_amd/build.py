@@ -10,6 +10,7 @@ from __future__ import annotations
 import os
 import subprocess
 import sys
+from concurrent.futures import ThreadPoolExecutor
 
 HERE = os.path.dirname(os.path.abspath(__file__))
 CSRC = os.path.join(HERE, "csrc")
@@ -45,15 +46,11 @@ def build(verbose: bool = False) -> str:
             print(" ".join(cmd), flush=True)
         subprocess.run(cmd, check=True)
 
-    objs = []
-    for src in _sources(".cpp"):
-        obj = os.path.join(BUILD_DIR, os.path.basename(src) + ".o")
-        run([cxx, *CXX_FLAGS, "-I", INCLUDE, "-c", src, "-o", obj])
-        objs.append(obj)
-    for src in _sources(".hip"):
-        obj = os.path.join(BUILD_DIR, os.path.basename(src) + ".o")
-        run([hipcc, *HIP_FLAGS, "-I", INCLUDE, "-c", src, "-o", obj])
-        objs.append(obj)
+    cmds = [([cxx, *CXX_FLAGS], src) for src in _sources(".cpp")] + [([hipcc, *HIP_FLAGS], src) for src in _sources(".hip")]
+    objs = [os.path.join(BUILD_DIR, os.path.basename(src) + ".o") for _, src in cmds]
+    with ThreadPoolExecutor(max_workers=min(8, len(os.sched_getaffinity(0)))) as pool:
+        for f in [pool.submit(run, [*cmd, "-I", INCLUDE, "-c", src, "-o", obj]) for (cmd, src), obj in zip(cmds, objs)]:
+            f.result()
     run([hipcc, "--offload-arch=gfx950", "-shared", "-fPIC", "-o", LIB + ".tmp", *objs, "-lquadmath", "-lgomp"])
     os.replace(LIB + ".tmp", LIB)
     return LIB

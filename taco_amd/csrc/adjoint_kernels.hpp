@@ -7,438 +7,6 @@
 // i dLoss/dIm z (torch's convention for real losses).
 #pragma once
 
-// y = L^H x (column r of L conjugated, column stride ld), summed over c in order.
-// (General D: column blocks of kMvBlk loads issued ahead, as in matvec_rows.)
-template <int DT>
-__device__ __forceinline__ void matvec_h(const double2* __restrict__ L, int ld, const double2* x, double2* y, int D) {
-    const int n = DT ? DT : D;
-    for (int r = threadIdx.x; r < n; r += blockDim.x) {
-        double2 s = make_double2(0.0, 0.0);
-        const double2* col = L + static_cast<long>(r) * ld;
-        if constexpr (DT == 0) {
-            int c = 0;
-            for (; c + kMvBlk <= n; c += kMvBlk) {
-                double2 v[kMvBlk];
-#pragma unroll
-                for (int j = 0; j < kMvBlk; ++j) v[j] = col[c + j];
-#pragma unroll
-                for (int j = 0; j < kMvBlk; ++j) s = cadd(s, cmul(cconj(v[j]), x[c + j]));
-            }
-            for (; c < n; ++c) s = cadd(s, cmul(cconj(col[c]), x[c]));
-        } else {
-#pragma unroll
-            for (int c = 0; c < DT; ++c) s = cadd(s, cmul(cconj(col[c]), x[c]));
-        }
-        y[r] = s;
-    }
-}
-
-// y = (0.5 (L0 + L1))^H x.
-template <int DT>
-__device__ __forceinline__ void matvec_h_half(const double2* __restrict__ L0, const double2* __restrict__ L1, int ld,
-                                              const double2* x, double2* y, int D) {
-    const int n = DT ? DT : D;
-    for (int r = threadIdx.x; r < n; r += blockDim.x) {
-        double2 s = make_double2(0.0, 0.0);
-        const long o = static_cast<long>(r) * ld;
-        if constexpr (DT == 0) {
-            int c = 0;
-            for (; c + kMvBlk <= n; c += kMvBlk) {
-                double2 v0[kMvBlk], v1[kMvBlk];
-#pragma unroll
-                for (int j = 0; j < kMvBlk; ++j) {
-                    v0[j] = L0[o + c + j];
-                    v1[j] = L1[o + c + j];
-                }
-#pragma unroll
-                for (int j = 0; j < kMvBlk; ++j) s = cadd(s, cmul(cconj(cscale(cadd(v0[j], v1[j]), 0.5)), x[c + j]));
-            }
-            for (; c < n; ++c) s = cadd(s, cmul(cconj(cscale(cadd(L0[o + c], L1[o + c]), 0.5)), x[c]));
-        } else {
-#pragma unroll
-            for (int c = 0; c < DT; ++c)
-                s = cadd(s, cmul(cconj(cscale(cadd(L0[o + c], L1[o + c]), 0.5)), x[c]));
-        }
-        y[r] = s;
-    }
-}
-
-// ---------------------------------------------------------------------------
-// RK4 adjoint.  Forward step n (rk4_step): k1 = L0 r, u1 = r + h k1,
-// k2 = Lh u1, u2 = r + h k2, k3 = Lh u2, u3 = r + dt k3, k4 = L1 u3,
-// r' = r + s (k1 + 2 k2 + 2 k3 + k4), h = dt/2, s = dt/6, Lh = (L0 + L1)/2.
-// Two launches.  k_rk4_recompute: one workgroup per checkpoint segment (K
-// steps) recomputes, from the checkpoint ck[q] = r_{qK} and with the forward
-// step's own arithmetic, the states r_n and stage points u1..u3 of its
-// segment; segments are independent, so all run at once.  k_rk4_adjoint:
-// one workgroup walks n = steps-1 .. 0, mapping lam_{n+1} to
-// lam_n = M_n^H lam_{n+1} + gbar_n and forming the cotangents of L_n and
-// L_{n+1}.  LDS: vectors of D, then (nstage >= 2) a window of generators
-// staged with column stride D + 1.  Lbar(t) collects the L1 part of step t-1
-// and the L0 part of step t: the latter is carried in registers
-// (D^2 <= 16 x 256) and each Lbar(t) stored once.  Larger D (generators read
-// from global memory): the walk reads the conjugate transposes LsH (written
-// beforehand by k_conj_transpose, so every product is a row-coalesced
-// matrix-vector product with the same terms in the same order), stores only
-// the step's cotangent vectors kb1..kb4, and k_rk4_lbar forms every Lbar(t)
-// afterwards, all times at once, with the walk's own sums.
-// ---------------------------------------------------------------------------
-struct Rk4AdjArgs {
-    const double2* Ls;    // [steps + 1][D * D] generators
-    const double2* ck;    // [ceil(steps / K)][D] checkpoint states r_{qK}
-    const double2* gbar;  // [steps + 1][D] dLoss/dr_n
-    double2* Lbar;        // [steps + 1][D * D]
-    double2* seg;         // [steps][4][D] state r_n and stage points u1, u2, u3 of step n
-    double2* r0bar;       // [D]
-    long steps;
-    int D;
-    int K;
-    double dt;
-    int nstage;
-    const double2* LsH = nullptr;  // [steps + 1][D * D] conjugate transposes (walk without staging)
-    const double2* LhH = nullptr;  // [steps][D * D] their midpoints (null: formed on the fly)
-    double2* vec = nullptr;        // [steps][4][D] kb1..kb4 of every step (Lbar formed by k_rk4_lbar)
-};
-
-constexpr int kRkCarry = 16;
-
-// Makes generators L_a..L_b resident in the LDS window M (column stride
-// D + 1), restaging the window [first, last] when they are not.
-struct GenWindow {
-    long lo = 0, hi = -1;
-    __device__ __forceinline__ void need(double2* M, const double2* Ls, long a, long b, long first, long last, int D) {
-        if (a >= lo && b <= hi) return;
-        __syncthreads();
-        lo = first;
-        hi = last;
-        stage_mats(M, Ls, lo, static_cast<int>(hi - lo + 1), D);
-        __syncthreads();
-    }
-};
-
-template <int DT, bool STAGED>
-__device__ __forceinline__ void rk4_recompute_body(double2* sh, const Rk4AdjArgs& A, long sg) {
-    const int D = A.D;
-    double2* x = sh;
-    double2* k1 = x + D;
-    double2* k2 = k1 + D;
-    double2* k3 = k2 + D;
-    double2* k4 = k3 + D;
-    double2* tmp = k4 + D;
-    double2* M = tmp + D;
-    const long D2 = static_cast<long>(D) * D;
-    const int ld = STAGED ? D + 1 : D;
-    GenWindow w;
-    const long s0 = sg * A.K, s1 = min(s0 + A.K, A.steps);
-    for (int e = threadIdx.x; e < D; e += blockDim.x) x[e] = A.ck[sg * D + e];
-    __syncthreads();
-    for (long n = s0; n < s1; ++n) {
-        double2* row = A.seg + n * 4 * D;
-        for (int e = threadIdx.x; e < D; e += blockDim.x) row[e] = x[e];
-        if constexpr (STAGED) {
-            w.need(M, A.Ls, n, n + 1, n, min(n + A.nstage - 1, s1), D);
-            rk4_step<DT>(M + (n - w.lo) * D * ld, M + (n + 1 - w.lo) * D * ld, ld, nullptr, x, k1, k2, k3, k4, tmp,
-                         D, A.dt, row + D);
-        } else {
-            rk4_step<DT>(A.Ls + n * D2, A.Ls + (n + 1) * D2, ld, nullptr, x, k1, k2, k3, k4, tmp, D, A.dt, row + D);
-        }
-    }
-}
-
-// Row-group recompute (rk4_rows with the stage points stashed) for the sizes
-// that have one: the same arithmetic as the forward run, so the states equal
-// the forward's bit for bit.  One workgroup per checkpoint segment.
-template <int DT>
-__global__ __launch_bounds__(64 * RowGroup<DT>::W) void k_rk4_recompute_rows(Rk4AdjArgs A) {
-    extern __shared__ double2 sh[];
-    const long sg = blockIdx.x;
-    const long s0 = sg * A.K, s1 = min(s0 + A.K, A.steps);
-    rk4_rows<DT, true>(sh, A.Ls, s0, s1, A.ck + sg * DT, nullptr, A.dt, 1, nullptr, nullptr, A.seg);
-}
-
-__global__ __launch_bounds__(kBlock) void k_rk4_recompute(Rk4AdjArgs A) {
-    extern __shared__ double2 sh[];
-    const long sg = blockIdx.x;
-    if (A.nstage >= 2) {
-#define TACO_RK4_CALL(DT) rk4_recompute_body<DT, true>(sh, A, sg)
-        TACO_RK4_DISPATCH(A.D, TACO_RK4_CALL)
-#undef TACO_RK4_CALL
-    } else {
-#define TACO_RK4_CALL(DT) rk4_recompute_body<DT, false>(sh, A, sg)
-        TACO_RK4_DISPATCH(A.D, TACO_RK4_CALL)
-#undef TACO_RK4_CALL
-    }
-}
-
-template <int DT, bool STAGED>
-__device__ __forceinline__ void rk4_adjoint_body(double2* sh, const Rk4AdjArgs& A) {
-    const int D = A.D;
-    double2* x = sh;          // r_n
-    double2* k3 = x + D;      // cotangent of k3
-    double2* k4 = k3 + D;     // cotangent of k4
-    double2* tmp = k4 + D;
-    double2* lam = tmp + D;   // cotangent of r_{n+1}, then of r_n
-    double2* u1 = lam + D;
-    double2* u2 = u1 + D;
-    double2* u3 = u2 + D;
-    double2* kb1 = u3 + D;    // cotangents of k1, k2
-    double2* kb2 = kb1 + D;
-    double2* rb = kb2 + D;    // cotangent of r_n being accumulated
-    double2* M = rb + D;      // staged generators
-    const long D2 = static_cast<long>(D) * D;
-    const int ld = STAGED ? D + 1 : D;
-    const bool carry = D2 <= static_cast<long>(kRkCarry) * blockDim.x;
-    double2 Lc[kRkCarry];     // L0 part of the step after the current one (carry mode)
-#pragma unroll
-    for (int q = 0; q < kRkCarry; ++q) Lc[q] = make_double2(0.0, 0.0);
-    GenWindow w;
-    const double h = 0.5 * A.dt, s6 = A.dt / 6.0;
-    for (int e = threadIdx.x; e < D; e += blockDim.x) lam[e] = A.gbar[A.steps * D + e];
-    __syncthreads();
-    for (long n = A.steps - 1; n >= 0; --n) {
-        const double2* L0;
-        const double2* L1;
-        const double2* H0 = nullptr;  // conjugate transposes (LsH path)
-        const double2* H1 = nullptr;
-        if constexpr (STAGED) {
-            w.need(M, A.Ls, n, n + 1, max(0L, n + 2 - A.nstage), n + 1, D);
-            L0 = M + (n - w.lo) * D * ld;
-            L1 = L0 + D * ld;
-        } else {
-            L0 = A.Ls + n * D2;
-            L1 = L0 + D2;
-            if (A.LsH) {
-                H0 = A.LsH + n * D2;
-                H1 = H0 + D2;
-            }
-        }
-        const double2* row = A.seg + n * 4 * D;
-        for (int e = threadIdx.x; e < D; e += blockDim.x) {
-            x[e] = row[e];
-            u1[e] = row[D + e];
-            u2[e] = row[2 * D + e];
-            u3[e] = row[3 * D + e];
-            k4[e] = cscale(lam[e], s6);                                                    // kb4
-        }
-        __syncthreads();
-        // reverse: r' = r + s (k1 + 2 k2 + 2 k3 + k4)
-        if (H1) matvec_rows<DT>(H1, D, k4, tmp, D); else matvec_h<DT>(L1, ld, k4, tmp, D);  // ub3
-        __syncthreads();
-        for (int e = threadIdx.x; e < D; e += blockDim.x) {
-            k3[e] = cadd(cscale(lam[e], 2.0 * s6), cscale(tmp[e], A.dt));                  // kb3
-            rb[e] = cadd(lam[e], tmp[e]);
-        }
-        __syncthreads();
-        if (A.LhH && H0) matvec_rows<DT>(A.LhH + n * D2, D, k3, tmp, D);                             // ub2
-        else if (H0) matvec_half<DT>(H0, H1, D, k3, tmp, D);
-        else matvec_h_half<DT>(L0, L1, ld, k3, tmp, D);
-        __syncthreads();
-        for (int e = threadIdx.x; e < D; e += blockDim.x) {
-            kb2[e] = cadd(cscale(lam[e], 2.0 * s6), cscale(tmp[e], h));
-            rb[e] = cadd(rb[e], tmp[e]);
-        }
-        __syncthreads();
-        if (A.LhH && H0) matvec_rows<DT>(A.LhH + n * D2, D, kb2, tmp, D);                            // ub1
-        else if (H0) matvec_half<DT>(H0, H1, D, kb2, tmp, D);
-        else matvec_h_half<DT>(L0, L1, ld, kb2, tmp, D);
-        __syncthreads();
-        for (int e = threadIdx.x; e < D; e += blockDim.x) {
-            kb1[e] = cadd(cscale(lam[e], s6), cscale(tmp[e], h));
-            rb[e] = cadd(rb[e], tmp[e]);
-        }
-        __syncthreads();
-        if (H0) matvec_rows<DT>(H0, D, kb1, tmp, D); else matvec_h<DT>(L0, ld, kb1, tmp, D);
-        __syncthreads();
-        // generator cotangents: Lbar_h = kb3 u2^H + kb2 u1^H, split half/half
-        double2* Lb0 = A.Lbar + n * D2;
-        double2* Lb1 = A.Lbar + (n + 1) * D2;
-        if (!carry && A.vec) {
-            double2* v = A.vec + n * 4 * D;
-            for (int e = threadIdx.x; e < D; e += blockDim.x) {
-                v[e] = kb1[e];
-                v[D + e] = kb2[e];
-                v[2 * D + e] = k3[e];
-                v[3 * D + e] = k4[e];
-            }
-        } else if (carry) {
-#pragma unroll
-            for (int q = 0; q < kRkCarry; ++q) {
-                const long e = threadIdx.x + static_cast<long>(q) * blockDim.x;
-                if (e < D2) {
-                    const int r = static_cast<int>(e % D), c = static_cast<int>(e / D);
-                    const double2 lh = cadd(cmul(k3[r], cconj(u2[c])), cmul(kb2[r], cconj(u1[c])));
-                    Lb1[e] = cadd(Lc[q], cadd(cmul(k4[r], cconj(u3[c])), cscale(lh, 0.5)));
-                    Lc[q] = cadd(cmul(kb1[r], cconj(x[c])), cscale(lh, 0.5));
-                }
-            }
-        } else {
-            // in place, kU elements per thread at a time with their loads issued
-            // first (the same expressions as the remainder loop)
-            constexpr int kU = 8;
-            const long stride = blockDim.x;
-            long e0 = threadIdx.x;
-            for (; e0 + (kU - 1) * stride < D2; e0 += kU * stride) {
-                double2 a0[kU], a1[kU];
-#pragma unroll
-                for (int u = 0; u < kU; ++u) {
-                    a0[u] = Lb0[e0 + u * stride];
-                    a1[u] = Lb1[e0 + u * stride];
-                }
-#pragma unroll
-                for (int u = 0; u < kU; ++u) {
-                    const long e = e0 + u * stride;
-                    const int r = static_cast<int>(e % D), c = static_cast<int>(e / D);
-                    const double2 lh = cadd(cmul(k3[r], cconj(u2[c])), cmul(kb2[r], cconj(u1[c])));
-                    Lb0[e] = cadd(a0[u], cadd(cmul(kb1[r], cconj(x[c])), cscale(lh, 0.5)));
-                    Lb1[e] = cadd(a1[u], cadd(cmul(k4[r], cconj(u3[c])), cscale(lh, 0.5)));
-                }
-            }
-            for (long e = e0; e < D2; e += stride) {
-                const int r = static_cast<int>(e % D), c = static_cast<int>(e / D);
-                const double2 lh = cadd(cmul(k3[r], cconj(u2[c])), cmul(kb2[r], cconj(u1[c])));
-                Lb0[e] = cadd(Lb0[e], cadd(cmul(kb1[r], cconj(x[c])), cscale(lh, 0.5)));
-                Lb1[e] = cadd(Lb1[e], cadd(cmul(k4[r], cconj(u3[c])), cscale(lh, 0.5)));
-            }
-        }
-        for (int e = threadIdx.x; e < D; e += blockDim.x) lam[e] = cadd(cadd(rb[e], tmp[e]), A.gbar[n * D + e]);
-        __syncthreads();
-    }
-    if (carry) {
-#pragma unroll
-        for (int q = 0; q < kRkCarry; ++q) {
-            const long e = threadIdx.x + static_cast<long>(q) * blockDim.x;
-            if (e < D2) A.Lbar[e] = Lc[q];
-        }
-    }
-    for (int e = threadIdx.x; e < D; e += blockDim.x) A.r0bar[e] = lam[e];
-}
-
-// Row-group reverse walk for D <= 16 (one wave of 64 threads).
-template <int DT>
-__global__ __launch_bounds__(64) void k_rk4_adjoint_rows(Rk4AdjArgs A) {
-    extern __shared__ double2 sh[];
-    if (A.vec)
-        rk4_rows_adjoint<DT, Rk4AdjArgs, true>(sh, A);
-    else
-        rk4_rows_adjoint<DT>(sh, A);
-}
-
-__global__ __launch_bounds__(kBlock) void k_rk4_adjoint(Rk4AdjArgs A) {
-    extern __shared__ double2 sh[];
-    if (A.nstage >= 2) {
-#define TACO_RK4_CALL(DT) rk4_adjoint_body<DT, true>(sh, A)
-        TACO_RK4_DISPATCH(A.D, TACO_RK4_CALL)
-#undef TACO_RK4_CALL
-    } else {
-#define TACO_RK4_CALL(DT) rk4_adjoint_body<DT, false>(sh, A)
-        TACO_RK4_DISPATCH(A.D, TACO_RK4_CALL)
-#undef TACO_RK4_CALL
-    }
-}
-
-// dst[t] = src[t]^H for count D x D matrices (tiles of 16 x 16 through LDS,
-// coalesced reads and writes).  Grid: (tiles of one matrix, count).
-__global__ __launch_bounds__(kBlock) void k_conj_transpose(const double2* __restrict__ src, double2* __restrict__ dst,
-                                                           int D, long count) {
-    __shared__ double2 tile[16][17];
-    const int tiles = (D + 15) / 16;
-    const int ti = static_cast<int>(blockIdx.x) % tiles, tj = static_cast<int>(blockIdx.x) / tiles;
-    const long m = blockIdx.y;
-    if (m >= count) return;
-    const long D2 = static_cast<long>(D) * D;
-    const int lr = threadIdx.x % 16, lc = threadIdx.x / 16;
-    const int r = ti * 16 + lr, c = tj * 16 + lc;  // source element (r, c)
-    if (r < D && c < D) tile[lc][lr] = src[m * D2 + r + static_cast<long>(c) * D];
-    __syncthreads();
-    const int r2 = tj * 16 + lr, c2 = ti * 16 + lc;  // destination element (r2, c2) = conj(src(c2, r2))
-    if (r2 < D && c2 < D) dst[m * D2 + r2 + static_cast<long>(c2) * D] = cconj(tile[lr][lc]);
-}
-
-// Lbar(t), t = 0..steps, from the walk's vectors: the L0 part of step t
-// (kb1 x^H + (kb3 u2^H + kb2 u1^H)/2) added to zero, then the L1 part of
-// step t-1 (kb4 u3^H + (kb3 u2^H + kb2 u1^H)/2): the sums the in-place walk
-// forms, in its order.  Grid: (element blocks of D^2, steps + 1[, tapes]).
-__device__ __forceinline__ void rk4_lbar_body(const Rk4AdjArgs& A) {
-    const int D = A.D;
-    const long D2 = static_cast<long>(D) * D;
-    const long e = static_cast<long>(blockIdx.x) * kBlock + threadIdx.x;
-    const long t = blockIdx.y;
-    if (e >= D2 || t > A.steps) return;
-    const int r = static_cast<int>(e % D), c = static_cast<int>(e / D);
-    double2 acc = make_double2(0.0, 0.0);
-    if (t < A.steps) {
-        const double2* v = A.vec + t * 4 * D;
-        const double2* sg = A.seg + t * 4 * D;
-        const double2 lh = cadd(cmul(v[2 * D + r], cconj(sg[2 * D + c])), cmul(v[D + r], cconj(sg[D + c])));
-        acc = cadd(acc, cadd(cmul(v[r], cconj(sg[c])), cscale(lh, 0.5)));
-    }
-    if (t >= 1) {
-        const double2* v = A.vec + (t - 1) * 4 * D;
-        const double2* sg = A.seg + (t - 1) * 4 * D;
-        const double2 lh = cadd(cmul(v[2 * D + r], cconj(sg[2 * D + c])), cmul(v[D + r], cconj(sg[D + c])));
-        acc = cadd(acc, cadd(cmul(v[3 * D + r], cconj(sg[3 * D + c])), cscale(lh, 0.5)));
-    }
-    A.Lbar[t * D2 + e] = acc;
-}
-
-__global__ __launch_bounds__(kBlock) void k_rk4_lbar(Rk4AdjArgs A) { rk4_lbar_body(A); }
-
-__global__ __launch_bounds__(kBlock) void k_rk4_lbar_multi(const Rk4AdjArgs* As) {
-    const Rk4AdjArgs A = As[blockIdx.z];
-    rk4_lbar_body(A);
-}
-
-// Many tapes of one D, steps and K in one launch: the recompute with
-// blockIdx.y choosing the tape, the walk with one workgroup per tape; each
-// workgroup runs the single-tape body on its own arguments.
-template <int DT>
-__global__ __launch_bounds__(64 * RowGroup<DT>::W) void k_rk4_recompute_rows_multi(const Rk4AdjArgs* As) {
-    extern __shared__ double2 sh[];
-    const Rk4AdjArgs A = As[blockIdx.y];
-    const long sg = blockIdx.x;
-    const long s0 = sg * A.K, s1 = min(s0 + A.K, A.steps);
-    rk4_rows<DT, true>(sh, A.Ls, s0, s1, A.ck + sg * DT, nullptr, A.dt, 1, nullptr, nullptr, A.seg);
-}
-
-__global__ __launch_bounds__(kBlock) void k_rk4_recompute_multi(const Rk4AdjArgs* As) {
-    extern __shared__ double2 sh[];
-    const Rk4AdjArgs A = As[blockIdx.y];
-    const long sg = blockIdx.x;
-    if (A.nstage >= 2) {
-#define TACO_RK4_CALL(DT) rk4_recompute_body<DT, true>(sh, A, sg)
-        TACO_RK4_DISPATCH(A.D, TACO_RK4_CALL)
-#undef TACO_RK4_CALL
-    } else {
-#define TACO_RK4_CALL(DT) rk4_recompute_body<DT, false>(sh, A, sg)
-        TACO_RK4_DISPATCH(A.D, TACO_RK4_CALL)
-#undef TACO_RK4_CALL
-    }
-}
-
-template <int DT>
-__global__ __launch_bounds__(64) void k_rk4_adjoint_rows_multi(const Rk4AdjArgs* As) {
-    extern __shared__ double2 sh[];
-    const Rk4AdjArgs A = As[blockIdx.x];
-    if (A.vec)
-        rk4_rows_adjoint<DT, Rk4AdjArgs, true>(sh, A);
-    else
-        rk4_rows_adjoint<DT>(sh, A);
-}
-
-__global__ __launch_bounds__(kBlock) void k_rk4_adjoint_multi(const Rk4AdjArgs* As) {
-    extern __shared__ double2 sh[];
-    const Rk4AdjArgs A = As[blockIdx.x];
-    if (A.nstage >= 2) {
-#define TACO_RK4_CALL(DT) rk4_adjoint_body<DT, true>(sh, A)
-        TACO_RK4_DISPATCH(A.D, TACO_RK4_CALL)
-#undef TACO_RK4_CALL
-    } else {
-#define TACO_RK4_CALL(DT) rk4_adjoint_body<DT, false>(sh, A)
-        TACO_RK4_DISPATCH(A.D, TACO_RK4_CALL)
-#undef TACO_RK4_CALL
-    }
-}
-
 // ---------------------------------------------------------------------------
 // Fused L4 adjoint, one workgroup per time t.  From Lbar(t) (the RK4 layout of
 // L4(n,m;i,j) = GW(n,i;m,j)) it forms Tbar = GWbar + GWbar^H (GW = T + T^H)

@@ -12,13 +12,14 @@
 //   phase B  forward stages a+1..L of the groups {k = k1 mod 2^a}, the
 //            spectral products with the per-bucket spectra of g2 (F) and
 //            conj(g2) (C), then inverse stages 1..b of the same groups,
-//   phase C  inverse stages b+1..L of the groups {t = q mod 2^b}, keeping
+//            storing only the rows t mod 2^b < T,
+//   phase C  inverse stages b+1..L of the columns {t = q mod 2^b}, keeping
 //            only t < T (the requested window),
 //
-// with a = ceil(L/2), b = L - a.  Every butterfly is the reference's
-// u +/- w*x with the same w, a plain (non-fused) complex product, so the
-// spectra equal the reference's bit for bit.  Groups are processed
-// Stockham-style in LDS, 2048 complex values per workgroup.
+// with b = 11 or 10 on the register groups of group_fft.hip, and b = L / 2 on
+// tiles of 2048 values in LDS for short lengths (fft_shape).  Every butterfly
+// is the reference's u +/- w*x with the same w, a plain (non-fused) complex
+// product, so the spectra equal the reference's bit for bit.
 //
 // The per-time stage (tcl4_mikx.cpp:46-136, tcl4_assemble.cpp:29-205) is one
 // fused kernel per time index that gathers M/I/K/X on the fly from the nf^3
@@ -50,6 +51,9 @@
 
 #include "cr_sincos.hpp"
 #include "cr_exp.hpp"
+#include "fcr_device.hpp"
+#include "group_fft.hpp"
+#include "rk4.hpp"
 
 namespace taco_engine {
 
@@ -64,17 +68,6 @@ static std::size_t g_pad_factor = 0;
         if (e_ != hipSuccess)                                                                 \
             throw Error(TACO_ERR_RUNTIME, std::string(#expr) + ": " + hipGetErrorString(e_)); \
     } while (0)
-
-// ---------------------------------------------------------------------------
-// Device helpers
-// ---------------------------------------------------------------------------
-__device__ __forceinline__ double2 cmul(double2 a, double2 b) {
-    return make_double2(a.x * b.x - a.y * b.y, a.x * b.y + a.y * b.x);
-}
-__device__ __forceinline__ double2 cadd(double2 a, double2 b) { return make_double2(a.x + b.x, a.y + b.y); }
-__device__ __forceinline__ double2 csub(double2 a, double2 b) { return make_double2(a.x - b.x, a.y - b.y); }
-__device__ __forceinline__ double2 cconj(double2 a) { return make_double2(a.x, -a.y); }
-__device__ __forceinline__ double2 cscale(double2 a, double s) { return make_double2(a.x * s, a.y * s); }
 
 // sin/cos(j/64) double-double table of the correctly rounded phase routine.
 __constant__ double c_crtab[4 * taco_cr::kTabN];
@@ -95,8 +88,7 @@ constexpr int kBlock = 256;
 // loads the 2^r values of a closed butterfly set, performs r radix-2 stages
 // on them (each butterfly exactly u +/- w*x with the stage's table
 // twiddle), and writes them back, Stockham-style.  Two barriers per pass.
-// Tile configurations (values per workgroup, threads); the autotuner picks
-// one per FFT length and phase.  kLds leaves room for the padding slots.
+// kLds leaves room for the padding slots.
 template <int TILE, int NT>
 struct FftCfg {
     static constexpr int kTile = TILE;
@@ -104,14 +96,8 @@ struct FftCfg {
     static constexpr int kPT = TILE / NT;  // values per thread (8 or 16)
     static constexpr int kLds = TILE + TILE / 8;
 };
-using Cfg8k = FftCfg<8192, 512>;
-using Cfg4k = FftCfg<4096, 256>;
-using Cfg4kW = FftCfg<4096, 512>;
 using Cfg2k = FftCfg<2048, 256>;
-using Cfg4kX = FftCfg<4096, 1024>;
 using Cfg2kW = FftCfg<2048, 512>;
-using Cfg8kX = FftCfg<8192, 1024>;
-constexpr int kNumFftCfg = 7;
 
 // Physical LDS slot of (group, position): one pad slot per 16 values and an
 // odd group stride keep strided accesses off a single bank.
@@ -275,70 +261,9 @@ __device__ __forceinline__ void tile_fft(double2* buf, const TileLayout& T, cons
     }
 }
 
-// Block -> (job, group block).  Workgroups are dispatched to the 8 XCDs
-// round-robin by id; when possible each XCD keeps a fixed eighth of the
-// group blocks for every job, so its L2 holds only that eighth of the
-// per-group twiddle tables.
-__device__ __forceinline__ void xcd_map(int bid, int bpj, int& job, int& gb) {
-    if ((bpj & 7) == 0) {
-        const int x = bid & 7, i = bid >> 3, per = bpj >> 3;
-        gb = x + 8 * (i % per);
-        job = i / per;
-    } else {
-        job = bid / bpj;
-        gb = bid % bpj;
-    }
-}
-
-struct FcrArgs {
-    const double2* gamma;   // [nf][Nt]
-    const double* omegas;   // [nf]
-    const int* mirror;      // [nf]
-    int nf;
-    long Nt;                // Gamma column stride
-    long Nin;               // Gamma rows that enter the FFT inputs (Nt, or T in the window mode)
-    double dt;
-    int L, a, b;
-    long n;
-    const double2* twStd;   // stages 1..max(a,b), standard layout
-    const double2* twB;     // phase B forward stages, per k1 group
-    const double2* twC;     // phase C inverse stages, per q group
-    const int* job_tri;     // sorted position -> triple id (triples grouped by equal Omega)
-    const unsigned char* job_mask;  // per sorted position: bit0 F needed, bit1 C needed, bit2 R needed
-    long nfft_jobs;         // positions [0, nfft_jobs) need FFTs; the rest only R
-    const int* ajob_start;  // [nA + 1] first sorted position of each A-job (the triples
-                            // of one Omega class with the same i: identical phase-A input)
-    const int* cls_start;   // [ncls + 1] first A-job of each Omega-class piece
-    const int* bperm;       // phase B processing order: grid slot (per chunk) -> A-job
-    long job0;              // first sorted position of the FFT chunk
-    int njobs;              // triples in the FFT chunk
-    long a0;                // first A-job of the FFT chunk
-    int na;                 // A-jobs in the FFT chunk
-    int cls0;               // first class piece touching the chunk
-    long comb0;             // first sorted position of the combine batch
-    long cconv;             // combine-batch capacity (conv slots)
-    double2* inter1;        // [njobs][2^a][2^b]
-    double2* inter2;        // [2][njobs][2^b][2^a]
-    double2* spec;          // [2 nf][2^a][2^b]   spectra of g_b (even) and conj(g_b) (odd)
-    double2* conv;          // [2][njobs][T]
-    long T;
-    // Phase mode TACO_PHASE_LIBM: host table of exp(+i Omega (t dt)), one row
-    // of ph_len values per distinct Omega, and the row of each sorted
-    // position; null in TACO_PHASE_CR (the kernels evaluate cexpi).
-    const double2* ph_tab;
-    const int* job_row;
-    long ph_len;
-};
-
 // exp(+i Omega (t dt)) of a triple: its table row, or the correctly rounded value.
 __device__ __forceinline__ double2 phase_plus(const double2* row, long t, double omega, double dt) {
     return row ? row[t] : cexpi(omega * (static_cast<double>(t) * dt));
-}
-
-__device__ __forceinline__ void decode_triple(long tri, int nf, int& i, int& j, int& k) {
-    k = static_cast<int>(tri % nf);
-    j = static_cast<int>((tri / nf) % nf);
-    i = static_cast<int>(tri / (static_cast<long>(nf) * nf));
 }
 
 // Phase A of the per-bucket spectra: input g_b (even job) or conj(g_b) (odd job).
@@ -509,10 +434,10 @@ __global__ __launch_bounds__(Cfg::kFT) TACO_FFT_OCC(Cfg) void k_phase_b(FcrArgs 
             __syncthreads();
             if (pn < pend) load_spec(Y, pn, pathn);
             tile_fft<Cfg, true>(buf, Tl, P.twStd, 0, true);
-            double2* out = P.inter2 + (static_cast<long>(path) * P.njobs + (p - P.job0)) * P.n;
+            double2* out = P.inter2 + ((static_cast<long>(path) * P.njobs + (p - P.job0)) << P.a) * P.Tq;
             for (int e = threadIdx.x; e < total; e += kFT) {
-                const int grp = Tl.grp_of(e), pos = Tl.pos_of(e);
-                out[(static_cast<long>(pos) << P.a) + k1b + grp] = buf[Tl.at(grp, pos)];
+                const int grp = e >> Tl.lg, pos = e & (gs - 1);
+                if (pos < P.Tq) out[static_cast<long>(k1b + grp) * P.Tq + pos] = buf[Tl.at(grp, pos)];
             }
             __syncthreads();
             p = pn;
@@ -536,10 +461,10 @@ __global__ __launch_bounds__(Cfg::kFT) TACO_FFT_OCC(Cfg) void k_phase_b(FcrArgs 
             }
             __syncthreads();
             tile_fft<Cfg, true>(buf, Tl, P.twStd, 0, true);
-            double2* out = P.inter2 + (static_cast<long>(path) * P.njobs + (p - P.job0)) * P.n;
+            double2* out = P.inter2 + ((static_cast<long>(path) * P.njobs + (p - P.job0)) << P.a) * P.Tq;
             for (int e = threadIdx.x; e < total; e += kFT) {
-                const int grp = Tl.grp_of(e), pos = Tl.pos_of(e);
-                out[(static_cast<long>(pos) << P.a) + k1b + grp] = buf[Tl.at(grp, pos)];
+                const int grp = e >> Tl.lg, pos = e & (gs - 1);
+                if (pos < P.Tq) out[static_cast<long>(k1b + grp) * P.Tq + pos] = buf[Tl.at(grp, pos)];
             }
             __syncthreads();
         }
@@ -581,16 +506,18 @@ __global__ __launch_bounds__(Cfg::kFT) void k_phase_c(FcrArgs P, int ntiles) {
 #pragma unroll
     for (int q = 0; q < kPT; ++q) {
         const int e = threadIdx.x + q * kFT;
-        vA[q] = (liveA && e < total) ? P.inter2[static_cast<long>(jpA) * P.n + static_cast<long>(q0A) * gs + e]
-                                     : make_double2(0.0, 0.0);
-        vB[q] = (liveB && e < total) ? P.inter2[static_cast<long>(jpB) * P.n + static_cast<long>(q0B) * gs + e]
-                                     : make_double2(0.0, 0.0);
+        vA[q] = (liveA && e < total && q0A + Tl.grp_of(e) < P.Tq)
+                    ? P.inter2[((static_cast<long>(jpA) << P.a) + Tl.pos_of(e)) * P.Tq + q0A + Tl.grp_of(e)]
+                    : make_double2(0.0, 0.0);
+        vB[q] = (liveB && e < total && q0B + Tl.grp_of(e) < P.Tq)
+                    ? P.inter2[((static_cast<long>(jpB) << P.a) + Tl.pos_of(e)) * P.Tq + q0B + Tl.grp_of(e)]
+                    : make_double2(0.0, 0.0);
     }
 #define TACO_PHASE_C_TILE(JP, Q0, V)                                                                         \
     {                                                                                                         \
         _Pragma("unroll") for (int q = 0; q < kPT; ++q) {                                                     \
             const int e = threadIdx.x + q * kFT;                                                              \
-            if (e < total) buf[Tl.at(e >> Tl.lg, e & (gs - 1))] = V[q];                                       \
+            if (e < total) buf[Tl.at(Tl.grp_of(e), Tl.pos_of(e))] = V[q];                                     \
         }                                                                                                     \
         __syncthreads();                                                                                      \
         /* only rows v2 with (Q0) + v2 * 2^b < T are kept */                                                 \
@@ -1541,288 +1468,11 @@ static void launch_k_l4f(unsigned grid, int N, std::size_t lds, hipStream_t st, 
         hipLaunchKernelGGL(k_l4f<kBlock>, dim3(grid), dim3(kBlock), lds, st, F);
 }
 
-// ---------------------------------------------------------------------------
-// RK4 on vec(rho) with prebuilt generators (rk4_dense.cpp:133-160, 246-320),
-// one workgroup, D <= 1024.  Matvecs sum over j in order per row.
-// ---------------------------------------------------------------------------
-// Matrices are read as L[r + c * ld]: ld = D in global memory, D + 1 when
-// staged in LDS (the padded column stride spreads the column reads of L^H
-// products over the banks).  Everything down to the kernels is inlined and
-// each code path sees either LDS or global matrices, so the compiler knows
-// the address space of every access (LDS reads, not flat ones).  Every product sums over c in order per row, so
-// staged and unstaged runs, and every instantiation below, give identical
-// values.  DT > 0 fixes D at compile time (the row loop is unrolled, so its
-// loads issue together); DT = 0 is the general case.
-// In the general case (DT = 0, D a runtime value) the columns are taken in
-// blocks of kMvBlk whose loads are issued before the block's products, so a
-// thread keeps kMvBlk generator loads in flight (the sum order is unchanged).
-constexpr int kMvBlk = 16;
-
-template <int DT>
-__device__ __forceinline__ void matvec_rows(const double2* __restrict__ L, int ld, const double2* x, double2* y,
-                                            int D) {
-    const int n = DT ? DT : D;
-    for (int r = threadIdx.x; r < n; r += blockDim.x) {
-        double2 s = make_double2(0.0, 0.0);
-        if constexpr (DT == 0) {
-            int c = 0;
-            for (; c + kMvBlk <= n; c += kMvBlk) {
-                double2 v[kMvBlk];
-#pragma unroll
-                for (int j = 0; j < kMvBlk; ++j) v[j] = L[r + static_cast<long>(c + j) * ld];
-#pragma unroll
-                for (int j = 0; j < kMvBlk; ++j) s = cadd(s, cmul(v[j], x[c + j]));
-            }
-            for (; c < n; ++c) s = cadd(s, cmul(L[r + static_cast<long>(c) * ld], x[c]));
-        } else {
-#pragma unroll
-            for (int c = 0; c < DT; ++c) s = cadd(s, cmul(L[r + static_cast<long>(c) * ld], x[c]));
-        }
-        y[r] = s;
-    }
-}
-
-// y = 0.5 (L0 + L1) x, the midpoint generator formed per element.
-template <int DT>
-__device__ __forceinline__ void matvec_half(const double2* __restrict__ L0, const double2* __restrict__ L1, int ld,
-                                            const double2* x, double2* y, int D) {
-    const int n = DT ? DT : D;
-    for (int r = threadIdx.x; r < n; r += blockDim.x) {
-        double2 s = make_double2(0.0, 0.0);
-        if constexpr (DT == 0) {
-            int c = 0;
-            for (; c + kMvBlk <= n; c += kMvBlk) {
-                double2 v0[kMvBlk], v1[kMvBlk];
-#pragma unroll
-                for (int j = 0; j < kMvBlk; ++j) {
-                    const long e = r + static_cast<long>(c + j) * ld;
-                    v0[j] = L0[e];
-                    v1[j] = L1[e];
-                }
-#pragma unroll
-                for (int j = 0; j < kMvBlk; ++j) s = cadd(s, cmul(cscale(cadd(v0[j], v1[j]), 0.5), x[c + j]));
-            }
-            for (; c < n; ++c) {
-                const long e = r + static_cast<long>(c) * ld;
-                s = cadd(s, cmul(cscale(cadd(L0[e], L1[e]), 0.5), x[c]));
-            }
-        } else {
-#pragma unroll
-            for (int c = 0; c < DT; ++c) {
-                const long e = r + static_cast<long>(c) * ld;
-                const double2 h = cscale(cadd(L0[e], L1[e]), 0.5);
-                s = cadd(s, cmul(h, x[c]));
-            }
-        }
-        y[r] = s;
-    }
-}
-
-// One RK4 step x <- x + dt/6 (k1 + 2 k2 + 2 k3 + k4) by the whole workgroup
-// (rk4_dense.cpp:133-160); Lh null: midpoint 0.5 (L0 + L1) per element.
-// L0 and L1 have column stride ld; Lh (global) has D.
-template <int DT>
-__device__ __forceinline__ void rk4_step(const double2* L0, const double2* L1, int ld, const double2* Lh, double2* x,
-                                         double2* k1, double2* k2, double2* k3, double2* k4, double2* tmp, int D,
-                                         double dt, double2* stash = nullptr) {
-    // stash (optional): receives the stage points u1, u2, u3 (3 x D)
-    const double hdt = 0.5 * dt;
-    const double s6 = dt / 6.0;
-    matvec_rows<DT>(L0, ld, x, k1, D);
-    __syncthreads();
-    for (int e = threadIdx.x; e < D; e += blockDim.x) {
-        tmp[e] = cadd(x[e], cscale(k1[e], hdt));
-        if (stash) stash[e] = tmp[e];
-    }
-    __syncthreads();
-    if (Lh) matvec_rows<DT>(Lh, D, tmp, k2, D); else matvec_half<DT>(L0, L1, ld, tmp, k2, D);
-    __syncthreads();
-    for (int e = threadIdx.x; e < D; e += blockDim.x) {
-        tmp[e] = cadd(x[e], cscale(k2[e], hdt));
-        if (stash) stash[D + e] = tmp[e];
-    }
-    __syncthreads();
-    if (Lh) matvec_rows<DT>(Lh, D, tmp, k3, D); else matvec_half<DT>(L0, L1, ld, tmp, k3, D);
-    __syncthreads();
-    for (int e = threadIdx.x; e < D; e += blockDim.x) {
-        tmp[e] = cadd(x[e], cscale(k3[e], dt));
-        if (stash) stash[2 * D + e] = tmp[e];
-    }
-    __syncthreads();
-    matvec_rows<DT>(L1, ld, tmp, k4, D);
-    __syncthreads();
-    for (int e = threadIdx.x; e < D; e += blockDim.x) {
-        const double2 acc = cadd(cadd(cadd(k1[e], cscale(k2[e], 2.0)), cscale(k3[e], 2.0)), k4[e]);
-        x[e] = cadd(x[e], cscale(acc, s6));
-    }
-    __syncthreads();
-}
-
-// Copies generators L_first .. L_first+count-1 into LDS with column stride D + 1.
-__device__ __forceinline__ void stage_mats(double2* dst, const double2* Ls, long first, int count, int D) {
-    const long D2 = static_cast<long>(D) * D;
-    const int ld = D + 1;
-    const double2* src = Ls + first * D2;
-    for (long e = threadIdx.x; e < count * D2; e += blockDim.x) {
-        const long m = e / D2, w = e % D2;
-        const int r = static_cast<int>(w % D), c = static_cast<int>(w / D);
-        dst[m * D * ld + r + static_cast<long>(c) * ld] = src[e];
-    }
-}
-
-// One system's RK4 run by the whole workgroup; x, k1..k4, tmp in LDS, then
-// (nstage >= 2, no Lh) the generators staged nstage at a time.  Reads the
-// initial vector from r_in and writes the final one to r_out.
-template <int DT>
-__device__ __forceinline__ void rk4_body(double2* sh, int nstage, const double2* Ls, const double2* Lh, long steps, int D,
-                         const double2* r_in, double2* r_out, double dt, long every, double2* samples,
-                         long* nsamples) {
-    double2* x = sh;
-    double2* k1 = x + D;
-    double2* k2 = k1 + D;
-    double2* k3 = k2 + D;
-    double2* k4 = k3 + D;
-    double2* tmp = k4 + D;
-    double2* M = tmp + D;
-    for (int e = threadIdx.x; e < D; e += blockDim.x) x[e] = r_in[e];
-    __syncthreads();
-    const long D2 = static_cast<long>(D) * D;
-    const int ld = D + 1;
-    long ns = 0;
-    if (nstage >= 2 && !Lh) {
-        for (long s = 0; s < steps; s += nstage - 1) {
-            const int cnt = static_cast<int>(min(static_cast<long>(nstage), steps - s + 1));
-            stage_mats(M, Ls, s, cnt, D);
-            __syncthreads();
-            for (int q = 0; q + 1 < cnt; ++q) {
-                const long st = s + q;
-                if (samples && st % every == 0) {
-                    for (int e = threadIdx.x; e < D; e += blockDim.x) samples[ns * D + e] = x[e];
-                    ++ns;
-                }
-                rk4_step<DT>(M + static_cast<long>(q) * D * ld, M + static_cast<long>(q + 1) * D * ld, ld, nullptr,
-                             x, k1, k2, k3, k4, tmp, D, dt);
-            }
-        }
-    } else {
-        for (long st = 0; st < steps; ++st) {
-            if (samples && st % every == 0) {
-                for (int e = threadIdx.x; e < D; e += blockDim.x) samples[ns * D + e] = x[e];
-                ++ns;
-            }
-            rk4_step<DT>(Ls + st * D2, Ls + (st + 1) * D2, D, Lh ? Lh + st * D2 : nullptr, x, k1, k2, k3, k4, tmp,
-                         D, dt);
-        }
-    }
-    if (samples) {
-        for (int e = threadIdx.x; e < D; e += blockDim.x) samples[ns * D + e] = x[e];
-        ++ns;
-    }
-    for (int e = threadIdx.x; e < D; e += blockDim.x) r_out[e] = x[e];
-    if (threadIdx.x == 0 && nsamples) *nsamples = ns;
-}
-
-// Dispatch on D = N^2 for the sizes of N = 2..8 (unrolled rows), else general.
-#define TACO_RK4_DISPATCH(D, CALL)      \
-    switch (D) {                        \
-        case 4: CALL(4); break;         \
-        case 9: CALL(9); break;         \
-        case 16: CALL(16); break;       \
-        case 25: CALL(25); break;       \
-        case 36: CALL(36); break;       \
-        case 49: CALL(49); break;       \
-        case 64: CALL(64); break;       \
-        default: CALL(0); break;        \
-    }
-
-#include "rk4_rows.hpp"
-
-// Largest RK4 workgroup: the row-group path at D = 64.
-constexpr int kRkBlockMax = 512;
-
-// Row-group path for the sizes that have one (no separate midpoint series),
-// else the general path above.
-template <int DT>
-__device__ __forceinline__ void rk4_any(double2* sh, int nstage, const double2* Ls, const double2* Lh, long steps,
-                                        int D, const double2* r_in, double2* r_out, double dt, long every,
-                                        double2* samples, long* nsamples) {
-    if constexpr (DT != 0) {
-        if (!Lh) {
-            rk4_rows<DT, false>(sh, Ls, 0, steps, r_in, r_out, dt, every, samples, nsamples, nullptr);
-            return;
-        }
-    }
-    rk4_body<DT>(sh, nstage, Ls, Lh, steps, D, r_in, r_out, dt, every, samples, nsamples);
-}
-
-// One system on the row-group path (D = N^2, N = 2..8), 64 W threads.
-template <int DT>
-__global__ __launch_bounds__(64 * RowGroup<DT>::W) void k_rk4_rows(const double2* Ls, long steps, double2* r,
-                                                                   double dt, long every, double2* samples,
-                                                                   long* nsamples) {
-    extern __shared__ double2 sh[];
-    rk4_rows<DT, false>(sh, Ls, 0, steps, r, r, dt, every, samples, nsamples, nullptr);
-}
-
-// Calls f(std::integral_constant<int, D>) for a D with a row-group path.
-template <class F>
-static bool rows_dispatch(int D, F&& f) {
-    switch (D) {
-        case 4: f(std::integral_constant<int, 4>{}); return true;
-        case 9: f(std::integral_constant<int, 9>{}); return true;
-        case 16: f(std::integral_constant<int, 16>{}); return true;
-        case 25: f(std::integral_constant<int, 25>{}); return true;
-        case 36: f(std::integral_constant<int, 36>{}); return true;
-        case 49: f(std::integral_constant<int, 49>{}); return true;
-        case 64: f(std::integral_constant<int, 64>{}); return true;
-        default: return false;
-    }
-}
-
-__global__ __launch_bounds__(kBlock) void k_rk4(const double2* Ls, const double2* Lh, long steps, int D, double2* r,
-                                                double dt, long every, double2* samples, long* nsamples, int nstage) {
-    extern __shared__ double2 sh[];
-#define TACO_RK4_CALL(DT) rk4_body<DT>(sh, nstage, Ls, Lh, steps, D, r, r, dt, every, samples, nsamples)
-    TACO_RK4_DISPATCH(D, TACO_RK4_CALL)
-#undef TACO_RK4_CALL
-}
-
-// Many independent systems, one workgroup each, in a single launch.
-struct Rk4Sys {
-    const double2* Ls;   // [steps + 1][D x D]
-    int nstage;          // generators staged in LDS at a time (0: read from global)
-    const double2* r0;   // [D]
-    double2* r;          // [D] final vector
-    double2* samples;    // [steps + 1][D]
-    long steps;
-    double dt;
-    int D;
-    const double2* Lh = nullptr;  // [steps][D x D] midpoints (large D), else formed on the fly
-};
-
-__global__ __launch_bounds__(kRkBlockMax) void k_rk4_batch(const Rk4Sys* sys) {
-    extern __shared__ double2 sh[];
-    const Rk4Sys S = sys[blockIdx.x];
-#define TACO_RK4_CALL(DT) rk4_any<DT>(sh, S.nstage, S.Ls, S.Lh, S.steps, S.D, S.r0, S.r, S.dt, 1, S.samples, nullptr)
-    TACO_RK4_DISPATCH(S.D, TACO_RK4_CALL)
-#undef TACO_RK4_CALL
-}
-
 // dst[q] = src[rows[q]] for rows of `len` complex values.
 __global__ __launch_bounds__(kBlock) void k_gather_rows(const double2* src, const int* rows, long len, double2* dst) {
     const double2* s = src + static_cast<long>(rows[blockIdx.x]) * len;
     double2* d = dst + static_cast<long>(blockIdx.x) * len;
     for (long e = threadIdx.x; e < len; e += kBlock) d[e] = s[e];
-}
-
-// out[n] = (L[n] + L[n + 1]) / 2 elementwise for n < count (midpoint
-// generators, formed with the expression the RK4 products use on the fly).
-__global__ __launch_bounds__(kBlock) void k_midpoints(const double2* __restrict__ L, long count, long D2,
-                                                      double2* __restrict__ out) {
-    const long total = count * D2;
-    for (long i = blockIdx.x * static_cast<long>(kBlock) + threadIdx.x; i < total;
-         i += static_cast<long>(gridDim.x) * kBlock)
-        out[i] = cscale(cadd(L[i], L[i + D2]), 0.5);
 }
 
 __global__ __launch_bounds__(kBlock) void k_fill_zero(double2* dst, long count) {
@@ -2252,7 +1902,7 @@ struct taco_ctx {
     hipStream_t stream = nullptr;
     hipEvent_t ev0 = nullptr, ev1 = nullptr;
     taco_engine::Profiler prof;
-    std::map<int, std::array<int, 3>> fft_choice;  // per FFT log-length: tile config of phases A, B, C
+    std::map<int, int> fft_shape;  // per FFT log-length: group bits of the last pass (0: tile kernels)
     std::map<int, std::unique_ptr<taco_engine::Twiddles>> tw;
     taco_engine::DevBuf gamma, omegas, mirror, p2f, ops, spec, inter1, inter2, conv, slices, t2pos, l4, gw, misc,
         rk, eps, jobtri, clsstart, jobmask, jobrow, comb, t2scr, rkmid, bred;
@@ -2292,10 +1942,11 @@ static void timed(taco_ctx* c, int id, double bytes, Fn&& launch) {
     c->prof.pending.push_back({id, a, b, bytes});
 }
 
-// Twiddle tables of length 2^L: the reference's recurrence values, or (exact)
-// each entry rounded once from quad precision (the window mode).
-static const Twiddles& twiddles_for(taco_ctx* c, int L, bool exact = false) {
-    const int key = L + (exact ? 64 : 0);
+// Twiddle tables of length 2^L for groups of 2^b values: the reference's
+// recurrence values, or (exact) each entry rounded once from quad precision
+// (the window mode).
+static const Twiddles& twiddles_for(taco_ctx* c, int L, int b, bool exact = false) {
+    const int key = L + 32 * b + (exact ? 1024 : 0);
     auto it = c->tw.find(key);
     if (it != c->tw.end()) return *it->second;
     auto t = std::make_unique<Twiddles>();
@@ -2305,8 +1956,8 @@ static const Twiddles& twiddles_for(taco_ctx* c, int L, bool exact = false) {
         make_twiddles_exact(L, tab);
     else
         make_twiddles(L, tab);  // stage-major standard table, 2^L - 1 entries
-    const int a = (L + 1) / 2, b = L - a;
-    const std::size_t nstd = (std::size_t{1} << std::max(a, b)) - 1;
+    const int a = L - b;
+    const std::size_t nstd = (std::size_t{1} << L) - 1;
     // Phase B forward stages s = a+1..L for group k1 < 2^a: T_s[k1 + v 2^a], v < 2^(s-1-a).
     const std::size_t bstride = (std::size_t{1} << b) - 1;
     std::vector<double> tb(2 * (std::size_t{1} << a) * bstride + 2);
@@ -2344,6 +1995,36 @@ static const Twiddles& twiddles_for(taco_ctx* c, int L, bool exact = false) {
     return ref;
 }
 
+static int env_int(const char* name, int dflt) {
+    const char* v = std::getenv(name);
+    return v ? std::atoi(v) : dflt;
+}
+
+// How a pass of FFT length 2^L over na A-jobs is laid out: groups of 2^b
+// values, run by the group kernels (group) or the tile kernels.
+struct FftShape {
+    int a, b;
+    bool group;
+};
+
+// Groups of 2^11 halve the rows a window of T > 2^9 times writes and phase C
+// reads (d = 8, Nfft 2^15, T = 1001: 24.1 ms a call against 28.4 with 2^10;
+// d = 4, Nfft 2^19, T = 10001: 12.0 against 14.0).  For T <= 2^9 the rows fall
+// off either way and one wave per group is the faster butterfly (d = 16,
+// Nfft 2^13, T = 201: 313 ms a gradient against 326), as it is when the
+// groups of 2^11 would leave compute units idle.  Lengths below 2^10 run on
+// tiles.  TACO_FFT_TILE forces a shape (every one performs the same
+// butterflies): 0, 1 the tiles on 256 / 512 threads, 2, 3 groups of 2^10, 2^11.
+static FftShape fft_shape(int L, long na, std::size_t T) {
+    const int forced = env_int("TACO_FFT_TILE", -1);
+    if (L < kGroupBitsMin || forced == 0 || forced == 1) return {(L + 1) / 2, L / 2, false};
+    int b = std::min(kGroupBitsMax, L);
+    const bool small = T <= (std::size_t{1} << (kGroupBitsMin - 1)) || (na << (L - b)) < 512;
+    if ((small || forced == 2) && forced != 3) b = kGroupBitsMin;
+    b = std::max(b, L - kTileBitsMax);
+    return {L - b, b, true};
+}
+
 // Launch phase kernels for a tile configuration index.
 enum Phase { PH_A_TRIPLE, PH_A_SPEC, PH_B_TRIPLE, PH_B_SPEC, PH_C };
 
@@ -2378,21 +2059,22 @@ static void launch_phase_cfg(Phase ph, const FcrArgs& P, long njobs, hipStream_t
     }
 }
 
-static void launch_phase(int cfg, Phase ph, const FcrArgs& P, long njobs, hipStream_t st) {
-    switch (cfg) {
-        case 0: launch_phase_cfg<Cfg8k>(ph, P, njobs, st); break;
-        case 1: launch_phase_cfg<Cfg4k>(ph, P, njobs, st); break;
-        case 2: launch_phase_cfg<Cfg4kW>(ph, P, njobs, st); break;
-        case 3: launch_phase_cfg<Cfg2k>(ph, P, njobs, st); break;
-        case 4: launch_phase_cfg<Cfg4kX>(ph, P, njobs, st); break;
-        case 5: launch_phase_cfg<Cfg2kW>(ph, P, njobs, st); break;
-        default: launch_phase_cfg<Cfg8kX>(ph, P, njobs, st); break;
+static void launch_phase(Phase ph, const FcrArgs& P, bool group, long njobs, hipStream_t st) {
+    if (group && (ph == PH_B_TRIPLE || ph == PH_B_SPEC)) {
+        launch_group_b(P, njobs, ph == PH_B_SPEC, st);
+        return;
     }
-}
-
-static int env_int(const char* name, int dflt) {
-    const char* v = std::getenv(name);
-    return v ? std::atoi(v) : dflt;
+    if (ph == PH_C) {
+        if (group && P.a == 0) return;  // phase B stored the convolutions
+        if (group_c_fits(P)) {
+            launch_group_c(P, st);
+            return;
+        }
+    }
+    if (env_int("TACO_FFT_TILE", -1) == 1)
+        launch_phase_cfg<Cfg2kW>(ph, P, njobs, st);
+    else
+        launch_phase_cfg<Cfg2k>(ph, P, njobs, st);
 }
 
 // Read at each launch (a test compares the two paths in one process).
@@ -2407,43 +2089,6 @@ static std::size_t chunk_budget_bytes() {
         return s ? static_cast<std::size_t>(std::strtoull(s, nullptr, 10)) : (std::size_t{12} << 30);
     }();
     return v;
-}
-
-// Times every tile configuration on this chunk, phase by phase in pipeline
-// order (each run rewrites the same values), and records the fastest.
-static void autotune(taco_ctx* c, const FcrArgs& P, long ncls, long na, long nj, std::array<int, 3>& choice) {
-    const Phase phases[3] = {PH_A_TRIPLE, PH_B_TRIPLE, PH_C};
-    const long units[3] = {ncls, na, nj};
-    hipEvent_t e0, e1;
-    HIP_OK(hipEventCreate(&e0));
-    HIP_OK(hipEventCreate(&e1));
-    for (int ph = 0; ph < 3; ++ph) {
-        float best = 0.f;
-        int best_cfg = 0;
-        for (int cfg = 0; cfg < kNumFftCfg; ++cfg) {
-            launch_phase(cfg, phases[ph], P, units[ph], c->stream);  // warm
-            // the fastest of three runs, so one noisy launch does not decide
-            float ms = 0.f;
-            for (int rep = 0; rep < 3; ++rep) {
-                HIP_OK(hipEventRecord(e0, c->stream));
-                launch_phase(cfg, phases[ph], P, units[ph], c->stream);
-                HIP_OK(hipEventRecord(e1, c->stream));
-                HIP_OK(hipEventSynchronize(e1));
-                float m = 0.f;
-                HIP_OK(hipEventElapsedTime(&m, e0, e1));
-                if (rep == 0 || m < ms) ms = m;
-            }
-            if (cfg == 0 || ms < best) {
-                best = ms;
-                best_cfg = cfg;
-            }
-        }
-        choice[ph] = best_cfg;
-        launch_phase(best_cfg, phases[ph], P, units[ph], c->stream);  // leave this phase's output in place
-    }
-    HIP_OK(hipGetLastError());
-    (void)hipEventDestroy(e0);
-    (void)hipEventDestroy(e1);
 }
 
 // Device-side F/C/R for all nf^3 triples over t < T; outputs per CombineArgs.
@@ -2531,6 +2176,7 @@ struct FcrJob {
     long nfft_jobs = 0, ncomb = 0, chunk = 1, cconv = 1, spec_jobs = 0;
     std::size_t n = 0, Nt = 0, T = 0;
     int L = 0;
+    bool group = false;
 };
 
 // Where a pass keeps its device job lists.
@@ -2621,8 +2267,6 @@ static FcrJob fcr_prepare(taco_ctx* c, const FcrPlan& pl, const FcrLists& lists)
     int L = 0;
     while ((std::size_t{1} << L) < n) ++L;
     if (L > 22) throw Error(TACO_ERR_INVALID, "FFT length above 2^22 (Nt above 2^21) is not supported");
-    const int a = (L + 1) / 2, b = L - a;
-    const Twiddles& tw = twiddles_for(c, L, window);
     const int nf = pl.nf;
     const long nf3 = static_cast<long>(nf) * nf * nf;
 
@@ -2659,6 +2303,10 @@ static FcrJob fcr_prepare(taco_ctx* c, const FcrPlan& pl, const FcrLists& lists)
     }
     const long nA = static_cast<long>(ajs.size());
     ajs.push_back(static_cast<int>(nfft_jobs));
+    const FftShape shape = fft_shape(L, nA, pl.T);
+    const Twiddles& tw = twiddles_for(c, L, shape.b, window);
+    const std::size_t Tq = std::min<std::size_t>(std::max<std::size_t>(pl.T, 1), std::size_t{1} << shape.b);
+    const std::size_t half_n = Tq << shape.a;  // values of one half-inverse product
     // Class pieces over A-jobs; a class with more than TACO_CLASS_MAX A-jobs
     // (default 4) is cut into pieces, each recomputing the same phases, so no
     // phase-A workgroup loops much longer than the others.
@@ -2673,7 +2321,7 @@ static FcrJob fcr_prepare(taco_ctx* c, const FcrPlan& pl, const FcrLists& lists)
     // running at the same time read the same two spectra (of g_mirror(j) and
     // conj(g_j)) and share them through L2.  The chunk length is fixed here
     // (chunks start at multiples of it).
-    const std::size_t per_job_b = 3 * n * 16;
+    const std::size_t per_job_b = (n + 2 * half_n) * 16;
     long chunk_len = static_cast<long>(std::max<std::size_t>(1, chunk_budget_bytes() / per_job_b));
     chunk_len = std::max(1L, std::min(chunk_len, std::max(nfft_jobs, 1L)));
     // FFT chunks: whole A-jobs, at most chunk_len triples (a longer A-job alone)
@@ -2745,7 +2393,7 @@ static FcrJob fcr_prepare(taco_ctx* c, const FcrPlan& pl, const FcrLists& lists)
     const long spec_jobs = 2L * nf;
     c->spec.ensure(static_cast<std::size_t>(spec_jobs) * n * 16);
     c->inter1.ensure(static_cast<std::size_t>(std::max(chunk, spec_jobs)) * n * 16);
-    c->inter2.ensure(static_cast<std::size_t>(2 * chunk) * n * 16);
+    c->inter2.ensure(static_cast<std::size_t>(2 * chunk) * half_n * 16);
     c->conv.ensure(static_cast<std::size_t>(2 * cconv) * Tpad * 16);
     for (const FcrJob::Batch& bt : batches)
         if (const long nblk = combine_split_blocks(bt.cb, pl.T))
@@ -2760,9 +2408,10 @@ static FcrJob fcr_prepare(taco_ctx* c, const FcrPlan& pl, const FcrLists& lists)
     P.Nin = static_cast<long>(Nin);
     P.dt = pl.dt;
     P.L = L;
-    P.a = a;
-    P.b = b;
+    P.a = shape.a;
+    P.b = shape.b;
     P.n = static_cast<long>(n);
+    P.Tq = static_cast<long>(Tq);
     P.twStd = tw.std_.as<double2>();
     P.twB = tw.b_.as<double2>();
     P.twC = tw.c_.as<double2>();
@@ -2799,37 +2448,29 @@ static FcrJob fcr_prepare(taco_ctx* c, const FcrPlan& pl, const FcrLists& lists)
     J.Nt = pl.Nt;
     J.T = pl.T;
     J.L = L;
+    J.group = shape.group;
     return J;
 }
 
-// Launches one prepared pass on the context stream.  The first pass of an
-// FFT length picks the tile configurations (autotune synchronises the
-// stream); later passes of that length only launch kernels.
+// Launches one prepared pass on the context stream.
 static void fcr_launch(taco_ctx* c, FcrJob& J, const CombineArgs& out) {
     FcrArgs& P = J.P;
     P.inter1 = c->inter1.as<double2>();
     P.inter2 = c->inter2.as<double2>();
     P.spec = c->spec.as<double2>();
     P.conv = c->conv.as<double2>();
-    const int L = J.L;
     const long spec_jobs = J.spec_jobs;
     const std::vector<int>& cls_start = J.cls_start;
-    // Tile configuration per phase: TACO_FFT_TILE=<0..6> forces one; otherwise
-    // the first chunk of each FFT length is run with every configuration
-    // (identical butterflies, identical results) and the fastest is kept.
-    auto it = c->fft_choice.find(L);
-    if (it == c->fft_choice.end()) it = c->fft_choice.emplace(L, std::array<int, 3>{-1, -1, -1}).first;
-    auto& choice = it->second;
-    const int forced = env_int("TACO_FFT_TILE", -1);
-    if (forced >= 0 && forced < kNumFftCfg) choice = {forced, forced, forced};
+    c->fft_shape[J.L] = J.group ? P.b : 0;
+    const double ch = static_cast<double>(P.Tq << P.a) * 16.0;  // the kept rows of one half-inverse product
     const double cn = static_cast<double>(J.n) * 16.0;      // one complex series of length Nfft
     const double cNt = static_cast<double>(J.Nt) * 16.0;
     const double cT = static_cast<double>(J.T) * 16.0;
     // Spectra of every Gamma column and its conjugate.
     P.njobs = static_cast<int>(spec_jobs);
     timed(c, K_SPECTRA, spec_jobs * (cNt + 3 * cn), [&] {
-        launch_phase(choice[0] >= 0 ? choice[0] : 0, PH_A_SPEC, P, spec_jobs, c->stream);
-        launch_phase(choice[1] >= 0 ? choice[1] : 0, PH_B_SPEC, P, spec_jobs, c->stream);
+        launch_phase(PH_A_SPEC, P, J.group, spec_jobs, c->stream);
+        launch_phase(PH_B_SPEC, P, J.group, spec_jobs, c->stream);
     });
     HIP_OK(hipGetLastError());
     auto class_of = [&](long aj) {
@@ -2849,17 +2490,16 @@ static void fcr_launch(taco_ctx* c, FcrJob& J, const CombineArgs& out) {
             P.cls0 = class_of(a0);
             const long ncls = class_of(a1 - 1) - P.cls0 + 1;
             const double na = static_cast<double>(a1 - a0);
-            if (choice[0] < 0 || choice[1] < 0 || choice[2] < 0) autotune(c, P, ncls, a1 - a0, nj, choice);
             // phase A: read the Gamma column, write the half-transformed signal, once per A-job
-            timed(c, K_PHASE_A, na * (cNt + cn), [&] { launch_phase(choice[0], PH_A_TRIPLE, P, ncls, c->stream); });
+            timed(c, K_PHASE_A, na * (cNt + cn), [&] { launch_phase(PH_A_TRIPLE, P, J.group, ncls, c->stream); });
             // F and C paths of the chunk (one or both per triple)
             const double np_ = static_cast<double>(J.paths[job0 + nj] - J.paths[job0]);
-            // phase B: read each A-job's signal once and one spectrum per path, write one
-            // half-inverse product per path
-            timed(c, K_PHASE_B, na * cn + np_ * 2 * cn,
-                  [&] { launch_phase(choice[1], PH_B_TRIPLE, P, a1 - a0, c->stream); });
+            // phase B: read each A-job's signal once and one spectrum per path, write the
+            // kept rows of one half-inverse product per path
+            timed(c, K_PHASE_B, na * cn + np_ * (cn + ch),
+                  [&] { launch_phase(PH_B_TRIPLE, P, J.group, a1 - a0, c->stream); });
             // phase C: read each path's product, write its convolution for t < T
-            timed(c, K_PHASE_C, np_ * (cn + cT), [&] { launch_phase(choice[2], PH_C, P, nj, c->stream); });
+            timed(c, K_PHASE_C, np_ * (ch + cT), [&] { launch_phase(PH_C, P, J.group, nj, c->stream); });
             HIP_OK(hipGetLastError());
         }
         // combine: read three Gamma columns and each path's convolution over
@@ -3286,8 +2926,7 @@ static void batch_enqueue(taco_ctx* c, BatchRun& B) {
     for (auto& s : B.sys) batch_enqueue_system(c, *s);
     if (B.nrk) {
         timed(c, K_RK4, B.rk_bytes, [&] {
-            hipLaunchKernelGGL(k_rk4_batch, dim3(static_cast<unsigned>(B.nrk)), dim3(B.rk_block), B.rk_lds, c->stream,
-                               B.rkargs.as<Rk4Sys>());
+            launch_rk4_batch(static_cast<unsigned>(B.nrk), B.rkargs.as<Rk4Sys>(), B.rk_block, B.rk_lds, c->stream);
         });
         HIP_OK(hipGetLastError());
     }
@@ -3326,10 +2965,7 @@ struct taco_tape {
 
 namespace taco_engine {
 
-// LDS of the RK4 workgroups: `vecs` vectors of D, then generators staged
-// nstage at a time (column stride D + 1) within the 160 KiB of a CU.
-constexpr std::size_t kRkLds = 160 * 1024;
-
+// Generators staged at a time beside `vecs` vectors of D.
 static int rk4_nstage(int D, int vecs, long max_mats) {
     const std::size_t per = static_cast<std::size_t>(D) * (D + 1) * 16;
     const std::size_t base = static_cast<std::size_t>(vecs) * D * 16;
@@ -3345,7 +2981,6 @@ static std::size_t rk4_lds(int D, int vecs, int nstage) {
 
 // Threads of an RK4 workgroup: TACO_RK4_BLOCK (64..256, multiple of 64),
 // else 256 (measured faster than one wave for D = 16..64).
-static int env_int(const char* name, int dflt);
 static int rk4_block(int D) {
     (void)D;
     const int b = env_int("TACO_RK4_BLOCK", 0);
@@ -3360,10 +2995,7 @@ static bool rk4_midpoints_fit(int D, std::size_t steps) {
 static const double2* rk4_midpoints(taco_ctx* c, DevBuf& buf, const double2* Ls, std::size_t steps, int D) {
     const long D2 = static_cast<long>(D) * D;
     buf.ensure(steps * static_cast<std::size_t>(D2) * 16);
-    const long total = static_cast<long>(steps) * D2;
-    const unsigned grid = static_cast<unsigned>(std::min<long>((total + kBlock - 1) / kBlock, 65536));
-    hipLaunchKernelGGL(k_midpoints, dim3(grid), dim3(kBlock), 0, c->stream, Ls, static_cast<long>(steps), D2,
-                       buf.as<double2>());
+    launch_midpoints(Ls, static_cast<long>(steps), D2, buf.as<double2>(), c->stream);
     HIP_OK(hipGetLastError());
     return buf.as<double2>();
 }
@@ -3375,11 +3007,8 @@ static void rk4_launch(taco_ctx* ctx, const double2* dLs, const double2* dLh, st
     const double rk_bytes = gen_bytes + (dsamples ? static_cast<double>(steps / every + 2) * D * 16.0 : 0.0);
     if (!dLh && rk4_rows_threads(D) > 0) {
         timed(ctx, K_RK4, rk_bytes, [&] {
-            rows_dispatch(D, [&](auto dc) {
-                constexpr int DT = decltype(dc)::value;
-                hipLaunchKernelGGL(k_rk4_rows<DT>, dim3(1), dim3(rk4_rows_threads(DT)), 3 * DT * 16, ctx->stream, dLs,
-                                   static_cast<long>(steps), dr, dt, static_cast<long>(every), dsamples, dns);
-            });
+            launch_rk4_rows(D, dLs, static_cast<long>(steps), dr, dt, static_cast<long>(every), dsamples, dns,
+                            ctx->stream);
         });
         HIP_OK(hipGetLastError());
         return;
@@ -3394,8 +3023,8 @@ static void rk4_launch(taco_ctx* ctx, const double2* dLs, const double2* dLh, st
     const std::size_t lds = rk4_lds(D, 6, nstage);
     if (lds > kRkLds) throw Error(TACO_ERR_INVALID, "RK4 kernel supports D <= 1706");
     timed(ctx, K_RK4, rk_bytes, [&] {
-        hipLaunchKernelGGL(k_rk4, dim3(1), dim3(rk4_block(D)), lds, ctx->stream, dLs, dLh, static_cast<long>(steps), D,
-                           dr, dt, static_cast<long>(every), dsamples, dns, nstage);
+        launch_rk4(D, dLs, dLh, static_cast<long>(steps), dr, dt, static_cast<long>(every), dsamples, dns, nstage,
+                   rk4_block(D), lds, ctx->stream);
     });
     HIP_OK(hipGetLastError());
 }
@@ -3706,13 +3335,8 @@ static void rk_rev_run(taco_tape& tp, const RkRev& b) {
     const RkRevShape sh = rk_rev_shape(tp, b);
     const int Di = static_cast<int>(D);
     if (b.LsH) {
-        const int tiles = (Di + 15) / 16;
-        hipLaunchKernelGGL(k_conj_transpose, dim3(static_cast<unsigned>(tiles * tiles), static_cast<unsigned>(tp.T)),
-                           dim3(kBlock), 0, c->stream, tp.lgen.as<double2>(), b.LsH, Di, static_cast<long>(tp.T));
-        const long D2l = static_cast<long>(D2), total = static_cast<long>(tp.steps) * D2l;
-        hipLaunchKernelGGL(k_midpoints, dim3(static_cast<unsigned>(std::min<long>((total + kBlock - 1) / kBlock, 65536))),
-                           dim3(kBlock), 0, c->stream, static_cast<const double2*>(b.LsH), static_cast<long>(tp.steps),
-                           D2l, b.LhH);
+        launch_conj_transpose(tp.lgen.as<double2>(), b.LsH, Di, static_cast<long>(tp.T), c->stream);
+        launch_midpoints(b.LsH, static_cast<long>(tp.steps), static_cast<long>(D2), b.LhH, c->stream);
     } else if (!sh.carry) {
         const long cntL = static_cast<long>(tp.T * D2);
         hipLaunchKernelGGL(k_fill_zero, dim3(static_cast<unsigned>((cntL + kBlock - 1) / kBlock)), dim3(kBlock), 0,
@@ -3720,29 +3344,9 @@ static void rk_rev_run(taco_tape& tp, const RkRev& b) {
     }
     timed(c, K_RK4, sh.bytes, [&] {
         // every segment's states and stage points from its checkpoint, all segments at once
-        if (sh.rows_f) {
-            rows_dispatch(Di, [&](auto dc) {
-                constexpr int DT = decltype(dc)::value;
-                hipLaunchKernelGGL(k_rk4_recompute_rows<DT>, dim3(static_cast<unsigned>(sh.nseg)),
-                                   dim3(rk4_rows_threads(DT)), 3 * DT * 16, c->stream, sh.Rf);
-            });
-        } else {
-            hipLaunchKernelGGL(k_rk4_recompute, dim3(static_cast<unsigned>(sh.nseg)), dim3(kBlock), sh.lds_f,
-                               c->stream, sh.Rf);
-        }
-        if (sh.rows_b) {
-            rows_dispatch(Di, [&](auto dc) {
-                constexpr int DT = decltype(dc)::value;
-                if constexpr (DT <= 16)
-                    hipLaunchKernelGGL(k_rk4_adjoint_rows<DT>, dim3(1), dim3(64), 5 * DT * 16, c->stream, sh.R);
-            });
-        } else {
-            hipLaunchKernelGGL(k_rk4_adjoint, dim3(1), dim3(kBlock), sh.lds_b, c->stream, sh.R);
-        }
-        if (b.vec)
-            hipLaunchKernelGGL(k_rk4_lbar, dim3(static_cast<unsigned>((D2 + kBlock - 1) / kBlock),
-                                                static_cast<unsigned>(tp.T)),
-                               dim3(kBlock), 0, c->stream, sh.R);
+        launch_rk4_recompute(sh.Rf, sh.rows_f, static_cast<unsigned>(sh.nseg), sh.lds_f, c->stream);
+        launch_rk4_walk(sh.R, sh.rows_b, sh.lds_b, c->stream);
+        if (b.vec) launch_rk4_lbar(sh.R, c->stream);
     });
     HIP_OK(hipGetLastError());
 }
@@ -4148,14 +3752,15 @@ static SpecOut fft_forward_dev(taco_ctx* c, double2* x, int L, double2* tw_tiny)
         HIP_OK(hipGetLastError());
         return {x, L, 0};
     }
-    const Twiddles& tw = twiddles_for(c, L);
+    const FftShape shape = fft_shape(L, 1, n);
+    const Twiddles& tw = twiddles_for(c, L, shape.b);
     FcrArgs P{};
     P.gamma = x;
     P.Nt = static_cast<long>(n);
     P.Nin = static_cast<long>(n);
     P.L = L;
-    P.a = (L + 1) / 2;
-    P.b = L - P.a;
+    P.a = shape.a;
+    P.b = shape.b;
     P.n = static_cast<long>(n);
     P.twStd = tw.std_.as<double2>();
     P.twB = tw.b_.as<double2>();
@@ -4165,11 +3770,8 @@ static SpecOut fft_forward_dev(taco_ctx* c, double2* x, int L, double2* tw_tiny)
     P.inter1 = c->inter1.as<double2>();
     P.spec = c->spec.as<double2>();
     P.njobs = 1;
-    auto it = c->fft_choice.find(L);
-    const int cfgA = it != c->fft_choice.end() && it->second[0] >= 0 ? it->second[0] : 2;
-    const int cfgB = it != c->fft_choice.end() && it->second[1] >= 0 ? it->second[1] : 2;
-    launch_phase(cfgA, PH_A_SPEC, P, 1, c->stream);
-    launch_phase(cfgB, PH_B_SPEC, P, 1, c->stream);
+    launch_phase(PH_A_SPEC, P, shape.group, 1, c->stream);
+    launch_phase(PH_B_SPEC, P, shape.group, 1, c->stream);
     HIP_OK(hipGetLastError());
     return {P.spec, P.a, P.b};
 }
@@ -4648,11 +4250,8 @@ static void mtape_forward(taco_mtape& mt, const taco_tape_set* in, double* const
         sys[s] = Rk4Sys{tp.lgen.as<double2>(), nstage, r0d + s * D, rend + s * D, samp + s * T * D,
                         static_cast<long>(tp.steps), tp.dt, Di};
         if (mids) {
-            const long D2 = static_cast<long>(D) * D, total = static_cast<long>(tp.steps) * D2;
             double2* m = mt.A->mid.as<double2>() + s * tp.steps * D * D;
-            hipLaunchKernelGGL(k_midpoints, dim3(static_cast<unsigned>(std::min<long>((total + kBlock - 1) / kBlock,
-                                                                                     65536))),
-                               dim3(kBlock), 0, c->stream, tp.lgen.as<double2>(), static_cast<long>(tp.steps), D2, m);
+            launch_midpoints(tp.lgen.as<double2>(), static_cast<long>(tp.steps), static_cast<long>(D) * D, m, c->stream);
             sys[s].Lh = m;
         }
     }
@@ -4660,8 +4259,8 @@ static void mtape_forward(taco_mtape& mt, const taco_tape_set* in, double* const
     HIP_OK(hipMemcpyAsync(mt.A->args.p, sys.data(), S * sizeof(Rk4Sys), hipMemcpyHostToDevice, c->stream));
     const double rk_bytes = static_cast<double>(S) * ((t0.steps + 1) * D * D * 16.0 + (t0.steps + 1) * D * 16.0);
     timed(c, K_RK4, rk_bytes, [&] {
-        hipLaunchKernelGGL(k_rk4_batch, dim3(static_cast<unsigned>(S)), dim3(rows_thr > 0 ? rows_thr : rk4_block(Di)),
-                           lds, c->stream, mt.A->args.as<const Rk4Sys>());
+        launch_rk4_batch(static_cast<unsigned>(S), mt.A->args.as<const Rk4Sys>(),
+                         rows_thr > 0 ? rows_thr : rk4_block(Di), lds, c->stream);
     });
     HIP_OK(hipGetLastError());
     for (std::size_t s = 0; s < S; ++s) tape_checkpoints(*mt.sets[s], samp + s * T * D);
@@ -4690,15 +4289,9 @@ static void mtape_adjoint(taco_mtape& mt, const double* const* samples_bar, doub
         args[s] = sh.Rf;
         args[S + s] = sh.R;
         if (rv[s].LsH) {
-            const int tiles = (static_cast<int>(D) + 15) / 16;
-            hipLaunchKernelGGL(k_conj_transpose, dim3(static_cast<unsigned>(tiles * tiles), static_cast<unsigned>(T)),
-                               dim3(kBlock), 0, c->stream, mt.sets[s]->lgen.as<double2>(), rv[s].LsH,
-                               static_cast<int>(D), static_cast<long>(T));
-            const long D2l = static_cast<long>(D2), total = static_cast<long>(T - 1) * D2l;
-            hipLaunchKernelGGL(k_midpoints,
-                               dim3(static_cast<unsigned>(std::min<long>((total + kBlock - 1) / kBlock, 65536))),
-                               dim3(kBlock), 0, c->stream, static_cast<const double2*>(rv[s].LsH),
-                               static_cast<long>(T - 1), D2l, rv[s].LhH);
+            launch_conj_transpose(mt.sets[s]->lgen.as<double2>(), rv[s].LsH, static_cast<int>(D), static_cast<long>(T),
+                                  c->stream);
+            launch_midpoints(rv[s].LsH, static_cast<long>(T - 1), static_cast<long>(D2), rv[s].LhH, c->stream);
         } else if (!sh.carry) {
             const long cntL = static_cast<long>(T * D2);
             hipLaunchKernelGGL(k_fill_zero, dim3(static_cast<unsigned>((cntL + kBlock - 1) / kBlock)), dim3(kBlock),
@@ -4710,32 +4303,10 @@ static void mtape_adjoint(taco_mtape& mt, const double* const* samples_bar, doub
     HIP_OK(hipMemcpyAsync(mt.A->args.p, args.data(), 2 * S * sizeof(Rk4AdjArgs), hipMemcpyHostToDevice, c->stream));
     const int Di = static_cast<int>(D);
     timed(c, K_RK4, sh.bytes * static_cast<double>(S), [&] {
-        if (sh.rows_f) {
-            rows_dispatch(Di, [&](auto dc) {
-                constexpr int DT = decltype(dc)::value;
-                hipLaunchKernelGGL(k_rk4_recompute_rows_multi<DT>,
-                                   dim3(static_cast<unsigned>(sh.nseg), static_cast<unsigned>(S)),
-                                   dim3(rk4_rows_threads(DT)), 3 * DT * 16, c->stream, dargs);
-            });
-        } else {
-            hipLaunchKernelGGL(k_rk4_recompute_multi, dim3(static_cast<unsigned>(sh.nseg), static_cast<unsigned>(S)),
-                               dim3(kBlock), sh.lds_f, c->stream, dargs);
-        }
-        if (sh.rows_b) {
-            rows_dispatch(Di, [&](auto dc) {
-                constexpr int DT = decltype(dc)::value;
-                if constexpr (DT <= 16)
-                    hipLaunchKernelGGL(k_rk4_adjoint_rows_multi<DT>, dim3(static_cast<unsigned>(S)), dim3(64),
-                                       5 * DT * 16, c->stream, dargs + S);
-            });
-        } else {
-            hipLaunchKernelGGL(k_rk4_adjoint_multi, dim3(static_cast<unsigned>(S)), dim3(kBlock), sh.lds_b, c->stream,
-                               dargs + S);
-        }
-        if (rv[0].vec)
-            hipLaunchKernelGGL(k_rk4_lbar_multi, dim3(static_cast<unsigned>((D2 + kBlock - 1) / kBlock),
-                                                      static_cast<unsigned>(T), static_cast<unsigned>(S)),
-                               dim3(kBlock), 0, c->stream, dargs + S);
+        const unsigned nt = static_cast<unsigned>(S);
+        launch_rk4_recompute_multi(dargs, nt, Di, sh.rows_f, static_cast<unsigned>(sh.nseg), sh.lds_f, c->stream);
+        launch_rk4_walk_multi(dargs + S, nt, Di, sh.rows_b, sh.lds_b, c->stream);
+        if (rv[0].vec) launch_rk4_lbar_multi(dargs + S, nt, Di, static_cast<long>(T) - 1, c->stream);
     });
     HIP_OK(hipGetLastError());
     for (std::size_t s = 0; s < S; ++s) {
@@ -4887,12 +4458,7 @@ int taco_ctx_create(int device, taco_ctx** out) {
                                  hipMemcpyHostToDevice));
         HIP_OK(hipEventCreate(&c->ev0));
         HIP_OK(hipEventCreate(&c->ev1));
-        for (const void* fn : {reinterpret_cast<const void*>(k_rk4), reinterpret_cast<const void*>(k_rk4_batch),
-                               reinterpret_cast<const void*>(k_rk4_adjoint),
-                               reinterpret_cast<const void*>(k_rk4_recompute),
-                               reinterpret_cast<const void*>(k_rk4_adjoint_multi),
-                               reinterpret_cast<const void*>(k_rk4_recompute_multi)})
-            HIP_OK(hipFuncSetAttribute(fn, hipFuncAttributeMaxDynamicSharedMemorySize, static_cast<int>(kRkLds)));
+        HIP_OK(rk4_set_lds_limits());
         *out = c.release();
     });
 }
@@ -4946,8 +4512,10 @@ int taco_profile_get(taco_ctx* ctx, int kernel, double* total_ms, long* launches
 int taco_fft_tile_choice(taco_ctx* ctx, int log2_nfft, int* cfg3) {
     return guarded([&] {
         check_ctx(ctx);
-        auto it = ctx->fft_choice.find(log2_nfft);
-        for (int k = 0; k < 3; ++k) cfg3[k] = it == ctx->fft_choice.end() ? -1 : it->second[k];
+        auto it = ctx->fft_shape.find(log2_nfft);
+        const int v = it == ctx->fft_shape.end() ? -1 : it->second ? it->second : 3;
+        cfg3[0] = v < 0 ? v : 3;  // phase A always runs on tiles
+        cfg3[1] = cfg3[2] = v;
     });
 }
 

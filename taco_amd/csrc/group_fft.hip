@@ -1,0 +1,407 @@
+// group_fft.hip — phases B and C of the F/C/R passes on register groups.
+//
+// The forward FFT's last b stages and the inverse's first b stages of a
+// residue group {k = k1 mod 2^a} are closed (engine.hip).  Here one workgroup
+// of 2^b / 16 threads runs them with the group's values in registers, 16 per
+// thread: three radix-2^r passes with two LDS exchanges, the forward values
+// kept in registers for every product of the A-job, spectra and results
+// straight between registers and memory.  Only the rows t mod 2^b < T of a
+// half-inverse feed kept times, so a group writes min(T, 2^b) values and
+// phase C combines 2^a of them per kept time.  Every butterfly is the
+// reference's u +/- w*x with the stage's table twiddle, as in the tile
+// kernels, so the values are bit-identical at every b.
+//
+// What bounds them (MI355X): phase B issues 53-59 % of the FP64 slots it has
+// (two waves per SIMD; the forward values and a pass's twiddles take the
+// registers of a third) at 1.8-1.9 GHz, next to 5 TB/s of traffic; phase C
+// reads at 4.3-4.8 TB/s, the rate of a plain copy.
+#include "group_fft.hpp"
+
+#pragma clang fp contract(off)
+
+namespace taco_engine {
+
+// A group of 2^LG values on 2^LG / 16 threads (one or two waves, so the
+// barriers cost little and four to eight groups share a CU; groups of 2^12
+// and 2^13 measured 1.5 and 2 times slower per value).  The stages run as
+// passes of radix 2^RL in registers with an LDS exchange between two passes.
+template <int LG>
+struct Group {
+    static constexpr int kNV = 16;
+    static constexpr int kNT = 1 << (LG - 4);
+    static constexpr int kPass = 3;
+    static constexpr int kLds = (1 << LG) + (1 << (LG - 4));  // a pad slot per 16 values
+    static __host__ __device__ constexpr int rl(int p) { return p == 0 || (p == 1 && LG == 11) ? 4 : 3; }
+    static __host__ __device__ constexpr int s_lo(int p) { return p == 0 ? 1 : s_lo(p - 1) + rl(p - 1); }
+};
+
+// Reads of kernel-constant data at a wave-uniform address, by scalar loads.
+template <class T>
+__device__ __forceinline__ T uload(const T* p) {
+    return *(const __attribute__((address_space(4))) T*)(unsigned long)(p);
+}
+__device__ __forceinline__ double2 uload2(const double2* p) {
+    const double* d = reinterpret_cast<const double*>(p);
+    return make_double2(uload(d), uload(d + 1));
+}
+// base[idx] with a wave-uniform base and a 32-bit byte offset per lane: one
+// offset register serves every access that differs by a uniform distance.
+__device__ __forceinline__ double2 vload(const double2* base, unsigned idx) {
+    return *reinterpret_cast<const double2*>(reinterpret_cast<const char*>(base) + idx * 16u);
+}
+__device__ __forceinline__ void vstore(double2* base, unsigned idx, double2 v) {
+    *reinterpret_cast<double2*>(reinterpret_cast<char*>(base) + idx * 16u) = v;
+}
+
+__device__ __forceinline__ unsigned lds_at(unsigned pos) { return pos + (pos >> 4); }
+
+// One pass: stages s_lo .. s_lo + RL - 1 (local, 1-based).  Set (k, u0) of a
+// thread holds the values at u0 + (k R + m) 2^ub on entry (v[q R + m]) and
+// those at u0 + (k + j 2^(s_lo-1)) 2^ub on return (v[q R + j]).
+template <int LG, int P>
+struct Pass {
+    using G = Group<LG>;
+    static constexpr int RL = G::rl(P), S = G::s_lo(P), R = 1 << RL, SETS = G::kNV / R;
+    static constexpr int UB = LG - S - RL + 1;
+    static __device__ __forceinline__ unsigned u0(int q) { return (threadIdx.x + q * G::kNT) & ((1u << UB) - 1); }
+    static __device__ __forceinline__ unsigned k(int q) { return (threadIdx.x + q * G::kNT) >> UB; }
+    // LDS slots of input m and output j of set q.  The m and j parts carry
+    // into no bit of the set's own low four (2^ub > u0, and k R 2^ub or
+    // 2^(s_lo-1+ub) clears them), so the padded slots add and the m and j
+    // parts are constants.
+    static __device__ __forceinline__ unsigned in_slot(int q, int m) {
+        return lds_at(u0(q) + ((k(q) * R) << UB)) + lds_at(m << UB);
+    }
+    static __device__ __forceinline__ unsigned out_slot(int q, int j) {
+        return lds_at(u0(q) + (k(q) << UB)) + lds_at(j << (S - 1 + UB));
+    }
+
+    static __device__ __forceinline__ void load_tw(double2 (&w)[SETS][R - 1], const double2* __restrict__ tw) {
+#pragma unroll
+        for (int q = 0; q < SETS; ++q)
+#pragma unroll
+            for (int i = 0; i < RL; ++i)
+#pragma unroll
+                for (int j = 0; j < (1 << i); ++j) {
+                    const double2* base = tw + ((1 << (S + i - 1)) - 1 + (j << (S - 1)));
+                    // pass 0 has k = 0: uniform twiddles
+                    w[q][(1 << i) - 1 + j] = P == 0 ? uload2(base) : vload(base, k(q));
+                }
+    }
+    template <bool CONJ>
+    static __device__ __forceinline__ void butterflies(double2 (&v)[16], const double2 (&w)[SETS][R - 1], int q) {
+#pragma unroll
+        for (int i = 0; i < RL; ++i) {
+            const int h = R >> (i + 1);
+            double2 y[R];
+#pragma unroll
+            for (int j = 0; j < (1 << i); ++j) {
+                double2 t = w[q][(1 << i) - 1 + j];
+                if (CONJ) t.y = -t.y;
+#pragma unroll
+                for (int m = 0; m < h; ++m) {
+                    const double2 E = v[q * R + m + 2 * h * j];
+                    const double2 x = cmul(t, v[q * R + m + h + 2 * h * j]);
+                    y[m + h * j] = cadd(E, x);
+                    y[m + h * j + R / 2] = csub(E, x);
+                }
+            }
+#pragma unroll
+            for (int m = 0; m < R; ++m) v[q * R + m] = y[m];
+        }
+    }
+    // Output j = 0 alone (the others are past the kept rows).
+    template <bool CONJ>
+    static __device__ __forceinline__ void butterflies_first(double2 (&v)[16], const double2 (&w)[SETS][R - 1], int q) {
+#pragma unroll
+        for (int i = 0; i < RL; ++i) {
+            const int h = R >> (i + 1);
+            double2 t = w[q][(1 << i) - 1];
+            if (CONJ) t.y = -t.y;
+#pragma unroll
+            for (int m = 0; m < h; ++m) v[q * R + m] = cadd(v[q * R + m], cmul(t, v[q * R + m + h]));
+        }
+    }
+};
+
+// Passes P.. of a group FFT.  v holds pass P's inputs; returns the group in
+// natural order, v[m] at threadIdx.x + m kNT.  need: positions at or above
+// it are not read afterwards (each pass then runs only the sets that feed
+// kept ones: a set of index k writes positions from k 2^ub on and reads the
+// R 2^ub positions from k R 2^ub).
+template <int LG, int P, bool CONJ>
+__device__ __forceinline__ void group_passes(double2 (&v)[16], double2* buf, const double2* __restrict__ tw, unsigned need) {
+    using G = Group<LG>;
+    using A = Pass<LG, P>;
+    constexpr bool last = P == G::kPass - 1;
+    // Sets of this pass that are needed: walk the bound back from the last pass.
+    unsigned kmax = 0;
+    {
+        unsigned bout = need;
+#pragma unroll
+        for (int p = G::kPass - 1; p >= P; --p) {
+            const int ub = LG - G::s_lo(p) - G::rl(p) + 1;
+            kmax = (bout + (1 << ub) - 1) >> ub;
+            bout = min(kmax << (ub + G::rl(p)), 1u << LG);
+        }
+    }
+    double2 w[A::SETS][A::R - 1];
+    A::load_tw(w, tw);  // in flight over the barrier and the LDS reads
+    if constexpr (P > 0) {
+        __syncthreads();
+#pragma unroll
+        for (int q = 0; q < A::SETS; ++q)
+            if (A::k(q) < kmax)
+#pragma unroll
+                for (int m = 0; m < A::R; ++m) v[q * A::R + m] = buf[A::in_slot(q, m)];
+    }
+#pragma unroll
+    for (int q = 0; q < A::SETS; ++q)
+        if (A::k(q) < kmax) {
+            if (last && need <= (1u << (A::S - 1)))
+                A::template butterflies_first<CONJ>(v, w, q);
+            else
+                A::template butterflies<CONJ>(v, w, q);
+        }
+    if constexpr (last) {
+        // set q's output j sits at threadIdx.x + (q + SETS j) kNT
+        double2 y[16];
+#pragma unroll
+        for (int q = 0; q < A::SETS; ++q)
+#pragma unroll
+            for (int j = 0; j < A::R; ++j) y[q + A::SETS * j] = v[q * A::R + j];
+#pragma unroll
+        for (int m = 0; m < 16; ++m) v[m] = y[m];
+    } else {
+        if constexpr (P > 0) __syncthreads();  // every read of this pass is done
+#pragma unroll
+        for (int q = 0; q < A::SETS; ++q)
+            if (A::k(q) < kmax)
+#pragma unroll
+                for (int j = 0; j < A::R; ++j) buf[A::out_slot(q, j)] = v[q * A::R + j];
+        group_passes<LG, P + 1, CONJ>(v, buf, tw, need);
+    }
+}
+
+// Phase B of one A-job (or spectrum) and one group k1.  SPEC stores the
+// forward group; otherwise every live (triple, path) of the A-job takes the
+// product with its bucket spectrum (path 0, F: g_mirror(j); path 1, C:
+// conj g_j) and the inverse's first b stages.  The forward values stay in
+// registers for all of the A-job's products.
+template <int LG, bool SPEC>
+__global__ __launch_bounds__(Group<LG>::kNT) __attribute__((amdgpu_waves_per_eu(2, 2))) void k_group_b(FcrArgs P,
+                                                                                                       long njobs) {
+    using G = Group<LG>;
+    constexpr int NT = G::kNT;
+    __shared__ double2 buf[G::kLds];
+    const int ngroups = 1 << P.a;
+    int job, k1;
+    if ((ngroups & 7) == 0) {
+        // each XCD keeps a fixed eighth of the groups: its L2 holds their
+        // twiddles and spectra
+        xcd_map(blockIdx.x, ngroups, job, k1);
+    } else {
+        // each XCD keeps a contiguous eighth of the A-jobs (sorted by j)
+        const long total = njobs << P.a, per = (total + 7) >> 3;
+        const long lin = (blockIdx.x & 7) * per + (blockIdx.x >> 3);
+        if ((blockIdx.x >> 3) >= per || lin >= total) return;
+        job = static_cast<int>(lin >> P.a);
+        k1 = static_cast<int>(lin & (ngroups - 1));
+    }
+    if constexpr (!SPEC) job = uload(P.bperm + P.a0 + job) - static_cast<int>(P.a0);  // A-job within the chunk
+    const long goff = static_cast<long>(k1) << LG;
+    const double2* in = P.inter1 + static_cast<long>(job) * P.n + goff;
+    double2 v[16];
+#pragma unroll
+    for (int m = 0; m < 16; ++m) v[m] = vload(in + m * NT, threadIdx.x);
+    const long bstride = (1L << LG) - 1;
+    group_passes<LG, 0, false>(v, buf, P.twB + static_cast<long>(k1) * bstride, 1 << LG);
+    if constexpr (SPEC) {
+        double2* out = P.spec + static_cast<long>(job) * P.n + goff;
+#pragma unroll
+        for (int m = 0; m < 16; ++m) vstore(out + m * NT, threadIdx.x, v[m]);
+        return;
+    }
+    double2 x[16];
+#pragma unroll
+    for (int m = 0; m < 16; ++m) x[m] = v[m];
+    const unsigned need = static_cast<unsigned>(P.Tq);
+    const double inv_n = 1.0 / static_cast<double>(P.n);
+    const int pend = uload(P.ajob_start + P.a0 + job + 1);
+    for (int p = uload(P.ajob_start + P.a0 + job); p < pend; ++p) {
+        int i, j, k;
+        decode_triple(uload(P.job_tri + p), P.nf, i, j, k);
+        const int bF = uload(P.mirror + j);
+        const int mask = __builtin_amdgcn_readfirstlane(P.job_mask[p]);
+        for (int path = 0; path < 2; ++path) {
+            if (!(mask & (1 << path))) continue;
+            const double2* sp = P.spec + static_cast<long>(path == 0 ? 2 * bF : 2 * j + 1) * P.n + goff;
+#pragma unroll
+            for (int m = 0; m < 16; ++m) v[m] = vload(sp + m * NT, threadIdx.x);
+#pragma unroll
+            for (int m = 0; m < 16; ++m) v[m] = cmul(x[m], v[m]);
+            __syncthreads();  // the previous transform's LDS reads are done
+            // loaded anew for every product: kept over the loop, the passes'
+            // twiddles would take over 200 registers
+            long zero = 0;
+            asm volatile("" : "+s"(zero));
+            group_passes<LG, 0, true>(v, buf, P.twStd + zero, need);
+            if (P.a == 0) {  // the whole inverse: no phase C
+                double2* out = P.conv + (path * P.cconv + (p - P.comb0)) * P.T;
+#pragma unroll
+                for (int m = 0; m < 16; ++m) {
+                    const unsigned t = threadIdx.x + m * NT;
+                    const double2 y = cscale(v[m], inv_n);
+                    if (t < need) vstore(out + m * NT, threadIdx.x, make_double2(P.dt * y.x, P.dt * y.y));
+                }
+            } else {
+                double2* out = P.inter2 + (((path * static_cast<long>(P.njobs) + (p - P.job0)) << P.a) + k1) * P.Tq;
+#pragma unroll
+                for (int m = 0; m < 16; ++m) {
+                    const unsigned t = threadIdx.x + m * NT;
+                    if (t < need) vstore(out + m * NT, threadIdx.x, v[m]);
+                }
+            }
+        }
+    }
+}
+
+template <int LG>
+static void launch_group_b_lg(const FcrArgs& P, long njobs, bool spec, hipStream_t st) {
+    const long total = njobs << P.a;
+    const unsigned blocks = static_cast<unsigned>(P.a >= 3 ? total : ((total + 7) / 8) * 8);
+    if (spec)
+        hipLaunchKernelGGL((k_group_b<LG, true>), dim3(blocks), dim3(Group<LG>::kNT), 0, st, P, njobs);
+    else
+        hipLaunchKernelGGL((k_group_b<LG, false>), dim3(blocks), dim3(Group<LG>::kNT), 0, st, P, njobs);
+}
+
+void launch_group_b(const FcrArgs& P, long njobs, bool spec, hipStream_t st) {
+    static_assert(kGroupBitsMin == 10 && kGroupBitsMax == 11, "one case per group size");
+    if (P.b == 10)
+        launch_group_b_lg<10>(P, njobs, spec, st);
+    else
+        launch_group_b_lg<11>(P, njobs, spec, st);
+}
+
+// Phase C on groups: the inverse's last a stages of the columns
+// {t = q mod 2^b}, NP = ceil(T / 2^b) kept rows each, from the 2^a group
+// values of a column.  A node of stage b + l is the DFT of the classes
+// k1 = r mod 2^(a-l); its value at t is E +/- w O over the classes r and
+// r + 2^(a-l) one stage below, w the stage's twiddle at t mod 2^(b+l-1).
+// Only the values that feed kept times are formed: min(2^l, NP) per node.
+//
+// A thread runs the first four stages of one subtree of 16 classes in
+// registers (16 reads in flight, coalesced over the columns); for a > 4 the
+// 2^(a-4) subtrees of a column sit in one workgroup and finish through LDS,
+// where every sign is + (2^4 >= NP).
+template <int A1>
+__global__ __launch_bounds__(A1 == 4 ? 1024 : 256) void k_group_c(FcrArgs P, int lgS, int lgQ, int NP) {
+    constexpr int R = 1 << A1;
+    extern __shared__ double2 nodes[];  // [2^lgS subtrees][NP][2^lgQ columns]
+    const int jp = blockIdx.x, path = jp / P.njobs, job = jp % P.njobs;
+    const int mask = P.job_mask[P.job0 + job];
+    if (!(mask & (1 << path))) return;
+    const int col = threadIdx.x & ((1 << lgQ) - 1), sub = threadIdx.x >> lgQ;
+    const long q = (static_cast<long>(blockIdx.y) << lgQ) + col;
+    const bool live = q < P.Tq;
+    const long b2 = 1L << P.b;
+    double2 v[R];
+    if (live) {
+        const double2* src = P.inter2 + ((static_cast<long>(jp) << P.a) + sub) * P.Tq + q;
+        const long step = P.Tq << lgS;
+#pragma unroll
+        for (int m = 0; m < R; ++m) v[m] = src[m * step];
+        // stage l: y[p] of node m from nodes m and m + R >> l, p < min(2^l, NP)
+        // rows; node m's rows sit at v[m + (R >> l) p]
+#pragma unroll
+        for (int l = 1; l <= A1; ++l) {
+            const int h = R >> l, rows = 1 << (l - 1);  // nodes after, rows per node before
+            const double2* tw = P.twStd + (static_cast<long>(rows) << P.b) - 1;
+            double2 y[R];
+#pragma unroll
+            for (int p = 0; p < rows; ++p) {
+                if (p < NP) {
+                    const double2 w = cconj(tw[q + p * b2]);
+                    const bool hi = p + rows < NP;
+#pragma unroll
+                    for (int m = 0; m < h; ++m) {
+                        const double2 E = v[m + 2 * h * p], x = cmul(w, v[m + h + 2 * h * p]);
+                        y[m + h * p] = cadd(E, x);
+                        if (hi) y[m + h * (p + rows)] = csub(E, x);
+                    }
+                }
+            }
+#pragma unroll
+            for (int m = 0; m < R; ++m) v[m] = y[m];
+        }
+    }
+    const double inv_n = 1.0 / static_cast<double>(P.n);
+    double2* out = P.conv + (path * P.cconv + (P.job0 + job - P.comb0)) * P.T;
+    if (lgS == 0) {
+        if (live)
+#pragma unroll
+            for (int p = 0; p < R; ++p) {
+                const long t = q + p * b2;
+                if (p < NP && t < P.T) {
+                    const double2 y = cscale(v[p], inv_n);
+                    out[t] = make_double2(P.dt * y.x, P.dt * y.y);
+                }
+            }
+        return;
+    }
+    if (live)
+#pragma unroll
+        for (int p = 0; p < R; ++p)
+            if (p < NP) nodes[((sub * NP + p) << lgQ) + col] = v[p];
+    __syncthreads();
+    const int rows = NP << lgQ;  // values per subtree
+    const int nt = 1 << (lgS + lgQ);
+    for (int l = 1; l <= lgS; ++l) {
+        const int h = 1 << (lgS - l);  // nodes after this stage
+        const double2* tw = P.twStd + (b2 << (A1 + l - 1)) - 1;
+        for (int e = threadIdx.x; e < h * rows; e += nt) {
+            const int m = e / rows, rest = e - m * rows;
+            const long c = (static_cast<long>(blockIdx.y) << lgQ) + (rest & ((1 << lgQ) - 1));
+            const long t = c + (rest >> lgQ) * b2;
+            if (c >= P.Tq || t >= P.T) continue;
+            const double2 E = nodes[e], x = cmul(cconj(tw[t]), nodes[e + h * rows]);
+            const double2 y = cadd(E, x);
+            if (l < lgS) {
+                nodes[e] = y;
+            } else {
+                const double2 z = cscale(y, inv_n);
+                out[t] = make_double2(P.dt * z.x, P.dt * z.y);
+            }
+        }
+        __syncthreads();
+    }
+}
+
+// Columns and subtrees of a workgroup: 256 threads, 32 columns (512 B runs)
+// at least.
+static int group_c_cols(int lgS) { return lgS <= 3 ? 8 - lgS : 5; }
+
+bool group_c_fits(const FcrArgs& P) {
+    const long NP = (P.T + (1L << P.b) - 1) >> P.b;
+    if (P.a <= 4) return true;
+    const int lgS = P.a - 4;
+    return lgS <= 5 && NP <= 16 && (NP << (lgS + group_c_cols(lgS) + 4)) <= 64 * 1024;
+}
+
+void launch_group_c(const FcrArgs& P, hipStream_t st) {
+    const int A1 = P.a < 4 ? P.a : 4, lgS = P.a - A1, lgQ = group_c_cols(lgS);
+    const int NP = static_cast<int>((P.T + (1L << P.b) - 1) >> P.b);
+    const std::size_t lds = lgS ? (static_cast<std::size_t>(NP) << (lgS + lgQ)) * sizeof(double2) : 0;
+    const dim3 grid(static_cast<unsigned>(2 * P.njobs), static_cast<unsigned>((P.Tq + (1L << lgQ) - 1) >> lgQ));
+    const dim3 block(1u << (lgS + lgQ));
+    switch (A1) {
+        case 0: hipLaunchKernelGGL(k_group_c<0>, grid, block, lds, st, P, lgS, lgQ, NP); break;
+        case 1: hipLaunchKernelGGL(k_group_c<1>, grid, block, lds, st, P, lgS, lgQ, NP); break;
+        case 2: hipLaunchKernelGGL(k_group_c<2>, grid, block, lds, st, P, lgS, lgQ, NP); break;
+        case 3: hipLaunchKernelGGL(k_group_c<3>, grid, block, lds, st, P, lgS, lgQ, NP); break;
+        default: hipLaunchKernelGGL(k_group_c<4>, grid, block, lds, st, P, lgS, lgQ, NP); break;
+    }
+}
+
+}  // namespace taco_engine

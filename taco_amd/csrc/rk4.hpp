@@ -1,0 +1,99 @@
+// rk4.hpp — kernel arguments and launches of the RK4 recursions and their
+// reverse (rk4.hip).
+#pragma once
+
+#include "fcr_device.hpp"
+
+namespace taco_engine {
+
+constexpr int kRkBlock = 256;  // threads of the general RK4 kernels
+
+// Largest RK4 workgroup: the row-group path at D = 64.
+constexpr int kRkBlockMax = 512;
+
+// LDS of the RK4 workgroups: vectors of D, then generators staged nstage at
+// a time (column stride D + 1) within the 160 KiB of a CU.
+constexpr std::size_t kRkLds = 160 * 1024;
+
+// L0 cotangent parts a thread of the reverse walk carries in registers.
+constexpr int kRkCarry = 16;
+
+template <int DT>
+struct RowGroup {
+    static constexpr int G = DT <= 16 ? 4 : 8;   // lanes per output element
+    static constexpr int R = 64 / G;             // output elements per wave
+    static constexpr int W = (DT + R - 1) / R;   // waves
+    static constexpr int CK = (DT + G - 1) / G;  // terms per lane
+    static constexpr int S = DT <= 16 ? 4 : 3;   // generator ring slots (forward)
+    static constexpr int SA = 3;                 // ring slots of the reverse walk
+};
+
+// Threads of a row-group workgroup for D (0 when D has no row-group path).
+__host__ __device__ constexpr int rk4_rows_threads(int D) {
+    return D == 4 ? 64 * RowGroup<4>::W
+         : D == 9 ? 64 * RowGroup<9>::W
+         : D == 16 ? 64 * RowGroup<16>::W
+         : D == 25 ? 64 * RowGroup<25>::W
+         : D == 36 ? 64 * RowGroup<36>::W
+         : D == 49 ? 64 * RowGroup<49>::W
+         : D == 64 ? 64 * RowGroup<64>::W
+         : 0;
+}
+
+// Many independent systems, one workgroup each, in a single launch.
+struct Rk4Sys {
+    const double2* Ls;   // [steps + 1][D x D]
+    int nstage;          // generators staged in LDS at a time (0: read from global)
+    const double2* r0;   // [D]
+    double2* r;          // [D] final vector
+    double2* samples;    // [steps + 1][D]
+    long steps;
+    double dt;
+    int D;
+    const double2* Lh = nullptr;  // [steps][D x D] midpoints (large D), else formed on the fly
+};
+
+struct Rk4AdjArgs {
+    const double2* Ls;    // [steps + 1][D * D] generators
+    const double2* ck;    // [ceil(steps / K)][D] checkpoint states r_{qK}
+    const double2* gbar;  // [steps + 1][D] dLoss/dr_n
+    double2* Lbar;        // [steps + 1][D * D]
+    double2* seg;         // [steps][4][D] state r_n and stage points u1, u2, u3 of step n
+    double2* r0bar;       // [D]
+    long steps;
+    int D;
+    int K;
+    double dt;
+    int nstage;
+    const double2* LsH = nullptr;  // [steps + 1][D * D] conjugate transposes (walk without staging)
+    const double2* LhH = nullptr;  // [steps][D * D] their midpoints (null: formed on the fly)
+    double2* vec = nullptr;        // [steps][4][D] kb1..kb4 of every step (Lbar formed by k_rk4_lbar)
+};
+
+// Raises the kernels' dynamic LDS limit to kRkLds on the current device.
+hipError_t rk4_set_lds_limits();
+
+// One system, row-group path (rk4_rows_threads(D) > 0).
+void launch_rk4_rows(int D, const double2* Ls, long steps, double2* r, double dt, long every, double2* samples,
+                     long* nsamples, hipStream_t st);
+// One system, general path.
+void launch_rk4(int D, const double2* Ls, const double2* Lh, long steps, double2* r, double dt, long every,
+                double2* samples, long* nsamples, int nstage, int block, std::size_t lds, hipStream_t st);
+// nsys systems, one workgroup each.
+void launch_rk4_batch(unsigned nsys, const Rk4Sys* sys, int block, std::size_t lds, hipStream_t st);
+// out[n] = (L[n] + L[n + 1]) / 2, n < count.
+void launch_midpoints(const double2* L, long count, long D2, double2* out, hipStream_t st);
+// dst[t] = src[t]^H, t < count.
+void launch_conj_transpose(const double2* src, double2* dst, int D, long count, hipStream_t st);
+
+// Reverse of one tape (A) or of ntapes tapes of one D, steps and K (As on
+// the device): the segments' recompute, the walk, the generator cotangents.
+void launch_rk4_recompute(const Rk4AdjArgs& A, bool rows, unsigned nseg, std::size_t lds, hipStream_t st);
+void launch_rk4_walk(const Rk4AdjArgs& A, bool rows, std::size_t lds, hipStream_t st);
+void launch_rk4_lbar(const Rk4AdjArgs& A, hipStream_t st);
+void launch_rk4_recompute_multi(const Rk4AdjArgs* As, unsigned ntapes, int D, bool rows, unsigned nseg,
+                                std::size_t lds, hipStream_t st);
+void launch_rk4_walk_multi(const Rk4AdjArgs* As, unsigned ntapes, int D, bool rows, std::size_t lds, hipStream_t st);
+void launch_rk4_lbar_multi(const Rk4AdjArgs* As, unsigned ntapes, int D, long steps, hipStream_t st);
+
+}  // namespace taco_engine

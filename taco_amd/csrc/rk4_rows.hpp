@@ -1,7 +1,7 @@
 // Row-group RK4 kernels bodies for D = N^2 with N = 2..8 (rk4_dense.cpp:133-160,
 // 246-320 for the step; the reverse walk has no reference counterpart).
 //
-// Included by engine.hip inside namespace taco_engine, after the complex
+// Included by rk4.hip inside namespace taco_engine, after the complex
 // helpers.  G consecutive lanes own one output element of every
 // matrix-vector product: lane g sums the terms k = g, g + G, g + 2G, ... in
 // order with fused multiply-adds, and the G partial sums are combined by a
@@ -14,28 +14,6 @@
 // one barrier per RK4 stage.  Forward, batched forward and segment
 // recompute share rk4_rows, so their states are identical bit for bit.
 #pragma once
-
-template <int DT>
-struct RowGroup {
-    static constexpr int G = DT <= 16 ? 4 : 8;   // lanes per output element
-    static constexpr int R = 64 / G;             // output elements per wave
-    static constexpr int W = (DT + R - 1) / R;   // waves
-    static constexpr int CK = (DT + G - 1) / G;  // terms per lane
-    static constexpr int S = DT <= 16 ? 4 : 3;   // generator ring slots (forward)
-    static constexpr int SA = 3;                 // ring slots of the reverse walk
-};
-
-// Threads of a row-group workgroup for D (0 when D has no row-group path).
-__host__ __device__ constexpr int rk4_rows_threads(int D) {
-    return D == 4 ? 64 * RowGroup<4>::W
-         : D == 9 ? 64 * RowGroup<9>::W
-         : D == 16 ? 64 * RowGroup<16>::W
-         : D == 25 ? 64 * RowGroup<25>::W
-         : D == 36 ? 64 * RowGroup<36>::W
-         : D == 49 ? 64 * RowGroup<49>::W
-         : D == 64 ? 64 * RowGroup<64>::W
-         : 0;
-}
 
 // One 64-bit value from another lane of the same row of 16 (DPP control CTRL).
 template <int CTRL>

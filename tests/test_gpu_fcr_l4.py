@@ -367,6 +367,30 @@ def test_fft_tile_configs_bitwise_identical(orc, cfg):
     assert max_rel_err(got, oref)[0] <= TOL
 
 
+@pytest.mark.parametrize("Nt,keep", [
+    (512, 1), (512, 512),            # one group of 2^10: phase B stores the convolutions
+    (513, 513), (1024, 300),         # Nfft 2^11
+    (1025, 512), (1025, 513), (1025, 1025),
+    (9001, 1023), (9001, 1024), (9001, 1025), (9001, 2048), (9001, 2049),  # 2^15: 16 or 32 groups, 1-3 rows
+    (9001, 9001),                    # every row kept
+    (40000, 5000),                   # 2^17: subtrees through LDS
+])
+def test_fft_groups_equal_tiles(Nt, keep, monkeypatch):
+    """Groups of 2^10 and 2^11 values (phases B and C in registers) and the
+    default choice give the tile kernels' F and C bit for bit."""
+    w = W.spin_boson(Nt=Nt, tmax=min(Nt - 1, 300))
+    out = {}
+    for shape in ("0", "2", "3", None):
+        if shape is None:
+            monkeypatch.delenv("TACO_FFT_TILE")
+        else:
+            monkeypatch.setenv("TACO_FFT_TILE", shape)
+        out[shape] = taco_amd.compute_triple_kernels(w.system, w.gamma, w.dt, keep=keep)
+    for shape in ("2", "3", None):
+        assert np.array_equal(out[shape].F, out["0"].F)
+        assert np.array_equal(out[shape].C, out["0"].C)
+
+
 @pytest.mark.parametrize("case", ["gue_pair", "d8"])
 def test_l4_factorised_matches_oracle(orc, case, monkeypatch):
     """The factorised L4 (O(N^5 + N^3 nf) per time; the kernel for N > 8)
