@@ -2064,6 +2064,10 @@ static void launch_phase(Phase ph, const FcrArgs& P, bool group, long njobs, hip
         launch_group_b(P, njobs, ph == PH_B_SPEC, st);
         return;
     }
+    if (group && (ph == PH_A_TRIPLE || ph == PH_A_SPEC) && column_a_fits(P)) {
+        launch_column_a(P, njobs, ph == PH_A_SPEC, st);
+        return;
+    }
     if (ph == PH_C) {
         if (group && P.a == 0) return;  // phase B stored the convolutions
         if (group_c_fits(P)) {
@@ -4458,6 +4462,7 @@ int taco_ctx_create(int device, taco_ctx** out) {
                                  hipMemcpyHostToDevice));
         HIP_OK(hipEventCreate(&c->ev0));
         HIP_OK(hipEventCreate(&c->ev1));
+        HIP_OK(group_fft_set_table(cr_table()));
         HIP_OK(rk4_set_lds_limits());
         *out = c.release();
     });

@@ -17,6 +17,8 @@
 // reads at 4.3-4.8 TB/s, the rate of a plain copy.
 #include "group_fft.hpp"
 
+#include "cr_sincos.hpp"
+
 #pragma clang fp contract(off)
 
 namespace taco_engine {
@@ -401,6 +403,194 @@ void launch_group_c(const FcrArgs& P, hipStream_t st) {
         case 2: hipLaunchKernelGGL(k_group_c<2>, grid, block, lds, st, P, lgS, lgQ, NP); break;
         case 3: hipLaunchKernelGGL(k_group_c<3>, grid, block, lds, st, P, lgS, lgQ, NP); break;
         default: hipLaunchKernelGGL(k_group_c<4>, grid, block, lds, st, P, lgS, lgQ, NP); break;
+    }
+}
+
+// ---------------------------------------------------------------------------
+// Phase A in registers: forward stages 1..a, a <= 8, of the columns
+// {t = r mod 2^b}, a thread per column (a <= 4) or 2^(a-4) threads of 16
+// values with one LDS exchange.  At most the lower half of a column is
+// nonzero (Nin <= n / 2), so stage 1 copies and the upper half is never read.
+// Consecutive threads hold consecutive columns: runs of 256 B and more both
+// ways.
+// ---------------------------------------------------------------------------
+__constant__ double c_crtab_a[4 * taco_cr::kTabN];  // table of sincos_cr
+
+hipError_t group_fft_set_table(const double* cr_tab) {
+    return hipMemcpyToSymbol(HIP_SYMBOL(c_crtab_a), cr_tab, sizeof(double) * 4 * taco_cr::kTabN, 0,
+                             hipMemcpyHostToDevice);
+}
+
+template <int A>
+struct ColA {
+    static constexpr int L1 = A < 4 ? A : 4;   // stages of pass 1
+    static constexpr int L2 = A - L1;          // stages of pass 2 (0: none)
+    static constexpr int V = 1 << L1;
+    static constexpr int H = A == 0 ? 1 : V / 2;
+    static constexpr int TPC = 1 << L2;        // threads per column
+    static constexpr int COLS = 256 / TPC;     // columns of a workgroup
+};
+
+// The column's stages on x[0..H) (position u0 + m 2^L2, u0 = the thread's
+// place in its column); stores out[k 2^b + r].
+template <int A>
+__device__ __forceinline__ void column_stages(double2 (&x)[ColA<A>::V], double2* buf, const double2* __restrict__ tw,
+                                              double2* out, int b) {
+    using C = ColA<A>;
+    constexpr int V = C::V;
+    // pass 1: stage 1 has a zero upper half, stages 2..L1 as in Pass (k = 0)
+    if constexpr (A > 0) {
+#pragma unroll
+        for (int m = 0; m < V / 2; ++m) x[m + V / 2] = x[m];
+#pragma unroll
+        for (int i = 1; i < C::L1; ++i) {
+            const int h = V >> (i + 1);
+            double2 y[V];
+#pragma unroll
+            for (int j = 0; j < (1 << i); ++j) {
+                const double2 t = uload2(tw + (1 << i) - 1 + j);
+#pragma unroll
+                for (int m = 0; m < h; ++m) {
+                    const double2 E = x[m + 2 * h * j], z = cmul(t, x[m + h + 2 * h * j]);
+                    y[m + h * j] = cadd(E, z);
+                    y[m + h * j + V / 2] = csub(E, z);
+                }
+            }
+#pragma unroll
+            for (int m = 0; m < V; ++m) x[m] = y[m];
+        }
+    }
+    if constexpr (C::L2 == 0) {
+#pragma unroll
+        for (int k = 0; k < V; ++k) out[static_cast<long>(k) << b] = x[k];
+    } else {
+        constexpr int R = C::TPC, SETS = 16 / R;
+        const int col = threadIdx.x % C::COLS, u = threadIdx.x / C::COLS;
+        __syncthreads();  // the previous column's reads are done
+#pragma unroll
+        for (int j = 0; j < 16; ++j) buf[(j * R + u) * C::COLS + col] = x[j];
+        __syncthreads();
+        // pass 2: sets k = u + R s of R positions k R + m, stages 5..a
+#pragma unroll
+        for (int s = 0; s < SETS; ++s) {
+            const int k = u + R * s;
+            double2 v[R];
+#pragma unroll
+            for (int m = 0; m < R; ++m) v[m] = buf[(k * R + m) * C::COLS + col];
+#pragma unroll
+            for (int i = 0; i < C::L2; ++i) {
+                const int h = R >> (i + 1);
+                double2 y[R];
+#pragma unroll
+                for (int j = 0; j < (1 << i); ++j) {
+                    const double2 t = tw[(16 << i) - 1 + k + 16 * j];
+#pragma unroll
+                    for (int m = 0; m < h; ++m) {
+                        const double2 E = v[m + 2 * h * j], z = cmul(t, v[m + h + 2 * h * j]);
+                        y[m + h * j] = cadd(E, z);
+                        y[m + h * j + R / 2] = csub(E, z);
+                    }
+                }
+#pragma unroll
+                for (int m = 0; m < R; ++m) v[m] = y[m];
+            }
+#pragma unroll
+            for (int j = 0; j < R; ++j) out[static_cast<long>(k + 16 * j) << b] = v[j];
+        }
+    }
+}
+
+// One workgroup per (Omega-class piece, columns): the phases of its columns
+// are formed once and applied to the Gamma column g_i of every A-job of the
+// piece inside the chunk.  SPEC: the spectra's inputs g_b (even job) and
+// conj g_b (odd job) instead.
+template <int A, bool SPEC>
+__global__ __launch_bounds__(256) void k_column_a(FcrArgs P) {
+    using C = ColA<A>;
+    extern __shared__ double2 buf[];  // [2^A][COLS] when A > 4
+    int cj, cb;
+    xcd_map(blockIdx.x, ((1 << P.b) + C::COLS - 1) / C::COLS, cj, cb);
+    const int u = threadIdx.x / C::COLS;
+    const long r = static_cast<long>(cb) * C::COLS + threadIdx.x % C::COLS;
+    const long stride = static_cast<long>(C::TPC) << P.b;       // between a thread's positions
+    const long t0 = r + (static_cast<long>(u) << P.b);
+    if constexpr (SPEC) {
+        const double2* src = P.gamma + static_cast<long>(cj >> 1) * P.Nt;
+        double2 x[C::V];
+#pragma unroll
+        for (int m = 0; m < C::H; ++m) {
+            const long t = t0 + m * stride;
+            x[m] = t < P.Nin ? src[t] : make_double2(0.0, 0.0);
+            if (cj & 1) x[m].y = -x[m].y;
+        }
+        column_stages<A>(x, buf, P.twStd, P.inter1 + static_cast<long>(cj) * P.n + r, P.b);
+    } else {
+        const int cls = P.cls0 + cj;
+        const long abeg = max(static_cast<long>(uload(P.cls_start + cls)), P.a0);
+        const long aend = min(static_cast<long>(uload(P.cls_start + cls + 1)), P.a0 + P.na);
+        if (abeg >= aend) return;
+        const int pfirst = uload(P.ajob_start + abeg);
+        int i, j, k;
+        decode_triple(uload(P.job_tri + pfirst), P.nf, i, j, k);
+        const double omega = (uload(P.omegas + i) + uload(P.omegas + j)) + uload(P.omegas + k);
+        const double2* prow =
+            P.ph_tab ? P.ph_tab + static_cast<long>(uload(P.job_row + pfirst)) * P.ph_len : nullptr;
+        double2 ph[C::H];
+        if (prow) {
+#pragma unroll
+            for (int m = 0; m < C::H; ++m) {
+                const long t = t0 + m * stride;
+                ph[m] = t < P.Nin ? cconj(prow[t]) : make_double2(0.0, 0.0);
+            }
+        } else {
+#pragma unroll
+            for (int m = 0; m < C::H; ++m) {
+                const long t = t0 + m * stride;
+                double s, c;
+                taco_cr::sincos_cr(omega * (static_cast<double>(t) * P.dt), &s, &c, c_crtab_a);
+                ph[m] = make_double2(c, -s);
+            }
+        }
+        for (long aj = abeg; aj < aend; ++aj) {
+            const int gi = uload(P.job_tri + uload(P.ajob_start + aj)) / (P.nf * P.nf);
+            const double2* src = P.gamma + static_cast<long>(gi) * P.Nt;
+            double2 x[C::V];
+#pragma unroll
+            for (int m = 0; m < C::H; ++m) {
+                const long t = t0 + m * stride;
+                x[m] = t < P.Nin ? cmul(src[t], ph[m]) : make_double2(0.0, 0.0);
+            }
+            column_stages<A>(x, buf, P.twStd, P.inter1 + (aj - P.a0) * P.n + r, P.b);
+        }
+    }
+}
+
+bool column_a_fits(const FcrArgs& P) {
+    return P.a <= 8 && P.b >= 8 && 2 * P.Nin <= P.n;
+}
+
+template <int A>
+static void launch_column_a_n(const FcrArgs& P, long njobs, bool spec, hipStream_t st) {
+    using C = ColA<A>;
+    const std::size_t lds = C::L2 ? (static_cast<std::size_t>(C::COLS) << A) * sizeof(double2) : 0;
+    const dim3 grid(static_cast<unsigned>(njobs * ((1L << P.b) / C::COLS)));
+    if (spec)
+        hipLaunchKernelGGL((k_column_a<A, true>), grid, dim3(256), lds, st, P);
+    else
+        hipLaunchKernelGGL((k_column_a<A, false>), grid, dim3(256), lds, st, P);
+}
+
+void launch_column_a(const FcrArgs& P, long njobs, bool spec, hipStream_t st) {
+    switch (P.a) {
+        case 0: launch_column_a_n<0>(P, njobs, spec, st); break;
+        case 1: launch_column_a_n<1>(P, njobs, spec, st); break;
+        case 2: launch_column_a_n<2>(P, njobs, spec, st); break;
+        case 3: launch_column_a_n<3>(P, njobs, spec, st); break;
+        case 4: launch_column_a_n<4>(P, njobs, spec, st); break;
+        case 5: launch_column_a_n<5>(P, njobs, spec, st); break;
+        case 6: launch_column_a_n<6>(P, njobs, spec, st); break;
+        case 7: launch_column_a_n<7>(P, njobs, spec, st); break;
+        default: launch_column_a_n<8>(P, njobs, spec, st); break;
     }
 }
 
