@@ -2848,6 +2848,9 @@ struct BatchSys {
 struct BatchRun {
     std::vector<std::unique_ptr<BatchSys>> sys;
     DevBuf rkargs;
+    DevBuf rkchunks;                 // chunk products and first states of the chunked systems
+    std::map<int, long> rk_chunked;  // D -> longest chunked run
+    bool rk_plain = false;           // some system runs unchunked
     long nrk = 0;
     std::size_t rk_lds = 0;
     int rk_block = 64;  // raised to the workgroup size each system needs
@@ -2930,7 +2933,10 @@ static void batch_enqueue(taco_ctx* c, BatchRun& B) {
     for (auto& s : B.sys) batch_enqueue_system(c, *s);
     if (B.nrk) {
         timed(c, K_RK4, B.rk_bytes, [&] {
-            launch_rk4_batch(static_cast<unsigned>(B.nrk), B.rkargs.as<Rk4Sys>(), B.rk_block, B.rk_lds, c->stream);
+            for (const auto& [D, steps] : B.rk_chunked)
+                launch_rk4_chunked(D, B.rkargs.as<Rk4Sys>(), Rk4Sys{}, static_cast<unsigned>(B.nrk), steps, c->stream);
+            if (B.rk_plain)
+                launch_rk4_batch(static_cast<unsigned>(B.nrk), B.rkargs.as<Rk4Sys>(), B.rk_block, B.rk_lds, c->stream);
         });
         HIP_OK(hipGetLastError());
     }
@@ -3004,11 +3010,33 @@ static const double2* rk4_midpoints(taco_ctx* c, DevBuf& buf, const double2* Ls,
     return buf.as<double2>();
 }
 
+// Places a chunked run's products and first states at `base`.
+static void rk4_set_chunks(Rk4Sys& S, double2* base) {
+    S.q = base;
+    S.xs = base + rk4_chunk_values(S.D, S.steps) - static_cast<std::size_t>((S.steps + kRkChunk - 1) / kRkChunk) * S.D;
+}
+
 static void rk4_launch(taco_ctx* ctx, const double2* dLs, const double2* dLh, std::size_t steps, int D, double2* dr,
                        double dt, std::size_t every, double2* dsamples, long* dns) {
     // algorithmic bytes: every generator read once, every sample written once
     const double gen_bytes = static_cast<double>(steps + 1) * D * D * 16.0 * (dLh ? 2.0 : 1.0);
     const double rk_bytes = gen_bytes + (dsamples ? static_cast<double>(steps / every + 2) * D * 16.0 : 0.0);
+    if (!dLh && rk4_chunked(D, static_cast<long>(steps))) {
+        ctx->rkmid.ensure(rk4_chunk_values(D, static_cast<long>(steps)) * 16);
+        Rk4Sys S{};
+        S.Ls = dLs;
+        S.r0 = S.r = dr;
+        S.samples = dsamples;
+        S.steps = static_cast<long>(steps);
+        S.dt = dt;
+        S.D = D;
+        S.every = static_cast<long>(every);
+        S.nsamples = dns;
+        rk4_set_chunks(S, ctx->rkmid.as<double2>());
+        timed(ctx, K_RK4, rk_bytes, [&] { launch_rk4_chunked(D, nullptr, S, 1, S.steps, ctx->stream); });
+        HIP_OK(hipGetLastError());
+        return;
+    }
     if (!dLh && rk4_rows_threads(D) > 0) {
         timed(ctx, K_RK4, rk_bytes, [&] {
             launch_rk4_rows(D, dLs, static_cast<long>(steps), dr, dt, static_cast<long>(every), dsamples, dns,
@@ -3238,6 +3266,7 @@ struct RkRev {
     double2 *gb, *Lb, *seg, *rb;
     double2 *LsH = nullptr, *vec = nullptr;  // deferred walk: conjugate transposes, cotangent vectors
     double2* LhH = nullptr;                  // and their midpoints
+    double2 *q = nullptr, *lam = nullptr, *bv = nullptr;  // chunked walk
 };
 
 // The walk reads transposed generators and leaves Lbar to k_rk4_lbar when it
@@ -3255,6 +3284,7 @@ static bool rk_rev_deferred(const taco_tape& tp) {
 // The row-group walk (D = 4, 9, 16) stores kb1..kb4 per step and leaves
 // Lbar to k_rk4_lbar as well (TACO_RK4_DEFER=0: Lbar formed in the walk).
 static bool rk_rev_rows_deferred(const taco_tape& tp) {
+    if (rk4_chunked_walk(tp.N * tp.N, static_cast<long>(tp.steps))) return true;
     if (env_int("TACO_RK4_DEFER", 1) == 0) return false;
     const int D = tp.N * tp.N;
     return D == 4 || D == 9 || D == 16;
@@ -3263,6 +3293,9 @@ static bool rk_rev_rows_deferred(const taco_tape& tp) {
 static std::size_t rk_rev_values(const taco_tape& tp) {
     const std::size_t D = static_cast<std::size_t>(tp.N) * tp.N;
     const std::size_t base = tp.T * D + tp.T * D * D + 4 * tp.steps * D + D;
+    if (rk4_chunked_walk(static_cast<int>(D), static_cast<long>(tp.steps)))
+        return base + 4 * tp.steps * D + rk4_chunk_values(static_cast<int>(D), static_cast<long>(tp.steps)) +
+               (tp.steps + kRkChunk - 1) / kRkChunk * D;
     if (rk_rev_rows_deferred(tp)) return base + 4 * tp.steps * D;
     return rk_rev_deferred(tp) ? base + tp.T * D * D + 4 * tp.steps * D + tp.steps * D * D : base;
 }
@@ -3276,6 +3309,12 @@ static RkRev rk_rev_at(const taco_tape& tp, double2* base) {
     b.rb = b.seg + 4 * tp.steps * D;
     if (rk_rev_rows_deferred(tp)) {
         b.vec = b.rb + D;
+        if (rk4_chunked_walk(static_cast<int>(D), static_cast<long>(tp.steps))) {
+            const std::size_t nch = (tp.steps + kRkChunk - 1) / kRkChunk;
+            b.q = b.vec + 4 * tp.steps * D;
+            b.lam = b.q + nch * D * D;
+            b.bv = b.lam + nch * D;
+        }
     } else if (rk_rev_deferred(tp)) {
         b.LsH = b.rb + D;
         b.vec = b.LsH + tp.T * D * D;
@@ -3313,6 +3352,9 @@ static RkRevShape rk_rev_shape(const taco_tape& tp, const RkRev& b) {
     R.LsH = b.LsH;
     R.vec = b.vec;
     R.LhH = b.LhH;
+    R.q = b.q;
+    R.lam = b.lam;
+    R.bv = b.bv;
     sh.carry = D2 <= static_cast<std::size_t>(kRkCarry) * kBlock;
     sh.nseg = (steps + K - 1) / K;
     const int Di = static_cast<int>(D);
@@ -3349,7 +3391,10 @@ static void rk_rev_run(taco_tape& tp, const RkRev& b) {
     timed(c, K_RK4, sh.bytes, [&] {
         // every segment's states and stage points from its checkpoint, all segments at once
         launch_rk4_recompute(sh.Rf, sh.rows_f, static_cast<unsigned>(sh.nseg), sh.lds_f, c->stream);
-        launch_rk4_walk(sh.R, sh.rows_b, sh.lds_b, c->stream);
+        if (b.q)
+            launch_rk4_chunked_walk(Di, nullptr, sh.R, 1, sh.R.steps, c->stream);
+        else
+            launch_rk4_walk(sh.R, sh.rows_b, sh.lds_b, c->stream);
         if (b.vec) launch_rk4_lbar(sh.R, c->stream);
     });
     HIP_OK(hipGetLastError());
@@ -4259,12 +4304,22 @@ static void mtape_forward(taco_mtape& mt, const taco_tape_set* in, double* const
             sys[s].Lh = m;
         }
     }
+    const bool chunked = rk4_chunked(Di, static_cast<long>(t0.steps));
+    if (chunked) {
+        const std::size_t per = rk4_chunk_values(Di, static_cast<long>(t0.steps));
+        mt.A->mid.ensure(S * per * 16);
+        for (std::size_t s = 0; s < S; ++s) rk4_set_chunks(sys[s], mt.A->mid.as<double2>() + s * per);
+    }
     mt.A->args.ensure(std::max(S * sizeof(Rk4Sys), 2 * S * sizeof(Rk4AdjArgs)));
     HIP_OK(hipMemcpyAsync(mt.A->args.p, sys.data(), S * sizeof(Rk4Sys), hipMemcpyHostToDevice, c->stream));
     const double rk_bytes = static_cast<double>(S) * ((t0.steps + 1) * D * D * 16.0 + (t0.steps + 1) * D * 16.0);
     timed(c, K_RK4, rk_bytes, [&] {
-        launch_rk4_batch(static_cast<unsigned>(S), mt.A->args.as<const Rk4Sys>(),
-                         rows_thr > 0 ? rows_thr : rk4_block(Di), lds, c->stream);
+        if (chunked)
+            launch_rk4_chunked(Di, mt.A->args.as<const Rk4Sys>(), Rk4Sys{}, static_cast<unsigned>(S),
+                               static_cast<long>(t0.steps), c->stream);
+        else
+            launch_rk4_batch(static_cast<unsigned>(S), mt.A->args.as<const Rk4Sys>(),
+                             rows_thr > 0 ? rows_thr : rk4_block(Di), lds, c->stream);
     });
     HIP_OK(hipGetLastError());
     for (std::size_t s = 0; s < S; ++s) tape_checkpoints(*mt.sets[s], samp + s * T * D);
@@ -4309,7 +4364,10 @@ static void mtape_adjoint(taco_mtape& mt, const double* const* samples_bar, doub
     timed(c, K_RK4, sh.bytes * static_cast<double>(S), [&] {
         const unsigned nt = static_cast<unsigned>(S);
         launch_rk4_recompute_multi(dargs, nt, Di, sh.rows_f, static_cast<unsigned>(sh.nseg), sh.lds_f, c->stream);
-        launch_rk4_walk_multi(dargs + S, nt, Di, sh.rows_b, sh.lds_b, c->stream);
+        if (rv[0].q)
+            launch_rk4_chunked_walk(Di, dargs + S, sh.R, nt, sh.R.steps, c->stream);
+        else
+            launch_rk4_walk_multi(dargs + S, nt, Di, sh.rows_b, sh.lds_b, c->stream);
         if (rv[0].vec) launch_rk4_lbar_multi(dargs + S, nt, Di, static_cast<long>(T) - 1, c->stream);
     });
     HIP_OK(hipGetLastError());
@@ -5253,6 +5311,21 @@ int taco_batch_create(taco_ctx* ctx, const taco_batch_system* systems, int nsys,
         B.nrk = static_cast<long>(rk.size());
         if (B.nrk) {
             if (B.rk_lds > kRkLds) throw Error(TACO_ERR_INVALID, "RK4 kernel supports D <= 1706");
+            std::size_t values = 0;
+            for (const Rk4Sys& r : rk)
+                if (rk4_chunked(r.D, r.steps)) values += rk4_chunk_values(r.D, r.steps);
+            B.rkchunks.ensure(values * 16);
+            double2* base = B.rkchunks.as<double2>();
+            for (Rk4Sys& r : rk) {
+                if (!rk4_chunked(r.D, r.steps)) {
+                    B.rk_plain = true;
+                    continue;
+                }
+                rk4_set_chunks(r, base);
+                base += rk4_chunk_values(r.D, r.steps);
+                long& longest = B.rk_chunked[r.D];
+                longest = std::max(longest, r.steps);
+            }
             B.rkargs.ensure(rk.size() * sizeof(Rk4Sys));
             HIP_OK(hipMemcpy(B.rkargs.p, rk.data(), rk.size() * sizeof(Rk4Sys), hipMemcpyHostToDevice));
         }

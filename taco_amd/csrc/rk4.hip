@@ -203,21 +203,6 @@ __device__ __forceinline__ void rk4_body(double2* sh, int nstage, const double2*
 
 #include "rk4_rows.hpp"
 
-// Row-group path for the sizes that have one (no separate midpoint series),
-// else the general path above.
-template <int DT>
-__device__ __forceinline__ void rk4_any(double2* sh, int nstage, const double2* Ls, const double2* Lh, long steps,
-                                        int D, const double2* r_in, double2* r_out, double dt, long every,
-                                        double2* samples, long* nsamples) {
-    if constexpr (DT != 0) {
-        if (!Lh) {
-            rk4_rows<DT, false>(sh, Ls, 0, steps, r_in, r_out, dt, every, samples, nsamples, nullptr);
-            return;
-        }
-    }
-    rk4_body<DT>(sh, nstage, Ls, Lh, steps, D, r_in, r_out, dt, every, samples, nsamples);
-}
-
 // One system on the row-group path (D = N^2, N = 2..8), 64 W threads.
 template <int DT>
 __global__ __launch_bounds__(64 * RowGroup<DT>::W) void k_rk4_rows(const double2* Ls, long steps, double2* r,
@@ -229,7 +214,7 @@ __global__ __launch_bounds__(64 * RowGroup<DT>::W) void k_rk4_rows(const double2
 
 // Calls f(std::integral_constant<int, D>) for a D with a row-group path.
 template <class F>
-static bool rows_dispatch(int D, F&& f) {
+__host__ __device__ inline bool rows_dispatch(int D, F&& f) {
     switch (D) {
         case 4: f(std::integral_constant<int, 4>{}); return true;
         case 9: f(std::integral_constant<int, 9>{}); return true;
@@ -253,9 +238,13 @@ __global__ __launch_bounds__(kRkBlock) void k_rk4(const double2* Ls, const doubl
 __global__ __launch_bounds__(kRkBlockMax) void k_rk4_batch(const Rk4Sys* sys) {
     extern __shared__ double2 sh[];
     const Rk4Sys S = sys[blockIdx.x];
-#define TACO_RK4_CALL(DT) rk4_any<DT>(sh, S.nstage, S.Ls, S.Lh, S.steps, S.D, S.r0, S.r, S.dt, 1, S.samples, nullptr)
-    TACO_RK4_DISPATCH(S.D, TACO_RK4_CALL)
-#undef TACO_RK4_CALL
+    if (S.q) return;  // chunked
+    // sizes with a row-group path have no separate midpoint series here
+    if (!rows_dispatch(S.D, [&](auto dc) {
+            constexpr int DT = decltype(dc)::value;
+            rk4_rows<DT, false>(sh, S.Ls, 0, S.steps, S.r0, S.r, S.dt, 1, S.samples, nullptr, nullptr);
+        }))
+        rk4_body<0>(sh, S.nstage, S.Ls, S.Lh, S.steps, S.D, S.r0, S.r, S.dt, 1, S.samples, nullptr);
 }
 
 // out[n] = (L[n] + L[n + 1]) / 2 elementwise for n < count (midpoint
@@ -403,13 +392,9 @@ __global__ __launch_bounds__(kRkBlock) void k_rk4_recompute(Rk4AdjArgs A) {
     extern __shared__ double2 sh[];
     const long sg = blockIdx.x;
     if (A.nstage >= 2) {
-#define TACO_RK4_CALL(DT) rk4_recompute_body<DT, true>(sh, A, sg)
-        TACO_RK4_DISPATCH(A.D, TACO_RK4_CALL)
-#undef TACO_RK4_CALL
+        rk4_recompute_body<0, true>(sh, A, sg);
     } else {
-#define TACO_RK4_CALL(DT) rk4_recompute_body<DT, false>(sh, A, sg)
-        TACO_RK4_DISPATCH(A.D, TACO_RK4_CALL)
-#undef TACO_RK4_CALL
+        rk4_recompute_body<0, false>(sh, A, sg);
     }
 }
 
@@ -560,22 +545,25 @@ __device__ __forceinline__ void rk4_adjoint_body(double2* sh, const Rk4AdjArgs& 
 template <int DT>
 __global__ __launch_bounds__(64) void k_rk4_adjoint_rows(Rk4AdjArgs A) {
     extern __shared__ double2 sh[];
+    const double2* lam = A.gbar + A.steps * DT;
     if (A.vec)
-        rk4_rows_adjoint<DT, Rk4AdjArgs, true>(sh, A);
+        rk4_rows_adjoint<DT, WALK_VEC>(sh, A, 0, A.steps, lam, A.r0bar);
     else
-        rk4_rows_adjoint<DT>(sh, A);
+        rk4_rows_adjoint<DT, WALK_LBAR>(sh, A, 0, A.steps, lam, A.r0bar);
 }
 
 __global__ __launch_bounds__(kRkBlock) void k_rk4_adjoint(Rk4AdjArgs A) {
     extern __shared__ double2 sh[];
     if (A.nstage >= 2) {
-#define TACO_RK4_CALL(DT) rk4_adjoint_body<DT, true>(sh, A)
-        TACO_RK4_DISPATCH(A.D, TACO_RK4_CALL)
-#undef TACO_RK4_CALL
+        switch (A.D) {  // 4, 9 and 16 have the row-group walk
+            case 25: rk4_adjoint_body<25, true>(sh, A); break;
+            case 36: rk4_adjoint_body<36, true>(sh, A); break;
+            case 49: rk4_adjoint_body<49, true>(sh, A); break;
+            case 64: rk4_adjoint_body<64, true>(sh, A); break;
+            default: rk4_adjoint_body<0, true>(sh, A); break;
+        }
     } else {
-#define TACO_RK4_CALL(DT) rk4_adjoint_body<DT, false>(sh, A)
-        TACO_RK4_DISPATCH(A.D, TACO_RK4_CALL)
-#undef TACO_RK4_CALL
+        rk4_adjoint_body<0, false>(sh, A);  // sizes to 64 always stage
     }
 }
 
@@ -648,13 +636,9 @@ __global__ __launch_bounds__(kRkBlock) void k_rk4_recompute_multi(const Rk4AdjAr
     const Rk4AdjArgs A = As[blockIdx.y];
     const long sg = blockIdx.x;
     if (A.nstage >= 2) {
-#define TACO_RK4_CALL(DT) rk4_recompute_body<DT, true>(sh, A, sg)
-        TACO_RK4_DISPATCH(A.D, TACO_RK4_CALL)
-#undef TACO_RK4_CALL
+        rk4_recompute_body<0, true>(sh, A, sg);
     } else {
-#define TACO_RK4_CALL(DT) rk4_recompute_body<DT, false>(sh, A, sg)
-        TACO_RK4_DISPATCH(A.D, TACO_RK4_CALL)
-#undef TACO_RK4_CALL
+        rk4_recompute_body<0, false>(sh, A, sg);
     }
 }
 
@@ -662,24 +646,245 @@ template <int DT>
 __global__ __launch_bounds__(64) void k_rk4_adjoint_rows_multi(const Rk4AdjArgs* As) {
     extern __shared__ double2 sh[];
     const Rk4AdjArgs A = As[blockIdx.x];
+    const double2* lam = A.gbar + A.steps * DT;
     if (A.vec)
-        rk4_rows_adjoint<DT, Rk4AdjArgs, true>(sh, A);
+        rk4_rows_adjoint<DT, WALK_VEC>(sh, A, 0, A.steps, lam, A.r0bar);
     else
-        rk4_rows_adjoint<DT>(sh, A);
+        rk4_rows_adjoint<DT, WALK_LBAR>(sh, A, 0, A.steps, lam, A.r0bar);
 }
 
 __global__ __launch_bounds__(kRkBlock) void k_rk4_adjoint_multi(const Rk4AdjArgs* As) {
     extern __shared__ double2 sh[];
     const Rk4AdjArgs A = As[blockIdx.x];
     if (A.nstage >= 2) {
-#define TACO_RK4_CALL(DT) rk4_adjoint_body<DT, true>(sh, A)
-        TACO_RK4_DISPATCH(A.D, TACO_RK4_CALL)
-#undef TACO_RK4_CALL
+        switch (A.D) {  // 4, 9 and 16 have the row-group walk
+            case 25: rk4_adjoint_body<25, true>(sh, A); break;
+            case 36: rk4_adjoint_body<36, true>(sh, A); break;
+            case 49: rk4_adjoint_body<49, true>(sh, A); break;
+            case 64: rk4_adjoint_body<64, true>(sh, A); break;
+            default: rk4_adjoint_body<0, true>(sh, A); break;
+        }
     } else {
-#define TACO_RK4_CALL(DT) rk4_adjoint_body<DT, false>(sh, A)
-        TACO_RK4_DISPATCH(A.D, TACO_RK4_CALL)
-#undef TACO_RK4_CALL
+        rk4_adjoint_body<0, false>(sh, A);  // sizes to 64 always stage
     }
+}
+
+// ---------------------------------------------------------------------------
+// Chunked runs.  One RK4 step is linear, r_{n+1} = (I + E_n) r_n, so the
+// recursion over many steps splits in time:
+//   1. every chunk of kRkChunk steps forms Q_c = prod (I + E_n) - I, all
+//      chunks at once (four D x D products a step);
+//   2. one workgroup carries r over the chunks, r <- r + Q_c r, one product
+//      per chunk where the plain run has four per step;
+//   3. every chunk runs its steps from its first state with the plain step
+//      (rk4_rows), all chunks at once.
+// The dependent chain shrinks from 4 steps products to 4 kRkChunk (twice) and
+// steps / kRkChunk.  E_n and Q_c are kept without the identity, so a chunk
+// rounds r once where kRkChunk plain steps round it kRkChunk times.
+// The reverse walk, affine in lam, splits alike: each chunk's walk from lam = 0
+// gives its constant part, the carry is lam <- lam + Q_c^H lam + b_c, and every
+// chunk's walk then runs from its true lam.
+// Against an 80-bit run the states are 2 to 5 times closer than the plain
+// run's (D = 16, 4000 steps: 5e-16 against 1.4e-15).
+// Measured, forward: D = 16, 4000 steps 2.7 -> 0.12 ms (products 43 us, 250
+// carries 63 us, states 17 us); D = 4, 2000 steps 1.02 -> 0.05 ms; D = 36,
+// 800 steps 0.42 ms.  All three are latency: chunks of 16 keep the products
+// at one workgroup per CU for 4000 steps and the carry at 0.25 us a chunk.
+// ---------------------------------------------------------------------------
+template <int DT>
+struct Chunk {
+    static constexpr int NT = DT < 16 ? 64 : 256;        // threads of step 1
+    static constexpr int CPB = DT == 4 ? 4 : 1;          // chunks of a workgroup
+    static constexpr int LPC = NT / CPB;                 // threads of a chunk
+    static constexpr int EPT = (DT * DT + LPC - 1) / LPC;  // entries of a thread
+    static constexpr int D2 = DT * DT;
+};
+
+// acc[i] = sum_k A(r_i, k) B(k, c_i) for the thread's entries.
+template <int DT>
+__device__ __forceinline__ void chunk_product(double2 (&acc)[Chunk<DT>::EPT], const double2* A, const double2* B, int lane) {
+    using C = Chunk<DT>;
+#pragma unroll
+    for (int i = 0; i < C::EPT; ++i) acc[i] = make_double2(0.0, 0.0);
+#pragma unroll(DT <= 16 ? DT : 4)
+    for (int k = 0; k < DT; ++k) {
+        double2 a = make_double2(0.0, 0.0);
+#pragma unroll
+        for (int i = 0; i < C::EPT; ++i) {
+            const int e = lane + i * C::LPC, r = e % DT, c = e / DT;
+            if (i == 0 || C::LPC % DT != 0) a = A[r + k * DT];  // LPC a multiple of DT: one row per thread
+            if (e < C::D2) acc[i] = cfma(a, B[k + c * DT], acc[i]);
+        }
+    }
+}
+
+// Step 1.  arr: one argument block per system or tape (null: the single `one`).
+template <int DT, class S>
+__global__ __launch_bounds__(Chunk<DT>::NT) void k_chunk_products(const S* arr, S one) {
+    using C = Chunk<DT>;
+    __shared__ double2 sA[C::CPB][C::D2], sB[C::CPB][C::D2], sQ[C::CPB][C::D2];
+    const S s = arr ? arr[blockIdx.y] : one;
+    if (s.D != DT || !s.q) return;
+    const int sub = threadIdx.x / C::LPC, lane = threadIdx.x % C::LPC;
+    const long c = static_cast<long>(blockIdx.x) * C::CPB + sub;
+    if (static_cast<long>(blockIdx.x) * C::CPB * kRkChunk >= s.steps) return;
+    const long n0 = c * kRkChunk;
+    const double h2 = 0.5 * s.dt, s6 = s.dt / 6.0;
+    double2 *A = sA[sub], *B = sB[sub], *Q = sQ[sub];
+    double2 l0[C::EPT], l1[C::EPT], ln[C::EPT], q[C::EPT], acc[C::EPT];
+    auto load = [&](double2 (&v)[C::EPT], long n) {
+        const double2* L = s.Ls + min(n, s.steps) * C::D2;
+#pragma unroll
+        for (int i = 0; i < C::EPT; ++i) v[i] = L[min(lane + i * C::LPC, C::D2 - 1)];
+    };
+    auto put = [&](double2* M, const double2 (&v)[C::EPT]) {
+#pragma unroll
+        for (int i = 0; i < C::EPT; ++i)
+            if (lane + i * C::LPC < C::D2) M[lane + i * C::LPC] = v[i];
+    };
+    load(l0, n0);
+    load(l1, n0 + 1);
+#pragma unroll
+    for (int i = 0; i < C::EPT; ++i) q[i] = make_double2(0.0, 0.0);
+    for (int m = 0; m < kRkChunk; ++m) {
+        load(ln, n0 + m + 2);
+        double2 lh[C::EPT], k2[C::EPT], k3[C::EPT];
+#pragma unroll
+        for (int i = 0; i < C::EPT; ++i) lh[i] = cscale(cadd(l0[i], l1[i]), 0.5);
+        put(A, lh);
+        put(B, l0);
+        put(Q, q);
+        __syncthreads();
+        chunk_product<DT>(acc, A, B, lane);  // K2 = Lh (I + h/2 K1), K1 = L0
+#pragma unroll
+        for (int i = 0; i < C::EPT; ++i) k2[i] = cadd(lh[i], cscale(acc[i], h2));
+        __syncthreads();
+        put(B, k2);
+        __syncthreads();
+        chunk_product<DT>(acc, A, B, lane);  // K3 = Lh (I + h/2 K2)
+#pragma unroll
+        for (int i = 0; i < C::EPT; ++i) k3[i] = cadd(lh[i], cscale(acc[i], h2));
+        __syncthreads();
+        put(A, l1);
+        put(B, k3);
+        __syncthreads();
+        chunk_product<DT>(acc, A, B, lane);  // K4 = L1 (I + h K3)
+        double2 e[C::EPT];
+#pragma unroll
+        for (int i = 0; i < C::EPT; ++i) {
+            const double2 k4 = cadd(l1[i], cscale(acc[i], s.dt));
+            e[i] = cscale(cadd(cadd(l0[i], cscale(cadd(k2[i], k3[i]), 2.0)), k4), s6);
+        }
+        __syncthreads();
+        put(A, e);
+        __syncthreads();
+        chunk_product<DT>(acc, A, Q, lane);  // Q <- Q + E + E Q
+        const bool live = n0 + m < s.steps;
+#pragma unroll
+        for (int i = 0; i < C::EPT; ++i) {
+            if (live) q[i] = cadd(q[i], cadd(e[i], acc[i]));
+            l0[i] = l1[i];
+            l1[i] = ln[i];
+        }
+        __syncthreads();
+    }
+    if (n0 < s.steps) {
+        double2* out = s.q + c * C::D2;
+#pragma unroll
+        for (int i = 0; i < C::EPT; ++i)
+            if (lane + i * C::LPC < C::D2) out[lane + i * C::LPC] = q[i];
+    }
+}
+
+// Step 2 on the row groups of rk4_rows: x over the chunks (REV: lam from the
+// last chunk down), the products' loads a ring of R chunks ahead.
+template <int DT, bool REV>
+__device__ __forceinline__ void chunk_carry(double2* sh, const double2* Q, const double2* b, long nch, const double2* x_in,
+                                            double2* xs, double2* x_out) {
+    using RG = RowGroup<DT>;
+    constexpr int R = DT <= 16 ? 8 : 4;
+    constexpr long D2 = static_cast<long>(DT) * DT;
+    const int lane = static_cast<int>(threadIdx.x & 63), g = lane % RG::G;
+    const int r = static_cast<int>(threadIdx.x >> 6) * RG::R + lane / RG::G;
+    const bool own = r < DT && g == 0;
+    auto at = [&](long c) { return REV ? nch - 1 - c : c; };  // c-th chunk visited
+    double2 x = make_double2(0.0, 0.0);
+    if (r < DT) x = x_in[r];
+    double2 ring[R][RG::CK], rb[R];
+    auto load = [&](int j, long c) {
+        const long k = at(min(c, nch - 1));
+        load_gen<DT, !REV>(ring[j], Q + k * D2, r, g);
+        rb[j] = REV ? b[k * DT + (r < DT ? r : 0)] : make_double2(0.0, 0.0);
+    };
+#pragma unroll
+    for (int j = 0; j < R; ++j) load(j, j);
+    int p = 0;
+    if (own) sh[r] = x;
+    __syncthreads();
+    auto step = [&](int j, long c) {
+        if (own) xs[at(c) * DT + r] = x;
+        const double2 y = group_dot<DT, REV>(ring[j], sh + p * DT, g);
+        x = cadd(x, y);
+        if (REV) x = cadd(x, rb[j]);
+        p ^= 1;
+        if (own) sh[p * DT + r] = x;
+        __builtin_amdgcn_sched_barrier(0);
+        load(j, c + R);
+        __syncthreads();
+    };
+    long c = 0;
+    for (; c + R <= nch; c += R) {
+#pragma unroll
+        for (int j = 0; j < R; ++j) step(j, c + j);
+    }
+#pragma unroll
+    for (int j = 0; j + 1 < R; ++j)
+        if (c + j < nch) step(j, c + j);
+    if (own && x_out) x_out[r] = x;
+}
+
+__device__ __forceinline__ long chunk_count(long steps) { return (steps + kRkChunk - 1) / kRkChunk; }
+
+template <int DT>
+__global__ __launch_bounds__(64 * RowGroup<DT>::W) void k_chunk_carry(const Rk4Sys* arr, Rk4Sys one) {
+    __shared__ double2 sh[2 * DT];
+    const Rk4Sys s = arr ? arr[blockIdx.x] : one;
+    if (s.D != DT || !s.q) return;
+    chunk_carry<DT, false>(sh, s.q, nullptr, chunk_count(s.steps), s.r0, s.xs, nullptr);
+}
+
+template <int DT>
+__global__ __launch_bounds__(64 * RowGroup<DT>::W) void k_chunk_states(const Rk4Sys* arr, Rk4Sys one) {
+    __shared__ double2 sh[3 * DT];
+    const Rk4Sys s = arr ? arr[blockIdx.y] : one;
+    const long c = blockIdx.x, n0 = c * kRkChunk;
+    if (s.D != DT || !s.q || n0 >= s.steps) return;
+    const long n1 = min(n0 + kRkChunk, s.steps);
+    const bool last = n1 == s.steps;
+    rk4_rows<DT, false>(sh, s.Ls, n0, n1, s.xs + c * DT, last ? s.r : nullptr, s.dt, s.every, s.samples,
+                        last ? s.nsamples : nullptr, nullptr, last);
+}
+
+// The reverse's chunk walks: CONST from lam = 0 (constant part to bv), else
+// from the chunk's true lam, storing kb1..kb4.
+template <int DT, bool CONST>
+__global__ __launch_bounds__(64) void k_chunk_walk(const Rk4AdjArgs* arr, Rk4AdjArgs one) {
+    __shared__ double2 sh[5 * DT];
+    const Rk4AdjArgs A = arr ? arr[blockIdx.y] : one;
+    const long c = blockIdx.x, n0 = c * kRkChunk;
+    if (n0 >= A.steps) return;
+    const long n1 = min(n0 + kRkChunk, A.steps);
+    if constexpr (CONST)
+        rk4_rows_adjoint<DT, WALK_NONE>(sh, A, n0, n1, nullptr, A.bv + c * DT);
+    else  // lam at the chunk's first step is known from the carry: bv takes the repeated value
+        rk4_rows_adjoint<DT, WALK_VEC>(sh, A, n0, n1, A.lam + c * DT, A.bv + c * DT);
+}
+
+template <int DT>
+__global__ __launch_bounds__(64) void k_chunk_carry_rev(const Rk4AdjArgs* arr, Rk4AdjArgs one) {
+    __shared__ double2 sh[2 * DT];
+    const Rk4AdjArgs A = arr ? arr[blockIdx.x] : one;
+    chunk_carry<DT, true>(sh, A.q, A.bv, chunk_count(A.steps), A.gbar + A.steps * DT, A.lam, A.r0bar);
 }
 
 // ---------------------------------------------------------------------------
@@ -695,6 +900,46 @@ hipError_t rk4_set_lds_limits() {
         if (e != hipSuccess) return e;
     }
     return hipSuccess;
+}
+
+template <class F>
+static void chunk_dispatch(int D, F&& f) {
+    switch (D) {
+        case 4: f(std::integral_constant<int, 4>{}); break;
+        case 9: f(std::integral_constant<int, 9>{}); break;
+        case 16: f(std::integral_constant<int, 16>{}); break;
+        case 25: f(std::integral_constant<int, 25>{}); break;
+        case 36: f(std::integral_constant<int, 36>{}); break;
+        default: break;
+    }
+}
+
+void launch_rk4_chunked(int D, const Rk4Sys* arr, const Rk4Sys& one, unsigned nsys, long max_steps, hipStream_t st) {
+    const unsigned nch = static_cast<unsigned>((max_steps + kRkChunk - 1) / kRkChunk);
+    chunk_dispatch(D, [&](auto dc) {
+        constexpr int DT = decltype(dc)::value;
+        constexpr unsigned cpb = Chunk<DT>::CPB;
+        hipLaunchKernelGGL((k_chunk_products<DT, Rk4Sys>), dim3((nch + cpb - 1) / cpb, nsys), dim3(Chunk<DT>::NT), 0, st,
+                           arr, one);
+        hipLaunchKernelGGL(k_chunk_carry<DT>, dim3(nsys), dim3(rk4_rows_threads(DT)), 0, st, arr, one);
+        hipLaunchKernelGGL(k_chunk_states<DT>, dim3(nch, nsys), dim3(rk4_rows_threads(DT)), 0, st, arr, one);
+    });
+}
+
+void launch_rk4_chunked_walk(int D, const Rk4AdjArgs* arr, const Rk4AdjArgs& one, unsigned ntapes, long steps,
+                             hipStream_t st) {
+    const unsigned nch = static_cast<unsigned>((steps + kRkChunk - 1) / kRkChunk);
+    chunk_dispatch(D, [&](auto dc) {
+        constexpr int DT = decltype(dc)::value;
+        if constexpr (DT <= 16) {
+            constexpr unsigned cpb = Chunk<DT>::CPB;
+            hipLaunchKernelGGL((k_chunk_products<DT, Rk4AdjArgs>), dim3((nch + cpb - 1) / cpb, ntapes),
+                               dim3(Chunk<DT>::NT), 0, st, arr, one);
+            hipLaunchKernelGGL((k_chunk_walk<DT, true>), dim3(nch, ntapes), dim3(64), 0, st, arr, one);
+            hipLaunchKernelGGL(k_chunk_carry_rev<DT>, dim3(ntapes), dim3(64), 0, st, arr, one);
+            hipLaunchKernelGGL((k_chunk_walk<DT, false>), dim3(nch, ntapes), dim3(64), 0, st, arr, one);
+        }
+    });
 }
 
 void launch_rk4_rows(int D, const double2* Ls, long steps, double2* r, double dt, long every, double2* samples,

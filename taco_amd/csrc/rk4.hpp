@@ -51,6 +51,10 @@ struct Rk4Sys {
     double dt;
     int D;
     const double2* Lh = nullptr;  // [steps][D x D] midpoints (large D), else formed on the fly
+    double2* q = nullptr;         // chunked run: [chunks][D x D] products, null: one sequential run
+    double2* xs = nullptr;        // chunked run: [chunks][D] first states
+    long every = 1;               // sample distance
+    long* nsamples = nullptr;
 };
 
 struct Rk4AdjArgs {
@@ -68,7 +72,28 @@ struct Rk4AdjArgs {
     const double2* LsH = nullptr;  // [steps + 1][D * D] conjugate transposes (walk without staging)
     const double2* LhH = nullptr;  // [steps][D * D] their midpoints (null: formed on the fly)
     double2* vec = nullptr;        // [steps][4][D] kb1..kb4 of every step (Lbar formed by k_rk4_lbar)
+    double2* q = nullptr;          // chunked walk: [chunks][D * D] products,
+    double2* lam = nullptr;        // [chunks][D] lam after each chunk's last step,
+    double2* bv = nullptr;         // [chunks][D] constant parts
 };
+
+// Steps of a chunk of the chunked runs.
+constexpr int kRkChunk = 16;
+
+// Whether a run of `steps` steps at D is chunked (rk4.hip).  The chunked run
+// costs five or six launches and 2 kRkChunk steps of latency whatever its
+// length; below 256 steps the plain run (0.5-0.7 us a step at D <= 16) is as
+// fast.  The reverse has row groups for D <= 16 only.
+constexpr long kRkChunkedMin = 256;
+inline bool rk4_chunked(int D, long steps) {
+    return steps >= kRkChunkedMin && (D == 4 || D == 9 || D == 16 || D == 25 || D == 36);
+}
+inline bool rk4_chunked_walk(int D, long steps) { return D <= 16 && rk4_chunked(D, steps); }
+// Complex values of a chunked run's products and first states (or lam).
+inline std::size_t rk4_chunk_values(int D, long steps) {
+    const std::size_t nch = static_cast<std::size_t>((steps + kRkChunk - 1) / kRkChunk);
+    return nch * (static_cast<std::size_t>(D) * D + D);
+}
 
 // Raises the kernels' dynamic LDS limit to kRkLds on the current device.
 hipError_t rk4_set_lds_limits();
@@ -81,6 +106,12 @@ void launch_rk4(int D, const double2* Ls, const double2* Lh, long steps, double2
                 double2* samples, long* nsamples, int nstage, int block, std::size_t lds, hipStream_t st);
 // nsys systems, one workgroup each.
 void launch_rk4_batch(unsigned nsys, const Rk4Sys* sys, int block, std::size_t lds, hipStream_t st);
+// Chunked runs of the systems with q set and this D: `one`, or nsys of them on
+// the device (arr), of at most max_steps steps; and the chunked walk of `one`
+// tape or ntapes tapes.
+void launch_rk4_chunked(int D, const Rk4Sys* arr, const Rk4Sys& one, unsigned nsys, long max_steps, hipStream_t st);
+void launch_rk4_chunked_walk(int D, const Rk4AdjArgs* arr, const Rk4AdjArgs& one, unsigned ntapes, long steps,
+                             hipStream_t st);
 // out[n] = (L[n] + L[n + 1]) / 2, n < count.
 void launch_midpoints(const double2* L, long count, long D2, double2* out, hipStream_t st);
 // dst[t] = src[t]^H, t < count.

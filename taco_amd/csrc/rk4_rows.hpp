@@ -162,7 +162,8 @@ struct RowsForward {
 
 // RK4 steps n0 .. n1-1 on x (x_in -> x_out, if given), step n using Ls[n],
 // Ls[n + 1] and the midpoint 0.5 (Ls[n] + Ls[n + 1]).  samples (optional): x
-// before every step with (n - n0) % every == 0 and after the last one.
+// before every step with n % every == 0 (sample n / every) and, if `last`,
+// after the last one.
 // STASH: the state r_n and stage points u1, u2, u3 of step n go to
 // seg[n][4][D].  LDS: 3 D values.  Whole blocks of S steps run in a loop with
 // no early exit (so each ring slot keeps its registers across iterations);
@@ -170,7 +171,7 @@ struct RowsForward {
 template <int DT, bool STASH>
 __device__ __forceinline__ void rk4_rows(double2* sh, const double2* __restrict__ Ls, long n0, long n1,
                                          const double2* x_in, double2* x_out, double dt, long every,
-                                         double2* samples, long* nsamples, double2* seg) {
+                                         double2* samples, long* nsamples, double2* seg, bool last = true) {
     using RG = RowGroup<DT>;
     constexpr int CK = RG::CK, S = RG::S;
     constexpr long D2 = static_cast<long>(DT) * DT;
@@ -184,8 +185,8 @@ __device__ __forceinline__ void rk4_rows(double2* sh, const double2* __restrict_
     F.seg = seg;
     F.n1 = n1;
     F.every = every;
-    F.ns = 0;
-    F.cnt = 0;
+    F.ns = (n0 + every - 1) / every;
+    F.cnt = F.ns * every - n0;
     F.dt = dt;
     F.hdt = 0.5 * dt;
     F.s6 = dt / 6.0;
@@ -208,7 +209,7 @@ __device__ __forceinline__ void rk4_rows(double2* sh, const double2* __restrict_
 #pragma unroll
     for (int j = 0; j + 1 < S; ++j)
         if (nb + j < n1) F.step(nb + j, Lr[j], Lr[(j + 1) % S]);
-    if (samples) {
+    if (samples && last) {
         if (F.own) samples[F.ns * DT + F.r] = F.xr;
         ++F.ns;
     }
@@ -226,7 +227,14 @@ __device__ __forceinline__ void load_points(double2 (&p)[4], double2& gb, const 
     gb = A.gbar[n * DT + cc];
 }
 
-// Reverse walk of rk4_rows over all steps (one wave: D <= 16).  Group c owns
+// What the reverse walk keeps of a step besides lam.
+enum WalkKeep {
+    WALK_LBAR,  // the generator cotangents, formed in place
+    WALK_VEC,   // kb1..kb4 (A.vec): k_rk4_lbar forms Lbar from them
+    WALK_NONE,  // nothing: only lam at the first step is wanted
+};
+
+// Reverse walk of rk4_rows over steps n1-1 .. n0 (one wave: D <= 16).  Group c owns
 // element c of every cotangent vector and column c of the generator
 // cotangents.  Per step n, with lam the cotangent of r_{n+1}:
 //   kb4 = s lam, ub3 = L1^H kb4, kb3 = 2 s lam + dt ub3,
@@ -237,7 +245,7 @@ __device__ __forceinline__ void load_points(double2 (&p)[4], double2& gb, const 
 //   Lbar_n     += kb1 r_n^H + (kb3 u2^H + kb2 u1^H) / 2,
 // the L0 part carried in registers to the next (earlier) step.  Generators,
 // stage points and gbar are prefetched S - 1 steps ahead.  LDS: 5 D values.
-template <int DT, class Args, bool DEFER = false>
+template <int DT, class Args, int KEEP>
 struct RowsAdjoint {
     using RG = RowGroup<DT>;
     static constexpr int CK = RG::CK, S = RG::SA, G = RG::G;
@@ -282,7 +290,7 @@ struct RowsAdjoint {
         __syncthreads();
         // ub0 = L0^H kb1
         const double2 ub0 = group_dot<DT, true>(L0, K1, g);
-        if constexpr (DEFER) {
+        if constexpr (KEEP == WALK_VEC) {
             // the step's kb1..kb4 for k_rk4_lbar, which forms every Lbar(t)
             // afterwards with these sums (all times in parallel)
             if (own) {
@@ -292,7 +300,7 @@ struct RowsAdjoint {
                 v[2 * DT + c] = kb3;
                 v[3 * DT + c] = kb4;
             }
-        } else {
+        } else if constexpr (KEEP == WALK_LBAR) {
             // generator cotangents of column c, rows g + k G
             const double2 xc = Sg[0], u1c = Sg[1], u2c = Sg[2], u3c = Sg[3];
             double2* Lb1 = A->Lbar + (n + 1) * D2;
@@ -315,17 +323,18 @@ struct RowsAdjoint {
     }
 };
 
-// DEFER: the walk stores each step's kb1..kb4 (A.vec) instead of forming
-// Lbar; k_rk4_lbar then forms Lbar(t) from them and the stage points, with
-// the walk's own sums (the same values; off the walk's sequential path).
-template <int DT, class Args, bool DEFER = false>
-__device__ __forceinline__ void rk4_rows_adjoint(double2* sh, const Args& A) {
+// lam_in: the cotangent of r_{n1} (null: zero); lam_out: that of r_{n0}.
+// WALK_VEC's kb1..kb4 and the stage points give k_rk4_lbar the walk's own
+// sums (the same values; off the walk's sequential path).
+template <int DT, int KEEP, class Args>
+__device__ __forceinline__ void rk4_rows_adjoint(double2* sh, const Args& A, long n0, long n1, const double2* lam_in,
+                                                 double2* lam_out) {
     using RG = RowGroup<DT>;
     static_assert(RG::W == 1, "one wave");
     constexpr int CK = RG::CK, S = RG::SA, G = RG::G;
     constexpr long D2 = static_cast<long>(DT) * DT;
     const int lane = static_cast<int>(threadIdx.x & 63);
-    RowsAdjoint<DT, Args, DEFER> B;
+    RowsAdjoint<DT, Args, KEEP> B;
     B.A = &A;
     B.K4 = sh;  // two buffers, alternating by step
     B.K3 = sh + 2 * DT;
@@ -338,37 +347,36 @@ __device__ __forceinline__ void rk4_rows_adjoint(double2* sh, const Args& A) {
     B.col = B.c < DT;
     B.own = B.col && B.g == 0;
     B.par = 0;
-    const long steps = A.steps;
     // lam first: its load is then the oldest one in flight when the loop
     // starts, so no wait for the ring loads lands in the loop
-    B.lam = A.gbar[steps * DT + (B.col ? B.c : 0)];
-    // ring slot (steps - m) % S holds generator m; slot (steps - 1 - n) % S
+    B.lam = lam_in ? lam_in[B.col ? B.c : 0] : make_double2(0.0, 0.0);
+    // ring slot (n1 - m) % S holds generator m; slot (n1 - 1 - n) % S
     // the stage points and gbar of step n
     double2 Lr[S][CK], Sg[S][4], Gb[S];
 #pragma unroll
     for (int q = 0; q < S; ++q) {
-        load_gen<DT, false>(Lr[q], A.Ls + max(steps - q, 0L) * D2, B.c, B.g);
-        load_points<DT>(Sg[q], Gb[q], A, max(steps - 1 - q, 0L), B.c);
+        load_gen<DT, false>(Lr[q], A.Ls + max(n1 - q, 0L) * D2, B.c, B.g);
+        load_points<DT>(Sg[q], Gb[q], A, max(n1 - 1 - q, 0L), B.c);
     }
 #pragma unroll
     for (int k = 0; k < CK; ++k) B.Lc[k] = make_double2(0.0, 0.0);
     if (B.own) B.K4[B.c] = cscale(B.lam, B.s6);
     __syncthreads();
     // whole blocks of S steps (no early exit), then the rest
-    long nb = steps - 1;
-    for (; nb + 1 >= S; nb -= S) {
+    long nb = n1 - 1;
+    for (; nb + 1 >= n0 + S; nb -= S) {
 #pragma unroll
         for (int j = 0; j < S; ++j) B.step(nb - j, Lr[j], Lr[(j + 1) % S], Sg[j], Gb[j]);
     }
 #pragma unroll
     for (int j = 0; j + 1 < S; ++j)
-        if (nb - j >= 0) B.step(nb - j, Lr[j], Lr[(j + 1) % S], Sg[j], Gb[j]);
-    if constexpr (!DEFER) {
+        if (nb - j >= n0) B.step(nb - j, Lr[j], Lr[(j + 1) % S], Sg[j], Gb[j]);
+    if constexpr (KEEP == WALK_LBAR) {
 #pragma unroll
         for (int k = 0; k < CK; ++k) {
             const int rr = B.g + k * G;
             if (B.col && rr < DT) A.Lbar[rr + B.c * DT] = B.Lc[k];
         }
     }
-    if (B.own) A.r0bar[B.c] = B.lam;
+    if (B.own) lam_out[B.c] = B.lam;
 }

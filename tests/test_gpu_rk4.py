@@ -29,6 +29,25 @@ def test_rk4_matches_oracle(orc, D, steps):
     assert max_rel_err(np.array(got_samples), ref_samples)[0] <= 1e-12
 
 
+@pytest.mark.parametrize("D", [4, 9, 16, 25, 36])
+@pytest.mark.parametrize("steps,every", [(255, 1), (256, 1), (257, 16), (272, 7), (273, 300), (1003, 10)])
+def test_chunked_rk4_matches_oracle(orc, D, steps, every):
+    """Runs of 256 steps and more are split into chunks of 16 steps: states at
+    every sample and at the end against the oracle's sequential run, at the
+    bound of the runs above."""
+    rng = np.random.default_rng(100 + D)
+    base = (rng.standard_normal((D, D)) + 1j * rng.standard_normal((D, D))) * (0.5 / np.sqrt(D))
+    Ls = np.array([base * np.cos(0.01 * s) - 0.1 * np.eye(D) for s in range(steps + 1)])
+    r0 = rng.standard_normal(D) + 1j * rng.standard_normal(D)
+    seen = []
+    r = taco_amd.propagate_rk4_dense(Ls, r0, 0.0, 0.005, on_sample=lambda t, v: seen.append(v.copy()),
+                                     sample_every=every)
+    rr, ref = orc.propagate(Ls, r0, 0.005, every=every)
+    assert np.abs(r - rr).max() <= 1e-12 * np.abs(rr).max()
+    assert len(seen) == len(ref)
+    assert max_rel_err(np.array(seen), ref)[0] <= 1e-12
+
+
 def test_rk4_closed_forms():
     D = 4
     L = np.diag([0.1 - 0.03j, -0.07 + 0.05j, 0.02, -0.04 - 0.02j])
