@@ -832,26 +832,33 @@ __device__ __forceinline__ double spectral_J_dev(int kind, double p0, double p1,
 
 // kms[k] = r^k for k = 1..posCount by the reference's recurrence KMS *= r.
 // One lane; the chain is unrolled 32 deep (loop overhead, not the multiply's
-// latency, bounds a shallower loop: 9.3 -> 6.2 ns per factor).
-__global__ void k_bcf_kms(double r, long pos_count, double* kms) {
-    if (blockIdx.x != 0 || threadIdx.x != 0) return;
-    constexpr int kU = 32;
-    double v = r;
-    long k = 1;
-    for (; k + kU <= pos_count + 1; k += kU) {  // the same chain, stored kU at a time
-        double t[kU];
+// latency, bounds a shallower loop: 9.3 -> 6.2 ns per factor).  Once a factor
+// is zero every later one is, and the whole wave fills them in: a chain of
+// 2^18 factors that underflows half way takes 0.85 ms instead of 1.65.
+__global__ __launch_bounds__(64) void k_bcf_kms(double r, long pos_count, double* kms) {
+    __shared__ long zero_from;
+    if (threadIdx.x == 0) {
+        constexpr int kU = 32;
+        double v = r;
+        long k = 1;
+        for (; k + kU <= pos_count + 1 && v != 0.0; k += kU) {  // the same chain, stored kU at a time
+            double t[kU];
 #pragma unroll
-        for (int j = 0; j < kU; ++j) {
-            t[j] = v;
+            for (int j = 0; j < kU; ++j) {
+                t[j] = v;
+                v *= r;
+            }
+#pragma unroll
+            for (int j = 0; j < kU; ++j) kms[k + j] = t[j];
+        }
+        for (; k <= pos_count && v != 0.0; ++k) {
+            kms[k] = v;
             v *= r;
         }
-#pragma unroll
-        for (int j = 0; j < kU; ++j) kms[k + j] = t[j];
+        zero_from = k;
     }
-    for (; k <= pos_count; ++k) {
-        kms[k] = v;
-        v *= r;
-    }
+    __syncthreads();
+    for (long k = zero_from + threadIdx.x; k <= pos_count; k += 64) kms[k] = 0.0;
 }
 
 // S[k], k < nfft: the KMS spectrum of bcf_fft_fun, one entry per thread.
@@ -926,16 +933,32 @@ __global__ __launch_bounds__(kBlock) void k_bcf_gather(const double2* spec, int 
     C[n] = make_double2(x.x * scale, x.y * scale);
 }
 
+// v of lane I of each row of 16, in every lane of the row.
+template <int I>
+__device__ __forceinline__ double row_bcast(double v) {
+    return __builtin_amdgcn_update_dpp(v, v, 0x150 + I, 0xF, 0xF, true);
+}
+
+// One step of the phase chain on lanes 0 and 1: x' = x c - y s, y' = x s + y c
+// as x kx + y ky with (kx, ky) = (c, -s) and (s, c) -- the same products and
+// sum, in three FP64 operations instead of six.
+__device__ __forceinline__ double phase_step(double phi, double kx, double ky) {
+    return row_bcast<0>(phi) * kx + row_bcast<1>(phi) * ky;
+}
+
 // Gamma[j][k] = trapz prefix of exp(i omega_j tau) C(tau), one workgroup per
 // bucket, with the reference's chains (phi_k = phi_{k-1} step; acc_k =
 // acc_{k-1} + dt/2 (phi_{k-1} C_{k-1} + phi_k C_k)) split so that only the
-// two recurrences are sequential.  Per chunk of kTzChunk times, in a
-// pipeline: lane 0 of wave 0 runs the phase chain of chunk c, lane 0 of wave
-// 1 the sum chain of chunk c - 1, waves 2-3 load C of chunk c and write Gamma
-// of chunk c - 2; then every thread forms chunk c's terms, each exactly the
-// reference's expression.  Over full chunks the chains run unrolled 64 (phase)
-// and 32 (sum) deep: a shallower loop's overhead rivals the arithmetic (5
-// buckets x 65536 times: 2.12 -> 1.99 ms).
+// two recurrences are sequential.  Per chunk of kTzChunk times, in a pipeline
+// with one barrier a chunk: lanes 0-1 of wave 0 run the phase chain of chunk c,
+// waves 2-3 load C of chunk c, form the terms of chunk c - 1 (each exactly the
+// reference's expression) and write Gamma of chunk c - 3, lane 0 of wave 1
+// runs the sum chain of chunk c - 2.  The phase chain bounds it, by the
+// latency of a broadcast, a product and a sum per step (26 ns): one lane with
+// six operations a step and every wave forming the terms between two barriers
+// took 6.2 ms for 13 buckets x 200001 times, this 5.3.  Over full chunks the
+// chains run unrolled 64 (phase) and 32 (sum) deep: a shallower loop's
+// overhead rivals the arithmetic.
 constexpr int kTzChunk = 1024;
 static_assert(kTzChunk % (kBlock - 128) == 0, "loader waves cover a chunk exactly");
 static_assert(kTzChunk % 64 == 0, "unrolled chains cover a full chunk exactly");
@@ -945,110 +968,106 @@ __global__ __launch_bounds__(kBlock) void k_gamma_trapz(const double2* C, long n
     __shared__ double2 ph[2][kTzChunk];    // phi_k of chunk c
     __shared__ double2 uu[2][kTzChunk];    // terms of chunk c
     __shared__ double2 gout[2][kTzChunk];  // Gamma of chunk c
-    __shared__ double2 last_phi[2], last_c[2];
+    __shared__ double2 last_phi[4], last_c[4];  // of chunk c (c % 4)
     double2* col = G + static_cast<long>(blockIdx.x) * nc;
     const double2 half_dt = make_double2(dt / 2.0, 0.0);
-    double2 step = make_double2(1.0, 0.0), phi = make_double2(1.0, 0.0), acc = make_double2(0.0, 0.0);
-    // the phase step exp(i omega_b dt): the host's value (TACO_PHASE_LIBM) or correctly rounded
-    if (threadIdx.x == 0) step = steps ? steps[blockIdx.x] : cexpi(omegas[blockIdx.x] * dt);
+    double2 acc = make_double2(0.0, 0.0);
+    // the phase chain's lanes: lane 0 carries Re phi, lane 1 Im phi, each with
+    // its factors of Re phi and Im phi in phi step.  The phase step
+    // exp(i omega_b dt) is the host's value (TACO_PHASE_LIBM) or correctly rounded.
+    double phi = threadIdx.x == 0 ? 1.0 : 0.0, kx = 0.0, ky = 0.0;
+    if (threadIdx.x < 2) {
+        const double2 step = steps ? steps[blockIdx.x] : cexpi(omegas[blockIdx.x] * dt);
+        kx = threadIdx.x == 0 ? step.x : step.y;
+        ky = threadIdx.x == 0 ? -step.y : step.x;
+    }
     const long nch = (nc + kTzChunk - 1) / kTzChunk;
-    for (long c = 0; c <= nch + 1; ++c) {
+    for (long c = 0; c <= nch + 2; ++c) {
         const int cb = static_cast<int>(c & 1), pb = cb ^ 1;
-        if (threadIdx.x == 0) {
-            if (c < nch) {  // phase chain of chunk c
+        if (threadIdx.x < 2) {
+            if (c < nch) {  // phase chain of chunk c, this lane's component
                 const long k0 = c * kTzChunk;
                 const int e_end = static_cast<int>(min(static_cast<long>(kTzChunk), nc - k0));
+                double* dst = reinterpret_cast<double*>(ph[cb]) + threadIdx.x;
                 int e = 0;
                 if (k0 == 0) {
-                    ph[cb][0] = phi;  // phi_0 = 1
+                    dst[0] = phi;  // phi_0 = 1
                     e = 1;
                 }
                 if (e_end == kTzChunk) {  // full chunk: to a multiple of 64, then 64 deep
-                    for (; e % 64 != 0; ++e) {
-                        phi = cmul(phi, step);
-                        ph[cb][e] = phi;
-                    }
+                    for (; e % 64 != 0; ++e) dst[2 * e] = phi = phase_step(phi, kx, ky);
                     for (; e < kTzChunk; e += 64) {
 #pragma unroll
-                        for (int j = 0; j < 64; ++j) {
-                            phi = cmul(phi, step);
-                            ph[cb][e + j] = phi;
-                        }
+                        for (int j = 0; j < 64; ++j) dst[2 * (e + j)] = phi = phase_step(phi, kx, ky);
                     }
                 }
-                for (; e < e_end; ++e) {
-                    phi = cmul(phi, step);
-                    ph[cb][e] = phi;
-                }
+                for (; e < e_end; ++e) dst[2 * e] = phi = phase_step(phi, kx, ky);
+                reinterpret_cast<double*>(last_phi + (c & 3))[threadIdx.x] = phi;
             }
         } else if (threadIdx.x == 64) {
-            if (c >= 1 && c - 1 < nch) {  // sum chain of chunk c - 1
-                const long k0 = (c - 1) * kTzChunk;
+            if (c >= 2 && c - 2 < nch) {  // sum chain of chunk c - 2
+                const long k0 = (c - 2) * kTzChunk;
                 const int e_end = static_cast<int>(min(static_cast<long>(kTzChunk), nc - k0));
                 int e = 0;
                 if (k0 == 0) {
-                    gout[pb][0] = make_double2(0.0, 0.0);
+                    gout[cb][0] = make_double2(0.0, 0.0);
                     e = 1;
                 }
                 if (e_end == kTzChunk) {  // full chunk: to a multiple of 32, then 32 deep
                     for (; e % 32 != 0; ++e) {
-                        acc = cadd(acc, uu[pb][e]);
-                        gout[pb][e] = acc;
+                        acc = cadd(acc, uu[cb][e]);
+                        gout[cb][e] = acc;
                     }
                     for (; e < kTzChunk; e += 32) {
                         double2 u[32];
 #pragma unroll
-                        for (int j = 0; j < 32; ++j) u[j] = uu[pb][e + j];
+                        for (int j = 0; j < 32; ++j) u[j] = uu[cb][e + j];
 #pragma unroll
                         for (int j = 0; j < 32; ++j) {
                             acc = cadd(acc, u[j]);
-                            gout[pb][e + j] = acc;
+                            gout[cb][e + j] = acc;
                         }
                     }
                 }
                 for (; e < e_end; ++e) {
-                    acc = cadd(acc, uu[pb][e]);
-                    gout[pb][e] = acc;
+                    acc = cadd(acc, uu[cb][e]);
+                    gout[cb][e] = acc;
                 }
             }
         } else if (threadIdx.x >= 128) {
-            // kLd values per loader thread, all loads issued before the LDS writes
-            constexpr int kLd = kTzChunk / (kBlock - 128);
+            // kLd values per thread, all loads issued before the LDS writes
+            constexpr int kW = kBlock - 128, kLd = kTzChunk / kW;
             const int e0 = threadIdx.x - 128;
-            if (c < nch) {
-                double2 v[kLd];
+            double2 v[kLd];
+            if (c < nch) {  // C of chunk c
 #pragma unroll
                 for (int q = 0; q < kLd; ++q) {
-                    const long k = c * kTzChunk + e0 + q * (kBlock - 128);
+                    const long k = c * kTzChunk + e0 + q * kW;
                     v[q] = k < nc ? C[k] : make_double2(0.0, 0.0);
                 }
-#pragma unroll
-                for (int q = 0; q < kLd; ++q) cin[cb][e0 + q * (kBlock - 128)] = v[q];
             }
-            if (c >= 2) {
-                double2 v[kLd];
-#pragma unroll
-                for (int q = 0; q < kLd; ++q) v[q] = gout[cb][e0 + q * (kBlock - 128)];
+            if (c >= 3) {  // Gamma of chunk c - 3
 #pragma unroll
                 for (int q = 0; q < kLd; ++q) {
-                    const long k = (c - 2) * kTzChunk + e0 + q * (kBlock - 128);
-                    if (k < nc) col[k] = v[q];
+                    const long k = (c - 3) * kTzChunk + e0 + q * kW;
+                    if (k < nc) col[k] = gout[pb][e0 + q * kW];
                 }
             }
-        }
-        __syncthreads();
-        if (c < nch) {  // terms of chunk c
-            const long k0 = c * kTzChunk;
-            const int e_end = static_cast<int>(min(static_cast<long>(kTzChunk), nc - k0));
-            for (int e = threadIdx.x; e < e_end; e += kBlock) {
-                if (k0 + e == 0) continue;
-                const double2 pm = e > 0 ? ph[cb][e - 1] : last_phi[pb];
-                const double2 cm = e > 0 ? cin[cb][e - 1] : last_c[pb];
-                uu[cb][e] = cmul(half_dt, cadd(cmul(pm, cm), cmul(ph[cb][e], cin[cb][e])));
+            if (c >= 1 && c - 1 < nch) {  // terms of chunk c - 1
+                const long k0 = (c - 1) * kTzChunk;
+#pragma unroll
+                for (int q = 0; q < kLd; ++q) {
+                    const int e = e0 + q * kW;
+                    if (k0 + e >= nc || k0 + e == 0) continue;
+                    const double2 pm = e > 0 ? ph[pb][e - 1] : last_phi[(c - 2) & 3];
+                    const double2 cm = e > 0 ? cin[pb][e - 1] : last_c[(c - 2) & 3];
+                    uu[pb][e] = cmul(half_dt, cadd(cmul(pm, cm), cmul(ph[pb][e], cin[pb][e])));
+                }
             }
-            if (threadIdx.x == 0 && e_end == kTzChunk) {
-                last_phi[cb] = ph[cb][kTzChunk - 1];
-                last_c[cb] = cin[cb][kTzChunk - 1];
+            if (c < nch) {
+#pragma unroll
+                for (int q = 0; q < kLd; ++q) cin[cb][e0 + q * kW] = v[q];
+                if (e0 == kW - 1) last_c[c & 3] = v[kLd - 1];
             }
         }
         __syncthreads();
