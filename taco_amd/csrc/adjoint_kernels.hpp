@@ -191,12 +191,12 @@ struct L4fAdjArgs {
     int N, nf, num_ops;
     long nf3;
     long T;
-    double2* sbar;        // [T][3][nf3]; zero on entry unless lds_slices
+    double2* sbar;        // [T][3][nf3], the entries of the lists below written
     double2* Abar;        // [T][num_ops][N^2]
     int lds_slices;
     int lds_tb;           // Tbar in LDS (else after U in the scratch)
     double2* scr;         // [gridDim.x][scr_per]
-    long scr_per;         // 4 N^2 nf + 3 N^2 + N^4, + N^4 when !lds_tb
+    long scr_per;         // 4 N^2 nf + 3 N^2 + N^4, + N^4 when !lds_tb, + nxp nf with xtab
     // Gather lists (host-built from the pair map) that give every cotangent
     // entry one owner thread summing its terms in a fixed order:
     // X-form pairs (x, z) with their (a, i, b, form) terms; F and R slice
@@ -209,10 +209,12 @@ struct L4fAdjArgs {
     const int* f_start;   // [nft + 1]
     const int* f_ent;     // n | i << 8 | a << 16 | b << 24 (kind in bit 31)
     int nft;
-    const int* r_tgt;
+    const int* r_tgt;     // [nrt] bit 31: no X-form pair writes this entry
     const int* r_start;
     const int* r_ent;
     int nrt;
+    int parts;            // room for entry_parts in LDS
+    const int* xtab;      // [nf * nf] x nf + z -> pair index (null: X read from the slices)
 };
 
 // LDS_SLICES: slice cotangents accumulate in LDS (else in global memory);
@@ -227,7 +229,8 @@ __device__ __forceinline__ void l4f_adjoint_body(double2* sm, const L4fAdjArgs& 
     double2* Tb = LDS_TB ? sm : scr0 + 4 * N2nf + 3 * N2 + N4;  // N^4
     double2* opsS = LDS_TB ? Tb + N4 : sm;              // num_ops N^2
     double2* Ab = opsS + A.num_ops * N2;                // num_ops N^2
-    double2* sb = Ab + A.num_ops * N2;                  // 3 nf3 (LDS_SLICES)
+    double2* part = A.parts ? Ab + A.num_ops * N2 : nullptr;                 // 2 BS
+    double2* sb = Ab + A.num_ops * N2 + (A.parts ? 2 * BS : 0);              // 3 nf3 (LDS_SLICES)
     int* f = reinterpret_cast<int*>(sb + (LDS_SLICES ? 3 * A.nf3 : 0));
     for (int e = threadIdx.x; e < A.num_ops * N2; e += BS) opsS[e] = A.ops[e];
     for (int e = threadIdx.x; e < N2; e += BS) f[e] = A.p2f[e];
@@ -239,6 +242,7 @@ __device__ __forceinline__ void l4f_adjoint_body(double2* sm, const L4fAdjArgs& 
     double2* S123b = S123 + N2;
     double2* Db = S123b + N2;
     double2* U = Db + N2;                               // U(n,i,b,j) at (n + i N) + (b + j N) N^2
+    double2* Xc = U + N4 + (LDS_TB ? 0 : N4);           // X at [g][pair] (xtab)
     const long nfl = nf;
     auto id3 = [nfl](int x, int y, int z) { return (static_cast<long>(x) * nfl + y) * nfl + z; };
     auto F2 = [f, N](int r, int c) { return f[r + c * N]; };
@@ -251,12 +255,28 @@ __device__ __forceinline__ void l4f_adjoint_body(double2* sm, const L4fAdjArgs& 
             Tb[idx] = cadd(Lb[(n + m * N) + (i + j * N) * N2], cconj(Lb[(m + n * N) + (j + i * N) * N2]));
         }
         for (int e = threadIdx.x; e < A.num_ops * N2; e += BS) Ab[e] = make_double2(0.0, 0.0);
-        if constexpr (LDS_SLICES)
+        if constexpr (LDS_SLICES)  // entries that no list writes
             for (long e = threadIdx.x; e < 3 * A.nf3; e += BS) sb[e] = make_double2(0.0, 0.0);
         __syncthreads();
         const double2* Fp = A.Fs + t * A.nf3;
         const double2* Cp = A.Cs + t * A.nf3;
         const double2* Rp = A.Rs + t * A.nf3;
+        // X = C + R at (x, g, z): its row over g starts at xrow(x, z) with stride
+        // xstep.  The sums below read every X several times in orders that
+        // touch a line for each 16 bytes; with xtab they read the pairs
+        // gathered once per time, in the order of the slices.
+        const bool packed = A.xtab != nullptr;
+        const long xstep = packed ? A.nxp : nfl;
+        auto xrow = [&](int x, int z) { return packed ? static_cast<long>(A.xtab[x * nf + z]) : x * nfl * nfl + z; };
+        auto xval = [&](long e) { return packed ? Xc[e] : cadd(Cp[e], Rp[e]); };
+        if (packed) {
+            for (int e = threadIdx.x; e < A.nxp * nf; e += BS) {
+                const int xz = A.xp_xz[e % A.nxp];
+                const long x = id3(xz & 65535, e / A.nxp, xz >> 16);
+                Xc[e] = cadd(Cp[x], Rp[x]);
+            }
+            __syncthreads();
+        }
         double2* sF = LDS_SLICES ? sb : A.sbar + t * 3 * A.nf3;
         double2* sC = sF + A.nf3;
         double2* sR = sC + A.nf3;
@@ -266,6 +286,7 @@ __device__ __forceinline__ void l4f_adjoint_body(double2* sm, const L4fAdjArgs& 
                 const double2* Bp = opsS + iB * N2;
                 double2* AbA = Ab + iA * N2;
                 double2* AbB = Ab + iB * N2;
+                const bool first = iA == 0 && iB == 0;  // stores the slice cotangents that later pairs add to
 #define AA(r, c) Ap[(r) + (c) * N]
 #define BB(r, c) Bp[(r) + (c) * N]
 #define TB(n, i, m, j) Tb[((n) + (i) * N) + ((m) + (j) * N) * N2]
@@ -275,17 +296,18 @@ __device__ __forceinline__ void l4f_adjoint_body(double2* sm, const L4fAdjArgs& 
                     const int g = static_cast<int>(e / N2);
                     double2 y = make_double2(0.0, 0.0);
                     for (int b = 0; b < N; ++b) {
-                        const long x1 = id3(F2(b, a), g, F2(a, i)), x2 = id3(F2(i, b), g, F2(a, i));
-                        y = cadd(y, cmul(cmul(AA(a, b), BB(b, i)), cadd(Cp[x1], Rp[x1])));
-                        y = csub(y, cmul(cmul(BB(a, b), AA(b, i)), cadd(Cp[x2], Rp[x2])));
+                        const long x1 = xrow(F2(b, a), F2(a, i)) + g * xstep, x2 = xrow(F2(i, b), F2(a, i)) + g * xstep;
+                        y = cadd(y, cmul(cmul(AA(a, b), BB(b, i)), xval(x1)));
+                        y = csub(y, cmul(cmul(BB(a, b), AA(b, i)), xval(x2)));
                     }
                     Q[e] = y;
                 }
-                for (int e = threadIdx.x; e < N2; e += BS) {
-                    const int n = e % N, i = e / N;
-                    double2 s = make_double2(0.0, 0.0);
-                    for (int a = 0; a < N; ++a)
-                        for (int b = 0; b < N; ++b) {
+                entry_parts<BS>(
+                    N2, part,
+                    [&](int e, int p, int np, double2& s, double2&) {
+                        const int n = e % N, i = e / N;
+                        for (int q = p; q < N2; q += np) {
+                            const int a = q / N, b = q % N;
                             const double2 Mv = csub(Fp[id3(F2(b, a), F2(b, i), F2(n, b))],
                                                     Rp[id3(F2(b, a), F2(n, a), F2(a, i))]);
                             const double2 Iv = Fp[id3(F2(a, n), F2(b, i), F2(n, b))];
@@ -294,8 +316,8 @@ __device__ __forceinline__ void l4f_adjoint_body(double2* sm, const L4fAdjArgs& 
                             s = cadd(s, cmul(cmul(cmul(AA(n, a), BB(a, b)), BB(b, i)), Iv));
                             s = csub(s, cmul(cmul(cmul(BB(n, a), BB(a, b)), AA(b, i)), Kv));
                         }
-                    S123[e] = s;
-                }
+                    },
+                    [&](int e, double2 s, double2) { S123[e] = s; });
                 __syncthreads();
                 // 2: S67; S123bar, Dbar, S67bar, U from Tbar; A-bar of the A(j,m) S123 term
                 for (long e = threadIdx.x; e < N2nf; e += BS) {
@@ -311,27 +333,33 @@ __device__ __forceinline__ void l4f_adjoint_body(double2* sm, const L4fAdjArgs& 
                             if (F2(j, m) == g) sb7 = cadd(sb7, cmul(cconj(BB(j, m)), Tb[ni + (m + j * N) * N2]));
                     S67b[e] = sb7;
                 }
-                for (int e = threadIdx.x; e < N2; e += BS) {
-                    double2 s = make_double2(0.0, 0.0), d = s;
-                    for (int j = 0; j < N; ++j) {
-                        for (int m = 0; m < N; ++m) s = cadd(s, cmul(cconj(AA(j, m)), Tb[e + (m + j * N) * N2]));
-                        d = cadd(d, Tb[e + (j + j * N) * N2]);
-                    }
-                    S123b[e] = s;
-                    Db[e] = d;
-                }
+                entry_parts<BS>(
+                    N2, part,
+                    [&](int e, int p, int np, double2& s, double2& d) {
+                        for (int q = p; q < N2; q += np) {  // q = m + j N
+                            const int j = q / N, m = q % N;
+                            const double2 tb = Tb[e + q * N2];
+                            s = cadd(s, cmul(cconj(AA(j, m)), tb));
+                            if (j == m) d = cadd(d, tb);
+                        }
+                    },
+                    [&](int e, double2 s, double2 d) {
+                        S123b[e] = s;
+                        Db[e] = d;
+                    });
                 for (int e = threadIdx.x; e < N4; e += BS) {
                     const int r = e % N2, c = e / N2, b = c % N, j = c / N;
                     double2 s = make_double2(0.0, 0.0);
                     for (int m = 0; m < N; ++m) s = cadd(s, cmul(cconj(AA(b, m)), Tb[r + (m + j * N) * N2]));
                     U[e] = s;
                 }
-                for (int e = threadIdx.x; e < N2; e += BS) {
-                    const int j = e % N, m = e / N;
-                    double2 s = make_double2(0.0, 0.0);
-                    for (int r = 0; r < N2; ++r) s = cadd(s, cmul(cconj(S123[r]), Tb[r + (m + j * N) * N2]));
-                    AbA[j + m * N] = cadd(AbA[j + m * N], s);
-                }
+                entry_parts<BS>(
+                    N2, part,
+                    [&](int e, int p, int np, double2& s, double2&) {
+                        const int j = e % N, m = e / N;
+                        for (int r = p; r < N2; r += np) s = cadd(s, cmul(cconj(S123[r]), Tb[r + (m + j * N) * N2]));
+                    },
+                    [&](int e, double2 s, double2) { AbA[e] = cadd(AbA[e], s); });
                 __syncthreads();
                 // 3: Qbar; S123bar gets the D term; operator cotangents of the S67,
                 // Q and D terms of T and of S67 = A Q and D = -A S123
@@ -351,13 +379,14 @@ __device__ __forceinline__ void l4f_adjoint_body(double2* sm, const L4fAdjArgs& 
                     for (int n = 0; n < N; ++n) s = csub(s, cmul(cconj(AA(n, a)), Db[n + i * N]));
                     S123b[e] = s;
                 }
-                for (int e = threadIdx.x; e < N2; e += BS) {
-                    const int j = e % N, m = e / N;
-                    const long go = static_cast<long>(F2(j, m)) * N2;
-                    double2 s = make_double2(0.0, 0.0);
-                    for (int r = 0; r < N2; ++r) s = cadd(s, cmul(cconj(S67[go + r]), Tb[r + (m + j * N) * N2]));
-                    AbB[j + m * N] = cadd(AbB[j + m * N], s);
-                }
+                entry_parts<BS>(
+                    N2, part,
+                    [&](int e, int p, int np, double2& s, double2&) {
+                        const int j = e % N, m = e / N;
+                        const long go = static_cast<long>(F2(j, m)) * N2;
+                        for (int r = p; r < N2; r += np) s = cadd(s, cmul(cconj(S67[go + r]), Tb[r + (m + j * N) * N2]));
+                    },
+                    [&](int e, double2 s, double2) { AbB[e] = cadd(AbB[e], s); });
                 __syncthreads();
                 // v(j,b,m) = sum_r conj(Q(r, f(j,b))) Tbar(r; m,j), in U's space (U is done)
                 double2* V = U;
@@ -384,20 +413,18 @@ __device__ __forceinline__ void l4f_adjoint_body(double2* sm, const L4fAdjArgs& 
                     AbB[j + b * N] = csub(AbB[j + b * N], s);
                 }
                 __syncthreads();
-                for (int e = threadIdx.x; e < N2; e += BS) {
-                    const int n = e % N, a = e / N;
-                    double2 s = make_double2(0.0, 0.0);
-                    for (int i = 0; i < N; ++i) {
-                        s = csub(s, cmul(cconj(S123[a + i * N]), Db[n + i * N]));
-                        for (int g = 0; g < nf; ++g)
-                            s = cadd(s, cmul(cconj(Q[a + i * N + g * N2]), S67b[n + i * N + g * N2]));
-                    }
-                    AbA[n + a * N] = cadd(AbA[n + a * N], s);
-                }
+                entry_parts<BS>(
+                    N2, part,
+                    [&](int e, int p, int np, double2& s, double2&) {
+                        const int n = e % N, a = e / N;
+                        for (int q = p; q < N * nf; q += np)  // q = i + g N
+                            s = cadd(s, cmul(cconj(Q[a + q * N]), S67b[n + q * N]));
+                        for (int i = p; i < N; i += np) s = csub(s, cmul(cconj(S123[a + i * N]), Db[n + i * N]));
+                    },
+                    [&](int e, double2 s, double2) { AbA[e] = cadd(AbA[e], s); });
                 __syncthreads();
                 // 4: slice and operator cotangents of Q and of S123, each entry owned by
                 // one thread that sums its terms in a fixed order (no atomics)
-                auto Xv = [&](long x) { return cadd(Cp[x], Rp[x]); };
                 // X = C + R slices: pair (x, z) and bucket g gather the Q-bar terms
                 for (long e = threadIdx.x; e < static_cast<long>(A.nxp) * nf; e += BS) {
                     const int pp = static_cast<int>(e % A.nxp), g = static_cast<int>(e / A.nxp);
@@ -413,8 +440,8 @@ __device__ __forceinline__ void l4f_adjoint_body(double2* sm, const L4fAdjArgs& 
                     }
                     const int xz = A.xp_xz[pp];
                     const long x = id3(xz & 65535, g, xz >> 16);
-                    sC[x] = cadd(sC[x], acc);
-                    sR[x] = cadd(sR[x], acc);
+                    sC[x] = first ? acc : cadd(sC[x], acc);
+                    sR[x] = first ? acc : cadd(sR[x], acc);
                 }
                 __syncthreads();
                 // F and R slices of the M, I, K terms of S123
@@ -429,7 +456,7 @@ __device__ __forceinline__ void l4f_adjoint_body(double2* sm, const L4fAdjArgs& 
                         else          // -B(n,a) A(a,b) B(b,i) M, M = F - R
                             acc = csub(acc, cmul(cconj(cmul(cmul(BB(n, a), AA(a, b)), BB(b, i))), sv));
                     }
-                    sF[A.f_tgt[e]] = cadd(sF[A.f_tgt[e]], acc);
+                    sF[A.f_tgt[e]] = first ? acc : cadd(sF[A.f_tgt[e]], acc);
                 }
                 for (int e = threadIdx.x; e < A.nrt; e += BS) {
                     double2 acc = make_double2(0.0, 0.0);
@@ -442,7 +469,8 @@ __device__ __forceinline__ void l4f_adjoint_body(double2* sm, const L4fAdjArgs& 
                         else          // the -R part of M
                             acc = cadd(acc, cmul(cconj(cmul(cmul(BB(n, a), AA(a, b)), BB(b, i))), sv));
                     }
-                    sR[A.r_tgt[e]] = cadd(sR[A.r_tgt[e]], acc);
+                    const int x = A.r_tgt[e] & 0x7fffffff;
+                    sR[x] = first && A.r_tgt[e] < 0 ? acc : cadd(sR[x], acc);
                 }
                 __syncthreads();
                 auto Mv = [&](int n, int i, int a, int b) {
@@ -451,61 +479,72 @@ __device__ __forceinline__ void l4f_adjoint_body(double2* sm, const L4fAdjArgs& 
                 auto Iv = [&](int n, int i, int a, int b) { return Fp[id3(F2(a, n), F2(b, i), F2(n, b))]; };
                 auto Kv = [&](int n, int i, int a, int b) { return Rp[id3(F2(i, b), F2(n, a), F2(a, i))]; };
                 // operator entries at (a,b) of the Q and S123 terms
-                for (int e = threadIdx.x; e < N2; e += BS) {
-                    const int a = e % N, b = e / N;
-                    double2 sa = make_double2(0.0, 0.0), sbb = sa;
-                    for (int i = 0; i < N; ++i)
-                        for (int g = 0; g < nf; ++g) {
-                            const double2 qb = Qb[a + i * N + g * N2];
-                            sa = cadd(sa, cmul(cconj(cmul(BB(b, i), Xv(id3(F2(b, a), g, F2(a, i))))), qb));
-                            sbb = csub(sbb, cmul(cconj(cmul(AA(b, i), Xv(id3(F2(i, b), g, F2(a, i))))), qb));
-                        }
-                    for (int n = 0; n < N; ++n)
-                        for (int i = 0; i < N; ++i) {
+                entry_parts<BS>(
+                    N2, part,
+                    [&](int e, int p, int np, double2& sa, double2& sbb) {
+                        const int a = e % N, b = e / N;
+                        for (int g = p; g < nf; g += np)  // a bucket's row of X serves every i
+                            for (int i = 0; i < N; ++i) {
+                                const int z = F2(a, i);
+                                const double2 qb = Qb[a + i * N + g * N2];
+                                sa = cadd(sa, cmul(cconj(cmul(BB(b, i), xval(xrow(F2(b, a), z) + g * xstep))), qb));
+                                sbb = csub(sbb, cmul(cconj(cmul(AA(b, i), xval(xrow(F2(i, b), z) + g * xstep))), qb));
+                            }
+                        for (int q = p; q < N2; q += np) {  // q = i + n N
+                            const int n = q / N, i = q % N;
                             const double2 sv = S123b[n + i * N];
                             sa = csub(sa, cmul(cconj(cmul(cmul(BB(n, a), BB(b, i)), Mv(n, i, a, b))), sv));
                             sbb = cadd(sbb, cmul(cconj(cmul(cmul(AA(n, a), BB(b, i)), Iv(n, i, a, b))), sv));
                             sbb = csub(sbb, cmul(cconj(cmul(cmul(BB(n, a), AA(b, i)), Kv(n, i, a, b))), sv));
                         }
-                    AbA[a + b * N] = cadd(AbA[a + b * N], sa);
-                    AbB[a + b * N] = cadd(AbB[a + b * N], sbb);
-                }
+                    },
+                    [&](int e, double2 sa, double2 sbb) {
+                        AbA[e] = cadd(AbA[e], sa);
+                        AbB[e] = cadd(AbB[e], sbb);
+                    });
                 __syncthreads();
                 // operator entries at (b,i)
-                for (int e = threadIdx.x; e < N2; e += BS) {
-                    const int b = e % N, i = e / N;
-                    double2 sa = make_double2(0.0, 0.0), sbb = sa;
-                    for (int a = 0; a < N; ++a)
-                        for (int g = 0; g < nf; ++g) {
-                            const double2 qb = Qb[a + i * N + g * N2];
-                            sbb = cadd(sbb, cmul(cconj(cmul(AA(a, b), Xv(id3(F2(b, a), g, F2(a, i))))), qb));
-                            sa = csub(sa, cmul(cconj(cmul(BB(a, b), Xv(id3(F2(i, b), g, F2(a, i))))), qb));
-                        }
-                    for (int n = 0; n < N; ++n)
-                        for (int a = 0; a < N; ++a) {
+                entry_parts<BS>(
+                    N2, part,
+                    [&](int e, int p, int np, double2& sa, double2& sbb) {
+                        const int b = e % N, i = e / N;
+                        for (int g = p; g < nf; g += np)
+                            for (int a = 0; a < N; ++a) {
+                                const int z = F2(a, i);
+                                const double2 qb = Qb[a + i * N + g * N2];
+                                sbb = cadd(sbb, cmul(cconj(cmul(AA(a, b), xval(xrow(F2(b, a), z) + g * xstep))), qb));
+                                sa = csub(sa, cmul(cconj(cmul(BB(a, b), xval(xrow(F2(i, b), z) + g * xstep))), qb));
+                            }
+                        for (int q = p; q < N2; q += np) {  // q = a + n N
+                            const int n = q / N, a = q % N;
                             const double2 sv = S123b[n + i * N];
                             sbb = csub(sbb, cmul(cconj(cmul(cmul(BB(n, a), AA(a, b)), Mv(n, i, a, b))), sv));
                             sbb = cadd(sbb, cmul(cconj(cmul(cmul(AA(n, a), BB(a, b)), Iv(n, i, a, b))), sv));
                             sa = csub(sa, cmul(cconj(cmul(cmul(BB(n, a), BB(a, b)), Kv(n, i, a, b))), sv));
                         }
-                    AbA[b + i * N] = cadd(AbA[b + i * N], sa);
-                    AbB[b + i * N] = cadd(AbB[b + i * N], sbb);
-                }
+                    },
+                    [&](int e, double2 sa, double2 sbb) {
+                        AbA[e] = cadd(AbA[e], sa);
+                        AbB[e] = cadd(AbB[e], sbb);
+                    });
                 __syncthreads();
                 // operator entries at (n,a)
-                for (int e = threadIdx.x; e < N2; e += BS) {
-                    const int n = e % N, a = e / N;
-                    double2 sa = make_double2(0.0, 0.0), sbb = sa;
-                    for (int i = 0; i < N; ++i)
-                        for (int b = 0; b < N; ++b) {
+                entry_parts<BS>(
+                    N2, part,
+                    [&](int e, int p, int np, double2& sa, double2& sbb) {
+                        const int n = e % N, a = e / N;
+                        for (int q = p; q < N2; q += np) {  // q = b + i N
+                            const int i = q / N, b = q % N;
                             const double2 sv = S123b[n + i * N];
                             sbb = csub(sbb, cmul(cconj(cmul(cmul(AA(a, b), BB(b, i)), Mv(n, i, a, b))), sv));
                             sa = cadd(sa, cmul(cconj(cmul(cmul(BB(a, b), BB(b, i)), Iv(n, i, a, b))), sv));
                             sbb = csub(sbb, cmul(cconj(cmul(cmul(BB(a, b), AA(b, i)), Kv(n, i, a, b))), sv));
                         }
-                    AbA[n + a * N] = cadd(AbA[n + a * N], sa);
-                    AbB[n + a * N] = cadd(AbB[n + a * N], sbb);
-                }
+                    },
+                    [&](int e, double2 sa, double2 sbb) {
+                        AbA[e] = cadd(AbA[e], sa);
+                        AbB[e] = cadd(AbB[e], sbb);
+                    });
                 __syncthreads();
 #undef AA
 #undef BB
@@ -521,10 +560,16 @@ __device__ __forceinline__ void l4f_adjoint_body(double2* sm, const L4fAdjArgs& 
 // only changes which thread owns it and the results are identical at any
 // size.  Large N (d >= 12: tens of thousands of entries per time, scattered
 // slice gathers) runs 1024 threads per time, whose sixteen waves per CU hide
-// the gathers' latency (d = 16: 23.2 -> 19.0 ms); small N keeps 256 threads
-// (d = 4: 0.43 ms, twice that at 1024).
+// the gathers' latency (d = 16, 201 times: 11.5 ms); small N keeps 256 threads
+// (d = 4, 4001 times: 0.28 ms; twice the time at 1024).
 constexpr int kL4AdjBlockLarge = 1024;
 constexpr int kL4AdjLargeN = 12;
+// Slices of nf^3 values and more (nf >= 26: 0.28 MB and more each) exceed what
+// the caches hold of a time: the reverse then gathers X once per time (d = 16,
+// nf = 81, with the rest of this layout: 19.3 -> 11.5 ms); smaller ones are read
+// in place from the caches,
+// without the extra pass.
+constexpr std::size_t kL4AdjPackedNf3 = std::size_t{1} << 14;
 template <int BS>
 __global__ __launch_bounds__(BS) void k_l4f_adjoint(L4fAdjArgs A) {
     extern __shared__ double2 sm[];
@@ -583,8 +628,12 @@ __device__ __forceinline__ double block_sum(double v, double* ws) {
     return tot;  // valid in thread 0
 }
 
-// Forward prefix scans and reverse suffix scans of one triple.
-__global__ __launch_bounds__(kBlock) void k_fcr_adj_scan(FcrAdjArgs P) {
+// Forward prefix scans and reverse suffix scans of one triple.  The suffix
+// pass takes the phases from the GM series, where the prefix pass leaves them.
+// Latency bounds it (a workgroup's chain of loads, phases and block scans), so
+// the registers are held to four waves per SIMD (d = 16, 201 times, 1.5e5
+// triples: 6.6 -> 6.0 ms).
+__global__ __launch_bounds__(kBlock) __attribute__((amdgpu_waves_per_eu(4, 8))) void k_fcr_adj_scan(FcrAdjArgs P) {
     __shared__ double wsum[8][4];
     __shared__ double wred[4];
     const long p = blockIdx.x;
@@ -634,6 +683,7 @@ __global__ __launch_bounds__(kBlock) void k_fcr_adj_scan(FcrAdjArgs P) {
         const double2 Cb = (mask & 2) ? sb[P.nf3 + tri] : z;
         const double2 Rb = (mask & 4) ? sb[2 * P.nf3 + tri] : z;
         const double2 w = cmul(x1, pm);
+        GM[t] = pp;
         W[t] = w;
         FB[t] = Fb;
         CB[t] = Cb;
@@ -667,7 +717,7 @@ __global__ __launch_bounds__(kBlock) void k_fcr_adj_scan(FcrAdjArgs P) {
         const double2 yF = make_double2(v[0] * dt, v[1] * dt), yC = make_double2(v[2] * dt, v[3] * dt);
         const double2 y3 = make_double2(v[4] * dt, v[5] * dt), y4 = make_double2(v[6] * dt, v[7] * dt);
         const double tdt = static_cast<double>(t) * dt;
-        const double2 pp = phase_plus(prow, t, omega, dt), pm = cconj(pp);
+        const double2 pp = GM[t], pm = cconj(pp);
         const double2 x1 = g1[t], x2 = g2[t], xm = gm[t];
         GM[t] = cmul(yF, cconj(pp));
         G2[t] = cadd(cadd(cmul(cconj(yC), pp), cmul(y3, pp)), cmul(y4, cconj(cmul(x1, pm))));
@@ -687,6 +737,8 @@ __global__ __launch_bounds__(kBlock) void k_fcr_adj_scan(FcrAdjArgs P) {
 //   wbar_u  += dt sum_{t>=u} (-Fbar_t conj(gm_{t-u}) - Cbar_t g2_{t-u})
 //   gmbar_u += dt sum_{t>=u} -Fbar_t conj(w_{t-u})
 //   g2bar_u += conj(dt sum_{t>=u} -Cbar_t conj(w_{t-u}))
+// Bound by FP64 operations: 16 fused multiply-adds per (t, u) pair (unfused
+// products and sums took 32 and twice the time).
 __global__ __launch_bounds__(kBlock) void k_fcr_adj_corr(FcrAdjArgs P) {
     __shared__ double2 fb[kBlock], cb[kBlock];
     __shared__ double2 wgm[2 * kBlock], wg2[2 * kBlock], ww[2 * kBlock];
@@ -728,18 +780,18 @@ __global__ __launch_bounds__(kBlock) void k_fcr_adj_corr(FcrAdjArgs P) {
             for (int q = qlo; q < qhi; ++q) {
                 const int e = static_cast<int>(t0 + q - u - dlo);
                 const double2 f = fb[q], c = cb[q];
-                xw = csub(xw, cadd(cmul(f, cconj(wgm[e])), cmul(c, wg2[e])));
-                xm = csub(xm, cmul(f, cconj(ww[e])));
-                xc = csub(xc, cmul(c, cconj(ww[e])));
+                xw = cfma_conj(wgm[e], f, cfma(wg2[e], c, xw));
+                xm = cfma_conj(ww[e], f, xm);
+                xc = cfma_conj(ww[e], c, xc);
             }
         }
         __syncthreads();
     }
     if (u < T) {
         const double dt = P.dt;
-        WB[u] = cadd(WB[u], cscale(xw, dt));
-        GM[u] = cadd(GM[u], cscale(xm, dt));
-        G2[u] = cadd(G2[u], cconj(cscale(xc, dt)));
+        WB[u] = csub(WB[u], cscale(xw, dt));
+        GM[u] = csub(GM[u], cscale(xm, dt));
+        G2[u] = csub(G2[u], cconj(cscale(xc, dt)));
     }
 }
 

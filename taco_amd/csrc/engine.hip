@@ -1306,21 +1306,22 @@ __global__ __launch_bounds__(kBlock) void k_gw_sym(double2* GW, int N2) {
 }
 
 // ---------------------------------------------------------------------------
-// Factorised L4 for any N (used for N > 8, where k_l4's N^4 LDS tile does
-// not fit).  Every NAKZWAN term of T(n,i;m,j) (tcl4_assemble.cpp:29-178)
-// factors through quantities of (n,i) and a bucket index:
+// Factorised L4 for any N.  Every NAKZWAN term of T(n,i;m,j)
+// (tcl4_assemble.cpp:29-178) factors through quantities of (n,i) and a bucket
+// index:
 //   -t1 + t2 - t3 = A(j,m) S123(n,i)
-//   t6 - t7       = B(j,m) S67(n,i, f(j,m)),  S67 = sum_a A(n,a) Yd(a,i,.)
-//   t4 - t5       = sum_b B(j,b) A(b,m) Wd(n,i, f(j,b))
-//   add1..3       = d(j,m) D(n,i),            D = sum_a A(n,a) E(a,i)
-// with Yd(a,i,beta) = sum_b [A(a,b)B(b,i) X[f(b,a)][beta][f(a,i)]
-//                            - B(a,b)A(b,i) X[f(i,b)][beta][f(a,i)]],
-// Wd(n,i,g) = sum_a [A(n,a)B(a,i) X[f(a,n)][g][f(n,i)]
-//                    - B(n,a)A(a,i) X[f(i,a)][g][f(n,i)]],  X = C + R,
+//   t6 - t7       = B(j,m) S67(n,i, f(j,m)),  S67 = sum_a A(n,a) Q(a,i,.)
+//   t4 - t5       = - sum_b B(j,b) A(b,m) Q(n,i, f(j,b))
+//   add1..3       = d(j,m) D(n,i),            D = - sum_a A(n,a) S123(a,i)
+// with Q(a,i,g) = sum_b [A(a,b)B(b,i) X[f(b,a)][g][f(a,i)]
+//                        - B(a,b)A(b,i) X[f(i,b)][g][f(a,i)]],  X = C + R,
 // so T costs O(N^5 + N^3 nf) per time instead of O(N^6).  The sums run in a
 // different order from the reference's, so values agree to rounding, not
-// bit for bit.  One workgroup per time; the intermediates of a time live in
-// its slice of a global scratch (L2-resident).
+// bit for bit.  One workgroup per time.  The N^2 sums of S123 are split over
+// the threads that N^2 entries leave idle (entry_parts).  The intermediates
+// of a time live in LDS with T while they fit (N <= 5), each T formed once
+// for its two entries of L4; else in the time's slice of a global scratch,
+// and T is formed where it is read.
 // ---------------------------------------------------------------------------
 struct L4fArgs {
     const double2* Fs;   // [npos][nf3]
@@ -1334,15 +1335,47 @@ struct L4fArgs {
     double2* GW;         // optional [npos][N^4]
     double2* scr;        // [npos][scr_per]
     long scr_per;        // complex values per position
+    bool parts;          // room for entry_parts in LDS
 };
 
-template <int BS>
+// Sums of N^2 entries by a workgroup of BS threads, P = BS / N^2 threads each:
+// body(e, p, P, s, u) adds part p of entry e's sums to s and u, and done(e, s, u)
+// takes the totals, the parts added in order.  part: 2 BS values of LDS (null:
+// one thread per entry).
+template <int BS, class Body, class Done>
+__device__ __forceinline__ void entry_parts(int N2, double2* part, Body&& body, Done&& done) {
+    const int EB = N2 < BS ? N2 : BS, P = part ? BS / EB : 1;
+    const int el = threadIdx.x % EB, p = threadIdx.x / EB;
+    for (int e0 = 0; e0 < N2; e0 += EB) {
+        const int e = e0 + el;
+        double2 s = make_double2(0.0, 0.0), u = s;
+        if (e < N2 && p < P) body(e, p, P, s, u);
+        if (P > 1) {
+            part[threadIdx.x] = s;
+            part[BS + threadIdx.x] = u;
+            __syncthreads();
+            if (p == 0)
+                for (int q = 1; q < P; ++q) {
+                    s = cadd(s, part[q * EB + el]);
+                    u = cadd(u, part[BS + q * EB + el]);
+                }
+        }
+        if (p == 0 && e < N2) done(e, s, u);
+        if (P > 1) __syncthreads();
+    }
+}
+
+template <int BS, bool LDS>
 __global__ __launch_bounds__(BS) void k_l4f(L4fArgs A) {
     extern __shared__ double2 sm[];
     const int N = A.N, N2 = N * N, nf = A.nf, P = A.num_ops * A.num_ops;
     const long pos = blockIdx.x;
     double2* opsS = sm;                                          // num_ops * N^2
-    int* f = reinterpret_cast<int*>(opsS + A.num_ops * N2);      // N^2
+    double2* part = A.parts ? opsS + A.num_ops * N2 : nullptr;   // 2 BS
+    double2* lds = opsS + A.num_ops * N2 + (A.parts ? 2 * BS : 0);  // LDS: intermediates, then T
+    const long per_pair = 2L * N2 + 2L * N2 * nf;                // [S123 N2][D N2][S67 N2 nf][Q N2 nf]
+    const long N4 = static_cast<long>(N2) * N2;
+    int* f = reinterpret_cast<int*>(lds + (LDS ? P * per_pair + N4 : 0));  // N^2
     for (int e = threadIdx.x; e < A.num_ops * N2; e += BS) opsS[e] = A.ops[e];
     int bad = 0;
     for (int e = threadIdx.x; e < N2; e += BS) {
@@ -1353,7 +1386,6 @@ __global__ __launch_bounds__(BS) void k_l4f(L4fArgs A) {
     // never saw) would index outside the slices: the time's L4 becomes NaN.
     if (__syncthreads_or(bad)) {
         const double nan = __builtin_nan("");
-        const long N4 = static_cast<long>(N2) * N2;
         for (long idx = threadIdx.x; idx < N4; idx += BS) {
             A.L4[pos * N4 + idx] = make_double2(nan, nan);
             if (A.GW) A.GW[pos * N4 + idx] = make_double2(nan, nan);
@@ -1367,77 +1399,54 @@ __global__ __launch_bounds__(BS) void k_l4f(L4fArgs A) {
     auto id3 = [nfl](int x, int y, int z) { return (static_cast<long>(x) * nfl + y) * nfl + z; };
     auto F2 = [f, N](int r, int c) { return f[r + c * N]; };
     auto X = [&](long e) { return cadd(Cp[e], Rp[e]); };
-    // scratch of this time: per pair [S123 N2][D N2][S67 N2 nf][Wd N2 nf], then Yd N2 nf and E N2
-    double2* base = A.scr + pos * A.scr_per;
-    const long per_pair = 2L * N2 + 2L * N2 * nf;
-    double2* Yd = base + P * per_pair;
-    double2* Ev = Yd + static_cast<long>(N2) * nf;
+    double2* base = LDS ? lds : A.scr + pos * A.scr_per;
     for (int iA = 0; iA < A.num_ops; ++iA)
         for (int iB = 0; iB < A.num_ops; ++iB) {
             const double2* Ap = opsS + iA * N2;
             const double2* Bp = opsS + iB * N2;
 #define AA(r, c) Ap[(r) + (c) * N]
 #define BB(r, c) Bp[(r) + (c) * N]
-            double2* pb = base + (iA * A.num_ops + iB) * per_pair;
-            double2* S123 = pb;
-            double2* Dv = pb + N2;
-            double2* S67 = pb + 2 * N2;
-            double2* Wd = S67 + static_cast<long>(N2) * nf;
-            // stage 1: Yd(a,i,beta), Wd(n,i,g), S123(n,i), E(a,i)
-            for (long e = threadIdx.x; e < static_cast<long>(N2) * nf; e += BS) {
-                const int a = static_cast<int>(e % N), i = static_cast<int>((e / N) % N);
-                const int g = static_cast<int>(e / N2);
-                double2 y = make_double2(0.0, 0.0), w = y;
+            double2* S123 = base + (iA * A.num_ops + iB) * per_pair;
+            double2* Dv = S123 + N2;
+            double2* S67 = Dv + N2;
+            double2* Q = S67 + static_cast<long>(N2) * nf;
+            // stage 1: Q(a,i,g) and S123(n,i)
+            for (int e = threadIdx.x; e < N2 * nf; e += BS) {
+                const int a = e % N, i = (e / N) % N, g = e / N2;
+                double2 y = make_double2(0.0, 0.0);
                 for (int b = 0; b < N; ++b) {
                     y = cadd(y, cmul(cmul(AA(a, b), BB(b, i)), X(id3(F2(b, a), g, F2(a, i)))));
                     y = csub(y, cmul(cmul(BB(a, b), AA(b, i)), X(id3(F2(i, b), g, F2(a, i)))));
                 }
-                // Wd uses (n, i) = (a, i) of this index
-                for (int c = 0; c < N; ++c) {
-                    w = cadd(w, cmul(cmul(AA(a, c), BB(c, i)), X(id3(F2(c, a), g, F2(a, i)))));
-                    w = csub(w, cmul(cmul(BB(a, c), AA(c, i)), X(id3(F2(i, c), g, F2(a, i)))));
-                }
-                Yd[e] = y;
-                Wd[e] = w;
+                Q[e] = y;
             }
-            for (int e = threadIdx.x; e < N2; e += BS) {
-                const int n = e % N, i = e / N;
-                double2 s = make_double2(0.0, 0.0), ev = s;
-                for (int a = 0; a < N; ++a)
-                    for (int b = 0; b < N; ++b) {
+            entry_parts<BS>(
+                N2, part,
+                [&](int e, int p, int np, double2& s, double2&) {
+                    const int n = e % N, i = e / N;
+                    for (int q = p; q < N2; q += np) {
+                        const int a = q / N, b = q % N;
                         const double2 Mv = csub(Fp[id3(F2(b, a), F2(b, i), F2(n, b))], Rp[id3(F2(b, a), F2(n, a), F2(a, i))]);
                         const double2 Iv = Fp[id3(F2(a, n), F2(b, i), F2(n, b))];
                         const double2 Kv = Rp[id3(F2(i, b), F2(n, a), F2(a, i))];
                         s = csub(s, cmul(cmul(cmul(BB(n, a), AA(a, b)), BB(b, i)), Mv));
                         s = cadd(s, cmul(cmul(cmul(AA(n, a), BB(a, b)), BB(b, i)), Iv));
                         s = csub(s, cmul(cmul(cmul(BB(n, a), BB(a, b)), AA(b, i)), Kv));
-                        // E(a', i) with a' = n: sum over (b, c) = (a, b) of this loop
-                        const int ap = n, bb = a, cc = b;
-                        const double2 M2 = csub(Fp[id3(F2(cc, bb), F2(cc, i), F2(ap, cc))],
-                                                Rp[id3(F2(cc, bb), F2(ap, bb), F2(bb, i))]);
-                        const double2 K2 = Rp[id3(F2(i, cc), F2(ap, bb), F2(bb, i))];
-                        const double2 I2 = Fp[id3(F2(bb, ap), F2(cc, i), F2(ap, cc))];
-                        ev = cadd(ev, cmul(cmul(cmul(BB(ap, bb), AA(bb, cc)), BB(cc, i)), M2));
-                        ev = cadd(ev, cmul(cmul(cmul(BB(ap, bb), BB(bb, cc)), AA(cc, i)), K2));
-                        ev = csub(ev, cmul(cmul(cmul(AA(ap, bb), BB(bb, cc)), BB(cc, i)), I2));
                     }
-                S123[e] = s;
-                Ev[e] = ev;
-            }
+                },
+                [&](int e, double2 s, double2) { S123[e] = s; });
             __syncthreads();
-            // stage 2: S67(n,i,beta) = sum_a A(n,a) Yd(a,i,beta); D(n,i) = sum_a A(n,a) E(a,i)
-            for (long e = threadIdx.x; e < static_cast<long>(N2) * nf; e += BS) {
-                const int n = static_cast<int>(e % N);
-                const long rest = e - n;  // (i, beta) part of the index
+            // stage 2: S67(n,i,g) = sum_a A(n,a) Q(a,i,g); D(n,i) = -sum_a A(n,a) S123(a,i)
+            for (int e = threadIdx.x; e < N2 * nf + N2; e += BS) {
+                const bool d = e >= N2 * nf;
+                const int w = d ? e - N2 * nf : e, n = w % N;
+                const double2* src = (d ? S123 : Q) + (w - n);
                 double2 s = make_double2(0.0, 0.0);
-                for (int a = 0; a < N; ++a) s = cadd(s, cmul(AA(n, a), Yd[rest + a]));
-                S67[e] = s;
-            }
-            for (int e = threadIdx.x; e < N2; e += BS) {
-                const int n = e % N, i = e / N;
-                double2 s = make_double2(0.0, 0.0);
-                for (int a = 0; a < N; ++a) s = cadd(s, cmul(AA(n, a), Ev[a + i * N]));
-                Dv[e] = s;
+                for (int a = 0; a < N; ++a) s = cadd(s, cmul(AA(n, a), src[a]));
+                if (d)
+                    Dv[w] = make_double2(-s.x, -s.y);
+                else
+                    S67[w] = s;
             }
             __syncthreads();
 #undef AA
@@ -1453,21 +1462,29 @@ __global__ __launch_bounds__(BS) void k_l4f(L4fArgs A) {
                 const double2* Bp = opsS + iB * N2;
                 const double2* pb = base + (iA * A.num_ops + iB) * per_pair;
                 const double2* S67 = pb + 2 * N2;
-                const double2* Wd = S67 + static_cast<long>(N2) * nf;
+                const double2* Q = S67 + static_cast<long>(N2) * nf;
                 t = cadd(t, cmul(Ap[j + m * N], pb[ni]));
-                t = cadd(t, cmul(Bp[j + m * N], S67[ni + static_cast<long>(F2(j, m)) * N2]));
+                t = cadd(t, cmul(Bp[j + m * N], S67[ni + F2(j, m) * N2]));
                 for (int b = 0; b < N; ++b)
-                    t = csub(t, cmul(cmul(Bp[j + b * N], Ap[b + m * N]), Wd[ni + static_cast<long>(F2(j, b)) * N2]));
+                    t = csub(t, cmul(cmul(Bp[j + b * N], Ap[b + m * N]), Q[ni + F2(j, b) * N2]));
                 if (j == m) t = cadd(t, pb[N2 + ni]);
             }
         return t;
     };
-    const long N4 = static_cast<long>(N2) * N2;
     double2* L = A.L4 + pos * N4;
+    double2* Tt = lds + P * per_pair;
+    if constexpr (LDS) {
+        for (int idx = threadIdx.x; idx < N4; idx += BS) {
+            const int r = idx % N2, c = idx / N2;  // r = (n, i), c = (m, j)
+            Tt[idx] = Tval(r % N, r / N, c % N, c / N);
+        }
+        __syncthreads();
+    }
     for (long idx = threadIdx.x; idx < N4; idx += BS) {
         const int r = static_cast<int>(idx % N2), c = static_cast<int>(idx / N2);  // r = (n, i), c = (m, j)
         const int n = r % N, i = r / N, m = c % N, j = c / N;
-        const double2 g = cadd(Tval(n, i, m, j), cconj(Tval(m, j, n, i)));
+        const double2 g = LDS ? cadd(Tt[idx], cconj(Tt[c + static_cast<long>(r) * N2]))
+                              : cadd(Tval(n, i, m, j), cconj(Tval(m, j, n, i)));
         if (A.GW) A.GW[pos * N4 + idx] = g;
         L[(n + m * N) + static_cast<long>(i + j * N) * N2] = g;
     }
@@ -1480,11 +1497,31 @@ __global__ __launch_bounds__(BS) void k_l4f(L4fArgs A) {
 // waves per CU hide the scattered slice and Gamma reads; small N keeps 256.
 constexpr int kFwdBlockLarge = 1024;
 constexpr int kFwdLargeN = 12;
-static void launch_k_l4f(unsigned grid, int N, std::size_t lds, hipStream_t st, const L4fArgs& F) {
-    if (N >= kFwdLargeN)
-        hipLaunchKernelGGL(k_l4f<kFwdBlockLarge>, dim3(grid), dim3(kFwdBlockLarge), lds, st, F);
+// LDS of k_l4f: operators and pair map, the parts of entry_parts, and (small
+// N) the intermediates with T.
+static std::size_t l4f_lds(int N, int nf, int num_ops, int parts, bool inter) {
+    const std::size_t N2 = static_cast<std::size_t>(N) * N, P = static_cast<std::size_t>(num_ops) * num_ops;
+    return (num_ops * N2 + 2 * static_cast<std::size_t>(parts) + (inter ? P * (2 * N2 + 2 * N2 * nf) + N2 * N2 : 0)) * 16 +
+           N2 * 4;
+}
+constexpr std::size_t kL4fInterLds = 48 * 1024;  // three workgroups per CU and more
+static void launch_k_l4f(unsigned grid, hipStream_t st, L4fArgs F) {
+    F.parts = true;
+    std::size_t lds = l4f_lds(F.N, F.nf, F.num_ops, kBlock, true);
+    if (F.N < kFwdLargeN && lds <= kL4fInterLds) {
+        hipLaunchKernelGGL((k_l4f<kBlock, true>), dim3(grid), dim3(kBlock), lds, st, F);
+        return;
+    }
+    const int bs = F.N >= kFwdLargeN ? kFwdBlockLarge : kBlock;
+    lds = l4f_lds(F.N, F.nf, F.num_ops, bs, false);
+    if (lds > 63 * 1024) {  // large operators: one thread per entry
+        F.parts = false;
+        lds = l4f_lds(F.N, F.nf, F.num_ops, 0, false);
+    }
+    if (bs == kFwdBlockLarge)
+        hipLaunchKernelGGL((k_l4f<kFwdBlockLarge, false>), dim3(grid), dim3(kFwdBlockLarge), lds, st, F);
     else
-        hipLaunchKernelGGL(k_l4f<kBlock>, dim3(grid), dim3(kBlock), lds, st, F);
+        hipLaunchKernelGGL((k_l4f<kBlock, false>), dim3(grid), dim3(kBlock), lds, st, F);
 }
 
 // dst[q] = src[rows[q]] for rows of `len` complex values.
@@ -2657,7 +2694,7 @@ static void launch_l4f(taco_ctx* c, const L4Args& A, long npos) {
         F.L4 = A.L4 + p0 * static_cast<long>(N4);
         if (A.GW) F.GW = A.GW + p0 * static_cast<long>(N4);
         timed(c, K_L4, np * (3.0 * A.nf3 + N4) * 16.0, [&] {
-            launch_k_l4f(static_cast<unsigned>(np), F.N, lds, c->stream, F);
+            launch_k_l4f(static_cast<unsigned>(np), c->stream, F);
         });
         HIP_OK(hipGetLastError());
     }
@@ -3208,7 +3245,7 @@ static void tape_forward(taco_tape& tp, const double* r0, double* samples_out) {
 // (n, i, a, b, kind) and every R slice index with its M and K terms, in a
 // fixed order.  Packed 8 bits per index (N <= 128).
 struct L4AdjLists {
-    std::vector<int> xp_xz, xp_start, xp_ent, f_tgt, f_start, f_ent, r_tgt, r_start, r_ent;
+    std::vector<int> xp_xz, xp_start, xp_ent, f_tgt, f_start, f_ent, r_tgt, r_start, r_ent, xtab;
 };
 
 // CSR of (key, word) pairs: the distinct keys ascending, each key's words in
@@ -3236,7 +3273,7 @@ static L4AdjLists l4_adjoint_lists(const int* p2f, int N, int nf) {
     const long nfl = nf;
     auto id3 = [nfl](long x, long y, long z) { return static_cast<int>((x * nfl + y) * nfl + z); };
     L4AdjLists L;
-    // X-form pairs keyed z nf + x (the order of x + 65536 z), stored as x + 65536 z
+    // X-form pairs keyed x nf + z (the order of the slices), stored as x + 65536 z
     std::vector<int> xk, xw;
     xk.reserve(2 * static_cast<std::size_t>(N) * N * N);
     xw.reserve(xk.capacity());
@@ -3244,13 +3281,18 @@ static L4AdjLists l4_adjoint_lists(const int* p2f, int N, int nf) {
         for (int i = 0; i < N; ++i)
             for (int b = 0; b < N; ++b) {
                 const int w = a | (i << 8) | (b << 16);
-                xk.push_back(f(a, i) * nf + f(b, a));
+                xk.push_back(f(b, a) * nf + f(a, i));
                 xw.push_back(w);
-                xk.push_back(f(a, i) * nf + f(i, b));
+                xk.push_back(f(i, b) * nf + f(a, i));
                 xw.push_back(w | (1 << 24));
             }
     csr_by_key(xk, xw, nfl * nfl, L.xp_xz, L.xp_start, L.xp_ent);
-    for (int& k : L.xp_xz) k = (k % nf) + 65536 * (k / nf);
+    L.xtab.assign(static_cast<std::size_t>(nf) * nf, 0);
+    for (std::size_t q = 0; q < L.xp_xz.size(); ++q) {
+        int& k = L.xp_xz[q];
+        L.xtab[static_cast<std::size_t>(k)] = static_cast<int>(q);
+        k = (k / nf) + 65536 * (k % nf);
+    }
     std::vector<int> fk, fw, rk, rw;
     const std::size_t n4 = static_cast<std::size_t>(N) * N * N * N;
     fk.reserve(2 * n4);
@@ -3275,6 +3317,11 @@ static L4AdjLists l4_adjoint_lists(const int* p2f, int N, int nf) {
                 }
     csr_by_key(fk, fw, nfl * nfl * nfl, L.f_tgt, L.f_start, L.f_ent);
     csr_by_key(rk, rw, nfl * nfl * nfl, L.r_tgt, L.r_start, L.r_ent);
+    // R entries that no X-form pair (x, any g, z) writes: bit 31
+    std::vector<char> outer(static_cast<std::size_t>(nf) * nf, 0);
+    for (int xz : L.xp_xz) outer[static_cast<std::size_t>(xz & 65535) * nf + (xz >> 16)] = 1;
+    for (int& t : L.r_tgt)
+        if (!outer[static_cast<std::size_t>(t / (nf * nf)) * nf + t % nf]) t |= static_cast<int>(1u << 31);
     return L;
 }
 
@@ -3536,8 +3583,10 @@ static void tape_adjoint_tail(taco_tape& tp, const RkRev& rv, const double2* sl,
         const std::size_t sbar_n = T * 3 * nf3, abar_n = T * tp.num_ops * N2;
         const std::size_t nscr = static_cast<std::size_t>(ncomb) * 11 * T;
         const unsigned l4_grid = static_cast<unsigned>(std::min<std::size_t>(T, 1024));
-        const std::size_t l4_per =
-            4 * N2 * static_cast<std::size_t>(tp.nf) + 3 * N2 + N2 * N2 + (lds_tb ? 0 : N2 * N2);
+        const bool packed = !l4_direct && nf3 >= kL4AdjPackedNf3;
+        const std::size_t nxp = packed ? l4_adjoint_lists_cached(c, tp.h_p2f.data(), tp.N, tp.nf).xp_xz.size() : 0;
+        const std::size_t l4_per = 4 * N2 * static_cast<std::size_t>(tp.nf) + 3 * N2 + N2 * N2 + (lds_tb ? 0 : N2 * N2) +
+                                   nxp * static_cast<std::size_t>(tp.nf);
         const std::size_t l4_scr = l4_direct ? 0 : l4_grid * l4_per;
         c->inter2.ensure((sbar_n + abar_n + nscr + static_cast<std::size_t>(tp.nf) * T + l4_scr) * 16 +
                          static_cast<std::size_t>(ncomb) * 8 + 64);
@@ -3547,7 +3596,7 @@ static void tape_adjoint_tail(taco_tape& tp, const RkRev& rv, const double2* sl,
         double2* gb4 = scr + nscr;
         double2* l4s = gb4 + static_cast<std::size_t>(tp.nf) * T;
         double* om = reinterpret_cast<double*>(l4s + l4_scr);
-        if (!lds_sl)
+        if (!lds_sl && l4_direct)  // the factorised kernel stores every entry that is read
             hipLaunchKernelGGL(k_fill_zero, dim3(static_cast<unsigned>((sbar_n + kBlock - 1) / kBlock)), dim3(kBlock),
                                0, c->stream, sbar, static_cast<long>(sbar_n));
         L4AdjArgs A{};
@@ -3588,14 +3637,14 @@ static void tape_adjoint_tail(taco_tape& tp, const RkRev& rv, const double2* sl,
             Af.scr = l4s;
             Af.scr_per = static_cast<long>(l4_per);
             const L4AdjLists& LL = l4_adjoint_lists_cached(c, tp.h_p2f.data(), tp.N, tp.nf);
-            const std::vector<int>* parts_l[9] = {&LL.xp_xz, &LL.xp_start, &LL.xp_ent, &LL.f_tgt, &LL.f_start,
-                                                  &LL.f_ent, &LL.r_tgt, &LL.r_start, &LL.r_ent};
+            const std::vector<int>* parts_l[10] = {&LL.xp_xz, &LL.xp_start, &LL.xp_ent,  &LL.f_tgt, &LL.f_start,
+                                                   &LL.f_ent, &LL.r_tgt,    &LL.r_start, &LL.r_ent, &LL.xtab};
             std::size_t tot = 0;
             for (auto* v : parts_l) tot += v->size();
             tp.bufs.adjl.ensure(std::max<std::size_t>(tot, 1) * sizeof(int));
             int* dl = tp.bufs.adjl.as<int>();
-            const int* dp[9];
-            for (int q = 0; q < 9; ++q) {
+            const int* dp[10];
+            for (int q = 0; q < 10; ++q) {
                 dp[q] = dl;
                 if (!parts_l[q]->empty())
                     HIP_OK(hipMemcpyAsync(dl, parts_l[q]->data(), parts_l[q]->size() * sizeof(int),
@@ -3614,17 +3663,21 @@ static void tape_adjoint_tail(taco_tape& tp, const RkRev& rv, const double2* sl,
             Af.r_start = dp[7];
             Af.r_ent = dp[8];
             Af.nrt = static_cast<int>(LL.r_tgt.size());
+            Af.xtab = packed ? dp[9] : nullptr;
             HIP_OK(hipStreamSynchronize(c->stream));  // the host lists go out of scope
             const bool large = tp.N >= kL4AdjLargeN;
+            const std::size_t with_parts = lds + 2 * static_cast<std::size_t>(large ? kL4AdjBlockLarge : kBlock) * 16;
+            Af.parts = with_parts <= 160 * 1024 ? 1 : 0;
+            const std::size_t lds_f = Af.parts ? with_parts : lds;
             set_fn_lds(large ? reinterpret_cast<const void*>(k_l4f_adjoint<kL4AdjBlockLarge>)
                              : reinterpret_cast<const void*>(k_l4f_adjoint<kBlock>),
-                       lds);
+                       lds_f);
             timed(c, K_L4, 0.0, [&] {
                 if (large)
-                    hipLaunchKernelGGL(k_l4f_adjoint<kL4AdjBlockLarge>, dim3(l4_grid), dim3(kL4AdjBlockLarge), lds,
+                    hipLaunchKernelGGL(k_l4f_adjoint<kL4AdjBlockLarge>, dim3(l4_grid), dim3(kL4AdjBlockLarge), lds_f,
                                        c->stream, Af);
                 else
-                    hipLaunchKernelGGL(k_l4f_adjoint<kBlock>, dim3(l4_grid), dim3(kBlock), lds, c->stream, Af);
+                    hipLaunchKernelGGL(k_l4f_adjoint<kBlock>, dim3(l4_grid), dim3(kBlock), lds_f, c->stream, Af);
             });
         }
         HIP_OK(hipGetLastError());
@@ -4983,7 +5036,7 @@ int taco_l4_from_slices_noalloc(const void* Fs, const void* Cs, const void* Rs, 
             F.Rs = static_cast<const double2*>(Rs) + p0 * nf3;
             F.L4 = static_cast<double2*>(L4_out) + p0 * N4;
             F.GW = GW_out ? static_cast<double2*>(GW_out) + p0 * N4 : nullptr;
-            launch_k_l4f(static_cast<unsigned>(np), F.N, lds, st, F);
+            launch_k_l4f(static_cast<unsigned>(np), st, F);
             HIP_OK(hipGetLastError());
         }
     });

@@ -16,6 +16,21 @@ __device__ __forceinline__ double2 cadd(double2 a, double2 b) { return make_doub
 __device__ __forceinline__ double2 csub(double2 a, double2 b) { return make_double2(a.x - b.x, a.y - b.y); }
 __device__ __forceinline__ double2 cconj(double2 a) { return make_double2(a.x, -a.y); }
 __device__ __forceinline__ double2 cscale(double2 a, double s) { return make_double2(a.x * s, a.y * s); }
+// s + a b and s + conj(a) b with fused multiply-adds.
+__device__ __forceinline__ double2 cfma(double2 a, double2 b, double2 s) {
+    s.x = fma(a.x, b.x, s.x);
+    s.x = fma(-a.y, b.y, s.x);
+    s.y = fma(a.x, b.y, s.y);
+    s.y = fma(a.y, b.x, s.y);
+    return s;
+}
+__device__ __forceinline__ double2 cfma_conj(double2 a, double2 b, double2 s) {
+    s.x = fma(a.x, b.x, s.x);
+    s.x = fma(a.y, b.y, s.x);
+    s.y = fma(a.x, b.y, s.y);
+    s.y = fma(-a.y, b.x, s.y);
+    return s;
+}
 
 // Block -> (job, group block).  Workgroups are dispatched to the 8 XCDs
 // round-robin by id; when possible each XCD keeps a fixed eighth of the

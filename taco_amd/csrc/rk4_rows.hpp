@@ -43,22 +43,6 @@ __device__ __forceinline__ double2 group_sum(double2 v) {
     return v;
 }
 
-// s + a b and s + conj(a) b with fused multiply-adds.
-__device__ __forceinline__ double2 cfma(double2 a, double2 b, double2 s) {
-    s.x = fma(a.x, b.x, s.x);
-    s.x = fma(-a.y, b.y, s.x);
-    s.y = fma(a.x, b.y, s.y);
-    s.y = fma(a.y, b.x, s.y);
-    return s;
-}
-__device__ __forceinline__ double2 cfma_conj(double2 a, double2 b, double2 s) {
-    s.x = fma(a.x, b.x, s.x);
-    s.x = fma(a.y, b.y, s.x);
-    s.y = fma(a.x, b.y, s.y);
-    s.y = fma(-a.y, b.x, s.y);
-    return s;
-}
-
 // Lane's CK entries of a D x D column-major matrix M.  ROWS: lane owns row
 // `o` and columns g + k G (forward products); otherwise column `o` and rows
 // g + k G (adjoint products).  Entries outside the matrix read M[0]: a finite

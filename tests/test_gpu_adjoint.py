@@ -146,6 +146,33 @@ def test_factorised_l4_adjoint_matches_term_walk(monkeypatch, case):
         assert np.abs(x - y).max() <= 1e-12 * np.abs(y).max()
 
 
+@pytest.mark.parametrize("num_ops", [1, 2])
+def test_factorised_l4_adjoint_packed_slices_matches_term_walk(monkeypatch, num_ops):
+    # d = 6 without degenerate gaps has nf = 31 and slices of 31^3 >= 2^14
+    # values, which the factorised reverse gathers once per time; both forms
+    # sum products of the same terms, so they differ by rounding only
+    rng = W.SplitMix64(23)
+    H = W.gue(6, rng)
+    ops = [W.random_hermitian_unit(6, rng) for _ in range(num_ops)]
+    w = W.Workload("g6", H, ops, taco_amd.DrudeLorentz(0.1, 3.0), 0.8, 0.02, 63, list(range(4)), steps=3)
+    S = w.system
+    assert S.nf ** 3 >= 2 ** 14
+    rng = np.random.default_rng(9)
+    Wt = rng.standard_normal((4, 36)) + 1j * rng.standard_normal((4, 36))
+    out = []
+    for kernel in ("factorised", "direct"):
+        if kernel == "direct":
+            monkeypatch.setenv("TACO_L4_ADJ_KERNEL", "direct")
+        tp = AD.Tape(w.gamma, S.omegas, S.mirror, S.pair_to_freq, S.A_eig, S.eps, w.dt, 3, r0_for(6), 4, 2)
+        out.append(tp.adjoint(Wt))
+        tp.close()
+    a, b = out
+    for key in ("gamma", "omegas", "eps", "r0"):
+        assert np.abs(a[key] - b[key]).max() <= 1e-12 * np.abs(b[key]).max(), key
+    for x, y in zip(a["ops"], b["ops"]):
+        assert np.abs(x - y).max() <= 1e-12 * np.abs(y).max()
+
+
 def oracle_spin_pair_rho_lab(orc, prob, p):
     alpha, wc, beta, eps, delta = p
     H1 = 0.5 * eps * AD.SZ + 0.5 * delta * AD.SX
