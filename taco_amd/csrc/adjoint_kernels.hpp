@@ -566,9 +566,7 @@ constexpr int kL4AdjBlockLarge = 1024;
 constexpr int kL4AdjLargeN = 12;
 // Slices of nf^3 values and more (nf >= 26: 0.28 MB and more each) exceed what
 // the caches hold of a time: the reverse then gathers X once per time (d = 16,
-// nf = 81, with the rest of this layout: 19.3 -> 11.5 ms); smaller ones are read
-// in place from the caches,
-// without the extra pass.
+// nf = 81: 13.5 -> 11.5 ms; nf = 19 to 27 the same either way).
 constexpr std::size_t kL4AdjPackedNf3 = std::size_t{1} << 14;
 template <int BS>
 __global__ __launch_bounds__(BS) void k_l4f_adjoint(L4fAdjArgs A) {

@@ -3054,18 +3054,6 @@ static int rk4_block(int D) {
     return kBlock;
 }
 
-// Midpoint series of large-D generators kept while it fits 2 GiB.
-static bool rk4_midpoints_fit(int D, std::size_t steps) {
-    return steps * static_cast<std::size_t>(D) * D * 16 <= (std::size_t{2} << 30);
-}
-static const double2* rk4_midpoints(taco_ctx* c, DevBuf& buf, const double2* Ls, std::size_t steps, int D) {
-    const long D2 = static_cast<long>(D) * D;
-    buf.ensure(steps * static_cast<std::size_t>(D2) * 16);
-    launch_midpoints(Ls, static_cast<long>(steps), D2, buf.as<double2>(), c->stream);
-    HIP_OK(hipGetLastError());
-    return buf.as<double2>();
-}
-
 // Places a chunked run's products and first states at `base`.
 static void rk4_set_chunks(Rk4Sys& S, double2* base) {
     S.q = base;
@@ -3077,17 +3065,17 @@ static void rk4_launch(taco_ctx* ctx, const double2* dLs, const double2* dLh, st
     // algorithmic bytes: every generator read once, every sample written once
     const double gen_bytes = static_cast<double>(steps + 1) * D * D * 16.0 * (dLh ? 2.0 : 1.0);
     const double rk_bytes = gen_bytes + (dsamples ? static_cast<double>(steps / every + 2) * D * 16.0 : 0.0);
+    Rk4Sys S{};
+    S.Ls = dLs;
+    S.r0 = S.r = dr;
+    S.samples = dsamples;
+    S.steps = static_cast<long>(steps);
+    S.dt = dt;
+    S.D = D;
+    S.every = static_cast<long>(every);
+    S.nsamples = dns;
     if (!dLh && rk4_chunked(D, static_cast<long>(steps))) {
         ctx->rkmid.ensure(rk4_chunk_values(D, static_cast<long>(steps)) * 16);
-        Rk4Sys S{};
-        S.Ls = dLs;
-        S.r0 = S.r = dr;
-        S.samples = dsamples;
-        S.steps = static_cast<long>(steps);
-        S.dt = dt;
-        S.D = D;
-        S.every = static_cast<long>(every);
-        S.nsamples = dns;
         rk4_set_chunks(S, ctx->rkmid.as<double2>());
         timed(ctx, K_RK4, rk_bytes, [&] { launch_rk4_chunked(D, nullptr, S, 1, S.steps, ctx->stream); });
         HIP_OK(hipGetLastError());
@@ -3101,15 +3089,17 @@ static void rk4_launch(taco_ctx* ctx, const double2* dLs, const double2* dLh, st
         HIP_OK(hipGetLastError());
         return;
     }
-    int nstage = dLh ? 0 : rk4_nstage(D, 6, static_cast<long>(steps) + 1);
-    if (!dLh && nstage < 2 && steps > 0 && rk4_midpoints_fit(D, steps)) {
-        // generators read from global memory: the midpoints once, so each
-        // step reads four matrices instead of six (the same values)
-        dLh = rk4_midpoints(ctx, ctx->rkmid, dLs, steps, D);
-        nstage = 0;
-    }
+    const int nstage = dLh ? 0 : rk4_nstage(D, 6, static_cast<long>(steps) + 1);
     const std::size_t lds = rk4_lds(D, 6, nstage);
     if (lds > kRkLds) throw Error(TACO_ERR_INVALID, "RK4 kernel supports D <= 1706");
+    if (rk4_wide(D)) {
+        ctx->rkmid.ensure(static_cast<std::size_t>(kRkWideVecs) * D * 16);
+        S.Lh = dLh;
+        S.xs = ctx->rkmid.as<double2>();
+        timed(ctx, K_RK4, rk_bytes, [&] { launch_rk4_wide(D, nullptr, S, 1, S.steps, ctx->stream); });
+        HIP_OK(hipGetLastError());
+        return;
+    }
     timed(ctx, K_RK4, rk_bytes, [&] {
         launch_rk4(D, dLs, dLh, static_cast<long>(steps), dr, dt, static_cast<long>(every), dsamples, dns, nstage,
                    rk4_block(D), lds, ctx->stream);
@@ -3330,22 +3320,9 @@ static L4AdjLists l4_adjoint_lists(const int* p2f, int N, int nf) {
 // step (seg, [steps][4][D]) and dLoss/dr_0 (rb, [D]).
 struct RkRev {
     double2 *gb, *Lb, *seg, *rb;
-    double2 *LsH = nullptr, *vec = nullptr;  // deferred walk: conjugate transposes, cotangent vectors
-    double2* LhH = nullptr;                  // and their midpoints
-    double2 *q = nullptr, *lam = nullptr, *bv = nullptr;  // chunked walk
+    double2* vec = nullptr;                               // deferred and wide walks: kb1..kb4 of every step
+    double2 *q = nullptr, *lam = nullptr, *bv = nullptr;  // chunked walk (lam: wide walk)
 };
-
-// The walk reads transposed generators and leaves Lbar to k_rk4_lbar when it
-// neither has a row-group kernel nor stages generators in LDS nor carries
-// the L0 parts in registers (large D).
-// TACO_RK4_DEFER=0 keeps the in-place walk (a test compares the two).
-static bool rk_rev_deferred(const taco_tape& tp) {
-    if (env_int("TACO_RK4_DEFER", 1) == 0) return false;
-    const int D = tp.N * tp.N;
-    if (D == 4 || D == 9 || D == 16) return false;
-    if (static_cast<long>(D) * D <= static_cast<long>(kRkCarry) * kBlock) return false;
-    return rk4_nstage(D, 12, static_cast<long>(tp.steps) + 1) < 2;
-}
 
 // The row-group walk (D = 4, 9, 16) stores kb1..kb4 per step and leaves
 // Lbar to k_rk4_lbar as well (TACO_RK4_DEFER=0: Lbar formed in the walk).
@@ -3362,8 +3339,8 @@ static std::size_t rk_rev_values(const taco_tape& tp) {
     if (rk4_chunked_walk(static_cast<int>(D), static_cast<long>(tp.steps)))
         return base + 4 * tp.steps * D + rk4_chunk_values(static_cast<int>(D), static_cast<long>(tp.steps)) +
                (tp.steps + kRkChunk - 1) / kRkChunk * D;
-    if (rk_rev_rows_deferred(tp)) return base + 4 * tp.steps * D;
-    return rk_rev_deferred(tp) ? base + tp.T * D * D + 4 * tp.steps * D + tp.steps * D * D : base;
+    if (rk4_wide(static_cast<int>(D))) return base + 4 * tp.steps * D + kRkWideVecs * D;
+    return rk_rev_rows_deferred(tp) ? base + 4 * tp.steps * D : base;
 }
 
 static RkRev rk_rev_at(const taco_tape& tp, double2* base) {
@@ -3373,7 +3350,10 @@ static RkRev rk_rev_at(const taco_tape& tp, double2* base) {
     b.Lb = b.gb + tp.T * D;
     b.seg = b.Lb + tp.T * D * D;
     b.rb = b.seg + 4 * tp.steps * D;
-    if (rk_rev_rows_deferred(tp)) {
+    if (rk4_wide(static_cast<int>(D))) {
+        b.vec = b.rb + D;
+        b.lam = b.vec + 4 * tp.steps * D;
+    } else if (rk_rev_rows_deferred(tp)) {
         b.vec = b.rb + D;
         if (rk4_chunked_walk(static_cast<int>(D), static_cast<long>(tp.steps))) {
             const std::size_t nch = (tp.steps + kRkChunk - 1) / kRkChunk;
@@ -3381,10 +3361,6 @@ static RkRev rk_rev_at(const taco_tape& tp, double2* base) {
             b.lam = b.q + nch * D * D;
             b.bv = b.lam + nch * D;
         }
-    } else if (rk_rev_deferred(tp)) {
-        b.LsH = b.rb + D;
-        b.vec = b.LsH + tp.T * D * D;
-        b.LhH = b.vec + 4 * tp.steps * D;
     }
     return b;
 }
@@ -3396,7 +3372,7 @@ static RkRev rk_rev_at(const taco_tape& tp, double2* base) {
 struct RkRevShape {
     Rk4AdjArgs Rf, R;
     std::size_t lds_f = 0, lds_b = 0, nseg = 0;
-    bool carry = false, rows_f = false, rows_b = false;
+    bool rows_f = false, rows_b = false;
     double bytes = 0.0;
 };
 
@@ -3415,13 +3391,10 @@ static RkRevShape rk_rev_shape(const taco_tape& tp, const RkRev& b) {
     R.D = static_cast<int>(D);
     R.K = tp.K;
     R.dt = tp.dt;
-    R.LsH = b.LsH;
     R.vec = b.vec;
-    R.LhH = b.LhH;
     R.q = b.q;
     R.lam = b.lam;
     R.bv = b.bv;
-    sh.carry = D2 <= static_cast<std::size_t>(kRkCarry) * kBlock;
     sh.nseg = (steps + K - 1) / K;
     const int Di = static_cast<int>(D);
     sh.Rf = R;
@@ -3443,18 +3416,14 @@ static RkRevShape rk_rev_shape(const taco_tape& tp, const RkRev& b) {
 // Reverse RK4 of one tape: gb filled, Lb and rb written.
 static void rk_rev_run(taco_tape& tp, const RkRev& b) {
     taco_ctx* c = tp.ctx;
-    const std::size_t D = static_cast<std::size_t>(tp.N) * tp.N, D2 = D * D;
     const RkRevShape sh = rk_rev_shape(tp, b);
-    const int Di = static_cast<int>(D);
-    if (b.LsH) {
-        launch_conj_transpose(tp.lgen.as<double2>(), b.LsH, Di, static_cast<long>(tp.T), c->stream);
-        launch_midpoints(b.LsH, static_cast<long>(tp.steps), static_cast<long>(D2), b.LhH, c->stream);
-    } else if (!sh.carry) {
-        const long cntL = static_cast<long>(tp.T * D2);
-        hipLaunchKernelGGL(k_fill_zero, dim3(static_cast<unsigned>((cntL + kBlock - 1) / kBlock)), dim3(kBlock), 0,
-                           c->stream, b.Lb, cntL);
-    }
+    const int Di = tp.N * tp.N;
     timed(c, K_RK4, sh.bytes, [&] {
+        if (rk4_wide(Di)) {
+            launch_rk4_wide_reverse(Di, nullptr, sh.R, 1, sh.R.steps, sh.R.K, c->stream);
+            launch_rk4_lbar(sh.R, c->stream);
+            return;
+        }
         // every segment's states and stage points from its checkpoint, all segments at once
         launch_rk4_recompute(sh.Rf, sh.rows_f, static_cast<unsigned>(sh.nseg), sh.lds_f, c->stream);
         if (b.q)
@@ -4203,8 +4172,8 @@ __global__ __launch_bounds__(kBlock) void k_slices_pack(double2* whole, double2*
 
 // Several tapes of one N, step count and checkpoint interval (parameter
 // sets of one model): each set's F/C/R, L4 and TCL2 passes run in turn, the
-// forward RK4 of every set is one launch (a workgroup per set), and so are
-// the reverse RK4's recompute and walk.  The sets' F/C/R slices stay on the
+// forward RK4 runs for all sets together, and so do the reverse RK4's
+// recompute and walk.  The sets' F/C/R slices stay on the
 // device while they fit the context's slice budget: whole when every set's
 // do, else packed to the entries the L4 passes read (about a third of
 // 3 nf^3 at d = 16), set by set in order while the running total fits.  The
@@ -4220,8 +4189,8 @@ struct taco_mtape {
     std::vector<std::size_t> pk_at;          // packed sets: offset of their triple lists in A->pkidx (ints)
     std::vector<std::array<long, 3>> pk_n;   // packed sets: F, C and R entry counts per time
     // A->samp [S][T][D] sampled states, A->rv [S][rk_rev_values] reverse RK4
-    // state, A->args launch arguments, A->mid [S][steps][D^2] midpoint
-    // generators of the forward RK4 (large D)
+    // state, A->args launch arguments, A->mid scratch of the forward RK4
+    // (chunked or wide)
     taco_engine::MtapeArena own;
     taco_engine::MtapeArena* A = nullptr;
     ~taco_mtape() {
@@ -4364,17 +4333,13 @@ static void mtape_forward(taco_mtape& mt, const taco_tape_set* in, double* const
     const std::size_t lds = rows_thr > 0 ? static_cast<std::size_t>(3) * D * 16 : rk4_lds(Di, 6, nstage);
     if (lds > kRkLds) throw Error(TACO_ERR_INVALID, "RK4 kernel supports D <= 1706");
     std::vector<Rk4Sys> sys(S);
-    const bool mids = rows_thr == 0 && nstage < 2 && rk4_midpoints_fit(Di, t0.steps * S);
-    if (mids) mt.A->mid.ensure(S * t0.steps * D * D * 16);
+    const bool wide = rk4_wide(Di);
+    if (wide) mt.A->mid.ensure(S * kRkWideVecs * D * 16);
     for (std::size_t s = 0; s < S; ++s) {
         const taco_tape& tp = *mt.sets[s];
         sys[s] = Rk4Sys{tp.lgen.as<double2>(), nstage, r0d + s * D, rend + s * D, samp + s * T * D,
                         static_cast<long>(tp.steps), tp.dt, Di};
-        if (mids) {
-            double2* m = mt.A->mid.as<double2>() + s * tp.steps * D * D;
-            launch_midpoints(tp.lgen.as<double2>(), static_cast<long>(tp.steps), static_cast<long>(D) * D, m, c->stream);
-            sys[s].Lh = m;
-        }
+        if (wide) sys[s].xs = mt.A->mid.as<double2>() + s * kRkWideVecs * D;
     }
     const bool chunked = rk4_chunked(Di, static_cast<long>(t0.steps));
     if (chunked) {
@@ -4389,6 +4354,9 @@ static void mtape_forward(taco_mtape& mt, const taco_tape_set* in, double* const
         if (chunked)
             launch_rk4_chunked(Di, mt.A->args.as<const Rk4Sys>(), Rk4Sys{}, static_cast<unsigned>(S),
                                static_cast<long>(t0.steps), c->stream);
+        else if (wide)
+            launch_rk4_wide(Di, mt.A->args.as<const Rk4Sys>(), Rk4Sys{}, static_cast<unsigned>(S),
+                            static_cast<long>(t0.steps), c->stream);
         else
             launch_rk4_batch(static_cast<unsigned>(S), mt.A->args.as<const Rk4Sys>(),
                              rows_thr > 0 ? rows_thr : rk4_block(Di), lds, c->stream);
@@ -4419,15 +4387,6 @@ static void mtape_adjoint(taco_mtape& mt, const double* const* samples_bar, doub
         sh = rk_rev_shape(*mt.sets[s], rv[s]);
         args[s] = sh.Rf;
         args[S + s] = sh.R;
-        if (rv[s].LsH) {
-            launch_conj_transpose(mt.sets[s]->lgen.as<double2>(), rv[s].LsH, static_cast<int>(D), static_cast<long>(T),
-                                  c->stream);
-            launch_midpoints(rv[s].LsH, static_cast<long>(T - 1), static_cast<long>(D2), rv[s].LhH, c->stream);
-        } else if (!sh.carry) {
-            const long cntL = static_cast<long>(T * D2);
-            hipLaunchKernelGGL(k_fill_zero, dim3(static_cast<unsigned>((cntL + kBlock - 1) / kBlock)), dim3(kBlock),
-                               0, c->stream, rv[s].Lb, cntL);
-        }
     }
     mt.A->args.ensure(std::max(S * sizeof(Rk4Sys), 2 * S * sizeof(Rk4AdjArgs)));
     const Rk4AdjArgs* dargs = mt.A->args.as<const Rk4AdjArgs>();
@@ -4435,6 +4394,11 @@ static void mtape_adjoint(taco_mtape& mt, const double* const* samples_bar, doub
     const int Di = static_cast<int>(D);
     timed(c, K_RK4, sh.bytes * static_cast<double>(S), [&] {
         const unsigned nt = static_cast<unsigned>(S);
+        if (rk4_wide(Di)) {
+            launch_rk4_wide_reverse(Di, dargs + S, sh.R, nt, sh.R.steps, sh.R.K, c->stream);
+            launch_rk4_lbar_multi(dargs + S, nt, Di, sh.R.steps, c->stream);
+            return;
+        }
         launch_rk4_recompute_multi(dargs, nt, Di, sh.rows_f, static_cast<unsigned>(sh.nseg), sh.lds_f, c->stream);
         if (rv[0].q)
             launch_rk4_chunked_walk(Di, dargs + S, sh.R, nt, sh.R.steps, c->stream);

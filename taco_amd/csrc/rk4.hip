@@ -247,16 +247,6 @@ __global__ __launch_bounds__(kRkBlockMax) void k_rk4_batch(const Rk4Sys* sys) {
         rk4_body<0>(sh, S.nstage, S.Ls, S.Lh, S.steps, S.D, S.r0, S.r, S.dt, 1, S.samples, nullptr);
 }
 
-// out[n] = (L[n] + L[n + 1]) / 2 elementwise for n < count (midpoint
-// generators, formed with the expression the RK4 products use on the fly).
-__global__ __launch_bounds__(kRkBlock) void k_midpoints(const double2* __restrict__ L, long count, long D2,
-                                                      double2* __restrict__ out) {
-    const long total = count * D2;
-    for (long i = blockIdx.x * static_cast<long>(kRkBlock) + threadIdx.x; i < total;
-         i += static_cast<long>(gridDim.x) * kRkBlock)
-        out[i] = cscale(cadd(L[i], L[i + D2]), 0.5);
-}
-
 // y = L^H x (column r of L conjugated, column stride ld), summed over c in order.
 // (General D: column blocks of kMvBlk loads issued ahead, as in matvec_rows.)
 template <int DT>
@@ -319,19 +309,15 @@ __device__ __forceinline__ void matvec_h_half(const double2* __restrict__ L0, co
 // r' = r + s (k1 + 2 k2 + 2 k3 + k4), h = dt/2, s = dt/6, Lh = (L0 + L1)/2.
 // Two launches.  k_rk4_recompute: one workgroup per checkpoint segment (K
 // steps) recomputes, from the checkpoint ck[q] = r_{qK} and with the forward
-// step's own arithmetic, the states r_n and stage points u1..u3 of its
+// step's arithmetic, the states r_n and stage points u1..u3 of its
 // segment; segments are independent, so all run at once.  k_rk4_adjoint:
 // one workgroup walks n = steps-1 .. 0, mapping lam_{n+1} to
 // lam_n = M_n^H lam_{n+1} + gbar_n and forming the cotangents of L_n and
 // L_{n+1}.  LDS: vectors of D, then (nstage >= 2) a window of generators
 // staged with column stride D + 1.  Lbar(t) collects the L1 part of step t-1
 // and the L0 part of step t: the latter is carried in registers
-// (D^2 <= 16 x 256) and each Lbar(t) stored once.  Larger D (generators read
-// from global memory): the walk reads the conjugate transposes LsH (written
-// beforehand by k_conj_transpose, so every product is a row-coalesced
-// matrix-vector product with the same terms in the same order), stores only
-// the step's cotangent vectors kb1..kb4, and k_rk4_lbar forms every Lbar(t)
-// afterwards, all times at once, with the walk's own sums.
+// (D^2 <= 16 x 256) and each Lbar(t) stored once.  Larger D take the wide
+// runs below.
 // ---------------------------------------------------------------------------
 
 // Makes generators L_a..L_b resident in the LDS window M (column stride
@@ -348,7 +334,6 @@ struct GenWindow {
     }
 };
 
-template <int DT, bool STAGED>
 __device__ __forceinline__ void rk4_recompute_body(double2* sh, const Rk4AdjArgs& A, long sg) {
     const int D = A.D;
     double2* x = sh;
@@ -358,8 +343,7 @@ __device__ __forceinline__ void rk4_recompute_body(double2* sh, const Rk4AdjArgs
     double2* k4 = k3 + D;
     double2* tmp = k4 + D;
     double2* M = tmp + D;
-    const long D2 = static_cast<long>(D) * D;
-    const int ld = STAGED ? D + 1 : D;
+    const int ld = D + 1;
     GenWindow w;
     const long s0 = sg * A.K, s1 = min(s0 + A.K, A.steps);
     for (int e = threadIdx.x; e < D; e += blockDim.x) x[e] = A.ck[sg * D + e];
@@ -367,19 +351,15 @@ __device__ __forceinline__ void rk4_recompute_body(double2* sh, const Rk4AdjArgs
     for (long n = s0; n < s1; ++n) {
         double2* row = A.seg + n * 4 * D;
         for (int e = threadIdx.x; e < D; e += blockDim.x) row[e] = x[e];
-        if constexpr (STAGED) {
-            w.need(M, A.Ls, n, n + 1, n, min(n + A.nstage - 1, s1), D);
-            rk4_step<DT>(M + (n - w.lo) * D * ld, M + (n + 1 - w.lo) * D * ld, ld, nullptr, x, k1, k2, k3, k4, tmp,
-                         D, A.dt, row + D);
-        } else {
-            rk4_step<DT>(A.Ls + n * D2, A.Ls + (n + 1) * D2, ld, nullptr, x, k1, k2, k3, k4, tmp, D, A.dt, row + D);
-        }
+        w.need(M, A.Ls, n, n + 1, n, min(n + A.nstage - 1, s1), D);
+        rk4_step<0>(M + (n - w.lo) * D * ld, M + (n + 1 - w.lo) * D * ld, ld, nullptr, x, k1, k2, k3, k4, tmp, D, A.dt,
+                    row + D);
     }
 }
 
 // Row-group recompute (rk4_rows with the stage points stashed) for the sizes
-// that have one: the same arithmetic as the forward run, so the states equal
-// the forward's bit for bit.  One workgroup per checkpoint segment.
+// that have one: the plain forward step (a chunked forward's states differ from
+// it by rounding).  One workgroup per checkpoint segment.
 template <int DT>
 __global__ __launch_bounds__(64 * RowGroup<DT>::W) void k_rk4_recompute_rows(Rk4AdjArgs A) {
     extern __shared__ double2 sh[];
@@ -390,15 +370,10 @@ __global__ __launch_bounds__(64 * RowGroup<DT>::W) void k_rk4_recompute_rows(Rk4
 
 __global__ __launch_bounds__(kRkBlock) void k_rk4_recompute(Rk4AdjArgs A) {
     extern __shared__ double2 sh[];
-    const long sg = blockIdx.x;
-    if (A.nstage >= 2) {
-        rk4_recompute_body<0, true>(sh, A, sg);
-    } else {
-        rk4_recompute_body<0, false>(sh, A, sg);
-    }
+    rk4_recompute_body(sh, A, blockIdx.x);
 }
 
-template <int DT, bool STAGED>
+template <int DT>
 __device__ __forceinline__ void rk4_adjoint_body(double2* sh, const Rk4AdjArgs& A) {
     const int D = A.D;
     double2* x = sh;          // r_n
@@ -414,9 +389,8 @@ __device__ __forceinline__ void rk4_adjoint_body(double2* sh, const Rk4AdjArgs& 
     double2* rb = kb2 + D;    // cotangent of r_n being accumulated
     double2* M = rb + D;      // staged generators
     const long D2 = static_cast<long>(D) * D;
-    const int ld = STAGED ? D + 1 : D;
-    const bool carry = D2 <= static_cast<long>(kRkCarry) * blockDim.x;
-    double2 Lc[kRkCarry];     // L0 part of the step after the current one (carry mode)
+    const int ld = D + 1;
+    double2 Lc[kRkCarry];     // L0 part of the step after the current one
 #pragma unroll
     for (int q = 0; q < kRkCarry; ++q) Lc[q] = make_double2(0.0, 0.0);
     GenWindow w;
@@ -424,22 +398,9 @@ __device__ __forceinline__ void rk4_adjoint_body(double2* sh, const Rk4AdjArgs& 
     for (int e = threadIdx.x; e < D; e += blockDim.x) lam[e] = A.gbar[A.steps * D + e];
     __syncthreads();
     for (long n = A.steps - 1; n >= 0; --n) {
-        const double2* L0;
-        const double2* L1;
-        const double2* H0 = nullptr;  // conjugate transposes (LsH path)
-        const double2* H1 = nullptr;
-        if constexpr (STAGED) {
-            w.need(M, A.Ls, n, n + 1, max(0L, n + 2 - A.nstage), n + 1, D);
-            L0 = M + (n - w.lo) * D * ld;
-            L1 = L0 + D * ld;
-        } else {
-            L0 = A.Ls + n * D2;
-            L1 = L0 + D2;
-            if (A.LsH) {
-                H0 = A.LsH + n * D2;
-                H1 = H0 + D2;
-            }
-        }
+        w.need(M, A.Ls, n, n + 1, max(0L, n + 2 - A.nstage), n + 1, D);
+        const double2* L0 = M + (n - w.lo) * D * ld;
+        const double2* L1 = L0 + D * ld;
         const double2* row = A.seg + n * 4 * D;
         for (int e = threadIdx.x; e < D; e += blockDim.x) {
             x[e] = row[e];
@@ -450,93 +411,48 @@ __device__ __forceinline__ void rk4_adjoint_body(double2* sh, const Rk4AdjArgs& 
         }
         __syncthreads();
         // reverse: r' = r + s (k1 + 2 k2 + 2 k3 + k4)
-        if (H1) matvec_rows<DT>(H1, D, k4, tmp, D); else matvec_h<DT>(L1, ld, k4, tmp, D);  // ub3
+        matvec_h<DT>(L1, ld, k4, tmp, D);  // ub3
         __syncthreads();
         for (int e = threadIdx.x; e < D; e += blockDim.x) {
             k3[e] = cadd(cscale(lam[e], 2.0 * s6), cscale(tmp[e], A.dt));                  // kb3
             rb[e] = cadd(lam[e], tmp[e]);
         }
         __syncthreads();
-        if (A.LhH && H0) matvec_rows<DT>(A.LhH + n * D2, D, k3, tmp, D);                             // ub2
-        else if (H0) matvec_half<DT>(H0, H1, D, k3, tmp, D);
-        else matvec_h_half<DT>(L0, L1, ld, k3, tmp, D);
+        matvec_h_half<DT>(L0, L1, ld, k3, tmp, D);  // ub2
         __syncthreads();
         for (int e = threadIdx.x; e < D; e += blockDim.x) {
             kb2[e] = cadd(cscale(lam[e], 2.0 * s6), cscale(tmp[e], h));
             rb[e] = cadd(rb[e], tmp[e]);
         }
         __syncthreads();
-        if (A.LhH && H0) matvec_rows<DT>(A.LhH + n * D2, D, kb2, tmp, D);                            // ub1
-        else if (H0) matvec_half<DT>(H0, H1, D, kb2, tmp, D);
-        else matvec_h_half<DT>(L0, L1, ld, kb2, tmp, D);
+        matvec_h_half<DT>(L0, L1, ld, kb2, tmp, D);  // ub1
         __syncthreads();
         for (int e = threadIdx.x; e < D; e += blockDim.x) {
             kb1[e] = cadd(cscale(lam[e], s6), cscale(tmp[e], h));
             rb[e] = cadd(rb[e], tmp[e]);
         }
         __syncthreads();
-        if (H0) matvec_rows<DT>(H0, D, kb1, tmp, D); else matvec_h<DT>(L0, ld, kb1, tmp, D);
+        matvec_h<DT>(L0, ld, kb1, tmp, D);
         __syncthreads();
         // generator cotangents: Lbar_h = kb3 u2^H + kb2 u1^H, split half/half
-        double2* Lb0 = A.Lbar + n * D2;
         double2* Lb1 = A.Lbar + (n + 1) * D2;
-        if (!carry && A.vec) {
-            double2* v = A.vec + n * 4 * D;
-            for (int e = threadIdx.x; e < D; e += blockDim.x) {
-                v[e] = kb1[e];
-                v[D + e] = kb2[e];
-                v[2 * D + e] = k3[e];
-                v[3 * D + e] = k4[e];
-            }
-        } else if (carry) {
 #pragma unroll
-            for (int q = 0; q < kRkCarry; ++q) {
-                const long e = threadIdx.x + static_cast<long>(q) * blockDim.x;
-                if (e < D2) {
-                    const int r = static_cast<int>(e % D), c = static_cast<int>(e / D);
-                    const double2 lh = cadd(cmul(k3[r], cconj(u2[c])), cmul(kb2[r], cconj(u1[c])));
-                    Lb1[e] = cadd(Lc[q], cadd(cmul(k4[r], cconj(u3[c])), cscale(lh, 0.5)));
-                    Lc[q] = cadd(cmul(kb1[r], cconj(x[c])), cscale(lh, 0.5));
-                }
-            }
-        } else {
-            // in place, kU elements per thread at a time with their loads issued
-            // first (the same expressions as the remainder loop)
-            constexpr int kU = 8;
-            const long stride = blockDim.x;
-            long e0 = threadIdx.x;
-            for (; e0 + (kU - 1) * stride < D2; e0 += kU * stride) {
-                double2 a0[kU], a1[kU];
-#pragma unroll
-                for (int u = 0; u < kU; ++u) {
-                    a0[u] = Lb0[e0 + u * stride];
-                    a1[u] = Lb1[e0 + u * stride];
-                }
-#pragma unroll
-                for (int u = 0; u < kU; ++u) {
-                    const long e = e0 + u * stride;
-                    const int r = static_cast<int>(e % D), c = static_cast<int>(e / D);
-                    const double2 lh = cadd(cmul(k3[r], cconj(u2[c])), cmul(kb2[r], cconj(u1[c])));
-                    Lb0[e] = cadd(a0[u], cadd(cmul(kb1[r], cconj(x[c])), cscale(lh, 0.5)));
-                    Lb1[e] = cadd(a1[u], cadd(cmul(k4[r], cconj(u3[c])), cscale(lh, 0.5)));
-                }
-            }
-            for (long e = e0; e < D2; e += stride) {
+        for (int q = 0; q < kRkCarry; ++q) {
+            const long e = threadIdx.x + static_cast<long>(q) * blockDim.x;
+            if (e < D2) {
                 const int r = static_cast<int>(e % D), c = static_cast<int>(e / D);
                 const double2 lh = cadd(cmul(k3[r], cconj(u2[c])), cmul(kb2[r], cconj(u1[c])));
-                Lb0[e] = cadd(Lb0[e], cadd(cmul(kb1[r], cconj(x[c])), cscale(lh, 0.5)));
-                Lb1[e] = cadd(Lb1[e], cadd(cmul(k4[r], cconj(u3[c])), cscale(lh, 0.5)));
+                Lb1[e] = cadd(Lc[q], cadd(cmul(k4[r], cconj(u3[c])), cscale(lh, 0.5)));
+                Lc[q] = cadd(cmul(kb1[r], cconj(x[c])), cscale(lh, 0.5));
             }
         }
         for (int e = threadIdx.x; e < D; e += blockDim.x) lam[e] = cadd(cadd(rb[e], tmp[e]), A.gbar[n * D + e]);
         __syncthreads();
     }
-    if (carry) {
 #pragma unroll
-        for (int q = 0; q < kRkCarry; ++q) {
-            const long e = threadIdx.x + static_cast<long>(q) * blockDim.x;
-            if (e < D2) A.Lbar[e] = Lc[q];
-        }
+    for (int q = 0; q < kRkCarry; ++q) {
+        const long e = threadIdx.x + static_cast<long>(q) * blockDim.x;
+        if (e < D2) A.Lbar[e] = Lc[q];
     }
     for (int e = threadIdx.x; e < D; e += blockDim.x) A.r0bar[e] = lam[e];
 }
@@ -554,41 +470,19 @@ __global__ __launch_bounds__(64) void k_rk4_adjoint_rows(Rk4AdjArgs A) {
 
 __global__ __launch_bounds__(kRkBlock) void k_rk4_adjoint(Rk4AdjArgs A) {
     extern __shared__ double2 sh[];
-    if (A.nstage >= 2) {
-        switch (A.D) {  // 4, 9 and 16 have the row-group walk
-            case 25: rk4_adjoint_body<25, true>(sh, A); break;
-            case 36: rk4_adjoint_body<36, true>(sh, A); break;
-            case 49: rk4_adjoint_body<49, true>(sh, A); break;
-            case 64: rk4_adjoint_body<64, true>(sh, A); break;
-            default: rk4_adjoint_body<0, true>(sh, A); break;
-        }
-    } else {
-        rk4_adjoint_body<0, false>(sh, A);  // sizes to 64 always stage
+    switch (A.D) {  // 4, 9 and 16 have the row-group walk
+        case 25: rk4_adjoint_body<25>(sh, A); break;
+        case 36: rk4_adjoint_body<36>(sh, A); break;
+        case 49: rk4_adjoint_body<49>(sh, A); break;
+        case 64: rk4_adjoint_body<64>(sh, A); break;
+        default: rk4_adjoint_body<0>(sh, A); break;
     }
 }
 
-// dst[t] = src[t]^H for count D x D matrices (tiles of 16 x 16 through LDS,
-// coalesced reads and writes).  Grid: (tiles of one matrix, count).
-__global__ __launch_bounds__(kRkBlock) void k_conj_transpose(const double2* __restrict__ src, double2* __restrict__ dst,
-                                                           int D, long count) {
-    __shared__ double2 tile[16][17];
-    const int tiles = (D + 15) / 16;
-    const int ti = static_cast<int>(blockIdx.x) % tiles, tj = static_cast<int>(blockIdx.x) / tiles;
-    const long m = blockIdx.y;
-    if (m >= count) return;
-    const long D2 = static_cast<long>(D) * D;
-    const int lr = threadIdx.x % 16, lc = threadIdx.x / 16;
-    const int r = ti * 16 + lr, c = tj * 16 + lc;  // source element (r, c)
-    if (r < D && c < D) tile[lc][lr] = src[m * D2 + r + static_cast<long>(c) * D];
-    __syncthreads();
-    const int r2 = tj * 16 + lr, c2 = ti * 16 + lc;  // destination element (r2, c2) = conj(src(c2, r2))
-    if (r2 < D && c2 < D) dst[m * D2 + r2 + static_cast<long>(c2) * D] = cconj(tile[lr][lc]);
-}
-
-// Lbar(t), t = 0..steps, from the walk's vectors: the L0 part of step t
+// Lbar(t), t = 0..steps, from a walk's vectors: the L0 part of step t
 // (kb1 x^H + (kb3 u2^H + kb2 u1^H)/2) added to zero, then the L1 part of
-// step t-1 (kb4 u3^H + (kb3 u2^H + kb2 u1^H)/2): the sums the in-place walk
-// forms, in its order.  Grid: (element blocks of D^2, steps + 1[, tapes]).
+// step t-1 (kb4 u3^H + (kb3 u2^H + kb2 u1^H)/2): the sums a walk that forms
+// them in place takes, in its order.  Grid: (element blocks of D^2, steps + 1[, tapes]).
 __device__ __forceinline__ void rk4_lbar_body(const Rk4AdjArgs& A) {
     const int D = A.D;
     const long D2 = static_cast<long>(D) * D;
@@ -634,12 +528,7 @@ __global__ __launch_bounds__(64 * RowGroup<DT>::W) void k_rk4_recompute_rows_mul
 __global__ __launch_bounds__(kRkBlock) void k_rk4_recompute_multi(const Rk4AdjArgs* As) {
     extern __shared__ double2 sh[];
     const Rk4AdjArgs A = As[blockIdx.y];
-    const long sg = blockIdx.x;
-    if (A.nstage >= 2) {
-        rk4_recompute_body<0, true>(sh, A, sg);
-    } else {
-        rk4_recompute_body<0, false>(sh, A, sg);
-    }
+    rk4_recompute_body(sh, A, blockIdx.x);
 }
 
 template <int DT>
@@ -656,16 +545,12 @@ __global__ __launch_bounds__(64) void k_rk4_adjoint_rows_multi(const Rk4AdjArgs*
 __global__ __launch_bounds__(kRkBlock) void k_rk4_adjoint_multi(const Rk4AdjArgs* As) {
     extern __shared__ double2 sh[];
     const Rk4AdjArgs A = As[blockIdx.x];
-    if (A.nstage >= 2) {
-        switch (A.D) {  // 4, 9 and 16 have the row-group walk
-            case 25: rk4_adjoint_body<25, true>(sh, A); break;
-            case 36: rk4_adjoint_body<36, true>(sh, A); break;
-            case 49: rk4_adjoint_body<49, true>(sh, A); break;
-            case 64: rk4_adjoint_body<64, true>(sh, A); break;
-            default: rk4_adjoint_body<0, true>(sh, A); break;
-        }
-    } else {
-        rk4_adjoint_body<0, false>(sh, A);  // sizes to 64 always stage
+    switch (A.D) {  // 4, 9 and 16 have the row-group walk
+        case 25: rk4_adjoint_body<25>(sh, A); break;
+        case 36: rk4_adjoint_body<36>(sh, A); break;
+        case 49: rk4_adjoint_body<49>(sh, A); break;
+        case 64: rk4_adjoint_body<64>(sh, A); break;
+        default: rk4_adjoint_body<0>(sh, A); break;
     }
 }
 
@@ -888,6 +773,240 @@ __global__ __launch_bounds__(64) void k_chunk_carry_rev(const Rk4AdjArgs* arr, R
 }
 
 // ---------------------------------------------------------------------------
+// Wide runs: D > 64 whose generators do not fit the LDS (rk4_wide).  One
+// workgroup reads them at the rate of one CU (D = 256: 1 MB a product, 18 us);
+// here a product is a launch whose workgroups share the rows, so a step is four
+// dependent launches.  Every workgroup first forms the whole stage vector from
+// the earlier products, with the first generator loads already in flight, and
+// workgroup 0 keeps what later launches or the caller read.  Vectors that the
+// next step's first launch both reads and writes alternate by the step's parity.
+// The midpoint generators are formed on the fly: a step then touches one new
+// matrix, the rest is in the L2 slices (row blocks keep their XCD).
+// Sums: 32 (reverse: 64) partial sums a row, then a fixed tree.
+// ---------------------------------------------------------------------------
+constexpr int kWideRows = 8;    // rows of a workgroup: 128 B runs of a column
+constexpr int kWideGroups = kRkBlock / kWideRows;
+constexpr int kWideBlk = 8;     // generator loads in flight
+constexpr int kWideOut = kRkBlock / 64;  // outputs of a reverse workgroup, a wave each
+
+// y[r] = sum_c M(r, c) u[c] for the kWideRows rows of block rb, M = L0 (L1 null)
+// or (L0 + L1) / 2; form() fills u (LDS) in between the first loads and their use.
+template <class Form>
+__device__ __forceinline__ void wide_rows(const double2* __restrict__ L0, const double2* __restrict__ L1, int D, long rb,
+                                          const double2* u, double2* y, Form&& form) {
+    __shared__ double2 part[kRkBlock / 64][kWideRows];
+    const int lr = threadIdx.x % kWideRows, cg = threadIdx.x / kWideRows;
+    const int r = static_cast<int>(rb) * kWideRows + lr;
+    const double2* p0 = L0 + min(r, D - 1);
+    const double2* p1 = L1 ? L1 + min(r, D - 1) : nullptr;
+    double2 v0[kWideBlk], v1[kWideBlk];
+    auto load = [&](int c0) {
+#pragma unroll
+        for (int j = 0; j < kWideBlk; ++j) v0[j] = p0[static_cast<long>(min(c0 + cg + j * kWideGroups, D - 1)) * D];
+        if (p1) {
+#pragma unroll
+            for (int j = 0; j < kWideBlk; ++j) v1[j] = p1[static_cast<long>(min(c0 + cg + j * kWideGroups, D - 1)) * D];
+#pragma unroll
+            for (int j = 0; j < kWideBlk; ++j) v0[j] = cscale(cadd(v0[j], v1[j]), 0.5);
+        }
+    };
+    load(0);
+    form();
+    __syncthreads();
+    double2 s = make_double2(0.0, 0.0);
+    for (int c0 = 0;;) {
+#pragma unroll
+        for (int j = 0; j < kWideBlk; ++j) {
+            const int c = c0 + cg + j * kWideGroups;
+            if (c < D) s = cfma(v0[j], u[c], s);
+        }
+        c0 += kWideBlk * kWideGroups;
+        if (c0 >= D) break;
+        load(c0);
+    }
+#pragma unroll
+    for (int m = kWideRows; m < 64; m *= 2) {
+        s.x += __shfl_xor(s.x, m);
+        s.y += __shfl_xor(s.y, m);
+    }
+    if (threadIdx.x % 64 < kWideRows) part[threadIdx.x / 64][lr] = s;
+    __syncthreads();
+    if (threadIdx.x < kWideRows && r < D) {
+        double2 t = part[0][lr];
+#pragma unroll
+        for (int w = 1; w < kRkBlock / 64; ++w) t = cadd(t, part[w][lr]);
+        y[r] = t;
+    }
+}
+
+// y[r] = sum_c conj(M(c, r)) u[c], one wave per r (columns are contiguous).
+template <class Form>
+__device__ __forceinline__ void wide_columns(const double2* __restrict__ L0, const double2* __restrict__ L1, int D,
+                                             const double2* u, double2* y, Form&& form) {
+    const int lane = threadIdx.x % 64, r = static_cast<int>(blockIdx.x) * kWideOut + threadIdx.x / 64;
+    const long col = static_cast<long>(min(r, D - 1)) * D;
+    constexpr int kBlk = 4;
+    double2 v0[kBlk], v1[kBlk];
+    auto load = [&](int c0) {
+#pragma unroll
+        for (int j = 0; j < kBlk; ++j) v0[j] = L0[col + min(c0 + lane + 64 * j, D - 1)];
+        if (L1) {
+#pragma unroll
+            for (int j = 0; j < kBlk; ++j) v1[j] = L1[col + min(c0 + lane + 64 * j, D - 1)];
+#pragma unroll
+            for (int j = 0; j < kBlk; ++j) v0[j] = cscale(cadd(v0[j], v1[j]), 0.5);
+        }
+    };
+    load(0);
+    form();
+    __syncthreads();
+    double2 s = make_double2(0.0, 0.0);
+    for (int c0 = 0;;) {
+#pragma unroll
+        for (int j = 0; j < kBlk; ++j) {
+            const int c = c0 + lane + 64 * j;
+            if (c < D) s = cfma_conj(v0[j], u[c], s);
+        }
+        c0 += 64 * kBlk;
+        if (c0 >= D) break;
+        load(c0);
+    }
+#pragma unroll
+    for (int m = 1; m < 64; m *= 2) {
+        s.x += __shfl_xor(s.x, m);
+        s.y += __shfl_xor(s.y, m);
+    }
+    if (lane == 0 && r < D) y[r] = s;
+}
+
+__device__ __forceinline__ double2 wide_sum(double2 x, double2 k1, double2 k2, double2 k3, double2 k4, double s6) {
+    return cadd(x, cscale(cadd(cadd(cadd(k1, cscale(k2, 2.0)), cscale(k3, 2.0)), k4), s6));
+}
+
+// Stage STAGE (0..3) of step n of every system; stage 0 at n = steps closes the
+// run.  xs: r_n and k1 of both parities, k2, k3, k4.
+template <int STAGE>
+__global__ __launch_bounds__(kRkBlock) void k_wide_stage(const Rk4Sys* arr, Rk4Sys one, long n) {
+    extern __shared__ double2 u[];
+    const Rk4Sys S = arr ? arr[blockIdx.y] : one;
+    if (n > S.steps || (STAGE && n == S.steps)) return;
+    const int D = S.D;
+    const long D2 = static_cast<long>(D) * D, cur = n & 1;
+    double2 *x = S.xs + cur * D, *k1 = S.xs + (2 + cur) * D;
+    double2 *k2 = S.xs + 4 * D, *k3 = S.xs + 5 * D, *k4 = S.xs + 6 * D;
+    if constexpr (STAGE == 0) {
+        const double2 *xo = S.xs + (1 - cur) * D, *ko = S.xs + (3 - cur) * D;
+        auto form = [&] {
+            const bool keep = S.samples && (n == S.steps || n % S.every == 0);
+            double2* row = keep ? S.samples + (n + S.every - 1) / S.every * D : nullptr;
+            for (int e = threadIdx.x; e < D; e += kRkBlock) {
+                const double2 v = n ? wide_sum(xo[e], ko[e], k2[e], k3[e], k4[e], S.dt / 6.0) : S.r0[e];
+                u[e] = v;
+                if (blockIdx.x) continue;
+                x[e] = v;
+                if (keep) row[e] = v;
+                if (n == S.steps) S.r[e] = v;
+            }
+        };
+        if (n == S.steps) {
+            if (blockIdx.x) return;
+            form();
+            if (threadIdx.x == 0 && S.nsamples) *S.nsamples = S.samples ? (n + S.every - 1) / S.every + 1 : 0;
+            return;
+        }
+        wide_rows(S.Ls + n * D2, nullptr, D, blockIdx.x, u, k1, form);
+    } else {
+        const double2* k = STAGE == 1 ? k1 : STAGE == 2 ? k2 : k3;
+        const double f = STAGE == 3 ? S.dt : 0.5 * S.dt;
+        const double2* L0 = STAGE == 3 ? S.Ls + (n + 1) * D2 : S.Lh ? S.Lh + n * D2 : S.Ls + n * D2;
+        const double2* L1 = STAGE == 3 || S.Lh ? nullptr : S.Ls + (n + 1) * D2;
+        wide_rows(L0, L1, D, blockIdx.x, u, STAGE == 1 ? k2 : STAGE == 2 ? k3 : k4, [&] {
+            for (int e = threadIdx.x; e < D; e += kRkBlock) u[e] = cadd(x[e], cscale(k[e], f));
+        });
+    }
+}
+
+// Stage STAGE of step j of every checkpoint segment: the states and stage
+// points into seg.  The products of step n use vec's rows of n, which the walk
+// fills afterwards.  Grid: (segments x row blocks, tapes).
+template <int STAGE>
+__global__ __launch_bounds__(kRkBlock) void k_wide_segment(const Rk4AdjArgs* arr, Rk4AdjArgs one, int j) {
+    extern __shared__ double2 u[];
+    const Rk4AdjArgs A = arr ? arr[blockIdx.y] : one;
+    const int D = A.D, nrb = (D + kWideRows - 1) / kWideRows;
+    const long sg = blockIdx.x / nrb, rb = blockIdx.x % nrb;
+    const long n = sg * A.K + j, s1 = min((sg + 1) * A.K, A.steps);
+    if (n >= s1) return;
+    const long D2 = static_cast<long>(D) * D;
+    double2 *row = A.seg + n * 4 * D, *k = A.vec + n * 4 * D;
+    const double f = STAGE == 3 ? A.dt : 0.5 * A.dt;
+    const double2* L0 = A.Ls + (STAGE == 3 ? n + 1 : n) * D2;
+    const double2* L1 = STAGE == 1 || STAGE == 2 ? A.Ls + (n + 1) * D2 : nullptr;
+    wide_rows(L0, L1, D, rb, u, k + STAGE * D, [&] {
+        for (int e = threadIdx.x; e < D; e += kRkBlock) {
+            double2 v;
+            if (STAGE)
+                v = cadd(row[e], cscale(k[(STAGE - 1) * D + e], f));
+            else if (j == 0)
+                v = A.ck[sg * D + e];
+            else
+                v = wide_sum(row[e - 4 * D], k[e - 4 * D], k[e - 3 * D], k[e - 2 * D], k[e - D], A.dt / 6.0);
+            u[e] = v;
+            if (rb == 0) row[STAGE * D + e] = v;
+        }
+    });
+}
+
+// Stage STAGE of the reverse of step n: ub3 = L1^H kb4, ub2 = Lh^H kb3,
+// ub1 = Lh^H kb2, ub0 = L0^H kb1 (rk4_adjoint_body); stage 0 first forms
+// lam_{n+1} of the step before, at n = -1 the result.  lam: lam and ub3 of both
+// parities, ub2, ub1, ub0.
+template <int STAGE>
+__global__ __launch_bounds__(kRkBlock) void k_wide_walk(const Rk4AdjArgs* arr, Rk4AdjArgs one, long n) {
+    extern __shared__ double2 u[];
+    const Rk4AdjArgs A = arr ? arr[blockIdx.y] : one;
+    const int D = A.D;
+    const long D2 = static_cast<long>(D) * D, cur = n & 1;
+    double2 *lam = A.lam + cur * D, *ub3 = A.lam + (2 + cur) * D;
+    double2 *ub2 = A.lam + 4 * D, *ub1 = A.lam + 5 * D, *ub0 = A.lam + 6 * D;
+    const double s6 = A.dt / 6.0, h = 0.5 * A.dt;
+    double2* v = A.vec + n * 4 * D;  // kb1..kb4
+    if constexpr (STAGE == 0) {
+        const double2 *lo = A.lam + (1 - cur) * D, *uo = A.lam + (3 - cur) * D;
+        auto form = [&] {
+            for (int e = threadIdx.x; e < D; e += kRkBlock) {
+                double2 l = A.gbar[(n + 1) * D + e];
+                if (n + 1 < A.steps) l = cadd(cadd(cadd(cadd(cadd(lo[e], uo[e]), ub2[e]), ub1[e]), ub0[e]), l);
+                const double2 kb4 = cscale(l, s6);
+                u[e] = kb4;
+                if (blockIdx.x) continue;
+                if (n < 0) {
+                    A.r0bar[e] = l;
+                } else {
+                    lam[e] = l;
+                    v[3 * D + e] = kb4;
+                }
+            }
+        };
+        if (n < 0) {
+            if (blockIdx.x == 0) form();
+            return;
+        }
+        wide_columns(A.Ls + (n + 1) * D2, nullptr, D, u, ub3, form);
+    } else {
+        const double2* ub = STAGE == 1 ? ub3 : STAGE == 2 ? ub2 : ub1;
+        const double2 *L0 = A.Ls + n * D2, *L1 = STAGE == 3 ? nullptr : L0 + D2;
+        wide_columns(L0, L1, D, u, STAGE == 1 ? ub2 : STAGE == 2 ? ub1 : ub0, [&] {
+            for (int e = threadIdx.x; e < D; e += kRkBlock) {
+                const double2 kb = cadd(cscale(lam[e], STAGE == 3 ? s6 : 2.0 * s6), cscale(ub[e], STAGE == 1 ? A.dt : h));
+                u[e] = kb;
+                if (blockIdx.x == 0) v[(3 - STAGE) * D + e] = kb;
+            }
+        });
+    }
+}
+
+// ---------------------------------------------------------------------------
 // Launches
 // ---------------------------------------------------------------------------
 hipError_t rk4_set_lds_limits() {
@@ -960,16 +1079,39 @@ void launch_rk4_batch(unsigned nsys, const Rk4Sys* sys, int block, std::size_t l
     hipLaunchKernelGGL(k_rk4_batch, dim3(nsys), dim3(block), lds, st, sys);
 }
 
-void launch_midpoints(const double2* L, long count, long D2, double2* out, hipStream_t st) {
-    const long total = count * D2;
-    const unsigned grid = static_cast<unsigned>(total < 65536L * kRkBlock ? (total + kRkBlock - 1) / kRkBlock : 65536);
-    hipLaunchKernelGGL(k_midpoints, dim3(grid), dim3(kRkBlock), 0, st, L, count, D2, out);
+static dim3 wide_grid(int D, unsigned y, int per = kWideRows) { return dim3(static_cast<unsigned>((D + per - 1) / per), y); }
+
+void launch_rk4_wide(int D, const Rk4Sys* arr, const Rk4Sys& one, unsigned nsys, long max_steps, hipStream_t st) {
+    const dim3 grid = wide_grid(D, nsys), block(kRkBlock);
+    const std::size_t lds = static_cast<std::size_t>(D) * 16;
+    for (long n = 0; n < max_steps; ++n) {
+        hipLaunchKernelGGL(k_wide_stage<0>, grid, block, lds, st, arr, one, n);
+        hipLaunchKernelGGL(k_wide_stage<1>, grid, block, lds, st, arr, one, n);
+        hipLaunchKernelGGL(k_wide_stage<2>, grid, block, lds, st, arr, one, n);
+        hipLaunchKernelGGL(k_wide_stage<3>, grid, block, lds, st, arr, one, n);
+    }
+    hipLaunchKernelGGL(k_wide_stage<0>, dim3(1, nsys), block, lds, st, arr, one, max_steps);
 }
 
-void launch_conj_transpose(const double2* src, double2* dst, int D, long count, hipStream_t st) {
-    const int tiles = (D + 15) / 16;
-    hipLaunchKernelGGL(k_conj_transpose, dim3(static_cast<unsigned>(tiles * tiles), static_cast<unsigned>(count)),
-                       dim3(kRkBlock), 0, st, src, dst, D, count);
+void launch_rk4_wide_reverse(int D, const Rk4AdjArgs* arr, const Rk4AdjArgs& one, unsigned ntapes, long steps, int K,
+                             hipStream_t st) {
+    const dim3 block(kRkBlock);
+    const std::size_t lds = static_cast<std::size_t>(D) * 16;
+    const dim3 gs(wide_grid(D, 1).x * static_cast<unsigned>((steps + K - 1) / K), ntapes);
+    for (int j = 0; j < K && j < steps; ++j) {
+        hipLaunchKernelGGL(k_wide_segment<0>, gs, block, lds, st, arr, one, j);
+        hipLaunchKernelGGL(k_wide_segment<1>, gs, block, lds, st, arr, one, j);
+        hipLaunchKernelGGL(k_wide_segment<2>, gs, block, lds, st, arr, one, j);
+        hipLaunchKernelGGL(k_wide_segment<3>, gs, block, lds, st, arr, one, j);
+    }
+    const dim3 gw = wide_grid(D, ntapes, kWideOut);
+    for (long n = steps - 1; n >= 0; --n) {
+        hipLaunchKernelGGL(k_wide_walk<0>, gw, block, lds, st, arr, one, n);
+        hipLaunchKernelGGL(k_wide_walk<1>, gw, block, lds, st, arr, one, n);
+        hipLaunchKernelGGL(k_wide_walk<2>, gw, block, lds, st, arr, one, n);
+        hipLaunchKernelGGL(k_wide_walk<3>, gw, block, lds, st, arr, one, n);
+    }
+    hipLaunchKernelGGL(k_wide_walk<0>, dim3(1, ntapes), block, lds, st, arr, one, -1L);
 }
 
 void launch_rk4_recompute(const Rk4AdjArgs& A, bool rows, unsigned nseg, std::size_t lds, hipStream_t st) {

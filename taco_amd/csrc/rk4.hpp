@@ -50,9 +50,9 @@ struct Rk4Sys {
     long steps;
     double dt;
     int D;
-    const double2* Lh = nullptr;  // [steps][D x D] midpoints (large D), else formed on the fly
+    const double2* Lh = nullptr;  // [steps][D x D] given midpoints, else formed on the fly
     double2* q = nullptr;         // chunked run: [chunks][D x D] products, null: one sequential run
-    double2* xs = nullptr;        // chunked run: [chunks][D] first states
+    double2* xs = nullptr;        // chunked run: [chunks][D] first states; wide run: kRkWideVecs x D
     long every = 1;               // sample distance
     long* nsamples = nullptr;
 };
@@ -69,11 +69,9 @@ struct Rk4AdjArgs {
     int K;
     double dt;
     int nstage;
-    const double2* LsH = nullptr;  // [steps + 1][D * D] conjugate transposes (walk without staging)
-    const double2* LhH = nullptr;  // [steps][D * D] their midpoints (null: formed on the fly)
     double2* vec = nullptr;        // [steps][4][D] kb1..kb4 of every step (Lbar formed by k_rk4_lbar)
     double2* q = nullptr;          // chunked walk: [chunks][D * D] products,
-    double2* lam = nullptr;        // [chunks][D] lam after each chunk's last step,
+    double2* lam = nullptr;        // [chunks][D] lam after each chunk's last step (wide walk: kRkWideVecs x D),
     double2* bv = nullptr;         // [chunks][D] constant parts
 };
 
@@ -95,6 +93,15 @@ inline std::size_t rk4_chunk_values(int D, long steps) {
     return nch * (static_cast<std::size_t>(D) * D + D);
 }
 
+// Whether runs at D are wide (rk4.hip): two generators do not fit the LDS
+// beside the vectors, so one workgroup would read every product's generator
+// from memory (D = 256: 18 us a product; a wide product takes 4 us for one
+// system or four, and 300 steps gain 1.3 ms at D = 81, 4 ms at D = 144).
+inline bool rk4_wide(int D) {
+    return D > 64 && (6 * static_cast<std::size_t>(D) + 2 * static_cast<std::size_t>(D) * (D + 1)) * 16 > kRkLds;
+}
+constexpr int kRkWideVecs = 7;
+
 // Raises the kernels' dynamic LDS limit to kRkLds on the current device.
 hipError_t rk4_set_lds_limits();
 
@@ -112,10 +119,11 @@ void launch_rk4_batch(unsigned nsys, const Rk4Sys* sys, int block, std::size_t l
 void launch_rk4_chunked(int D, const Rk4Sys* arr, const Rk4Sys& one, unsigned nsys, long max_steps, hipStream_t st);
 void launch_rk4_chunked_walk(int D, const Rk4AdjArgs* arr, const Rk4AdjArgs& one, unsigned ntapes, long steps,
                              hipStream_t st);
-// out[n] = (L[n] + L[n + 1]) / 2, n < count.
-void launch_midpoints(const double2* L, long count, long D2, double2* out, hipStream_t st);
-// dst[t] = src[t]^H, t < count.
-void launch_conj_transpose(const double2* src, double2* dst, int D, long count, hipStream_t st);
+// Wide runs (rk4_wide) of `one` or nsys systems of this D (arr), and the
+// recompute and walk of `one` tape or ntapes tapes of this D, steps and K.
+void launch_rk4_wide(int D, const Rk4Sys* arr, const Rk4Sys& one, unsigned nsys, long max_steps, hipStream_t st);
+void launch_rk4_wide_reverse(int D, const Rk4AdjArgs* arr, const Rk4AdjArgs& one, unsigned ntapes, long steps, int K,
+                             hipStream_t st);
 
 // Reverse of one tape (A) or of ntapes tapes of one D, steps and K (As on
 // the device): the segments' recompute, the walk, the generator cotangents.

@@ -299,6 +299,40 @@ def test_d16_vjp_matches_fd_of_forward():
     check("r0", float(np.real(np.vdot(g["r0"], dr))), lambda s: loss(r0=r0_for(N) + s * dr), 1e-2)
 
 
+@pytest.mark.parametrize("d,steps,K", [(9, 1, 4), (9, 7, 3), (17, 4, 2)])
+def test_wide_reverse_matches_forward(d, steps, K):
+    """The reverse RK4 of D = 81 and 289 (products over many workgroups) at
+    order 2: a partial last segment, an odd and an even first step.  The run is
+    linear in r0, so <bar, F dr> = <r0bar, dr> to rounding; the generator
+    cotangents against central differences of the forward."""
+    rng = W.SplitMix64(29)
+    H = W.gue(d, rng)
+    w = W.Workload("g", H, [W.random_hermitian_unit(d, rng)], taco_amd.DrudeLorentz(0.1, 3.0), 0.8, 0.05, 63,
+                   list(range(steps + 1)), steps=steps)
+    S, G, dt = w.system, w.gamma, w.dt
+    rng = np.random.default_rng(7)
+    bar = rng.standard_normal((steps + 1, d * d)) + 1j * rng.standard_normal((steps + 1, d * d))
+
+    def forward(Gx, r0):
+        t = AD.Tape(Gx, S.omegas, S.mirror, S.pair_to_freq, S.A_eig, S.eps, dt, steps, r0, 2, K)
+        s = t.samples.copy()
+        t.close()
+        return s
+
+    tp = AD.Tape(G, S.omegas, S.mirror, S.pair_to_freq, S.A_eig, S.eps, dt, steps, r0_for(d), 2, K)
+    g = tp.adjoint(bar)
+    tp.close()
+    dr = rng.standard_normal(d * d) + 1j * rng.standard_normal(d * d)
+    ref, got = float(np.real(np.vdot(bar, forward(G, dr)))), float(np.real(np.vdot(g["r0"], dr)))
+    scale = float(np.linalg.norm(bar) * np.linalg.norm(forward(G, dr)))
+    assert abs(got - ref) <= 1e-13 * scale
+    dG = (rng.standard_normal(G.shape) + 1j * rng.standard_normal(G.shape)) * np.abs(G).max()
+    loss = lambda s: float(np.real(np.vdot(bar, forward(G + s * dG, r0_for(d)))))
+    h = 1e-4
+    ref, got = (loss(h) - loss(-h)) / (2 * h), float(np.real(np.vdot(g["gamma"], dG)))
+    assert abs(got - ref) <= FD_TOL * abs(ref) + 1e-14 * abs(loss(0.0)) / h
+
+
 def test_tfim_parameter_gradient_matches_fd():
     """Gradient of the d = 16 chain loss with respect to (lambda, gamma, beta,
     J, h) through the whole chain (Drude-Lorentz bath correlation, trapz

@@ -48,6 +48,28 @@ def test_chunked_rk4_matches_oracle(orc, D, steps, every):
     assert max_rel_err(np.array(seen), ref)[0] <= 1e-12
 
 
+@pytest.mark.parametrize("D", [69, 70, 81, 256, 257, 300])
+@pytest.mark.parametrize("steps,every", [(1, 1), (2, 7), (9, 4)])
+@pytest.mark.parametrize("half", [False, True])
+def test_wide_rk4_matches_oracle(orc, D, steps, every, half):
+    """D = 70 and more run each product over many workgroups (69: the last one
+    that stages two generators): remainders of the 8-row blocks and of the
+    256-column passes, an odd and an even last step, samples and the end
+    against the oracle at the bound of the runs above."""
+    rng = np.random.default_rng(100 + D)
+    base = (rng.standard_normal((D, D)) + 1j * rng.standard_normal((D, D))) * (0.5 / np.sqrt(D))
+    Ls = np.array([base * np.cos(0.1 * s) - 0.1 * np.eye(D) for s in range(steps + 1)])
+    Lh = 0.5 * (Ls[:-1] + Ls[1:])
+    r0 = rng.standard_normal(D) + 1j * rng.standard_normal(D)
+    seen = []
+    r = taco_amd.propagate_rk4_dense(Ls, r0, 0.0, 0.05, L_half_series=Lh if half else None,
+                                     on_sample=lambda t, v: seen.append(v.copy()), sample_every=every)
+    rr, ref = orc.propagate(Ls, r0, 0.05, every=every)
+    assert np.abs(r - rr).max() <= 1e-12 * np.abs(rr).max()
+    assert len(seen) == len(ref)
+    assert max_rel_err(np.array(seen), ref)[0] <= 1e-12
+
+
 def test_rk4_closed_forms():
     D = 4
     L = np.diag([0.1 - 0.03j, -0.07 + 0.05j, 0.02, -0.04 - 0.02j])
