@@ -609,7 +609,7 @@ struct FcrAdjArgs {
     long ncomb;
     const double2* sbar;    // [T][3][nf3]
     long nf3;
-    double2* scr;           // [ncomb][11][T]
+    double2* scr;           // [ncomb][11][T] (k_fcr_adj_short: [ncomb][3][T])
     double* om;             // [ncomb] Omega cotangent
     const double2* ph_tab;  // phase table of the forward pass (TACO_PHASE_LIBM) or null
     const int* job_row;
@@ -821,16 +821,164 @@ __global__ __launch_bounds__(kBlock) void k_fcr_adj_fin(FcrAdjArgs P) {
     if (threadIdx.x == 0) P.om[p] += tot;
 }
 
+// Scan, correlations and final sums of one triple of at most kAdjShort times by
+// one wave: lane l holds the times l + 64 r, the series that the correlations
+// shift stay in LDS, and only the three Gamma cotangents go to memory (the
+// three kernels above store and reload eleven series, and their correlations
+// read five LDS values for 16 fused multiply-adds; here up to four times of a
+// lane share the unshifted values, two of which are scalar loads).
+// d = 16, 201 times, 1.5e5 triples: 11.5 -> 5.9 ms.  Longer runs, whose series
+// would need more registers and LDS than a wave can have beside others, take
+// the three kernels.
+constexpr int kAdjShort = 256;
+
+// Sum over the lanes up to (UP) or from this one, plus carry; carry takes the total.
+template <bool UP, int Q>
+__device__ __forceinline__ void wave_scan_n(double (&v)[Q], double (&carry)[Q]) {
+    const int lane = threadIdx.x;
+#pragma unroll
+    for (int q = 0; q < Q; ++q) {
+#pragma unroll
+        for (int off = 1; off < 64; off <<= 1) {
+            const double nb = UP ? __shfl_up(v[q], off, 64) : __shfl_down(v[q], off, 64);
+            if (UP ? lane >= off : lane + off < 64) v[q] += nb;
+        }
+        const double tot = __shfl(v[q], UP ? 63 : 0, 64);
+        v[q] += carry[q];
+        carry[q] += tot;
+    }
+}
+
+__global__ __launch_bounds__(64) __attribute__((amdgpu_waves_per_eu(3, 8))) void k_fcr_adj_short(FcrAdjArgs P) {
+    constexpr int R = kAdjShort / 64;
+    __shared__ double2 fb[kAdjShort], cb[kAdjShort], ww[kAdjShort];
+    const long p = blockIdx.x;
+    const int lane = threadIdx.x, T = static_cast<int>(P.T), mask = P.job_mask[p];
+    const long tri = P.job_tri[p];
+    int i, j, k;
+    decode_triple(tri, P.nf, i, j, k);
+    const int mj = P.mirror[j];
+    const double omega = (P.omegas[i] + P.omegas[j]) + P.omegas[k];
+    const double2* prow = P.ph_tab ? P.ph_tab + static_cast<long>(P.job_row[p]) * P.ph_len : nullptr;
+    const double2* g1 = P.gamma + static_cast<long>(i) * P.Nt;
+    const double2* g2 = P.gamma + static_cast<long>(j) * P.Nt;
+    const double2* gm = P.gamma + static_cast<long>(mj) * P.Nt;
+    double2 *G1 = P.scr + p * 3 * T, *G2 = G1 + T, *GM = G2 + T;
+    const double dt = P.dt;
+    const double2 z = make_double2(0.0, 0.0);
+    double2 pp[R], Rb[R], wb[R], g1b[R];
+    double carry[6] = {0, 0, 0, 0, 0, 0};
+#pragma unroll
+    for (int r = 0; r < R; ++r) {
+        pp[r] = Rb[r] = wb[r] = g1b[r] = z;
+        if (64 * r >= T) continue;
+        const int t = lane + 64 * r;
+        const bool valid = t < T;
+        double2 a1 = z, a2 = z, a3 = z, w = z, Fb = z, Cb = z;
+        if (valid) {
+            const double2* sb = P.sbar + static_cast<long>(t) * 3 * P.nf3;
+            if (mask & 1) Fb = sb[tri];
+            if (mask & 2) Cb = sb[P.nf3 + tri];
+            if (mask & 4) Rb[r] = sb[2 * P.nf3 + tri];
+            pp[r] = phase_plus(prow, t, omega, dt);
+            const double2 pm = cconj(pp[r]), x2 = g2[t];
+            a1 = cmul(gm[t], pp[r]);
+            a2 = cmul(cconj(x2), pp[r]);
+            a3 = cmul(x2, pm);
+            w = cmul(g1[t], pm);
+        }
+        double v[6] = {a1.x, a1.y, a2.x, a2.y, a3.x, a3.y};
+        wave_scan_n<true>(v, carry);
+        const double2 PF = make_double2(v[0] * dt, v[1] * dt);
+        const double2 PC = make_double2(v[2] * dt, v[3] * dt);
+        const double2 P3 = make_double2(v[4] * dt, v[5] * dt);
+        fb[t] = Fb;
+        cb[t] = Cb;
+        ww[t] = w;
+        if (!valid) continue;
+        wb[r] = cadd(cmul(Fb, cconj(PF)), cmul(Cb, cconj(PC)));
+        g1b[r] = cmul(Rb[r], cconj(P3));
+    }
+    __syncthreads();
+    // correlations over the lags e: time t = u + e for u = lane + 64 r
+    double2 xw[R], xm[R], xc[R];
+#pragma unroll
+    for (int r = 0; r < R; ++r) xw[r] = xm[r] = xc[r] = z;
+    auto lags = [&](auto nr, int e0, int e1) {
+        constexpr int NR = decltype(nr)::value;
+        for (int e = e0; e < e1; ++e) {
+            const double2 m = uload2(gm + e), q = uload2(g2 + e), w = ww[e];
+#pragma unroll
+            for (int r = 0; r < NR; ++r) {
+                const int t = lane + 64 * r + e;
+                if (r + 1 < NR || t < T) {  // the blocks before the last one end below T
+                    const double2 f = fb[t], c = cb[t];
+                    xw[r] = cfma_conj(m, f, cfma(q, c, xw[r]));
+                    xm[r] = cfma_conj(w, f, xm[r]);
+                    xc[r] = cfma_conj(w, c, xc[r]);
+                }
+            }
+        }
+    };
+    if (mask & 3) {
+        lags(std::integral_constant<int, 4>{}, 0, T - 192);
+        lags(std::integral_constant<int, 3>{}, max(0, T - 192), T - 128);
+        lags(std::integral_constant<int, 2>{}, max(0, T - 128), T - 64);
+        lags(std::integral_constant<int, 1>{}, max(0, T - 64), T);
+    }
+    // suffix sums ybar_m = dt sum_{t >= m} Pbar_t, and the results
+    double sc[8] = {0, 0, 0, 0, 0, 0, 0, 0};
+    double om_part = 0.0, om_fin = 0.0;
+#pragma unroll
+    for (int r = R - 1; r >= 0; --r) {
+        if (64 * r >= T) continue;
+        const int t = lane + 64 * r;
+        const bool valid = t < T;
+        double2 x1 = z, x2 = z, xmir = z;
+        if (valid) {
+            x1 = g1[t];
+            x2 = g2[t];
+            xmir = gm[t];
+        }
+        const double2 Fb = fb[t], Cb = cb[t], w = ww[t], pm = cconj(pp[r]);
+        const double2 pF = cmul(Fb, cconj(w)), pC = cmul(Cb, cconj(w)), p3 = cmul(Rb[r], cconj(x1));
+        double v[8] = {pF.x, pF.y, pC.x, pC.y, p3.x, p3.y, -Rb[r].x, -Rb[r].y};
+        wave_scan_n<false>(v, sc);
+        if (!valid) continue;
+        const double2 yF = make_double2(v[0] * dt, v[1] * dt), yC = make_double2(v[2] * dt, v[3] * dt);
+        const double2 y3 = make_double2(v[4] * dt, v[5] * dt), y4 = make_double2(v[6] * dt, v[7] * dt);
+        const double tdt = static_cast<double>(t) * dt;
+        const double2 wbar = csub(wb[r], cscale(xw[r], dt));
+        GM[t] = csub(cmul(yF, pm), cscale(xm[r], dt));
+        G2[t] = csub(cadd(cadd(cmul(cconj(yC), pp[r]), cmul(y3, pp[r])), cmul(y4, cconj(cmul(x1, pm)))),
+                     cconj(cscale(xc[r], dt)));
+        G1[t] = cadd(cadd(g1b[r], cmul(y4, cconj(cmul(x2, pm)))), cmul(wbar, pp[r]));
+        const double2 ppb = cadd(cmul(yF, cconj(xmir)), cmul(yC, x2));
+        const double2 pmb = cadd(cmul(y3, cconj(x2)), cmul(y4, cconj(cmul(x1, x2)))), pmf = cmul(wbar, cconj(x1));
+        // d pp / d Omega = i t dt pp, d pm / d Omega = -i t dt pm
+        const double2 dpp = make_double2(-tdt * pp[r].y, tdt * pp[r].x);
+        const double2 dpm = make_double2(tdt * pm.y, -tdt * pm.x);
+        om_part += (ppb.x * dpp.x + ppb.y * dpp.y) + (pmb.x * dpm.x + pmb.y * dpm.y);
+        om_fin += pmf.x * dpm.x + pmf.y * dpm.y;
+    }
+    for (int off = 32; off > 0; off >>= 1) {
+        om_part += __shfl_down(om_part, off, 64);
+        om_fin += __shfl_down(om_fin, off, 64);
+    }
+    if (lane == 0) P.om[p] = om_part + om_fin;
+}
+
 // Gamma cotangent per bucket: gbar[b][t] = sum over the bucket's entries
-// (position, role) of series role (4 g1bar, 5 g2bar, 6 gmbar), in list order.
+// (position, role) of the series g1bar, g2bar, gmbar (from series `first` of a
+// position's `rows`), in list order.
 // Per bucket b (blockIdx.y), its list of (position, role) entries in
 // gridDim.z contiguous pieces: piece z (blockIdx.z) sums its entries in list
 // order into part[(z nf + b) T + t]; k_bucket_reduce_pieces adds the pieces
 // in order.  Enough workgroups to hide the gathers' latency (a bucket can
 // hold thousands of entries), and a fixed order.
 constexpr int kBredPieces = 32;
-__global__ __launch_bounds__(kBlock) void k_bucket_reduce(const double2* scr, long T, const int* ent_start,
-                                                          const int* ent, double2* part) {
+__global__ __launch_bounds__(kBlock) void k_bucket_reduce(const double2* scr, int rows, int first, long T,
+                                                          const int* ent_start, const int* ent, double2* part) {
     const int b = blockIdx.y, nf = gridDim.y, z = blockIdx.z, P = gridDim.z;
     const long t = static_cast<long>(blockIdx.x) * kBlock + threadIdx.x;
     if (t >= T) return;
@@ -839,8 +987,8 @@ __global__ __launch_bounds__(kBlock) void k_bucket_reduce(const double2* scr, lo
     double2 s = make_double2(0.0, 0.0);
     for (long q = lo; q < hi; ++q) {
         const int code = ent[q];
-        const long p = code / 3, role = 4 + code % 3;
-        s = cadd(s, scr[(p * 11 + role) * T + t]);
+        const long p = code / 3, role = first + code % 3;
+        s = cadd(s, scr[(p * rows + role) * T + t]);
     }
     part[(static_cast<long>(z) * nf + b) * T + t] = s;
 }

@@ -3550,7 +3550,9 @@ static void tape_adjoint_tail(taco_tape& tp, const RkRev& rv, const double2* sl,
         if (lds > 160 * 1024) throw Error(TACO_ERR_INVALID, "direct L4 adjoint kernel supports N <= 8");
         if (l4_direct) set_fn_lds(reinterpret_cast<const void*>(k_l4_adjoint), lds);
         const std::size_t sbar_n = T * 3 * nf3, abar_n = T * tp.num_ops * N2;
-        const std::size_t nscr = static_cast<std::size_t>(ncomb) * 11 * T;
+        const bool short_run = T <= static_cast<std::size_t>(kAdjShort);
+        const int scr_rows = short_run ? 3 : 11;
+        const std::size_t nscr = static_cast<std::size_t>(ncomb) * scr_rows * T;
         const unsigned l4_grid = static_cast<unsigned>(std::min<std::size_t>(T, 1024));
         const bool packed = !l4_direct && nf3 >= kL4AdjPackedNf3;
         const std::size_t nxp = packed ? l4_adjoint_lists_cached(c, tp.h_p2f.data(), tp.N, tp.nf).xp_xz.size() : 0;
@@ -3671,6 +3673,10 @@ static void tape_adjoint_tail(taco_tape& tp, const RkRev& rv, const double2* sl,
             P.ph_len = J.P.ph_len;
             const unsigned nub = static_cast<unsigned>((T + kBlock - 1) / kBlock);
             timed(c, K_COMBINE, 0.0, [&] {
+                if (short_run) {
+                    hipLaunchKernelGGL(k_fcr_adj_short, dim3(static_cast<unsigned>(ncomb)), dim3(64), 0, c->stream, P);
+                    return;
+                }
                 hipLaunchKernelGGL(k_fcr_adj_scan, dim3(static_cast<unsigned>(ncomb)), dim3(kBlock), 0, c->stream, P);
                 hipLaunchKernelGGL(k_fcr_adj_corr, dim3(static_cast<unsigned>(ncomb), nub), dim3(kBlock), 0,
                                    c->stream, P);
@@ -3703,7 +3709,8 @@ static void tape_adjoint_tail(taco_tape& tp, const RkRev& rv, const double2* sl,
             // list order), the pieces then summed in order
             c->bred.ensure(static_cast<std::size_t>(kBredPieces) * tp.nf * T * 16);
             hipLaunchKernelGGL(k_bucket_reduce, dim3(nub, static_cast<unsigned>(tp.nf), kBredPieces), dim3(kBlock), 0,
-                               c->stream, scr, static_cast<long>(T), dstart, dent, c->bred.as<double2>());
+                               c->stream, scr, scr_rows, short_run ? 0 : 4, static_cast<long>(T), dstart, dent,
+                               c->bred.as<double2>());
             hipLaunchKernelGGL(k_bucket_reduce_pieces, dim3(nub, static_cast<unsigned>(tp.nf)), dim3(kBlock), 0,
                                c->stream, c->bred.as<double2>(), static_cast<long>(T), static_cast<long>(T), gb4);
             HIP_OK(hipGetLastError());

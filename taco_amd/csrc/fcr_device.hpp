@@ -6,6 +6,16 @@
 
 namespace taco_engine {
 
+// Reads of kernel-constant data at a wave-uniform address, by scalar loads.
+template <class T>
+__device__ __forceinline__ T uload(const T* p) {
+    return *(const __attribute__((address_space(4))) T*)(unsigned long)(p);
+}
+__device__ __forceinline__ double2 uload2(const double2* p) {
+    const double* d = reinterpret_cast<const double*>(p);
+    return make_double2(uload(d), uload(d + 1));
+}
+
 // ---------------------------------------------------------------------------
 // Device helpers
 // ---------------------------------------------------------------------------

@@ -37,15 +37,6 @@ struct Group {
     static __host__ __device__ constexpr int s_lo(int p) { return p == 0 ? 1 : s_lo(p - 1) + rl(p - 1); }
 };
 
-// Reads of kernel-constant data at a wave-uniform address, by scalar loads.
-template <class T>
-__device__ __forceinline__ T uload(const T* p) {
-    return *(const __attribute__((address_space(4))) T*)(unsigned long)(p);
-}
-__device__ __forceinline__ double2 uload2(const double2* p) {
-    const double* d = reinterpret_cast<const double*>(p);
-    return make_double2(uload(d), uload(d + 1));
-}
 // base[idx] with a wave-uniform base and a 32-bit byte offset per lane: one
 // offset register serves every access that differs by a uniform distance.
 __device__ __forceinline__ double2 vload(const double2* base, unsigned idx) {

@@ -333,6 +333,32 @@ def test_wide_reverse_matches_forward(d, steps, K):
     assert abs(got - ref) <= FD_TOL * abs(ref) + 1e-14 * abs(loss(0.0)) / h
 
 
+@pytest.mark.parametrize("steps", [1, 62, 63, 64, 127, 128, 191, 192, 254, 255])
+def test_short_slice_reverse_matches_long(steps):
+    """Tapes of at most 256 times take the one-wave slice reverse.  A run of 256
+    steps or more whose later sample cotangents are zero has the same cotangents
+    at the first times and none after them (both sum the same terms)."""
+    rng = W.SplitMix64(11)
+    H = W.gue(3, rng)
+    A1, A2 = W.random_hermitian_unit(3, rng), W.random_hermitian_unit(3, rng)
+    w = W.Workload("g3", H, [A1, A2], taco_amd.DrudeLorentz(0.08, 4.0), 0.7, 0.01, 511, list(range(2)), steps=1)
+    S, G, N = w.system, w.gamma, 3
+    rng = np.random.default_rng(steps)
+    bar = rng.standard_normal((steps + 1, N * N)) + 1j * rng.standard_normal((steps + 1, N * N))
+    out = []
+    for n in (steps, 260):
+        b = np.zeros((n + 1, N * N), complex)
+        b[:steps + 1] = bar
+        tp = AD.Tape(G, S.omegas, S.mirror, S.pair_to_freq, S.A_eig, S.eps, w.dt, n, r0_for(N), 4, 16)
+        out.append(tp.adjoint(b))
+        tp.close()
+    a, b = out
+    for key in ("gamma", "omegas", "eps", "r0"):
+        assert np.abs(a[key] - b[key]).max() <= 1e-11 * np.abs(b[key]).max(), key
+    for x, y in zip(a["ops"], b["ops"]):
+        assert np.abs(x - y).max() <= 1e-11 * np.abs(y).max()
+
+
 def test_tfim_parameter_gradient_matches_fd():
     """Gradient of the d = 16 chain loss with respect to (lambda, gamma, beta,
     J, h) through the whole chain (Drude-Lorentz bath correlation, trapz
