@@ -173,7 +173,7 @@ def batched_record(a, steps: int | None = None, warmup: int | None = None):
     print(f"[bench] batch created in {time.perf_counter() - t0:.1f} s", file=sys.stderr, flush=True)
     with tcl4.Profile(0) as prof:
         t0 = time.perf_counter()
-        b.run()  # eager: tunes the FFT tiles; profiled per kernel
+        b.run()  # eager; profiled per kernel
         eager_s = time.perf_counter() - t0
         kern = prof.read()
     print(f"[bench] eager batch run {eager_s:.2f} s", file=sys.stderr, flush=True)
@@ -616,7 +616,7 @@ def main():
     print(f"[bench] workload {w.name}: d={S.N} nf={S.nf} Nt={G.shape[0]} ntau={ntau}; warmup {a.warmup}",
           file=sys.stderr, flush=True)
     # first call: builds the libm phase table (host std::exp per Omega class,
-    # cached in the context) and autotunes the FFT tiles; later calls reuse both
+    # cached in the context); later calls reuse it
     first = []
     for _ in range(max(a.warmup, 2)):
         torch.cuda.synchronize()
@@ -662,288 +662,6 @@ def main():
     _lib.check(_lib.lib().taco_fft_tile_choice(tcl4.context(0).handle, int(np.log2(nfft)), _lib.iptr(choice)))
     shapes = {-1: None, 3: "tiles of 2048"}
     fft_tiles = {ph: shapes.get(int(c), f"groups of {1 << int(c)}") for ph, c in zip("ABC", choice)}
-    L4 = out.cpu().numpy().reshape(ntau, S.N ** 2, S.N ** 2).transpose(0, 2, 1)
-        short = [t for t in w.tidx if t <= 500]
-        L4s = taco_amd.build_TCL4_generator_hip_fused_batch(S, G, w.dt, short)
-    rec = {"workload": f"{w.name} in the window FFT mode, Nfft {1 << int(np.ceil(np.log2(2 * (max(w.tidx) + 1) - 1)))}",
-           "value": ntau / el, "unit": "L4 time-points/s", "ms_per_step": 1e3 * el, "steps": steps}
-    if ref_libm is not None:
-        e, _ = per_t_rel_err(L4, ref_libm)
-        rec["max_per_t_rel_err_vs_parity_oracle"] = float(e.max())
-        rec["max_per_t_rel_err_vs_parity_oracle_t_ge_20"] = float(e[20:].max()) if ntau > 20 else None
-        t0 = time.perf_counter()
-        with oracle.phase_mode(oracle.PHASE_LIBM):
-            direct = oracle.l4_series(G, S.omegas, S.mirror, S.pair_to_freq, S.A_eig, w.dt, short, method="direct",
-                                      nthreads=threads)
-        ed, _ = per_t_rel_err(L4s, direct)
-        ep, _ = per_t_rel_err(ref_libm[: len(short)], direct)
-        rec["max_per_t_rel_err_vs_direct_t_le_500"] = float(ed.max())
-        rec["parity_oracle_vs_direct_t_le_500"] = float(ep.max())
-        rec["direct_seconds"] = time.perf_counter() - t0
-    return rec
-
-
-def host_pointer_record(w, steps: int = 3) -> dict:
-    """taco_l4_batch from host buffers: the Gamma table copied in, the L4
-    series copied out and repacked into per-time matrices, as the reference's
-    published timing includes (tests/tcl4_e2e_cuda_compare.cpp:208-214)."""
-    import taco_amd
-
-    S, G = w.system, w.gamma
-    taco_amd.build_TCL4_generator_hip_fused_batch(S, G, w.dt, w.tidx)  # tables, tiles, workspace
-    t0 = time.perf_counter()
-    for _ in range(steps):
-        L = taco_amd.build_TCL4_generator_hip_fused_batch(S, G, w.dt, w.tidx)
-        mats = [np.ascontiguousarray(L[q]) for q in range(L.shape[0])]  # per-time matrices
-    el = (time.perf_counter() - t0) / steps
-    del mats
-    return {"workload": w.name, "d": S.N, "nf": S.nf, "ntau": len(w.tidx), "Nt": int(G.shape[0]),
-            "seconds_per_call": el, "L4_per_s_with_host_copies": len(w.tidx) / el, "calls": steps}
-
-
-def cpu_model() -> str:
-    try:
-        for line in open("/proc/cpuinfo"):
-            if line.startswith("model name"):
-                return line.split(":", 1)[1].strip()
-    except OSError:
-        pass
-    return "unknown"
-
-
-def serial_cpu_record(w) -> dict:
-    """The oracle on one thread (the reference's serial path) over the whole
-    workload w."""
-    from oracle import oracle
-
-    S, G = w.system, w.gamma
-    with oracle.phase_mode(oracle.PHASE_LIBM):
-        t0 = time.perf_counter()
-        oracle.l4_series(G, S.omegas, S.mirror, S.pair_to_freq, S.A_eig, w.dt, w.tidx, nthreads=1)
-        el = time.perf_counter() - t0
-    return {"value": len(w.tidx) / el, "unit": "L4 time-points/s", "cores": 1, "kind": "port",
-            "sample": f"{w.name}: whole workload (d={S.N}, nf={S.nf}, Nt={G.shape[0]}, {len(w.tidx)} L4 times), "
-                      f"oracle serial, {el:.1f} s", "seconds": el}
-
-
-def tfim_adjoint_main(a):
-    """Gradients of the d = 16 loss (open 4-spin transverse-field Ising chain,
-    J = 1, h drawn from U[0.5, 1.5] (seed 5), A = sum sz_i, Drude-Lorentz
-    bath lambda 0.05, gamma 5, beta 1) with respect to (lambda, gamma, beta,
-    J, h), for --systems parameter sets (default 64) in one multi-set tape
-    (their RK4 recursions one launch each way), and set by set for the first
-    four (the single-tape path, timed for comparison).  The window is reduced from the 2^20-point grid and 20001 times of the full
-    configuration (its forward F/C/R pass alone moves ~10 TB per parameter
-    set) to a 2^12-point grid and 200 RK4 steps of TCL2 + L4, checkpoints
-    every 64.  One step = one gradient per parameter set (forward + reverse);
-    the value is gradients per second.  The gradient of the first set is
-    checked against central differences (h = 1e-6 relative) of the same GPU
-    pipeline, whose d = 16 forward the tests pin to the oracle; the oracle's
-    own d = 16 forward at this size (all 531441 F/C/R triples at Nfft 2^13
-    plus 201 O(N^6) L4 evaluations) is too slow to time as a baseline."""
-    import torch
-
-    from taco_amd import adjoint as AD
-
-    assert torch.cuda.is_available(), "bench needs an MI355X"
-    import taco_amd
-    # correctly rounded phases: each parameter set has its own ~10^5 Omega
-    # classes, whose libm table the host would rebuild for every gradient
-    taco_amd.set_phase_mode(taco_amd.PHASE_CR)
-    # F/C/R slices (5.1 GB per set at nf = 81 whole, 1.5 GB packed to the
-    # entries L4 reads) kept within 160 GiB of the 288 GB HBM; the multi-set
-    # reverse recomputes those of any set past it
-    slice_budget = 160 << 30
-    taco_amd.set_slice_budget(slice_budget)
-    nsets = a.systems or 64
-    rng = np.random.default_rng(5)
-    hs = rng.uniform(0.5, 1.5, size=nsets)
-    prob = AD.TfimChainProblem(Nt=2 ** 12, dt=0.005, steps=200, checkpoint_every=64)
-    P0 = [np.array([0.05, 5.0, 1.0, 1.0, h]) for h in hs]
-    u = np.where(np.random.default_rng(4).uniform(size=5) < 0.5, -1.0, 1.0)
-    with torch.no_grad():
-        targets = [prob.rho_lab(torch.tensor(p * (1 + 0.05 * u), dtype=torch.float64)).detach() for p in P0]
-    print(f"[bench] tfim_adjoint: {nsets} targets built", file=sys.stderr, flush=True)
-
-    def fwd(q):
-        with torch.no_grad():
-            return float(prob.loss(torch.tensor(P0[q], dtype=torch.float64), targets[q]))
-
-    def grad(q):
-        params = torch.tensor(P0[q], dtype=torch.float64, requires_grad=True)
-        loss = prob.loss(params, targets[q])
-        (g,) = torch.autograd.grad(loss, params)
-        return float(loss), g.numpy()
-
-    def grad_many():
-        params = [torch.tensor(p, dtype=torch.float64, requires_grad=True) for p in P0]
-        losses = prob.losses_many(params, targets)
-        gs = torch.autograd.grad(sum(losses), params)
-        return [(float(l), g.numpy()) for l, g in zip(losses, gs)]
-
-    for _ in range(a.warmup):
-        fwd(0)
-        grad(0)
-    # set by set (a few sets: each is a whole forward + reverse)
-    nseq = min(nsets, 4)
-    t0 = time.perf_counter()
-    for _ in range(a.steps):
-        for q in range(nseq):
-            fwd(q)
-    t_fwd = (time.perf_counter() - t0) / (a.steps * nseq)
-    t0 = time.perf_counter()
-    seq = []
-    for _ in range(a.steps):
-        seq = [grad(q) for q in range(nseq)]
-    t_seq = (time.perf_counter() - t0) / (a.steps * nseq)
-    print(f"[bench] set by set: forward {t_fwd * 1e3:.1f} ms, forward+reverse {t_seq * 1e3:.1f} ms per set",
-          file=sys.stderr, flush=True)
-    # every set in one multi-set tape
-    grad_many()
-    t0 = time.perf_counter()
-    grads = []
-    for _ in range(a.steps):
-        grads = grad_many()
-    t_grad = (time.perf_counter() - t0) / (a.steps * nsets)
-    same = sum(1 for q in range(nseq) if grads[q][0] == seq[q][0] and np.array_equal(grads[q][1], seq[q][1]))
-    modes = AD.MultiTape.last_slice_modes
-    slice_modes = {m: sum(1 for x in modes if x[0] == m) for m in ("whole", "packed", "recompute")}
-    slice_gib = sum(x[1] for x in modes) / 2 ** 30
-    print(f"[bench] multi-set tape: {t_grad * 1e3:.1f} ms per set over {nsets} sets; {same}/{nseq} sets bit-equal "
-          f"to the set-by-set gradients; slices {slice_modes}, {slice_gib:.1f} GiB", file=sys.stderr, flush=True)
-    from taco_amd import tcl4
-    # kernel figures of one multi-set gradient, per set; the roofline is phase
-    # B's (the HBM-bound kernel with the most time: the L4 and F/C/R reverses
-    # are FP64-latency bound and are timed under the forward kernels' names
-    # with no bytes of their own)
-    with tcl4.Profile(0) as prof:
-        grad_many()
-        kern = prof.read()
-    kernels, roofline = kernel_table(kern, nsets, dom="k_phase_b")
-    loss0, g0 = grads[0]
-    fdg = np.zeros(5)
-    for q in range(5):
-        h = 1e-6 * abs(P0[0][q])
-        pp, pm = P0[0].copy(), P0[0].copy()
-        pp[q] += h
-        pm[q] -= h
-        with torch.no_grad():
-            lp = float(prob.loss(torch.tensor(pp, dtype=torch.float64), targets[0]))
-            lm = float(prob.loss(torch.tensor(pm, dtype=torch.float64), targets[0]))
-        fdg[q] = (lp - lm) / (2 * h)
-    rel = np.abs(g0 - fdg) / np.abs(fdg)
-    rec = {
-        "metric": METRIC,
-        "value": 1.0 / t_grad,
-        "unit": "gradients/s",
-        "n_gpus": 1,
-        "steps": a.steps,
-        "warmup": a.warmup,
-        "ms_per_step": 1e3 * t_grad * nsets,
-        "higher_is_better": True,
-        "scaling": "weak",
-        "vs_baseline": None,
-        "dtype": "c128",
-        "data": "synthetic",
-        "config": {
-            "workload": f"tfim_adjoint (reduced window): d=16 open TFIM chain (nf=81 at generic h), J=1, "
-                        f"h~U[0.5,1.5] seed 5, "
-                        f"{nsets} parameter sets, Drude-Lorentz (0.05, 5, 1), Nt=2^12, dt=0.005, 200 RK4 steps of "
-                        f"TCL2+L4, checkpoints every 64, 5 parameters (lambda, gamma, beta, J, h)",
-            "path": "multi-set tape: every set's F/C/R, L4, TCL2 and their reverses in turn, the forward RK4 "
-                    "and the reverse RK4 (recompute, walk) of all sets one launch each; F/C/R slices kept "
-                    f"within a {slice_budget >> 30} GiB slice budget (whole, or packed to the entries L4 reads), "
-                    "recomputed in the reverse pass past it; bath correlation and Gamma made and reversed on the "
-                    "device; correctly rounded phases",
-            "slices": {"sets": slice_modes, "GiB": round(slice_gib, 2)},
-        },
-        "forward_ms": 1e3 * t_fwd,
-        "gradient_over_forward": t_grad / t_fwd,
-        "set_by_set": {"sets": nseq, "ms_per_gradient": 1e3 * t_seq, "forward_ms": 1e3 * t_fwd,
-                       "multi_set_speedup": t_seq / t_grad, "bit_equal_sets": same},
-        "check": {"params": list(prob.names), "h": float(hs[0]), "adjoint": g0.tolist(), "gpu_fd": fdg.tolist(),
-                  "max_rel_diff": float(rel.max()), "loss": loss0},
-        "roofline": roofline,
-        "cpu_baseline": None,
-        "kernels": kernels,
-        "kernels_note": "per parameter set over one multi-set gradient; k_l4 and k_combine include the L4 and "
-                        "F/C/R reverses' time but only the forward kernels' bytes",
-    }
-    print(json.dumps(rec), flush=True)
-
-
-def main():
-    a = parse()
-    if a.gpus != 1:
-        print(f"bench.py: this engine runs on one GPU; --gpus {a.gpus} is not supported (use --gpus 1)",
-              file=sys.stderr)
-        sys.exit(2)
-    if a.workload == "batched":
-        return batched_main(a)
-    if a.workload == "adjoint":
-        return adjoint_main(a)
-    if a.workload == "tfim_adjoint":
-        return tfim_adjoint_main(a)
-    import torch
-
-    import taco_amd
-    from taco_amd import tcl4
-
-    assert torch.cuda.is_available(), "bench needs an MI355X"
-    w = make_workload(a.workload, a.reduced)
-    S, G = w.system, w.gamma
-    ntau = len(w.tidx)
-    dsys = tcl4.DeviceSystem(S, G, 0)
-    out = torch.empty((ntau, S.N ** 4), dtype=torch.complex128, device="cuda:0")
-    print(f"[bench] workload {w.name}: d={S.N} nf={S.nf} Nt={G.shape[0]} ntau={ntau}; warmup {a.warmup}",
-          file=sys.stderr, flush=True)
-    # first call: builds the libm phase table (host std::exp per Omega class,
-    # cached in the context) and autotunes the FFT tiles; later calls reuse both
-    first = []
-    for _ in range(max(a.warmup, 2)):
-        torch.cuda.synchronize()
-        t0 = time.perf_counter()
-        tcl4.build_l4_dev(dsys, w.dt, w.tidx, out)
-        torch.cuda.synchronize()
-        first.append(time.perf_counter() - t0)
-    print(f"[bench] first call {first[0]:.2f} s, second {first[1] * 1e3:.1f} ms", file=sys.stderr, flush=True)
-    with tcl4.Profile(0) as prof:
-        torch.cuda.synchronize()
-        t0 = time.perf_counter()
-        for _ in range(a.steps):
-            tcl4.build_l4_dev(dsys, w.dt, w.tidx, out)
-        torch.cuda.synchronize()
-        elapsed = time.perf_counter() - t0
-        kern = prof.read()
-    print(f"[bench] timed {a.steps} steps in {elapsed:.3f} s", file=sys.stderr, flush=True)
-    if a.copy_bytes:
-        n = a.copy_bytes // 8
-        src = torch.ones(n, dtype=torch.float64, device="cuda:0")
-        dst = torch.empty_like(src)
-        torch.cuda.synchronize()
-        dst.copy_(src)
-        torch.cuda.synchronize()
-        del src, dst
-    ms_per_step = 1000.0 * elapsed / a.steps
-    value = ntau * a.steps / elapsed
-    kernels, roofline = kernel_table(kern, a.steps)
-    # HBM traffic of the dominant kernel measured by rocprofv3 FETCH_SIZE /
-    # WRITE_SIZE passes of this workload (committed summary), when present
-    tf = os.path.join(ROOT, "profiles", "fcr_l4_gue_pair_d4_traffic.json")
-    if a.workload == "gue_pair" and not a.reduced and os.path.exists(tf):
-        t = json.load(open(tf))
-        # only when it was measured on launches of the same size as these
-        same = abs(t.get("algo_bytes_per_launch", 0.0) - roofline["algo_bytes_per_launch"]) <= (
-            0.01 * roofline["algo_bytes_per_launch"])
-        if t.get("kernel") == roofline["kernel"] and same:
-            roofline["traffic"] = t["traffic_bytes_per_launch"]
-            roofline["traffic_source"] = t["source"]
-    from taco_amd import _lib
-    choice = np.zeros(3, np.int32)
-    nfft = 1 << int(np.ceil(np.log2(2 * G.shape[0] - 1)))
-    _lib.check(_lib.lib().taco_fft_tile_choice(tcl4.context(0).handle, int(np.log2(nfft)), _lib.iptr(choice)))
-    tiles = ["8192/512", "4096/256", "4096/512", "2048/256", "4096/1024", "2048/512", "8192/1024"]
-    fft_tiles = {ph: tiles[c] if c >= 0 else None for ph, c in zip("ABC", choice)}
     L4 = out.cpu().numpy().reshape(ntau, S.N ** 2, S.N ** 2).transpose(0, 2, 1)
     cpu, parity, ref_libm = None, None, None
     if not a.no_cpu:
