@@ -365,8 +365,8 @@ typedef struct taco_batch taco_batch;
  * workspace.  The host arrays are only read during this call. */
 int taco_batch_create(taco_ctx* ctx, const taco_batch_system* systems, int nsys, taco_batch** out);
 /* Runs the whole batch and synchronises.  use_graph = 1 captures the batch
- * into a hipGraph on the first call after an eager run (which also tunes the
- * FFT tiles) and replays it afterwards; results are identical either way. */
+ * into a hipGraph on the first call after an eager run and replays it
+ * afterwards; results are identical either way. */
 int taco_batch_run(taco_batch* b, int use_graph);
 /* System s's L4 at its tidx, request order: ntau blocks of N^2 x N^2. */
 int taco_batch_l4(taco_batch* b, int s, double* L4_out);

@@ -5383,8 +5383,7 @@ int taco_batch_run(taco_batch* b, int use_graph) {
         BatchRun& B = b->run;
         DeviceGuard g(c->device);
         if (!use_graph || !B.ran_eager) {
-            // The first run is eager: it picks the FFT tile configurations
-            // (autotune synchronises) that a captured graph then keeps.
+            // The first run is eager: it loads the kernels, so a capture only records launches.
             batch_enqueue(c, B);
             HIP_OK(hipStreamSynchronize(c->stream));
             B.ran_eager = true;

@@ -11,8 +11,9 @@
 // step in registers, and the loads of later generators are issued up to
 // S - 1 steps ahead (a ring of S register slots), which hides global latency
 // behind the sequential steps.  Vectors go through small LDS buffers with
-// one barrier per RK4 stage.  Forward, batched forward and segment
-// recompute share rk4_rows, so their states are identical bit for bit.
+// one barrier per RK4 stage.  Plain and batched forward runs, the states of a
+// chunked run and the segment recompute share rk4_rows; a chunked run's chunk
+// starts come from the chunk products and differ from a plain run's by rounding.
 #pragma once
 
 // One 64-bit value from another lane of the same row of 16 (DPP control CTRL).
