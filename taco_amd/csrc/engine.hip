@@ -3054,11 +3054,8 @@ static int rk4_block(int D) {
     return kBlock;
 }
 
-// Places a chunked run's products and first states at `base`.
-static void rk4_set_chunks(Rk4Sys& S, double2* base) {
-    S.q = base;
-    S.xs = base + rk4_chunk_values(S.D, S.steps) - static_cast<std::size_t>((S.steps + kRkChunk - 1) / kRkChunk) * S.D;
-}
+// Places a chunked run's products, first states and flags at `base`.
+static void rk4_set_chunks(Rk4Sys& S, double2* base) { rk4_place_chunks(S.D, S.steps, base, S.q, S.xs, S.plain); }
 
 static void rk4_launch(taco_ctx* ctx, const double2* dLs, const double2* dLh, std::size_t steps, int D, double2* dr,
                        double dt, std::size_t every, double2* dsamples, long* dns) {
@@ -3322,6 +3319,7 @@ struct RkRev {
     double2 *gb, *Lb, *seg, *rb;
     double2* vec = nullptr;                               // deferred and wide walks: kb1..kb4 of every step
     double2 *q = nullptr, *lam = nullptr, *bv = nullptr;  // chunked walk (lam: wide walk)
+    int* plain = nullptr;                                 // chunked walk
 };
 
 // The row-group walk (D = 4, 9, 16) stores kb1..kb4 per step and leaves
@@ -3338,7 +3336,7 @@ static std::size_t rk_rev_values(const taco_tape& tp) {
     const std::size_t base = tp.T * D + tp.T * D * D + 4 * tp.steps * D + D;
     if (rk4_chunked_walk(static_cast<int>(D), static_cast<long>(tp.steps)))
         return base + 4 * tp.steps * D + rk4_chunk_values(static_cast<int>(D), static_cast<long>(tp.steps)) +
-               (tp.steps + kRkChunk - 1) / kRkChunk * D;
+               rk4_chunks(static_cast<long>(tp.steps)) * D;
     if (rk4_wide(static_cast<int>(D))) return base + 4 * tp.steps * D + kRkWideVecs * D;
     return rk_rev_rows_deferred(tp) ? base + 4 * tp.steps * D : base;
 }
@@ -3356,10 +3354,11 @@ static RkRev rk_rev_at(const taco_tape& tp, double2* base) {
     } else if (rk_rev_rows_deferred(tp)) {
         b.vec = b.rb + D;
         if (rk4_chunked_walk(static_cast<int>(D), static_cast<long>(tp.steps))) {
-            const std::size_t nch = (tp.steps + kRkChunk - 1) / kRkChunk;
-            b.q = b.vec + 4 * tp.steps * D;
-            b.lam = b.q + nch * D * D;
-            b.bv = b.lam + nch * D;
+            const int Di = static_cast<int>(D);
+            const long steps = static_cast<long>(tp.steps);
+            double2* chunks = b.vec + 4 * tp.steps * D;
+            rk4_place_chunks(Di, steps, chunks, b.q, b.lam, b.plain);
+            b.bv = chunks + rk4_chunk_values(Di, steps);
         }
     }
     return b;
@@ -3395,6 +3394,7 @@ static RkRevShape rk_rev_shape(const taco_tape& tp, const RkRev& b) {
     R.q = b.q;
     R.lam = b.lam;
     R.bv = b.bv;
+    R.plain = b.plain;
     sh.nseg = (steps + K - 1) / K;
     const int Di = static_cast<int>(D);
     sh.Rf = R;

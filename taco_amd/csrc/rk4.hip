@@ -560,7 +560,8 @@ __global__ __launch_bounds__(kRkBlock) void k_rk4_adjoint_multi(const Rk4AdjArgs
 //   1. every chunk of kRkChunk steps forms Q_c = prod (I + E_n) - I, all
 //      chunks at once (four D x D products a step);
 //   2. one workgroup carries r over the chunks, r <- r + Q_c r, one product
-//      per chunk where the plain run has four per step;
+//      per chunk where the plain run has four per step; chunks in which r may
+//      decay (chunk_mild) take the plain steps here instead;
 //   3. every chunk runs its steps from its first state with the plain step
 //      (rk4_rows), all chunks at once.
 // The dependent chain shrinks from 4 steps products to 4 kRkChunk (twice) and
@@ -569,8 +570,6 @@ __global__ __launch_bounds__(kRkBlock) void k_rk4_adjoint_multi(const Rk4AdjArgs
 // The reverse walk, affine in lam, splits alike: each chunk's walk from lam = 0
 // gives its constant part, the carry is lam <- lam + Q_c^H lam + b_c, and every
 // chunk's walk then runs from its true lam.
-// Against an 80-bit run the states are 2 to 5 times closer than the plain
-// run's (D = 16, 4000 steps: 5e-16 against 1.4e-15).
 // Measured, forward: D = 16, 4000 steps 2.7 -> 0.12 ms (products 43 us, 250
 // carries 63 us, states 17 us); D = 4, 2000 steps 1.02 -> 0.05 ms; D = 36,
 // 800 steps 0.42 ms.  All three are latency: chunks of 16 keep the products
@@ -584,6 +583,42 @@ struct Chunk {
     static constexpr int EPT = (DT * DT + LPC - 1) / LPC;  // entries of a thread
     static constexpr int D2 = DT * DT;
 };
+
+// The kernels' arguments: arr[i], one block per system or tape, or the single
+// `one` (arr null), by scalar loads.  A pointer that comes from memory is taken to
+// be of any address space, and its loads wait with the LDS's (a step 25 % longer
+// at D = 16): in_global says that it is global.
+template <class T>
+__device__ __forceinline__ void in_global(T*& p) {
+    auto g = (__attribute__((address_space(1))) T*)p;
+    asm("" : "+s"(g));  // the plain cast there and back is folded away
+    p = (T*)g;
+}
+template <class S>
+__device__ __forceinline__ S scalar_args(const S* arr, const S& one, unsigned i) {
+    constexpr int W = sizeof(S) / 8;
+    static_assert(sizeof(S) % 8 == 0, "whole words");
+    S s = one;
+    if (arr) {
+        unsigned long w[W];
+#pragma unroll
+        for (int q = 0; q < W; ++q) w[q] = uload(reinterpret_cast<const unsigned long*>(arr + i) + q);
+        __builtin_memcpy(&s, w, sizeof(S));
+    }
+    return s;
+}
+__device__ __forceinline__ Rk4Sys chunk_args(const Rk4Sys* arr, const Rk4Sys& one, unsigned i) {
+    Rk4Sys s = scalar_args(arr, one, i);
+    in_global(s.Ls), in_global(s.r0), in_global(s.r), in_global(s.samples), in_global(s.q), in_global(s.xs);
+    in_global(s.plain), in_global(s.nsamples);
+    return s;
+}
+__device__ __forceinline__ Rk4AdjArgs chunk_args(const Rk4AdjArgs* arr, const Rk4AdjArgs& one, unsigned i) {
+    Rk4AdjArgs a = scalar_args(arr, one, i);
+    in_global(a.Ls), in_global(a.gbar), in_global(a.seg), in_global(a.r0bar), in_global(a.vec), in_global(a.q);
+    in_global(a.lam), in_global(a.bv), in_global(a.plain);
+    return a;
+}
 
 // acc[i] = sum_k A(r_i, k) B(k, c_i) for the thread's entries.
 template <int DT>
@@ -603,17 +638,108 @@ __device__ __forceinline__ void chunk_product(double2 (&acc)[Chunk<DT>::EPT], co
     }
 }
 
-// Step 1.  arr: one argument block per system or tape (null: the single `one`).
+// Whether the product may carry a chunk's state: dt kRkChunk times the Frobenius
+// norms of the entries' largest values over the chunk, of the generator
+// (kMildNorm) and of its Hermitian part (kMildDamp), the rate at which the state
+// or a decoupled part of it can shrink.  x + Q x then cancels at most to
+// exp(-kMildDamp) of x, and RK4's own damping of a rotation is below 1e-4 a chunk.
+// A chunk past either line is stepped: there the product loses what the state
+// decays by (scalar generators of dt times rate 0.2, 0.5 and 1, 256 steps: 1e-14,
+// 1e-12 and 5e-9 relative against 6e-15, 2e-14 and 4e-14 stepped).  Below the
+// lines both are alike: 400 complex scalars each, 512 steps, error of the product
+// over that of the steps 0.3 at norm 0.1, 0.8 at 0.5, 1.0 at 1 and 2; over 4096
+// steps of a nearly constant generator 0.4, 1.3, 1.2 and 0.9.  TCL generators of
+// baths up to coupling 0.2 and cutoff 12 at d = 2..5, dt = 0.01 reach norm 1.2,
+// Hermitian part 0.35.  NaN and infinities are past the lines.
+constexpr double kMildNorm = 2.0;
+constexpr double kMildDamp = 0.5;
+
+template <int DT>
+__device__ __forceinline__ bool chunk_mild(const double2* __restrict__ Ls, long n0, long steps, double dt, int lane) {
+    using C = Chunk<DT>;
+    constexpr int NP = DT * (DT + 1) / 2, PPT = (NP + C::LPC - 1) / C::LPC;  // pairs (r, c), r >= c
+    int lo[PPT], up[PPT];
+    double ml[PPT], mu[PPT], mh[PPT];  // largest |L(r, c)|^2, |L(c, r)|^2, |L(r, c) + conj(L(c, r))|^2
+#pragma unroll
+    for (int i = 0; i < PPT; ++i) {
+        int c = 0, r = min(lane + i * C::LPC, NP - 1);
+        while (r >= DT - c) r -= DT - c++;
+        r += c;
+        lo[i] = r + c * DT;
+        up[i] = c + r * DT;
+        ml[i] = mu[i] = mh[i] = 0.0;
+    }
+    auto raise = [](double& m, double a) { m = a > m || a != a ? a : m; };  // a NaN stays
+#pragma unroll(PPT == 1 ? kRkChunk + 1 : 6)
+    for (int m = 0; m <= kRkChunk; ++m) {
+        const double2* L = Ls + min(n0 + m, steps) * C::D2;
+#pragma unroll
+        for (int i = 0; i < PPT; ++i) {
+            const double2 v = L[lo[i]], w = L[up[i]], h = cadd(v, cconj(w));
+            raise(ml[i], v.x * v.x + v.y * v.y);
+            raise(mu[i], w.x * w.x + w.y * w.y);
+            raise(mh[i], h.x * h.x + h.y * h.y);
+        }
+    }
+    double f = 0.0, h = 0.0;
+#pragma unroll
+    for (int i = 0; i < PPT; ++i)
+        if (lane + i * C::LPC < NP) {
+            const bool diagonal = lo[i] == up[i];
+            f += diagonal ? ml[i] : ml[i] + mu[i];
+            h += diagonal ? mh[i] : 2.0 * mh[i];
+        }
+    constexpr int LW = C::LPC < 64 ? C::LPC : 64;
+#pragma unroll
+    for (int m = 1; m < LW; m *= 2) {
+        f += __shfl_xor(f, m, 64);
+        h += __shfl_xor(h, m, 64);
+    }
+    if constexpr (C::LPC > 64) {
+        __shared__ double2 part[C::LPC / 64];
+        if (threadIdx.x % 64 == 0) part[threadIdx.x / 64] = make_double2(f, h);
+        __syncthreads();
+        f = h = 0.0;
+#pragma unroll
+        for (int w = 0; w < C::LPC / 64; ++w) {
+            f += part[w].x;
+            h += part[w].y;
+        }
+    }
+    const double s = dt * kRkChunk;
+    return s * s * f <= kMildNorm * kMildNorm && s * s * (0.25 * h) <= kMildDamp * kMildDamp;
+}
+
+// A run with more than a quarter of its chunks past the lines is stepped whole by
+// step 3's first workgroup: the plain run and two launches that only end (600
+// steps: 2 % longer at D = 4..36).  The products of its other chunks are then
+// formed for nothing, 41 us at D = 16, 0.39 ms at D = 36 (four fifths of the chunks
+// past the lines: 8 and 27 % longer); flags from a launch of their own would save
+// that for 30 to 40 us on every run.
+__device__ __forceinline__ bool step_whole(const int* plain, long nch) {
+    long stepped = 0;
+    for (long j0 = 0; j0 < nch; j0 += 64) {
+        const long j = j0 + (threadIdx.x & 63);
+        stepped += __popcll(__ballot(j < nch && plain[j] != 0));
+    }
+    return 4 * stepped > nch;
+}
+constexpr int kWhole = 2;  // plain[0] of a run that step 3 steps whole
+
+// Step 1.
 template <int DT, class S>
 __global__ __launch_bounds__(Chunk<DT>::NT) void k_chunk_products(const S* arr, S one) {
     using C = Chunk<DT>;
     __shared__ double2 sA[C::CPB][C::D2], sB[C::CPB][C::D2], sQ[C::CPB][C::D2];
-    const S s = arr ? arr[blockIdx.y] : one;
+    const S s = chunk_args(arr, one, blockIdx.y);
     if (s.D != DT || !s.q) return;
     const int sub = threadIdx.x / C::LPC, lane = threadIdx.x % C::LPC;
     const long c = static_cast<long>(blockIdx.x) * C::CPB + sub;
     if (static_cast<long>(blockIdx.x) * C::CPB * kRkChunk >= s.steps) return;
     const long n0 = c * kRkChunk;
+    const bool mild = chunk_mild<DT>(s.Ls, n0, s.steps, s.dt, lane);
+    if (lane == 0 && n0 < s.steps) s.plain[c] = mild ? 0 : 1;
+    if (!__syncthreads_or(mild && n0 < s.steps)) return;
     const double h2 = 0.5 * s.dt, s6 = s.dt / 6.0;
     double2 *A = sA[sub], *B = sB[sub], *Q = sQ[sub];
     double2 l0[C::EPT], l1[C::EPT], ln[C::EPT], q[C::EPT], acc[C::EPT];
@@ -681,72 +807,105 @@ __global__ __launch_bounds__(Chunk<DT>::NT) void k_chunk_products(const S* arr, 
     }
 }
 
-// Step 2 on the row groups of rk4_rows: x over the chunks (REV: lam from the
-// last chunk down), the products' loads a ring of R chunks ahead.
+// Step 2 on the row groups of rk4_rows: x over the i0-th to the i1-th chunk
+// visited (REV: lam, visited from the last chunk down), the products' loads a
+// ring of R chunks ahead.
 template <int DT, bool REV>
-__device__ __forceinline__ void chunk_carry(double2* sh, const double2* Q, const double2* b, long nch, const double2* x_in,
-                                            double2* xs, double2* x_out) {
+__device__ __forceinline__ void chunk_carry(double2* sh, const double2* Q, const double2* b, long nch, long i0, long i1,
+                                            const double2* x_in, double2* xs, double2* x_out) {
     using RG = RowGroup<DT>;
     constexpr int R = DT <= 16 ? 8 : 4;
     constexpr long D2 = static_cast<long>(DT) * DT;
     const int lane = static_cast<int>(threadIdx.x & 63), g = lane % RG::G;
     const int r = static_cast<int>(threadIdx.x >> 6) * RG::R + lane / RG::G;
     const bool own = r < DT && g == 0;
-    auto at = [&](long c) { return REV ? nch - 1 - c : c; };  // c-th chunk visited
+    auto at = [&](long i) { return REV ? nch - 1 - i : i; };  // i-th chunk visited
     double2 x = make_double2(0.0, 0.0);
     if (r < DT) x = x_in[r];
     double2 ring[R][RG::CK], rb[R];
-    auto load = [&](int j, long c) {
-        const long k = at(min(c, nch - 1));
+    auto load = [&](int j, long i) {
+        const long k = at(min(i, i1 - 1));
         load_gen<DT, !REV>(ring[j], Q + k * D2, r, g);
         rb[j] = REV ? b[k * DT + (r < DT ? r : 0)] : make_double2(0.0, 0.0);
     };
 #pragma unroll
-    for (int j = 0; j < R; ++j) load(j, j);
+    for (int j = 0; j < R; ++j) load(j, i0 + j);
     int p = 0;
     if (own) sh[r] = x;
     __syncthreads();
-    auto step = [&](int j, long c) {
-        if (own) xs[at(c) * DT + r] = x;
+    auto step = [&](int j, long i) {
+        if (own) xs[at(i) * DT + r] = x;
         const double2 y = group_dot<DT, REV>(ring[j], sh + p * DT, g);
         x = cadd(x, y);
         if (REV) x = cadd(x, rb[j]);
         p ^= 1;
         if (own) sh[p * DT + r] = x;
         __builtin_amdgcn_sched_barrier(0);
-        load(j, c + R);
+        load(j, i + R);
         __syncthreads();
     };
-    long c = 0;
-    for (; c + R <= nch; c += R) {
+    long i = i0;
+    for (; i + R <= i1; i += R) {
 #pragma unroll
-        for (int j = 0; j < R; ++j) step(j, c + j);
+        for (int j = 0; j < R; ++j) step(j, i + j);
     }
 #pragma unroll
     for (int j = 0; j + 1 < R; ++j)
-        if (c + j < nch) step(j, c + j);
+        if (i + j < i1) step(j, i + j);
     if (own && x_out) x_out[r] = x;
+}
+
+// End of the run of chunks, in visiting order, whose flag is that of the i-th.
+template <bool REV>
+__device__ __forceinline__ long carry_run(const int* plain, long i, long nch) {
+    const long lane = threadIdx.x & 63;
+    auto flag = [&](long j) { return plain[REV ? nch - 1 - j : j] != 0; };
+    const bool first = flag(i);
+    for (long b = i; b < nch; b += 64) {
+        const unsigned long long other = __ballot(b + lane < nch && flag(b + lane) != first);
+        if (other) return b + __ffsll(other) - 1;
+    }
+    return nch;
 }
 
 __device__ __forceinline__ long chunk_count(long steps) { return (steps + kRkChunk - 1) / kRkChunk; }
 
 template <int DT>
 __global__ __launch_bounds__(64 * RowGroup<DT>::W) void k_chunk_carry(const Rk4Sys* arr, Rk4Sys one) {
-    __shared__ double2 sh[2 * DT];
-    const Rk4Sys s = arr ? arr[blockIdx.x] : one;
+    __shared__ double2 sh[3 * DT];
+    const Rk4Sys s = chunk_args(arr, one, blockIdx.x);
     if (s.D != DT || !s.q) return;
-    chunk_carry<DT, false>(sh, s.q, nullptr, chunk_count(s.steps), s.r0, s.xs, nullptr);
+    const long nch = chunk_count(s.steps);
+    if (step_whole(s.plain, nch)) {
+        if (threadIdx.x == 0) s.plain[0] = kWhole;
+        return;
+    }
+    const double2* x = s.r0;
+    for (long i = 0; i < nch;) {
+        const long e = carry_run<false>(s.plain, i, nch), last = min(e, nch - 1);
+        double2* out = s.xs + last * DT;
+        if (s.plain[i])  // first states as the run's samples
+            rk4_rows<DT, false>(sh, s.Ls, i * kRkChunk, last * kRkChunk, x, out, s.dt, kRkChunk, s.xs, nullptr, nullptr,
+                                false);
+        else
+            chunk_carry<DT, false>(sh, s.q, nullptr, nch, i, e, x, s.xs, e < nch ? out : nullptr);
+        __syncthreads();
+        x = out;
+        i = e;
+    }
 }
 
 template <int DT>
 __global__ __launch_bounds__(64 * RowGroup<DT>::W) void k_chunk_states(const Rk4Sys* arr, Rk4Sys one) {
     __shared__ double2 sh[3 * DT];
-    const Rk4Sys s = arr ? arr[blockIdx.y] : one;
+    const Rk4Sys s = chunk_args(arr, one, blockIdx.y);
     const long c = blockIdx.x, n0 = c * kRkChunk;
     if (s.D != DT || !s.q || n0 >= s.steps) return;
-    const long n1 = min(n0 + kRkChunk, s.steps);
+    const bool whole = s.plain[0] == kWhole;
+    if (whole && c) return;
+    const long n1 = whole ? s.steps : min(n0 + kRkChunk, s.steps);
     const bool last = n1 == s.steps;
-    rk4_rows<DT, false>(sh, s.Ls, n0, n1, s.xs + c * DT, last ? s.r : nullptr, s.dt, s.every, s.samples,
+    rk4_rows<DT, false>(sh, s.Ls, n0, n1, whole ? s.r0 : s.xs + c * DT, last ? s.r : nullptr, s.dt, s.every, s.samples,
                         last ? s.nsamples : nullptr, nullptr, last);
 }
 
@@ -755,21 +914,43 @@ __global__ __launch_bounds__(64 * RowGroup<DT>::W) void k_chunk_states(const Rk4
 template <int DT, bool CONST>
 __global__ __launch_bounds__(64) void k_chunk_walk(const Rk4AdjArgs* arr, Rk4AdjArgs one) {
     __shared__ double2 sh[5 * DT];
-    const Rk4AdjArgs A = arr ? arr[blockIdx.y] : one;
+    const Rk4AdjArgs A = chunk_args(arr, one, blockIdx.y);
     const long c = blockIdx.x, n0 = c * kRkChunk;
     if (n0 >= A.steps) return;
-    const long n1 = min(n0 + kRkChunk, A.steps);
-    if constexpr (CONST)
-        rk4_rows_adjoint<DT, WALK_NONE>(sh, A, n0, n1, nullptr, A.bv + c * DT);
-    else  // lam at the chunk's first step is known from the carry: bv takes the repeated value
-        rk4_rows_adjoint<DT, WALK_VEC>(sh, A, n0, n1, A.lam + c * DT, A.bv + c * DT);
+    if constexpr (CONST) {
+        if (!A.plain[c]) rk4_rows_adjoint<DT, WALK_NONE>(sh, A, n0, min(n0 + kRkChunk, A.steps), nullptr, A.bv + c * DT);
+    } else {
+        const bool whole = A.plain[0] == kWhole;
+        if (whole && c) return;
+        // lam at a chunk's first step is known from the carry: bv takes the repeated value
+        rk4_rows_adjoint<DT, WALK_VEC>(sh, A, n0, whole ? A.steps : min(n0 + kRkChunk, A.steps),
+                                       whole ? A.gbar + A.steps * DT : A.lam + c * DT, whole ? A.r0bar : A.bv + c * DT);
+    }
 }
 
 template <int DT>
 __global__ __launch_bounds__(64) void k_chunk_carry_rev(const Rk4AdjArgs* arr, Rk4AdjArgs one) {
-    __shared__ double2 sh[2 * DT];
-    const Rk4AdjArgs A = arr ? arr[blockIdx.x] : one;
-    chunk_carry<DT, true>(sh, A.q, A.bv, chunk_count(A.steps), A.gbar + A.steps * DT, A.lam, A.r0bar);
+    __shared__ double2 sh[5 * DT];
+    const Rk4AdjArgs A = chunk_args(arr, one, blockIdx.x);
+    const long nch = chunk_count(A.steps);
+    const double2* x = A.gbar + A.steps * DT;
+    if (step_whole(A.plain, nch)) {
+        if (threadIdx.x == 0) A.plain[0] = kWhole;
+        return;
+    }
+    for (long i = 0; i < nch;) {
+        const long e = carry_run<true>(A.plain, i, nch), top = nch - 1 - i;  // chunks top .. nch - e
+        double2* out = e < nch ? A.lam + (nch - 1 - e) * DT : A.r0bar;
+        if (A.plain[top]) {
+            if (threadIdx.x < DT) A.lam[top * DT + threadIdx.x] = x[threadIdx.x];
+            rk4_rows_adjoint<DT, WALK_LAM>(sh, A, (nch - e) * kRkChunk, min((top + 1) * kRkChunk, A.steps), x, out);
+        } else {
+            chunk_carry<DT, true>(sh, A.q, A.bv, nch, i, e, x, A.lam, out);
+        }
+        __syncthreads();
+        x = out;
+        i = e;
+    }
 }
 
 // ---------------------------------------------------------------------------
@@ -1037,9 +1218,8 @@ void launch_rk4_chunked(int D, const Rk4Sys* arr, const Rk4Sys& one, unsigned ns
     const unsigned nch = static_cast<unsigned>((max_steps + kRkChunk - 1) / kRkChunk);
     chunk_dispatch(D, [&](auto dc) {
         constexpr int DT = decltype(dc)::value;
-        constexpr unsigned cpb = Chunk<DT>::CPB;
-        hipLaunchKernelGGL((k_chunk_products<DT, Rk4Sys>), dim3((nch + cpb - 1) / cpb, nsys), dim3(Chunk<DT>::NT), 0, st,
-                           arr, one);
+        const dim3 grid((nch + Chunk<DT>::CPB - 1) / Chunk<DT>::CPB, nsys), block(Chunk<DT>::NT);
+        hipLaunchKernelGGL((k_chunk_products<DT, Rk4Sys>), grid, block, 0, st, arr, one);
         hipLaunchKernelGGL(k_chunk_carry<DT>, dim3(nsys), dim3(rk4_rows_threads(DT)), 0, st, arr, one);
         hipLaunchKernelGGL(k_chunk_states<DT>, dim3(nch, nsys), dim3(rk4_rows_threads(DT)), 0, st, arr, one);
     });
@@ -1051,9 +1231,8 @@ void launch_rk4_chunked_walk(int D, const Rk4AdjArgs* arr, const Rk4AdjArgs& one
     chunk_dispatch(D, [&](auto dc) {
         constexpr int DT = decltype(dc)::value;
         if constexpr (DT <= 16) {
-            constexpr unsigned cpb = Chunk<DT>::CPB;
-            hipLaunchKernelGGL((k_chunk_products<DT, Rk4AdjArgs>), dim3((nch + cpb - 1) / cpb, ntapes),
-                               dim3(Chunk<DT>::NT), 0, st, arr, one);
+            const dim3 grid((nch + Chunk<DT>::CPB - 1) / Chunk<DT>::CPB, ntapes), block(Chunk<DT>::NT);
+                hipLaunchKernelGGL((k_chunk_products<DT, Rk4AdjArgs>), grid, block, 0, st, arr, one);
             hipLaunchKernelGGL((k_chunk_walk<DT, true>), dim3(nch, ntapes), dim3(64), 0, st, arr, one);
             hipLaunchKernelGGL(k_chunk_carry_rev<DT>, dim3(ntapes), dim3(64), 0, st, arr, one);
             hipLaunchKernelGGL((k_chunk_walk<DT, false>), dim3(nch, ntapes), dim3(64), 0, st, arr, one);

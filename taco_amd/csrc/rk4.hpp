@@ -53,6 +53,7 @@ struct Rk4Sys {
     const double2* Lh = nullptr;  // [steps][D x D] given midpoints, else formed on the fly
     double2* q = nullptr;         // chunked run: [chunks][D x D] products, null: one sequential run
     double2* xs = nullptr;        // chunked run: [chunks][D] first states; wide run: kRkWideVecs x D
+    int* plain = nullptr;         // chunked run: [chunks] whether a chunk is stepped (chunk_mild)
     long every = 1;               // sample distance
     long* nsamples = nullptr;
 };
@@ -73,6 +74,7 @@ struct Rk4AdjArgs {
     double2* q = nullptr;          // chunked walk: [chunks][D * D] products,
     double2* lam = nullptr;        // [chunks][D] lam after each chunk's last step (wide walk: kRkWideVecs x D),
     double2* bv = nullptr;         // [chunks][D] constant parts
+    int* plain = nullptr;          // [chunks] whether a chunk is stepped (chunk_mild)
 };
 
 // Steps of a chunk of the chunked runs.
@@ -87,10 +89,18 @@ inline bool rk4_chunked(int D, long steps) {
     return steps >= kRkChunkedMin && (D == 4 || D == 9 || D == 16 || D == 25 || D == 36);
 }
 inline bool rk4_chunked_walk(int D, long steps) { return D <= 16 && rk4_chunked(D, steps); }
-// Complex values of a chunked run's products and first states (or lam).
+// A chunked run's products, first states (or lam) and flags, in that order, and
+// the complex values they take.
+inline std::size_t rk4_chunks(long steps) { return static_cast<std::size_t>((steps + kRkChunk - 1) / kRkChunk); }
 inline std::size_t rk4_chunk_values(int D, long steps) {
-    const std::size_t nch = static_cast<std::size_t>((steps + kRkChunk - 1) / kRkChunk);
-    return nch * (static_cast<std::size_t>(D) * D + D);
+    const std::size_t nch = rk4_chunks(steps);
+    return nch * (static_cast<std::size_t>(D) * D + D) + (nch + 3) / 4;
+}
+inline void rk4_place_chunks(int D, long steps, double2* base, double2*& q, double2*& x, int*& plain) {
+    const std::size_t nch = rk4_chunks(steps);
+    q = base;
+    x = q + nch * D * D;
+    plain = reinterpret_cast<int*>(x + nch * D);
 }
 
 // Whether runs at D are wide (rk4.hip): two generators do not fit the LDS

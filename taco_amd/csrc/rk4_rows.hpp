@@ -216,6 +216,7 @@ __device__ __forceinline__ void load_points(double2 (&p)[4], double2& gb, const 
 enum WalkKeep {
     WALK_LBAR,  // the generator cotangents, formed in place
     WALK_VEC,   // kb1..kb4 (A.vec): k_rk4_lbar forms Lbar from them
+    WALK_LAM,   // lam after every chunk's last step but the walk's own (A.lam)
     WALK_NONE,  // nothing: only lam at the first step is wanted
 };
 
@@ -300,6 +301,9 @@ struct RowsAdjoint {
             }
         }
         lam = cadd(cadd(rb, ub0), Gb);
+        if constexpr (KEEP == WALK_LAM) {
+            if (own && n > 0 && n % kRkChunk == 0) A->lam[(n / kRkChunk - 1) * DT + c] = lam;
+        }
         par ^= 1;
         if (own) K4[par * DT + c] = cscale(lam, s6);
         __builtin_amdgcn_sched_barrier(0);

@@ -333,6 +333,60 @@ def test_wide_reverse_matches_forward(d, steps, K):
     assert abs(got - ref) <= FD_TOL * abs(ref) + 1e-14 * abs(loss(0.0)) / h
 
 
+def dephasing_set(orc, N, rate, steps, dt, r0):
+    """Pure dephasing: H and A diagonal, Gamma constant in time, scaled so that
+    the fastest coherence decays by `rate` a step.  L is diagonal (order 2), so
+    every component of vec(rho) runs by itself.  Returns the tape's arguments and
+    the generators."""
+    H = np.diag(np.linspace(-0.5, 0.6, N) ** 2).astype(complex)
+    A = np.diag(np.linspace(-1.0, 0.8, N)).astype(complex)
+    S = orc.system_build(H, [A])
+    gamma = np.ones((steps + 1, S["nf"]), complex)
+    slow = orc.tcl2_at(S["eps"], S["A_eig"], S["pair_to_freq"], gamma[0])
+    gamma *= rate / (dt * -np.real(np.diag(slow)).min())
+    L = orc.tcl2_at(S["eps"], S["A_eig"], S["pair_to_freq"], gamma[0])
+    assert np.count_nonzero(L - np.diag(np.diag(L))) == 0
+    st = dict(gamma=gamma, omegas=S["omegas"], mirror=orc.mirror(S["omegas"]), pair_to_freq=S["pair_to_freq"],
+              ops=S["A_eig"], eps=S["eps"], dt=dt, steps=steps, r0=r0, order=2)
+    return st, np.repeat(L[None], steps + 1, axis=0)
+
+
+@pytest.mark.parametrize("N", [2, 3, 4])
+@pytest.mark.parametrize("rates", [(0.5, 1.0), (0.01, 0.7, 0.1)])
+@pytest.mark.parametrize("steps", [256, 403])
+def test_long_damped_reverse_matches_oracle(orc, N, rates, steps):
+    """The reverse RK4 of 256 steps and more keeps the relative accuracy of
+    cotangents that decay: with a cotangent of the last state only, component c of
+    r0's is conj(f_c) times it, f_c the oracle's sequential run from 1.  Sets of
+    different damping in one multi-set tape, which has the single tapes' values
+    bit for bit.  Both sides round once per sum and product, about 4 eps a step."""
+    rng = np.random.default_rng(3)
+    D, dt = N * N, 0.05
+    bar = np.zeros((steps + 1, D), complex)
+    bar[-1] = rng.standard_normal(D) + 1j * rng.standard_normal(D)
+    sets, want = [], []
+    for rate in rates:
+        st, L = dephasing_set(orc, N, rate, steps, dt, np.ones(D, complex))
+        sets.append(st)
+        want.append(orc.propagate(L, np.ones(D, complex), dt)[1])
+    mt = AD.MultiTape(sets, checkpoint_every=32)
+    got = mt.adjoint([bar] * len(sets))
+    samples = [s.copy() for s in mt.samples]
+    mt.close()
+    for k, (st, ref) in enumerate(zip(sets, want)):
+        ref = np.asarray(ref)
+        assert (np.abs(samples[k] - ref) <= 1e-12 * np.abs(ref)).all(), k
+        r0bar = np.conj(ref[-1]) * bar[-1]
+        assert (np.abs(got[k]["r0"] - r0bar) <= 1e-12 * np.abs(r0bar)).all(), k
+        tp = AD.Tape(st["gamma"], st["omegas"], st["mirror"], st["pair_to_freq"], st["ops"], st["eps"], dt, steps,
+                     st["r0"], 2, 32)
+        single = tp.adjoint(bar)
+        assert np.array_equal(samples[k], tp.samples), k
+        tp.close()
+        for key in ("gamma", "omegas", "eps", "r0"):
+            assert np.array_equal(got[k][key], single[key]), (k, key)
+
+
 @pytest.mark.parametrize("steps", [1, 62, 63, 64, 127, 128, 191, 192, 254, 255])
 def test_short_slice_reverse_matches_long(steps):
     """Tapes of at most 256 times take the one-wave slice reverse.  A run of 256

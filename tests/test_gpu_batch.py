@@ -78,6 +78,26 @@ def test_batch_matches_oracle(orc, batch_and_items):
             assert er <= TOL, names[s]
 
 
+def test_batch_of_long_runs_equals_plain_builders():
+    """Runs of 256 steps and more at D = 4, 9, 16 and 25, two lengths of one D,
+    one strongly damped system (its Gamma 100 times the others'), beside a short
+    run; eager and replayed.  (Order 2: L4 is not what is tested.)"""
+    items = []
+    for d, steps, scale in ((2, 300, 1), (2, 1000, 1), (3, 257, 100), (4, 400, 1), (4, 288, 100), (5, 256, 1), (3, 40, 1)):
+        rng = W.SplitMix64(40 + d)
+        w = W.Workload("g", W.gue(d, rng), [W.random_hermitian_unit(d, rng)], taco_amd.DrudeLorentz(0.1, 4.0), 0.9,
+                       0.02, 1023, [0], steps=steps)
+        items.append(taco_amd.BatchItem(w.system, scale * w.gamma, w.dt, [], steps=steps, r0=r0_for(d), order=2))
+    b = taco_amd.Batch(items).run()
+    ref = [taco_amd.tcl4_propagate(it.system, it.gamma, it.dt, it.steps, it.r0, order=2) for it in items]
+    for graph in (False, True, True):
+        if graph:
+            b.run(graph=True)
+        for s in range(len(items)):
+            assert np.array_equal(b.rho(s), ref[s]), (graph, s)
+    b.close()
+
+
 def test_graph_replays_equal_eager():
     """The captured hipGraph, replayed several times with eager engine work
     and synchronisations in between, reproduces the eager results exactly."""

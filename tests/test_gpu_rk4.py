@@ -48,6 +48,60 @@ def test_chunked_rk4_matches_oracle(orc, D, steps, every):
     assert max_rel_err(np.array(seen), ref)[0] <= 1e-12
 
 
+def damped_series(D, rate, steps, dt, seed):
+    """Generators of two uncoupled parts: D // 2 components that only decay and
+    rotate, dt times their rates from 0.2 to 1 times `rate`, and a dense part that
+    decays uniformly at rate / 2.  Strong over the first and the last third of the
+    run, 1 / 50 of that between."""
+    rng = np.random.default_rng(seed)
+    n = D // 2
+    base = np.zeros((D, D), complex)
+    base[np.arange(n), np.arange(n)] = -rate * np.linspace(0.2, 1.0, n) + 0.3j * rate * rng.standard_normal(n)
+    A = rng.standard_normal((D - n, D - n)) + 1j * rng.standard_normal((D - n, D - n))
+    base[n:, n:] = 0.2 * rate * (A - A.conj().T) / np.linalg.norm(A) - 0.5 * rate * np.eye(D - n)
+    s = np.arange(steps + 1)
+    f = np.where((s > steps // 3) & (s < 2 * steps // 3), 0.02, 1.0) * (1 + 0.05 * np.cos(0.01 * s))
+    return base[None] * f[:, None, None] / dt, n, rng.standard_normal(D) + 1j * rng.standard_normal(D)
+
+
+@pytest.mark.parametrize("D", [4, 9, 16, 25, 36])
+@pytest.mark.parametrize("rate", [0.005, 0.03, 0.1, 0.5, 1.0])
+@pytest.mark.parametrize("steps", [400, 777])
+def test_long_damped_rk4_matches_oracle(orc, D, rate, steps):
+    """Runs of 256 steps and more of generators that damp by `rate` a step keep
+    their relative accuracy: every decoupled component by itself and the dense
+    part in norm, at every step, against the oracle's sequential run.  Both round
+    once per sum and product: 777 steps of about 4 eps each, below 1e-12."""
+    Ls, n, r0 = damped_series(D, rate, steps, 0.05, 11 + D)
+    seen = []
+    r = taco_amd.propagate_rk4_dense(Ls, r0, 0.0, 0.05, on_sample=lambda t, v: seen.append(v.copy()))
+    rr, ref = orc.propagate(Ls, r0, 0.05)
+    got, ref = np.array(seen), np.asarray(ref)
+    assert got.shape == ref.shape and np.array_equal(got[-1], r)
+    assert (np.abs(got - ref)[:, :n] <= 1e-12 * np.abs(ref)[:, :n]).all()
+    e = np.linalg.norm((got - ref)[:, n:], axis=1) / np.linalg.norm(ref[:, n:], axis=1)
+    assert e.max() <= 1e-12
+
+
+@pytest.mark.parametrize("D", [4, 16, 36])
+def test_long_rk4_with_a_non_finite_generator(orc, D):
+    """A NaN or an infinity in one generator: the states before it are the
+    finite run's, those after it are not finite, as in the sequential run."""
+    steps, at = 400, 150
+    rng = np.random.default_rng(5)
+    Ls = np.array([0.1 * (rng.standard_normal((D, D)) + 1j * rng.standard_normal((D, D)))] * (steps + 1))
+    r0 = rng.standard_normal(D) + 0j
+    ref = np.asarray(orc.propagate(Ls, r0, 0.01)[1])
+    for bad in (np.nan, np.inf):
+        Lb = Ls.copy()
+        Lb[at, 0, D - 1] = bad
+        seen = []
+        taco_amd.propagate_rk4_dense(Lb, r0, 0.0, 0.01, on_sample=lambda t, v: seen.append(v.copy()))
+        got = np.array(seen)
+        assert np.abs(got[:at] - ref[:at]).max() <= 1e-12 * np.abs(ref[:at]).max()
+        assert not np.isfinite(got[at:]).any()
+
+
 @pytest.mark.parametrize("D", [69, 70, 81, 256, 257, 300])
 @pytest.mark.parametrize("steps,every", [(1, 1), (2, 7), (9, 4)])
 @pytest.mark.parametrize("half", [False, True])
