@@ -121,8 +121,8 @@ int taco_profile_get(taco_ctx* ctx, int kernel, double* total_ms, long* launches
 /* Shape of the FFT passes of length 2^log2_nfft last run in this context, per
  * phase A, B, C (3: tiles of 2048 values; 10, 11: groups of 2^10, 2^11 values,
  * one workgroup each; -1 if none ran yet).  Every shape performs the same
- * butterflies.  TACO_FFT_TILE forces one: 0, 1 the tiles on 256 / 512 threads,
- * 2, 3 groups of 2^10, 2^11.  No reference counterpart (the
+ * butterflies.  TACO_FFT_TILE forces one: 0, 1 tiles (1: of 8192 values in
+ * phases A and C), 2, 3 groups of 2^10, 2^11.  No reference counterpart (the
  * reference's cuFFT plans are internal, tcl4_fcr_kernels.cu:602-622). */
 int taco_fft_tile_choice(taco_ctx* ctx, int log2_nfft, int* cfg3);
 

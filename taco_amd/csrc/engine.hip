@@ -83,7 +83,7 @@ __device__ __forceinline__ double2 cexpi(double arg) {
 
 constexpr int kBlock = 256;
 
-// FFT phases: 512-thread workgroups on a tile of 8192 complex values (G
+// FFT phases on tiles: NT-thread workgroups on a tile of TILE complex values (G
 // groups of 2^lg) in LDS.  Stages run as radix-2^r register passes: a thread
 // loads the 2^r values of a closed butterfly set, performs r radix-2 stages
 // on them (each butterfly exactly u +/- w*x with the stage's table
@@ -96,8 +96,14 @@ struct FftCfg {
     static constexpr int kPT = TILE / NT;  // values per thread (8 or 16)
     static constexpr int kLds = TILE + TILE / 8;
 };
+// The wide tile takes phases A and C of 2^10 and 2^11 classes, of which a small one
+// holds 2 columns or 1 and so moves runs of 32 or 16 B.  One L4 call at 1001 times
+// up to 10^4, small tiles -> wide: FFT length 2^21, d = 4: 81.1 -> 63.8 ms; 2^22,
+// d = 4: 267 -> 144 ms, d = 2: 5.86 -> 3.97 ms.  At 2^9 classes the small one is the
+// faster (phase A, length 2^20, d = 4: 27.8 against 28.1 ms), as it is for long windows of
+// fewer (phase C, length 2^19, 30001 times, d = 4: 13.7 against 14.3 ms).
 using Cfg2k = FftCfg<2048, 256>;
-using Cfg2kW = FftCfg<2048, 512>;
+using CfgWide = FftCfg<8192, 1024>;
 
 // Physical LDS slot of (group, position): one pad slot per 16 values and an
 // odd group stride keep strided accesses off a single bank.
@@ -2070,7 +2076,8 @@ struct FftShape {
 // Nfft 2^13, T = 201: 313 ms a gradient against 326), as it is when the
 // groups of 2^11 would leave compute units idle.  Lengths below 2^10 run on
 // tiles.  TACO_FFT_TILE forces a shape (every one performs the same
-// butterflies): 0, 1 the tiles on 256 / 512 threads, 2, 3 groups of 2^10, 2^11.
+// butterflies): 0, 1 tiles (1: the wide one in phases A and C), 2, 3 groups of
+// 2^10, 2^11.
 static FftShape fft_shape(int L, long na, std::size_t T) {
     const int forced = env_int("TACO_FFT_TILE", -1);
     if (L < kGroupBitsMin || forced == 0 || forced == 1) return {(L + 1) / 2, L / 2, false};
@@ -2084,44 +2091,38 @@ static FftShape fft_shape(int L, long na, std::size_t T) {
 // Launch phase kernels for a tile configuration index.
 enum Phase { PH_A_TRIPLE, PH_A_SPEC, PH_B_TRIPLE, PH_B_SPEC, PH_C };
 
+// Phases A and C on tiles.
 template <class Cfg>
-static void launch_phase_cfg(Phase ph, const FcrArgs& P, long njobs, hipStream_t st) {
-    const int ngA = 1 << P.b, ngB = 1 << P.a;
-    switch (ph) {
-        case PH_A_TRIPLE: {  // njobs = number of Omega classes touching the chunk
-            const long blocks = njobs * (ngA / tile_groups<Cfg>(P.a, ngA));
-            hipLaunchKernelGGL(k_phase_a<Cfg>, dim3(static_cast<unsigned>(blocks)), dim3(Cfg::kFT), 0, st, P);
-            break;
-        }
-        case PH_A_SPEC: {
-            const long blocks = njobs * (ngA / tile_groups<Cfg>(P.a, ngA));
-            hipLaunchKernelGGL(k_phase_a_spec<Cfg>, dim3(static_cast<unsigned>(blocks)), dim3(Cfg::kFT), 0, st, P);
-            break;
-        }
-        case PH_B_TRIPLE:
-        case PH_B_SPEC: {
-            const long blocks = njobs * (ngB / tile_groups<Cfg>(P.b, ngB));
-            hipLaunchKernelGGL(k_phase_b<Cfg>, dim3(static_cast<unsigned>(blocks)), dim3(Cfg::kFT), 0, st, P,
-                               ph == PH_B_SPEC ? 1 : 0);
-            break;
-        }
-        case PH_C: {
-            const long tiles = 2 * njobs * (ngA / tile_groups<Cfg>(P.a, ngA));
-            const long blocks = (tiles + 1) / 2;
-            hipLaunchKernelGGL(k_phase_c<Cfg>, dim3(static_cast<unsigned>(blocks)), dim3(Cfg::kFT), 0, st, P,
-                               static_cast<int>(tiles));
-            break;
-        }
+static void launch_columns(Phase ph, const FcrArgs& P, long njobs, hipStream_t st) {
+    const long ngA = 1L << P.b, per = ngA / tile_groups<Cfg>(P.a, static_cast<int>(ngA));
+    if (ph == PH_C) {
+        const long tiles = 2 * njobs * per;
+        hipLaunchKernelGGL(k_phase_c<Cfg>, dim3(static_cast<unsigned>((tiles + 1) / 2)), dim3(Cfg::kFT), 0, st, P,
+                           static_cast<int>(tiles));
+        return;
     }
+    // A: njobs = number of Omega classes touching the chunk, or of spectra
+    const dim3 grid(static_cast<unsigned>(njobs * per));
+    if (ph == PH_A_TRIPLE)
+        hipLaunchKernelGGL(k_phase_a<Cfg>, grid, dim3(Cfg::kFT), 0, st, P);
+    else
+        hipLaunchKernelGGL(k_phase_a_spec<Cfg>, grid, dim3(Cfg::kFT), 0, st, P);
+}
+
+// Phase B on tiles.
+static void launch_tile_b(Phase ph, const FcrArgs& P, long njobs, hipStream_t st) {
+    const int ngB = 1 << P.a;
+    const long blocks = njobs * (ngB / tile_groups<Cfg2k>(P.b, ngB));
+    hipLaunchKernelGGL(k_phase_b<Cfg2k>, dim3(static_cast<unsigned>(blocks)), dim3(Cfg2k::kFT), 0, st, P,
+                       ph == PH_B_SPEC ? 1 : 0);
 }
 
 static void launch_phase(Phase ph, const FcrArgs& P, bool group, long njobs, hipStream_t st) {
-    if (group && (ph == PH_B_TRIPLE || ph == PH_B_SPEC)) {
-        launch_group_b(P, njobs, ph == PH_B_SPEC, st);
-        return;
-    }
-    if (group && (ph == PH_A_TRIPLE || ph == PH_A_SPEC) && column_a_fits(P)) {
-        launch_column_a(P, njobs, ph == PH_A_SPEC, st);
+    if (ph == PH_B_TRIPLE || ph == PH_B_SPEC) {
+        if (group)
+            launch_group_b(P, njobs, ph == PH_B_SPEC, st);
+        else
+            launch_tile_b(ph, P, njobs, st);
         return;
     }
     if (ph == PH_C) {
@@ -2130,11 +2131,15 @@ static void launch_phase(Phase ph, const FcrArgs& P, bool group, long njobs, hip
             launch_group_c(P, st);
             return;
         }
+    } else if (group && column_a_fits(P)) {
+        launch_column_a(P, njobs, ph == PH_A_SPEC, st);
+        return;
     }
-    if (env_int("TACO_FFT_TILE", -1) == 1)
-        launch_phase_cfg<Cfg2kW>(ph, P, njobs, st);
+    const int forced = env_int("TACO_FFT_TILE", -1);
+    if (forced == 1 || (forced != 0 && P.a > 9))
+        launch_columns<CfgWide>(ph, P, njobs, st);
     else
-        launch_phase_cfg<Cfg2k>(ph, P, njobs, st);
+        launch_columns<Cfg2k>(ph, P, njobs, st);
 }
 
 // Read at each launch (a test compares the two paths in one process).
