@@ -660,10 +660,9 @@ def main():
     choice = np.zeros(3, np.int32)
     nfft = 1 << int(np.ceil(np.log2(2 * G.shape[0] - 1)))
     _lib.check(_lib.lib().taco_fft_tile_choice(tcl4.context(0).handle, int(np.log2(nfft)), _lib.iptr(choice)))
-    shapes = {-1: None, 3: "tiles of 2048"}
-    fft_tiles = {ph: shapes.get(int(c), f"groups of {1 << int(c)}") for ph, c in zip("ABC", choice)}
-    if choice[1] > 3:
-        fft_tiles["A"] = "register columns"
+    shapes = {-1: None, 0: "tiles of 8192", 3: "tiles of 2048", 10: "groups of 1024", 11: "groups of 2048",
+              20: "register columns"}
+    fft_tiles = {ph: shapes[int(c)] for ph, c in zip("ABC", choice)}
     L4 = out.cpu().numpy().reshape(ntau, S.N ** 2, S.N ** 2).transpose(0, 2, 1)
     cpu, parity, ref_libm = None, None, None
     if not a.no_cpu:

@@ -118,12 +118,13 @@ int taco_profile_enable(taco_ctx* ctx, int on);
 int taco_profile_reset(taco_ctx* ctx);
 int taco_profile_get(taco_ctx* ctx, int kernel, double* total_ms, long* launches, double* algo_bytes);
 
-/* Shape of the FFT passes of length 2^log2_nfft last run in this context, per
- * phase A, B, C (3: tiles of 2048 values; 10, 11: groups of 2^10, 2^11 values,
- * one workgroup each; -1 if none ran yet).  Every shape performs the same
- * butterflies.  TACO_FFT_TILE forces one: 0, 1 tiles (1: of 8192 values in
- * phases A and C), 2, 3 groups of 2^10, 2^11.  No reference counterpart (the
- * reference's cuFFT plans are internal, tcl4_fcr_kernels.cu:602-622). */
+/* Kernels of the FFT pass of length 2^log2_nfft last run in this context, per
+ * phase A, B, C (0: tiles of 8192 values; 3: tiles of 2048; 10, 11: groups of
+ * 2^10, 2^11 values in registers, one workgroup each; 20: columns in registers;
+ * -1 if none ran yet).  All perform the same butterflies.  TACO_FFT_TILE forces
+ * 0, 1: tiles (1: of 8192 values in phases A and C), 2, 3: groups of 2^10, 2^11.
+ * No reference counterpart (the reference's cuFFT plans are internal,
+ * tcl4_fcr_kernels.cu:602-622). */
 int taco_fft_tile_choice(taco_ctx* ctx, int log2_nfft, int* cfg3);
 
 /* Correctly rounded sin/cos of each x[i] (|x| < 2^30): the phase routine of

@@ -1964,7 +1964,7 @@ struct taco_ctx {
     hipStream_t stream = nullptr;
     hipEvent_t ev0 = nullptr, ev1 = nullptr;
     taco_engine::Profiler prof;
-    std::map<int, int> fft_shape;  // per FFT log-length: group bits of the last pass (0: tile kernels)
+    std::map<int, std::array<int, 3>> fft_kernels;  // per FFT log-length: the last pass's kernels of phases A, B, C
     std::map<int, std::unique_ptr<taco_engine::Twiddles>> tw;
     taco_engine::DevBuf gamma, omegas, mirror, p2f, ops, spec, inter1, inter2, conv, slices, t2pos, l4, gw, misc,
         rk, eps, jobtri, clsstart, jobmask, jobrow, comb, t2scr, rkmid, bred;
@@ -2117,29 +2117,36 @@ static void launch_tile_b(Phase ph, const FcrArgs& P, long njobs, hipStream_t st
                        ph == PH_B_SPEC ? 1 : 0);
 }
 
-static void launch_phase(Phase ph, const FcrArgs& P, bool group, long njobs, hipStream_t st) {
+// The kernels of a phase, as taco_fft_tile_choice reports them (a group's is its b).
+enum FftKernel { FFT_WIDE_TILES = 0, FFT_TILES = 3, FFT_COLUMNS = 20 };
+
+// Launches a phase and returns which kernels took it.
+static int launch_phase(Phase ph, const FcrArgs& P, bool group, long njobs, hipStream_t st) {
     if (ph == PH_B_TRIPLE || ph == PH_B_SPEC) {
-        if (group)
+        if (group) {
             launch_group_b(P, njobs, ph == PH_B_SPEC, st);
-        else
-            launch_tile_b(ph, P, njobs, st);
-        return;
+            return P.b;
+        }
+        launch_tile_b(ph, P, njobs, st);
+        return FFT_TILES;
     }
     if (ph == PH_C) {
-        if (group && P.a == 0) return;  // phase B stored the convolutions
+        if (group && P.a == 0) return P.b;  // phase B stored the convolutions
         if (group_c_fits(P)) {
             launch_group_c(P, st);
-            return;
+            return FFT_COLUMNS;
         }
     } else if (group && column_a_fits(P)) {
         launch_column_a(P, njobs, ph == PH_A_SPEC, st);
-        return;
+        return FFT_COLUMNS;
     }
     const int forced = env_int("TACO_FFT_TILE", -1);
-    if (forced == 1 || (forced != 0 && P.a > 9))
+    if (forced == 1 || (forced != 0 && P.a > 9)) {
         launch_columns<CfgWide>(ph, P, njobs, st);
-    else
-        launch_columns<Cfg2k>(ph, P, njobs, st);
+        return FFT_WIDE_TILES;
+    }
+    launch_columns<Cfg2k>(ph, P, njobs, st);
+    return FFT_TILES;
 }
 
 // Read at each launch (a test compares the two paths in one process).
@@ -2526,7 +2533,7 @@ static void fcr_launch(taco_ctx* c, FcrJob& J, const CombineArgs& out) {
     P.conv = c->conv.as<double2>();
     const long spec_jobs = J.spec_jobs;
     const std::vector<int>& cls_start = J.cls_start;
-    c->fft_shape[J.L] = J.group ? P.b : 0;
+    std::array<int, 3> ran{-1, -1, -1};
     const double ch = static_cast<double>(P.Tq << P.a) * 16.0;  // the kept rows of one half-inverse product
     const double cn = static_cast<double>(J.n) * 16.0;      // one complex series of length Nfft
     const double cNt = static_cast<double>(J.Nt) * 16.0;
@@ -2556,15 +2563,15 @@ static void fcr_launch(taco_ctx* c, FcrJob& J, const CombineArgs& out) {
             const long ncls = class_of(a1 - 1) - P.cls0 + 1;
             const double na = static_cast<double>(a1 - a0);
             // phase A: read the Gamma column, write the half-transformed signal, once per A-job
-            timed(c, K_PHASE_A, na * (cNt + cn), [&] { launch_phase(PH_A_TRIPLE, P, J.group, ncls, c->stream); });
+            timed(c, K_PHASE_A, na * (cNt + cn), [&] { ran[0] = launch_phase(PH_A_TRIPLE, P, J.group, ncls, c->stream); });
             // F and C paths of the chunk (one or both per triple)
             const double np_ = static_cast<double>(J.paths[job0 + nj] - J.paths[job0]);
             // phase B: read each A-job's signal once and one spectrum per path, write the
             // kept rows of one half-inverse product per path
             timed(c, K_PHASE_B, na * cn + np_ * (cn + ch),
-                  [&] { launch_phase(PH_B_TRIPLE, P, J.group, a1 - a0, c->stream); });
+                  [&] { ran[1] = launch_phase(PH_B_TRIPLE, P, J.group, a1 - a0, c->stream); });
             // phase C: read each path's product, write its convolution for t < T
-            timed(c, K_PHASE_C, np_ * (ch + cT), [&] { launch_phase(PH_C, P, J.group, nj, c->stream); });
+            timed(c, K_PHASE_C, np_ * (ch + cT), [&] { ran[2] = launch_phase(PH_C, P, J.group, nj, c->stream); });
             HIP_OK(hipGetLastError());
         }
         // combine: read three Gamma columns and each path's convolution over
@@ -2588,6 +2595,7 @@ static void fcr_launch(taco_ctx* c, FcrJob& J, const CombineArgs& out) {
         });
         HIP_OK(hipGetLastError());
     }
+    c->fft_kernels[J.L] = ran;
 }
 
 // The Direct method over the pass's triples (every one, or the ones the L4
@@ -4622,10 +4630,8 @@ int taco_profile_get(taco_ctx* ctx, int kernel, double* total_ms, long* launches
 int taco_fft_tile_choice(taco_ctx* ctx, int log2_nfft, int* cfg3) {
     return guarded([&] {
         check_ctx(ctx);
-        auto it = ctx->fft_shape.find(log2_nfft);
-        const int v = it == ctx->fft_shape.end() ? -1 : it->second ? it->second : 3;
-        cfg3[0] = v < 0 ? v : 3;  // phase A always runs on tiles
-        cfg3[1] = cfg3[2] = v;
+        const auto it = ctx->fft_kernels.find(log2_nfft);
+        for (int ph = 0; ph < 3; ++ph) cfg3[ph] = it == ctx->fft_kernels.end() ? -1 : it->second[ph];
     });
 }
 

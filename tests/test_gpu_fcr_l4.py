@@ -367,6 +367,29 @@ def test_fft_tile_configs_bitwise_identical(orc, cfg):
     assert max_rel_err(got, oref)[0] <= TOL
 
 
+@pytest.mark.parametrize("Nt,keep,shape,want", [
+    (200, 200, None, (3, 3, 20)),         # 2^9: below the groups; phase C's columns fit the registers
+    (512, 512, None, (20, 10, 10)),       # one group: phase B stores the convolutions
+    (9001, 9001, "3", (20, 11, 20)),
+    (9001, 9001, "0", (3, 3, 3)),
+    (9001, 9001, "1", (0, 3, 0)),
+    (40000, 40000, None, (20, 11, 3)),    # 20 kept rows of 2^11
+    (300000, 700, None, (3, 11, 20)),     # 2^9 classes
+    (600000, 700, None, (0, 11, 0)),      # 2^10 classes
+])
+def test_fft_kernels_reported(Nt, keep, shape, want, monkeypatch):
+    """taco_fft_tile_choice names the kernels that ran in each phase."""
+    from taco_amd import _lib, tcl4
+    if shape is not None:
+        monkeypatch.setenv("TACO_FFT_TILE", shape)
+    w = W.spin_boson(Nt=Nt, tmax=150)
+    taco_amd.compute_triple_kernels(w.system, w.gamma, w.dt, keep=keep)
+    got = np.zeros(3, np.int32)
+    L = (2 * w.gamma.shape[0] - 2).bit_length()
+    _lib.check(_lib.lib().taco_fft_tile_choice(tcl4.context(0).handle, L, _lib.iptr(got)))
+    assert tuple(got) == want
+
+
 @pytest.mark.parametrize("Nt,keep", [
     (512, 1), (512, 512),            # one group of 2^10: phase B stores the convolutions
     (513, 513), (1024, 300),         # Nfft 2^11
