@@ -302,10 +302,10 @@ int taco_fcr_batched_dev(taco_ctx* ctx, const void* gamma, const void* omegas, c
  * ops [num_ops][N*N], L4_out [npos][N^4], GW_out [npos][N^4] (nullable).
  * Enqueued on `stream` (a hipStream_t; NULL = the default stream) of the
  * current device and not synchronised.  The factorised kernel's per-time
- * intermediates live in a 64 MiB file-scope device array that each GPU holds
- * until the process ends; times run in launches whose intermediates fit it,
- * and a single time that needs more than 64 MiB (N and nf with
- * (num_ops^2 (2N^2 + 2N^2 nf) + N^2 nf + N^2) * 16 bytes above it) is refused
+ * intermediates live in LDS at small N, else in a 64 MiB file-scope device array
+ * that each GPU holds until the process ends; times run in launches whose
+ * intermediates fit it, and N, nf and num_ops with
+ * (num_ops^2 (2N^2 + 2N^2 nf) + N^2 nf + N^2) * 16 bytes above 64 MiB are refused
  * with TACO_ERR_INVALID.  Calls that overlap on one GPU share the array and
  * race: serialise them (one stream, or events).  No hipMalloc, hipFree or
  * other allocation happens in this call. */

@@ -1511,10 +1511,13 @@ static std::size_t l4f_lds(int N, int nf, int num_ops, int parts, bool inter) {
            N2 * 4;
 }
 constexpr std::size_t kL4fInterLds = 48 * 1024;  // three workgroups per CU and more
+static bool l4f_in_lds(int N, int nf, int num_ops) {
+    return N < kFwdLargeN && l4f_lds(N, nf, num_ops, kBlock, true) <= kL4fInterLds;
+}
 static void launch_k_l4f(unsigned grid, hipStream_t st, L4fArgs F) {
     F.parts = true;
     std::size_t lds = l4f_lds(F.N, F.nf, F.num_ops, kBlock, true);
-    if (F.N < kFwdLargeN && lds <= kL4fInterLds) {
+    if (l4f_in_lds(F.N, F.nf, F.num_ops)) {
         hipLaunchKernelGGL((k_l4f<kBlock, true>), dim3(grid), dim3(kBlock), lds, st, F);
         return;
     }
@@ -2670,15 +2673,18 @@ static void set_l4_lds(taco_ctx* c, std::size_t lds) {
     }
 }
 
-// Scratch of the factorised L4: complex values per position, and positions
-// per launch (at most 1 GiB of scratch per launch).
+// Scratch of the factorised L4: complex values per position (none where the
+// intermediates live in LDS), and positions per launch (at most 1 GiB of scratch).
 static long l4f_per_pos(int N, int nf, int num_ops) {
+    if (l4f_in_lds(N, nf, num_ops)) return 0;
     const long N2 = static_cast<long>(N) * N, P = static_cast<long>(num_ops) * num_ops;
-    return P * (2 * N2 + 2 * N2 * nf) + N2 * nf + N2;
+    return P * (2 * N2 + 2 * N2 * nf);
+}
+static long l4f_chunk(long per, std::size_t scratch_bytes, long npos) {
+    return per ? std::max(1L, std::min(npos, static_cast<long>(scratch_bytes / (per * 16)))) : npos;
 }
 static long l4f_chunk(int N, int nf, int num_ops, long npos) {
-    const long per = l4f_per_pos(N, nf, num_ops);
-    return std::max(1L, std::min(npos, static_cast<long>((std::size_t{1} << 30) / (per * 16))));
+    return l4f_chunk(l4f_per_pos(N, nf, num_ops), std::size_t{1} << 30, npos);
 }
 
 // Factorised L4 (any N), positions in launches of at most 1 GiB of scratch.
@@ -4991,13 +4997,15 @@ int taco_l4_from_slices_noalloc(const void* Fs, const void* Cs, const void* Rs, 
         const long N2 = static_cast<long>(N) * N;
         const std::size_t lds = static_cast<std::size_t>(num_ops) * N2 * 16 + static_cast<std::size_t>(N2) * 4;
         if (lds > 64 * 1024) throw Error(TACO_ERR_INVALID, "factorised L4 kernel: coupling operators exceed 64 KiB of LDS");
-        const long per = l4f_per_pos(N, nf, num_ops);
-        const std::size_t per_bytes = static_cast<std::size_t>(per) * sizeof(double2);
+        // the documented limit, an upper bound of the scratch
+        const std::size_t per_bytes =
+            static_cast<std::size_t>(static_cast<long>(num_ops) * num_ops * (2 * N2 + 2 * N2 * nf) + N2 * nf + N2) * 16;
         if (per_bytes > kNoallocScratchBytes)
             throw Error(TACO_ERR_INVALID, "one time's L4 intermediates (" + std::to_string(per_bytes) +
                                               " bytes) exceed the 64 MiB scratch of the allocation-free entry point");
+        const long per = l4f_per_pos(N, nf, num_ops);
         double2* scr = scratch_on_current_device();
-        const long chunk = static_cast<long>(kNoallocScratchBytes / per_bytes);
+        const long chunk = l4f_chunk(per, kNoallocScratchBytes, static_cast<long>(npos));
         const long nf3 = static_cast<long>(nf) * nf * nf;
         const long N4 = N2 * N2;
         L4fArgs F{};

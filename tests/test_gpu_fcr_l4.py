@@ -417,6 +417,25 @@ def test_fft_groups_equal_tiles(Nt, keep, monkeypatch):
         assert np.array_equal(out[shape].C, out["0"].C)
 
 
+def test_l4_of_many_times_in_one_launch():
+    """d = 3 with two operators keeps its intermediates in LDS: no scratch is
+    reserved for them, so 105001 times (over 1 GiB at the intermediates' size) run
+    in one launch.  Values as in a call of few of the times, bit for bit."""
+    import torch
+
+    from taco_amd import tcl4
+    rng = W.SplitMix64(19)
+    w = W.Workload("g3", W.gue(3, rng), [W.random_hermitian_unit(3, rng) for _ in range(2)],
+                   taco_amd.DrudeLorentz(0.1, 3.0), 0.9, 0.001, 105000, [0], steps=1)
+    D = tcl4.DeviceSystem(w.system, w.gamma)
+    with tcl4.Profile(0) as prof:
+        L4 = tcl4.build_l4_dev(D, w.dt, list(range(105001)))
+        kern = prof.read()
+    assert kern["k_l4"]["launches"] == 1
+    few = [0, 1, 99999, 100000, 105000]
+    assert torch.equal(L4[few], tcl4.build_l4_dev(D, w.dt, few))
+
+
 @pytest.mark.parametrize("case", ["gue_pair", "d8"])
 def test_l4_factorised_matches_oracle(orc, case, monkeypatch):
     """The factorised L4 (O(N^5 + N^3 nf) per time; the kernel for N > 8)

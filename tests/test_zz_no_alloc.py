@@ -58,7 +58,7 @@ def noalloc_l4(S, sl, npos, ops, p2f):
 
 
 def test_noalloc_equals_context_entry_point_twice():
-    """d = 16 (one time's intermediates ~1 MB, so 200 times run in four
+    """d = 16 (one time's intermediates 0.67 MB, so 200 times run in three
     launches of the 64 MiB scratch), then d = 4 with fewer times: the second
     call reuses the scratch the first left behind."""
     cases = [(W.tfim_workload(0.9, Nt=64, tmax=10), 200, 11), (W.gue_pair(N_bath=100, tmax=10), 37, 12)]
