@@ -3385,8 +3385,7 @@ static RkRev rk_rev_at(const taco_tape& tp, double2* base) {
 
 // Launch shape of the reverse RK4 kernels of a tape (the same for every
 // tape of a D, steps and K): recompute (Rf) and walk (R) arguments, their
-// LDS, and whether the walk keeps the next step's L0 part in registers
-// (carry) instead of accumulating Lbar in place over a zeroed buffer.
+// LDS, the recompute's segments, and whether each runs on row groups.
 struct RkRevShape {
     Rk4AdjArgs Rf, R;
     std::size_t lds_f = 0, lds_b = 0, nseg = 0;

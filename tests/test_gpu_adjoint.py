@@ -413,6 +413,31 @@ def test_short_slice_reverse_matches_long(steps):
         assert np.abs(x - y).max() <= 1e-11 * np.abs(y).max()
 
 
+@pytest.mark.parametrize("N", [2, 4])
+def test_chunked_reverse_matches_plain(N):
+    """The chunked reverse walk (256 steps and more) at D = 4, whose workgroups hold
+    four chunks, and D = 16 against the plain one: a longer run whose later sample
+    cotangents are zero has the same cotangents (order 2: no slices)."""
+    rng = W.SplitMix64(11)
+    w = W.Workload("g", W.gue(N, rng), [W.random_hermitian_unit(N, rng)], taco_amd.DrudeLorentz(0.08, 4.0), 0.7, 0.01,
+                   1100, [0], steps=1)
+    S, G = w.system, w.gamma
+    rng = np.random.default_rng(N)
+    bar = rng.standard_normal((251, N * N)) + 1j * rng.standard_normal((251, N * N))
+    out = []
+    for n in (250, 256, 1001):
+        b = np.zeros((n + 1, N * N), complex)
+        b[:251] = bar
+        tp = AD.Tape(G, S.omegas, S.mirror, S.pair_to_freq, S.A_eig, S.eps, w.dt, n, r0_for(N), 2, 16)
+        out.append(tp.adjoint(b))
+        tp.close()
+    for a in out[1:]:
+        for key in ("gamma", "omegas", "eps", "r0"):
+            assert np.abs(a[key] - out[0][key]).max() <= 1e-11 * np.abs(out[0][key]).max(), key
+        for x, y in zip(a["ops"], out[0]["ops"]):
+            assert np.abs(x - y).max() <= 1e-11 * np.abs(y).max()
+
+
 def test_tfim_parameter_gradient_matches_fd():
     """Gradient of the d = 16 chain loss with respect to (lambda, gamma, beta,
     J, h) through the whole chain (Drude-Lorentz bath correlation, trapz
@@ -623,25 +648,14 @@ def test_tfim_losses_many_equal_set_by_set(chain):
         assert np.array_equal(g1.numpy(), grads[q].numpy()), q
 
 
-@pytest.mark.parametrize("kind", ["d16", "d10", "d4_rows", "d3_rows"])
+@pytest.mark.parametrize("kind", ["d2", "d3", "d4"])
 def test_deferred_reverse_walk_equals_in_place_walk(monkeypatch, kind):
-    """The reverse RK4 walk with the generator cotangents formed afterwards by
-    k_rk4_lbar (large D: over conjugate-transposed generators; D = 4, 9, 16:
-    the row-group walk storing kb1..kb4) gives the cotangents of the walk that
-    forms them in place, bit for bit (single and multi-set)."""
-    if kind == "d16":
-        S, G, dt = D16.system, D16.gamma, D16.dt
-        steps, K = D16_STEPS, D16_K
-    elif kind == "d4_rows":
-        name, S, G, dt, steps, K = CASES[1]
-    elif kind == "d3_rows":
-        name, S, G, dt, steps, K = CASES[2]
-    else:
-        rng = W.SplitMix64(17)
-        H = W.gue(10, rng)
-        w = W.Workload("g10", H, [W.random_hermitian_unit(10, rng)], taco_amd.DrudeLorentz(0.1, 3.0), 0.8, 0.02, 127,
-                       list(range(21)), steps=20)
-        S, G, dt, steps, K = w.system, w.gamma, w.dt, 20, 8
+    """Below 256 steps (longer runs of D = 4, 9, 16 are chunked) the row-group
+    reverse walk that stores kb1..kb4, with the generator cotangents formed
+    afterwards by k_rk4_lbar, gives the cotangents of the walk that forms them in
+    place (TACO_RK4_DEFER=0), bit for bit, single and multi-set."""
+    name, S, G, dt, steps, K = CASES[{"d2": 0, "d3": 2, "d4": 1}[kind]]
+    steps = min(steps, 255)
     N = S.N
     rng = np.random.default_rng(5)
     bar = rng.standard_normal((steps + 1, N * N)) + 1j * rng.standard_normal((steps + 1, N * N))
@@ -659,9 +673,41 @@ def test_deferred_reverse_walk_equals_in_place_walk(monkeypatch, kind):
     for key in ("gamma", "omegas", "eps", "r0"):
         assert np.array_equal(out["0"][key], out["1"][key]), key
         for q in range(2):
-            assert np.array_equal(out["0m"][q][key], out["1"][key]), key
+            assert np.array_equal(out["0m"][q][key], out["0"][key]), key
+            assert np.array_equal(out["1m"][q][key], out["1"][key]), key
     for x, y in zip(out["0"]["ops"], out["1"]["ops"]):
         assert np.array_equal(x, y)
+
+
+@pytest.mark.parametrize("kind", ["d16", "d10"])
+def test_wide_reverse_of_two_sets_equals_single(kind):
+    """D = 100 and 256: two sets in one multi-set tape (one launch a product for
+    both) have the single tape's cotangents bit for bit."""
+    if kind == "d16":
+        S, G, dt = D16.system, D16.gamma, D16.dt
+        steps, K = D16_STEPS, D16_K
+    else:
+        rng = W.SplitMix64(17)
+        H = W.gue(10, rng)
+        w = W.Workload("g10", H, [W.random_hermitian_unit(10, rng)], taco_amd.DrudeLorentz(0.1, 3.0), 0.8, 0.02, 127,
+                       list(range(21)), steps=20)
+        S, G, dt, steps, K = w.system, w.gamma, w.dt, 20, 8
+    N = S.N
+    rng = np.random.default_rng(5)
+    bars = [rng.standard_normal((steps + 1, N * N)) + 1j * rng.standard_normal((steps + 1, N * N)) for _ in range(2)]
+    st = dict(gamma=G, omegas=S.omegas, mirror=S.mirror, pair_to_freq=S.pair_to_freq, ops=S.A_eig, eps=S.eps,
+              dt=dt, steps=steps, r0=r0_for(N))
+    mt = AD.MultiTape([st, st], checkpoint_every=K)
+    got = mt.adjoint(bars)
+    mt.close()
+    tp = AD.Tape(G, S.omegas, S.mirror, S.pair_to_freq, S.A_eig, S.eps, dt, steps, r0_for(N), 4, K)
+    for q in range(2):
+        ref = tp.adjoint(bars[q])
+        for key in ("gamma", "omegas", "eps", "r0"):
+            assert np.array_equal(got[q][key], ref[key]), (q, key)
+        for x, y in zip(got[q]["ops"], ref["ops"]):
+            assert np.array_equal(x, y), q
+    tp.close()
 
 
 def _chain_grad(prob, p, target):
