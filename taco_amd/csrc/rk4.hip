@@ -716,13 +716,17 @@ __device__ __forceinline__ bool chunk_mild(const double2* __restrict__ Ls, long 
 // formed for nothing, 41 us at D = 16, 0.39 ms at D = 36 (four fifths of the chunks
 // past the lines: 8 and 27 % longer); flags from a launch of their own would save
 // that for 30 to 40 us on every run.
-__device__ __forceinline__ bool step_whole(const int* plain, long nch) {
-    long stepped = 0;
+__device__ __forceinline__ bool step_whole(long stepped, long nch) { return 4 * stepped > nch; }
+
+// How many chunks are past the lines (every wave counts them).
+__device__ __forceinline__ long stepped_chunks(const int* plain, long nch) {
+    long n = 0;
+#pragma unroll 4
     for (long j0 = 0; j0 < nch; j0 += 64) {
         const long j = j0 + (threadIdx.x & 63);
-        stepped += __popcll(__ballot(j < nch && plain[j] != 0));
+        n += __popcll(__ballot(plain[min(j, nch - 1)] != 0 && j < nch));
     }
-    return 4 * stepped > nch;
+    return n;
 }
 constexpr int kWhole = 2;  // plain[0] of a run that step 3 steps whole
 
@@ -875,16 +879,16 @@ __global__ __launch_bounds__(64 * RowGroup<DT>::W) void k_chunk_carry(const Rk4S
     __shared__ double2 sh[3 * DT];
     const Rk4Sys s = chunk_args(arr, one, blockIdx.x);
     if (s.D != DT || !s.q) return;
-    const long nch = chunk_count(s.steps);
-    if (step_whole(s.plain, nch)) {
+    const long nch = chunk_count(s.steps), stepped = stepped_chunks(s.plain, nch);
+    if (step_whole(stepped, nch)) {
         if (threadIdx.x == 0) s.plain[0] = kWhole;
         return;
     }
     const double2* x = s.r0;
     for (long i = 0; i < nch;) {
-        const long e = carry_run<false>(s.plain, i, nch), last = min(e, nch - 1);
+        const long e = stepped ? carry_run<false>(s.plain, i, nch) : nch, last = min(e, nch - 1);
         double2* out = s.xs + last * DT;
-        if (s.plain[i])  // first states as the run's samples
+        if (stepped && s.plain[i])  // first states as the run's samples
             rk4_rows<DT, false>(sh, s.Ls, i * kRkChunk, last * kRkChunk, x, out, s.dt, kRkChunk, s.xs, nullptr, nullptr,
                                 false);
         else
@@ -932,16 +936,16 @@ template <int DT>
 __global__ __launch_bounds__(64) void k_chunk_carry_rev(const Rk4AdjArgs* arr, Rk4AdjArgs one) {
     __shared__ double2 sh[5 * DT];
     const Rk4AdjArgs A = chunk_args(arr, one, blockIdx.x);
-    const long nch = chunk_count(A.steps);
+    const long nch = chunk_count(A.steps), stepped = stepped_chunks(A.plain, nch);
     const double2* x = A.gbar + A.steps * DT;
-    if (step_whole(A.plain, nch)) {
+    if (step_whole(stepped, nch)) {
         if (threadIdx.x == 0) A.plain[0] = kWhole;
         return;
     }
     for (long i = 0; i < nch;) {
-        const long e = carry_run<true>(A.plain, i, nch), top = nch - 1 - i;  // chunks top .. nch - e
+        const long e = stepped ? carry_run<true>(A.plain, i, nch) : nch, top = nch - 1 - i;  // chunks top .. nch - e
         double2* out = e < nch ? A.lam + (nch - 1 - e) * DT : A.r0bar;
-        if (A.plain[top]) {
+        if (stepped && A.plain[top]) {
             if (threadIdx.x < DT) A.lam[top * DT + threadIdx.x] = x[threadIdx.x];
             rk4_rows_adjoint<DT, WALK_LAM>(sh, A, (nch - e) * kRkChunk, min((top + 1) * kRkChunk, A.steps), x, out);
         } else {
