@@ -654,6 +654,11 @@ __device__ __forceinline__ void chunk_product(double2 (&acc)[Chunk<DT>::EPT], co
 constexpr double kMildNorm = 2.0;
 constexpr double kMildDamp = 0.5;
 
+// Of kProbes generators spread over the run, the same for every chunk, two past the
+// lines by themselves make it one to step whole (below): the chunk then forms no
+// product.
+constexpr int kProbes = 4;
+
 template <int DT>
 __device__ __forceinline__ bool chunk_mild(const double2* __restrict__ Ls, long n0, long steps, double dt, int lane) {
     using C = Chunk<DT>;
@@ -670,52 +675,68 @@ __device__ __forceinline__ bool chunk_mild(const double2* __restrict__ Ls, long 
         ml[i] = mu[i] = mh[i] = 0.0;
     }
     auto raise = [](double& m, double a) { m = a > m || a != a ? a : m; };  // a NaN stays
+    constexpr int NV = 2 * (kProbes + 1);
+    double sum[NV];  // squared norms: generator and Hermitian part (times 2) of the probes, then of the chunk
+#pragma unroll
+    for (int q = 0; q < NV; ++q) sum[q] = 0.0;
+    auto add = [&](int q, int i, double l, double u, double h) {
+        if (lane + i * C::LPC >= NP) return;
+        const bool diagonal = lo[i] == up[i];
+        sum[2 * q] += diagonal ? l : l + u;
+        sum[2 * q + 1] += diagonal ? h : 2.0 * h;
+    };
+    auto sq = [](double2 z) { return z.x * z.x + z.y * z.y; };
+#pragma unroll
+    for (int q = 0; q < kProbes; ++q) {
+        const double2* L = Ls + (2 * q + 1) * steps / (2 * kProbes) * C::D2;
+#pragma unroll
+        for (int i = 0; i < PPT; ++i) add(q, i, sq(L[lo[i]]), sq(L[up[i]]), sq(cadd(L[lo[i]], cconj(L[up[i]]))));
+    }
 #pragma unroll(PPT == 1 ? kRkChunk + 1 : 6)
     for (int m = 0; m <= kRkChunk; ++m) {
         const double2* L = Ls + min(n0 + m, steps) * C::D2;
 #pragma unroll
         for (int i = 0; i < PPT; ++i) {
-            const double2 v = L[lo[i]], w = L[up[i]], h = cadd(v, cconj(w));
-            raise(ml[i], v.x * v.x + v.y * v.y);
-            raise(mu[i], w.x * w.x + w.y * w.y);
-            raise(mh[i], h.x * h.x + h.y * h.y);
+            const double2 v = L[lo[i]], w = L[up[i]];
+            raise(ml[i], sq(v));
+            raise(mu[i], sq(w));
+            raise(mh[i], sq(cadd(v, cconj(w))));
         }
     }
-    double f = 0.0, h = 0.0;
 #pragma unroll
-    for (int i = 0; i < PPT; ++i)
-        if (lane + i * C::LPC < NP) {
-            const bool diagonal = lo[i] == up[i];
-            f += diagonal ? ml[i] : ml[i] + mu[i];
-            h += diagonal ? mh[i] : 2.0 * mh[i];
-        }
+    for (int i = 0; i < PPT; ++i) add(kProbes, i, ml[i], mu[i], mh[i]);
     constexpr int LW = C::LPC < 64 ? C::LPC : 64;
 #pragma unroll
-    for (int m = 1; m < LW; m *= 2) {
-        f += __shfl_xor(f, m, 64);
-        h += __shfl_xor(h, m, 64);
-    }
-    if constexpr (C::LPC > 64) {
-        __shared__ double2 part[C::LPC / 64];
-        if (threadIdx.x % 64 == 0) part[threadIdx.x / 64] = make_double2(f, h);
-        __syncthreads();
-        f = h = 0.0;
+    for (int m = 1; m < LW; m *= 2)
 #pragma unroll
-        for (int w = 0; w < C::LPC / 64; ++w) {
-            f += part[w].x;
-            h += part[w].y;
+        for (int q = 0; q < NV; ++q) sum[q] += __shfl_xor(sum[q], m, 64);
+    if constexpr (C::LPC > 64) {
+        __shared__ double part[C::LPC / 64][NV];
+        if (threadIdx.x % 64 == 0)
+#pragma unroll
+            for (int q = 0; q < NV; ++q) part[threadIdx.x / 64][q] = sum[q];
+        __syncthreads();
+#pragma unroll
+        for (int q = 0; q < NV; ++q) {
+            sum[q] = 0.0;
+#pragma unroll
+            for (int w = 0; w < C::LPC / 64; ++w) sum[q] += part[w][q];
         }
     }
     const double s = dt * kRkChunk;
-    return s * s * f <= kMildNorm * kMildNorm && s * s * (0.25 * h) <= kMildDamp * kMildDamp;
+    auto within = [&](int q) {
+        return s * s * sum[2 * q] <= kMildNorm * kMildNorm && s * s * (0.25 * sum[2 * q + 1]) <= kMildDamp * kMildDamp;
+    };
+    int past = 0;
+#pragma unroll
+    for (int q = 0; q < kProbes; ++q) past += within(q) ? 0 : 1;
+    return past < 2 && within(kProbes);
 }
 
 // A run with more than a quarter of its chunks past the lines is stepped whole by
-// step 3's first workgroup: the plain run and two launches that only end (600
-// steps: 2 % longer at D = 4..36).  The products of its other chunks are then
-// formed for nothing, 41 us at D = 16, 0.39 ms at D = 36 (four fifths of the chunks
-// past the lines: 8 and 27 % longer); flags from a launch of their own would save
-// that for 30 to 40 us on every run.
+// step 3's first workgroup: the plain run and launches that only end.  Products that
+// its other chunks still form (where fewer than two probes found them) take 41 us at
+// D = 16, 0.39 ms at D = 36.
 __device__ __forceinline__ bool step_whole(long stepped, long nch) { return 4 * stepped > nch; }
 
 // How many chunks are past the lines (every wave counts them).
