@@ -645,17 +645,6 @@ def main():
     ms_per_step = 1000.0 * elapsed / a.steps
     value = ntau * a.steps / elapsed
     kernels, roofline = kernel_table(kern, a.steps)
-    # HBM traffic of the dominant kernel measured by rocprofv3 FETCH_SIZE /
-    # WRITE_SIZE passes of this workload (committed summary), when present
-    tf = os.path.join(ROOT, "profiles", "fcr_l4_gue_pair_d4_traffic.json")
-    if a.workload == "gue_pair" and not a.reduced and os.path.exists(tf):
-        t = json.load(open(tf))
-        # only when it was measured on launches of the same size as these
-        same = abs(t.get("algo_bytes_per_launch", 0.0) - roofline["algo_bytes_per_launch"]) <= (
-            0.01 * roofline["algo_bytes_per_launch"])
-        if t.get("kernel") == roofline["kernel"] and same:
-            roofline["traffic"] = t["traffic_bytes_per_launch"]
-            roofline["traffic_source"] = t["source"]
     from taco_amd import _lib
     choice = np.zeros(3, np.int32)
     nfft = 1 << int(np.ceil(np.log2(2 * G.shape[0] - 1)))
@@ -663,6 +652,17 @@ def main():
     shapes = {-1: None, 0: "tiles of 8192", 3: "tiles of 2048", 10: "groups of 1024", 11: "groups of 2048",
               20: "register columns"}
     fft_tiles = {ph: shapes[int(c)] for ph, c in zip("ABC", choice)}
+    # HBM traffic of the dominant kernel measured by rocprofv3 FETCH_SIZE /
+    # WRITE_SIZE passes of this workload (committed summary), when present
+    tf = os.path.join(ROOT, "profiles", "fcr_l4_gue_pair_d4_traffic.json")
+    if a.workload == "gue_pair" and not a.reduced and os.path.exists(tf):
+        t = json.load(open(tf))
+        # only when it was measured on launches of the same size and shape as these
+        same = abs(t.get("algo_bytes_per_launch", 0.0) - roofline["algo_bytes_per_launch"]) <= (
+            0.01 * roofline["algo_bytes_per_launch"])
+        if t.get("kernel") == roofline["kernel"] and same and t.get("fft_tiles") == fft_tiles:
+            roofline["traffic"] = t["traffic_bytes_per_launch"]
+            roofline["traffic_source"] = t["source"]
     L4 = out.cpu().numpy().reshape(ntau, S.N ** 2, S.N ** 2).transpose(0, 2, 1)
     cpu, parity, ref_libm = None, None, None
     if not a.no_cpu:

@@ -11,10 +11,12 @@
 // reference's u +/- w*x with the stage's table twiddle, as in the tile
 // kernels, so the values are bit-identical at every b.
 //
-// What bounds them (MI355X): phase B issues 53-59 % of the FP64 slots it has
-// (two waves per SIMD; the forward values and a pass's twiddles take the
-// registers of a third) at 1.8-1.9 GHz, next to 5 TB/s of traffic; phase C
-// reads at 4.3-4.8 TB/s, the rate of a plain copy.
+// What bounds them (MI355X): phase B moves 5.5-6.2 TB/s past L2 at d = 4, Nfft 2^19
+// (1.01 times the algorithmic bytes; a plain copy reaches 4.9), the vector units
+// 49-52 % busy; at d = 8, Nfft 2^15, whose spectra stay in L2, 3.2 TB/s and 60 % busy
+// (53 % with groups of 2^10): two waves per SIMD, since the forward values and a
+// pass's twiddles take the registers of a third, at 1.8-1.9 GHz.  Phase C reads at
+// 4.0-4.4 TB/s at d = 4, the rate of a plain copy, and 5.2 at d = 8.
 #include "group_fft.hpp"
 
 #include "cr_sincos.hpp"

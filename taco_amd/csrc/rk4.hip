@@ -570,9 +570,9 @@ __global__ __launch_bounds__(kRkBlock) void k_rk4_adjoint_multi(const Rk4AdjArgs
 // The reverse walk, affine in lam, splits alike: each chunk's walk from lam = 0
 // gives its constant part, the carry is lam <- lam + Q_c^H lam + b_c, and every
 // chunk's walk then runs from its true lam.
-// Measured, forward: D = 16, 4000 steps 2.7 -> 0.12 ms (products 43 us, 250
-// carries 63 us, states 17 us); D = 4, 2000 steps 1.02 -> 0.05 ms; D = 36,
-// 800 steps 0.42 ms.  All three are latency: chunks of 16 keep the products
+// Measured, forward: D = 16, 4000 steps 2.7 -> 0.12 ms (products 45 us, 250
+// carries 59 us, states 15 us); D = 4, 2000 steps 1.02 -> 0.05 ms; D = 36,
+// 800 steps 0.45 ms.  All three are latency: chunks of 16 keep the products
 // at one workgroup per CU for 4000 steps and the carry at 0.25 us a chunk.
 // ---------------------------------------------------------------------------
 template <int DT>
@@ -644,13 +644,14 @@ __device__ __forceinline__ void chunk_product(double2 (&acc)[Chunk<DT>::EPT], co
 // or a decoupled part of it can shrink.  x + Q x then cancels at most to
 // exp(-kMildDamp) of x, and RK4's own damping of a rotation is below 1e-4 a chunk.
 // A chunk past either line is stepped: there the product loses what the state
-// decays by (scalar generators of dt times rate 0.2, 0.5 and 1, 256 steps: 1e-14,
-// 1e-12 and 5e-9 relative against 6e-15, 2e-14 and 4e-14 stepped).  Below the
+// decays by (scalar generators of dt times rate 0.2, 0.5 and 1, 384 steps: 1e-14,
+// 1e-12 and 5e-9 relative against 8e-15, 2e-14 and 4e-14 stepped).  Below the
 // lines both are alike: 400 complex scalars each, 512 steps, error of the product
 // over that of the steps 0.3 at norm 0.1, 0.8 at 0.5, 1.0 at 1 and 2; over 4096
 // steps of a nearly constant generator 0.4, 1.3, 1.2 and 0.9.  TCL generators of
-// baths up to coupling 0.2 and cutoff 12 at d = 2..5, dt = 0.01 reach norm 1.2,
-// Hermitian part 0.35.  NaN and infinities are past the lines.
+// d = 2..5 at dt = 0.01 have norms up to 1.3 and Hermitian parts of 0.2, up to 0.55
+// at coupling 0.2, cutoff 12 and beta 0.4 together.  NaN and infinities are past
+// the lines.
 constexpr double kMildNorm = 2.0;
 constexpr double kMildDamp = 0.5;
 
@@ -734,9 +735,10 @@ __device__ __forceinline__ bool chunk_mild(const double2* __restrict__ Ls, long 
 }
 
 // A run with more than a quarter of its chunks past the lines is stepped whole by
-// step 3's first workgroup: the plain run and launches that only end.  Products that
-// its other chunks still form (where fewer than two probes found them) take 41 us at
-// D = 16, 0.39 ms at D = 36.
+// step 3's first workgroup: the plain run and launches that only end (600 steps,
+// D = 4..36: 2 to 4 % longer than the plain run).  Products that its other chunks
+// still form, where fewer than two probes are past the lines, take 41 us at D = 16,
+// 0.39 ms at D = 36.
 __device__ __forceinline__ bool step_whole(long stepped, long nch) { return 4 * stepped > nch; }
 
 // How many chunks are past the lines (every wave counts them).
