@@ -10,7 +10,7 @@ in HBM.  The value is L4 time-points per second.
 
 The CPU baseline leg times the oracle (the C++ restatement of the reference
 serial/OpenMP path, with the platform libm phases the reference calls) on the
-host cores, and uses the oracle as the checker of the GPU result (per-t
+host cores, and checks the GPU result against the oracle (per-t
 relative Frobenius error of L4 against the oracle in the same libm phase
 convention; the error against the correctly rounded-phase oracle is reported
 beside it).
@@ -44,7 +44,7 @@ def parse():
     p.add_argument("--systems", type=int, default=None,
                    help="batched workload: number of systems (256); tfim_adjoint: parameter sets (64)")
     p.add_argument("--no-plain", action="store_true", help="batched workload: skip the plain per-system leg")
-    p.add_argument("--no-cpu", action="store_true", help="skip the CPU baseline / checker leg")
+    p.add_argument("--no-cpu", action="store_true", help="skip the CPU baseline / oracle leg")
     p.add_argument("--cpu-threads", type=int, default=0)
     p.add_argument("--reduced", action="store_true", help="small grid (for a quick functional run)")
     p.add_argument("--plain-only", action="store_true",
@@ -667,7 +667,7 @@ def main():
     cpu, parity, ref_libm = None, None, None
     if not a.no_cpu:
         threads = a.cpu_threads or len(os.sched_getaffinity(0))
-        print(f"[bench] cpu baseline / checker leg on {threads} threads", file=sys.stderr, flush=True)
+        print(f"[bench] cpu baseline / oracle leg on {threads} threads", file=sys.stderr, flush=True)
         cpu, parity, ref_libm = cpu_baseline_leg(w, L4, threads)
         print(f"[bench] cpu leg done in {cpu['seconds']:.1f} s", file=sys.stderr, flush=True)
     rec = {

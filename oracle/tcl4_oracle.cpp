@@ -8,7 +8,7 @@
 // plain (non-FMA) complex products.  Build flags pin `-ffp-contract=off`.
 //
 // Only tests/, __graft_entry__.smoke() and bench.py's cpu_baseline leg may
-// load this library, and only as the checker.  Nothing in taco_amd/ links it.
+// load this library, and only to check against it.  Nothing in taco_amd/ links it.
 //
 // Parity status of each function is listed in the header of oracle/oracle.py.
 
