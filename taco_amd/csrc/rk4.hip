@@ -570,7 +570,7 @@ __global__ __launch_bounds__(kRkBlock) void k_rk4_adjoint_multi(const Rk4AdjArgs
 // The reverse walk, affine in lam, splits alike: each chunk's walk from lam = 0
 // gives its constant part, the carry is lam <- lam + Q_c^H lam + b_c, and every
 // chunk's walk then runs from its true lam.
-// Measured, forward: D = 16, 4000 steps 2.7 -> 0.12 ms (products 45 us, 250
+// Measured, forward: D = 16, 4000 steps 2.7 -> 0.12 ms (products 43 us, 250
 // carries 59 us, states 15 us); D = 4, 2000 steps 1.02 -> 0.05 ms; D = 36,
 // 800 steps 0.45 ms.  All three are latency: chunks of 16 keep the products
 // at one workgroup per CU for 4000 steps and the carry at 0.25 us a chunk.
@@ -638,8 +638,8 @@ __device__ __forceinline__ void chunk_product(double2 (&acc)[Chunk<DT>::EPT], co
     }
 }
 
-// Whether the product may carry a chunk's state: dt kRkChunk times the Frobenius
-// norms of the entries' largest values over the chunk, of the generator
+// Whether the product may carry a chunk's state (chunk_mild): dt kRkChunk times the
+// Frobenius norms of the entries' largest values over the chunk, of the generator
 // (kMildNorm) and of its Hermitian part (kMildDamp), the rate at which the state
 // or a decoupled part of it can shrink.  x + Q x then cancels at most to
 // exp(-kMildDamp) of x, and RK4's own damping of a rotation is below 1e-4 a chunk.
@@ -655,90 +655,77 @@ __device__ __forceinline__ void chunk_product(double2 (&acc)[Chunk<DT>::EPT], co
 constexpr double kMildNorm = 2.0;
 constexpr double kMildDamp = 0.5;
 
-// Of kProbes generators spread over the run, the same for every chunk, two past the
-// lines by themselves make it one to step whole (below): the chunk then forms no
-// product.
-constexpr int kProbes = 4;
-
-template <int DT>
-__device__ __forceinline__ bool chunk_mild(const double2* __restrict__ Ls, long n0, long steps, double dt, int lane) {
+// Squared norms summed over a chunk's threads (LPC of them, consecutive).
+template <int DT, int M>
+__device__ __forceinline__ void chunk_sums(double (&sum)[M]) {
     using C = Chunk<DT>;
-    constexpr int NP = DT * (DT + 1) / 2, PPT = (NP + C::LPC - 1) / C::LPC;  // pairs (r, c), r >= c
-    int lo[PPT], up[PPT];
-    double ml[PPT], mu[PPT], mh[PPT];  // largest |L(r, c)|^2, |L(c, r)|^2, |L(r, c) + conj(L(c, r))|^2
-#pragma unroll
-    for (int i = 0; i < PPT; ++i) {
-        int c = 0, r = min(lane + i * C::LPC, NP - 1);
-        while (r >= DT - c) r -= DT - c++;
-        r += c;
-        lo[i] = r + c * DT;
-        up[i] = c + r * DT;
-        ml[i] = mu[i] = mh[i] = 0.0;
-    }
-    auto raise = [](double& m, double a) { m = a > m || a != a ? a : m; };  // a NaN stays
-    constexpr int NV = 2 * (kProbes + 1);
-    double sum[NV];  // squared norms: generator and Hermitian part (times 2) of the probes, then of the chunk
-#pragma unroll
-    for (int q = 0; q < NV; ++q) sum[q] = 0.0;
-    auto add = [&](int q, int i, double l, double u, double h) {
-        if (lane + i * C::LPC >= NP) return;
-        const bool diagonal = lo[i] == up[i];
-        sum[2 * q] += diagonal ? l : l + u;
-        sum[2 * q + 1] += diagonal ? h : 2.0 * h;
-    };
-    auto sq = [](double2 z) { return z.x * z.x + z.y * z.y; };
-#pragma unroll
-    for (int q = 0; q < kProbes; ++q) {
-        const double2* L = Ls + (2 * q + 1) * steps / (2 * kProbes) * C::D2;
-#pragma unroll
-        for (int i = 0; i < PPT; ++i) add(q, i, sq(L[lo[i]]), sq(L[up[i]]), sq(cadd(L[lo[i]], cconj(L[up[i]]))));
-    }
-#pragma unroll(PPT == 1 ? kRkChunk + 1 : 6)
-    for (int m = 0; m <= kRkChunk; ++m) {
-        const double2* L = Ls + min(n0 + m, steps) * C::D2;
-#pragma unroll
-        for (int i = 0; i < PPT; ++i) {
-            const double2 v = L[lo[i]], w = L[up[i]];
-            raise(ml[i], sq(v));
-            raise(mu[i], sq(w));
-            raise(mh[i], sq(cadd(v, cconj(w))));
-        }
-    }
-#pragma unroll
-    for (int i = 0; i < PPT; ++i) add(kProbes, i, ml[i], mu[i], mh[i]);
     constexpr int LW = C::LPC < 64 ? C::LPC : 64;
 #pragma unroll
     for (int m = 1; m < LW; m *= 2)
 #pragma unroll
-        for (int q = 0; q < NV; ++q) sum[q] += __shfl_xor(sum[q], m, 64);
+        for (int q = 0; q < M; ++q) sum[q] += __shfl_xor(sum[q], m, 64);
     if constexpr (C::LPC > 64) {
-        __shared__ double part[C::LPC / 64][NV];
+        __shared__ double part[C::LPC / 64][M];
         if (threadIdx.x % 64 == 0)
 #pragma unroll
-            for (int q = 0; q < NV; ++q) part[threadIdx.x / 64][q] = sum[q];
+            for (int q = 0; q < M; ++q) part[threadIdx.x / 64][q] = sum[q];
         __syncthreads();
 #pragma unroll
-        for (int q = 0; q < NV; ++q) {
+        for (int q = 0; q < M; ++q) {
             sum[q] = 0.0;
 #pragma unroll
             for (int w = 0; w < C::LPC / 64; ++w) sum[q] += part[w][q];
         }
     }
+}
+
+__device__ __forceinline__ double norm2(double2 z) { return z.x * z.x + z.y * z.y; }
+
+// gen: squared norm of a generator; herm: of L + L^H.  False for NaN.
+__device__ __forceinline__ bool chunk_mild(double gen, double herm, double dt) {
     const double s = dt * kRkChunk;
-    auto within = [&](int q) {
-        return s * s * sum[2 * q] <= kMildNorm * kMildNorm && s * s * (0.25 * sum[2 * q + 1]) <= kMildDamp * kMildDamp;
-    };
+    return s * s * gen <= kMildNorm * kMildNorm && s * s * (0.25 * herm) <= kMildDamp * kMildDamp;
+}
+
+// Of kProbes generators spread over the run, the same for every chunk, two past the
+// lines by themselves make it one to step whole (below): no product is formed.
+constexpr int kProbes = 4;
+
+template <int DT>
+__device__ __forceinline__ bool probes_mild(const double2* __restrict__ Ls, long steps, double dt, int lane) {
+    using C = Chunk<DT>;
+    constexpr int NP = DT * (DT + 1) / 2, PPT = (NP + C::LPC - 1) / C::LPC;  // pairs (r, c), r >= c
+    double sum[2 * kProbes];
+#pragma unroll
+    for (int q = 0; q < 2 * kProbes; ++q) sum[q] = 0.0;
+#pragma unroll
+    for (int i = 0; i < PPT; ++i) {
+        const int p = lane + i * C::LPC;
+        int c = 0, r = min(p, NP - 1);
+        while (r >= DT - c) r -= DT - c++;
+        r += c;
+#pragma unroll
+        for (int q = 0; q < kProbes; ++q) {
+            const double2* L = Ls + (2 * q + 1) * steps / (2 * kProbes) * C::D2;
+            const double2 v = L[r + c * DT], w = L[c + r * DT];
+            if (p >= NP) continue;
+            sum[2 * q] += r == c ? norm2(v) : norm2(v) + norm2(w);
+            sum[2 * q + 1] += (r == c ? 1.0 : 2.0) * norm2(cadd(v, cconj(w)));
+        }
+    }
+    chunk_sums<DT>(sum);
     int past = 0;
 #pragma unroll
-    for (int q = 0; q < kProbes; ++q) past += within(q) ? 0 : 1;
-    return past < 2 && within(kProbes);
+    for (int q = 0; q < kProbes; ++q) past += chunk_mild(sum[2 * q], sum[2 * q + 1], dt) ? 0 : 1;
+    return past < 2;
 }
 
 // A run with more than a quarter of its chunks past the lines is stepped whole by
 // step 3's first workgroup: the plain run and launches that only end (600 steps,
-// D = 4..36: 2 to 4 % longer than the plain run).  Products that its other chunks
-// still form, where fewer than two probes are past the lines, take 41 us at D = 16,
-// 0.39 ms at D = 36.
+// D = 4..36: 1 to 2 % longer than the plain run).  Products formed for nothing,
+// where fewer than two probes are past the lines, take 39 us at D = 16, 0.39 ms at
+// D = 36.  The norms cost a carried run nothing that shows: they are taken from the
+// generators as step 1 passes them through LDS (read beforehand: 3 to 20 us).
 __device__ __forceinline__ bool step_whole(long stepped, long nch) { return 4 * stepped > nch; }
 
 // How many chunks are past the lines (every wave counts them).
@@ -764,9 +751,6 @@ __global__ __launch_bounds__(Chunk<DT>::NT) void k_chunk_products(const S* arr, 
     const long c = static_cast<long>(blockIdx.x) * C::CPB + sub;
     if (static_cast<long>(blockIdx.x) * C::CPB * kRkChunk >= s.steps) return;
     const long n0 = c * kRkChunk;
-    const bool mild = chunk_mild<DT>(s.Ls, n0, s.steps, s.dt, lane);
-    if (lane == 0 && n0 < s.steps) s.plain[c] = mild ? 0 : 1;
-    if (!__syncthreads_or(mild && n0 < s.steps)) return;
     const double h2 = 0.5 * s.dt, s6 = s.dt / 6.0;
     double2 *A = sA[sub], *B = sB[sub], *Q = sQ[sub];
     double2 l0[C::EPT], l1[C::EPT], ln[C::EPT], q[C::EPT], acc[C::EPT];
@@ -782,8 +766,27 @@ __global__ __launch_bounds__(Chunk<DT>::NT) void k_chunk_products(const S* arr, 
     };
     load(l0, n0);
     load(l1, n0 + 1);
+    if (!probes_mild<DT>(s.Ls, s.steps, s.dt, lane)) {
+        if (lane == 0 && n0 < s.steps) s.plain[c] = 1;
+        return;
+    }
+    // the largest |L(r, c)|^2 and |L(r, c) + conj(L(c, r))|^2 of the thread's entries
+    // over the chunk, from the generators as they pass through LDS
+    double mx[C::EPT], hx[C::EPT];
+    auto raise = [](double& m, double a) { m = a > m || a != a ? a : m; };  // a NaN stays
+    auto norms = [&](const double2* M, const double2 (&v)[C::EPT]) {
 #pragma unroll
-    for (int i = 0; i < C::EPT; ++i) q[i] = make_double2(0.0, 0.0);
+        for (int i = 0; i < C::EPT; ++i) {
+            const int e = min(lane + i * C::LPC, C::D2 - 1);
+            raise(mx[i], norm2(v[i]));
+            raise(hx[i], norm2(cadd(v[i], cconj(M[e / DT + e % DT * DT]))));
+        }
+    };
+#pragma unroll
+    for (int i = 0; i < C::EPT; ++i) {
+        q[i] = make_double2(0.0, 0.0);
+        mx[i] = hx[i] = 0.0;
+    }
     for (int m = 0; m < kRkChunk; ++m) {
         load(ln, n0 + m + 2);
         double2 lh[C::EPT], k2[C::EPT], k3[C::EPT];
@@ -793,6 +796,7 @@ __global__ __launch_bounds__(Chunk<DT>::NT) void k_chunk_products(const S* arr, 
         put(B, l0);
         put(Q, q);
         __syncthreads();
+        if (m == 0) norms(B, l0);
         chunk_product<DT>(acc, A, B, lane);  // K2 = Lh (I + h/2 K1), K1 = L0
 #pragma unroll
         for (int i = 0; i < C::EPT; ++i) k2[i] = cadd(lh[i], cscale(acc[i], h2));
@@ -806,6 +810,7 @@ __global__ __launch_bounds__(Chunk<DT>::NT) void k_chunk_products(const S* arr, 
         put(A, l1);
         put(B, k3);
         __syncthreads();
+        norms(A, l1);
         chunk_product<DT>(acc, A, B, lane);  // K4 = L1 (I + h K3)
         double2 e[C::EPT];
 #pragma unroll
@@ -826,12 +831,20 @@ __global__ __launch_bounds__(Chunk<DT>::NT) void k_chunk_products(const S* arr, 
         }
         __syncthreads();
     }
-    if (n0 < s.steps) {
-        double2* out = s.q + c * C::D2;
+    double sum[2] = {0.0, 0.0};
 #pragma unroll
-        for (int i = 0; i < C::EPT; ++i)
-            if (lane + i * C::LPC < C::D2) out[lane + i * C::LPC] = q[i];
-    }
+    for (int i = 0; i < C::EPT; ++i)
+        if (lane + i * C::LPC < C::D2) {
+            sum[0] += mx[i];
+            sum[1] += hx[i];
+        }
+    chunk_sums<DT>(sum);
+    if (n0 >= s.steps) return;
+    if (lane == 0) s.plain[c] = chunk_mild(sum[0], sum[1], s.dt) ? 0 : 1;
+    double2* out = s.q + c * C::D2;
+#pragma unroll
+    for (int i = 0; i < C::EPT; ++i)
+        if (lane + i * C::LPC < C::D2) out[lane + i * C::LPC] = q[i];
 }
 
 // Step 2 on the row groups of rk4_rows: x over the i0-th to the i1-th chunk

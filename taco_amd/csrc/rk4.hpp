@@ -83,11 +83,11 @@ constexpr int kRkChunk = 16;
 // Whether a run of `steps` steps at D is chunked (rk4.hip).  The chunked run
 // costs five or six launches and 2 kRkChunk steps of latency whatever its
 // length; below 256 steps the plain run (0.5-0.7 us a step at D <= 16) is as
-// fast.  At D = 36 the products alone take 0.39 ms, and 384 steps it is (a call
-// of 256, 320, 384 and 448 steps: 0.74, 0.82, 0.90 and 0.97 ms against 0.70, 0.85,
-// 1.01 and 1.16 plain).  The reverse has row groups for D <= 16 only.
+// fast.  At D = 36 the products alone take 0.39 ms, and 320 steps it is (a call
+// of 256, 288, 320, 384 and 448 steps: 0.74, 0.78, 0.82, 0.89 and 0.96 ms against
+// 0.70, 0.78, 0.86, 1.01 and 1.16 plain).  The reverse has row groups for D <= 16 only.
 inline bool rk4_chunked(int D, long steps) {
-    return D == 36 ? steps >= 384 : steps >= 256 && (D == 4 || D == 9 || D == 16 || D == 25);
+    return D == 36 ? steps >= 320 : steps >= 256 && (D == 4 || D == 9 || D == 16 || D == 25);
 }
 inline bool rk4_chunked_walk(int D, long steps) { return D <= 16 && rk4_chunked(D, steps); }
 // A chunked run's products, first states (or lam) and flags, in that order, and

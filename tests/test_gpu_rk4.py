@@ -32,7 +32,7 @@ def test_rk4_matches_oracle(orc, D, steps):
 @pytest.mark.parametrize("D", [4, 9, 16, 25, 36])
 @pytest.mark.parametrize("steps,every", [(255, 1), (256, 1), (257, 16), (272, 7), (273, 300), (1003, 10)])
 def test_chunked_rk4_matches_oracle(orc, D, steps, every):
-    """Runs of 256 steps and more (D = 36: 384) are split into chunks of 16 steps: states at
+    """Runs of 256 steps and more (D = 36: 320) are split into chunks of 16 steps: states at
     every sample and at the end against the oracle's sequential run, at the
     bound of the runs above."""
     rng = np.random.default_rng(100 + D)
